@@ -11,6 +11,9 @@ LIB_PATH = os.path.join(_PKG, "libdisc_q8_ral.so")
 # selection and the MFMA layout probe, which the product library does not carry
 HOOKS_LIB_PATH = os.path.join(_PKG, "libdisc_q8_testhooks.so")
 
+# the native callers of kernels.py (csrc_torch/torch_calls.cc), a CPython module
+TORCH_CALLS_PATH = os.path.join(_PKG, "_torch_calls.so")
+
 _lib = None
 _hooks = None
 
@@ -125,6 +128,17 @@ def lib():
                 "(there is no CPU fallback)" % LIB_PATH)
         _lib = _bind(C.CDLL(LIB_PATH, mode=C.RTLD_GLOBAL), skip=_HOOKS)
     return _lib
+
+
+def torch_calls():
+    """The module of native callers (kernels.py); it links the product library."""
+    lib()
+    if not os.path.exists(TORCH_CALLS_PATH):
+        raise RuntimeError(
+            "%s is missing: build it with `python -m bladedisc_amd.build` "
+            "(there is no fallback)" % TORCH_CALLS_PATH)
+    from . import _torch_calls
+    return _torch_calls
 
 
 def check(status, what, L=None):

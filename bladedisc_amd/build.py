@@ -1,4 +1,5 @@
-"""Builds libdisc_q8_ral.so: the gfx950 kernels, their C ABI and the RAL runtime.
+"""Builds libdisc_q8_ral.so: the gfx950 kernels, their C ABI and the RAL runtime; and
+_torch_calls.so, the native callers behind kernels.py.
 
 Everything is compiled in-tree with hipcc for gfx950 only (hipcc cross-compiles
 without a GPU).  Usage: ``python -m bladedisc_amd.build [--force]``.
@@ -19,6 +20,10 @@ LIB = os.path.join(PKG, "libdisc_q8_ral.so")
 HOOKS_LIB = os.path.join(PKG, "libdisc_q8_testhooks.so")
 HOOKS_SRC = os.path.join(CSRC, "kernels", "qgemm.hip")     # compiled a second time with the hooks
 EXPORTS = os.path.join(CSRC, "exports.map")
+
+# a CPython module on torch's C++ headers (host code only)
+TORCH_CALLS_SRC = os.path.join(PKG, "csrc_torch", "torch_calls.cc")
+TORCH_CALLS = os.path.join(PKG, "_torch_calls.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
@@ -100,6 +105,33 @@ def _record_resources(obj, lines):
         json.dump(kernels, f, indent=0, sort_keys=True)
 
 
+def build_torch_calls(force=False):
+    """csrc_torch/torch_calls.cc -> _torch_calls.so, linked against the product library next to
+    it and the torch libraries of the running interpreter (loaded by `import torch` before)."""
+    import sysconfig
+
+    import torch
+    inputs = [TORCH_CALLS_SRC, os.path.join(ROOT, "include", "disc_q8.h")]
+    if (not force and os.path.exists(TORCH_CALLS)
+            and os.path.getmtime(TORCH_CALLS) > max(map(os.path.getmtime, inputs))):
+        return TORCH_CALLS
+    t = os.path.dirname(torch.__file__)
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
+           "-I" + os.path.join(ROOT, "include"), "-isystem", sysconfig.get_paths()["include"],
+           "-isystem", os.path.join(t, "include"),
+           "-isystem", os.path.join(t, "include", "torch", "csrc", "api", "include"),
+           "-isystem", "/opt/rocm/include", TORCH_CALLS_SRC, "-o", TORCH_CALLS,
+           "-L" + PKG, "-l:" + os.path.basename(LIB), "-L" + os.path.join(t, "lib"),
+           "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python",
+           "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed for %s:\n%s" % (TORCH_CALLS_SRC, r.stdout + r.stderr))
+    return TORCH_CALLS
+
+
 def build_test_code_objects():
     """Device code objects the GPU tests hand to ral_kernel_launch (tests/programs/*.hip ->
     *.hsaco next to the source), as a compiled program would carry them."""
@@ -147,6 +179,7 @@ def build(force=False, verbose=False, jobs=8):
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError("link of the test-hooks library failed:\n" + r.stdout + r.stderr)
+    build_torch_calls(force)
     return LIB
 
 

@@ -1,0 +1,480 @@
+// The host side of bladedisc_amd/kernels.py: takes torch tensors, fills in sizes, strides, the
+// result and the scratch, and calls the C ABI of include/disc_q8.h on the current stream.
+//
+// What bounds it: nothing but instructions on the calling thread.  A quantized linear of a small
+// batch runs 3-5 us on the GPU; driven through ctypes (one Python object per argument, a stream
+// object, three reshapes of one-element scales, two library calls for the scratch) the call
+// itself took 12-14 us and the GPU waited for it.  Here a call costs the launch plus about a
+// microsecond.  Results and scratch come from torch's caching allocator on the current stream,
+// as torch.empty does, so nothing outlives the call and streams and threads behave as before;
+// the interpreter lock is released around the launch.
+#define PY_SSIZE_T_CLEAN
+#include <torch/csrc/python_headers.h>
+
+#include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <string>
+
+#include "disc_q8.h"
+
+namespace {
+
+using at::ScalarType;
+using at::Tensor;
+
+struct PyFailure {};   // a Python exception has been set
+
+[[noreturn]] void raise(PyObject* type, const char* msg) {
+  PyErr_SetString(type, msg);
+  throw PyFailure{};
+}
+
+void check(int status, const char* what) {
+  if (status == 0) return;
+  PyErr_Format(PyExc_RuntimeError, "%s failed: %s", what, dq8_last_error());
+  throw PyFailure{};
+}
+
+void* stream() { return (void*)c10::hip::getCurrentHIPStream().stream(); }
+
+// The launch itself, without the interpreter lock.
+template <typename F>
+void launch(const char* what, F&& f) {
+  int status;
+  Py_BEGIN_ALLOW_THREADS
+  status = f();
+  Py_END_ALLOW_THREADS
+  check(status, what);
+}
+
+Tensor empty(at::IntArrayRef sizes, ScalarType t, const at::Device& dev) {
+  return Tensor(at::detail::empty_cuda(sizes, t, dev, std::nullopt));
+}
+
+const Tensor& tensor(PyObject* o) {
+  if (!THPVariable_Check(o)) raise(PyExc_TypeError, "expected a tensor");
+  return THPVariable_Unpack(o);
+}
+
+const Tensor& device_tensor(PyObject* o) {
+  const Tensor& t = tensor(o);
+  if (!t.is_cuda()) raise(PyExc_ValueError, "expected device tensors");
+  return t;
+}
+
+// None or a device tensor
+Tensor optional_device_tensor(PyObject* o) {
+  return o == Py_None ? Tensor() : device_tensor(o);
+}
+
+void* ptr(const Tensor& t) { return t.defined() ? const_cast<void*>(t.const_data_ptr()) : nullptr; }
+
+int64_t integer(PyObject* o) {
+  const int64_t v = PyLong_AsLongLong(o);
+  if (v == -1 && PyErr_Occurred()) throw PyFailure{};
+  return v;
+}
+
+bool truth(PyObject* o) {
+  const int v = PyObject_IsTrue(o);
+  if (v < 0) throw PyFailure{};
+  return v != 0;
+}
+
+Tensor dense(const Tensor& t) { return t.is_contiguous() ? t : t.contiguous(); }
+
+// A scale operand: a flat f32 device tensor, or a number.
+Tensor scale(PyObject* o, const at::Device& dev) {
+  if (o == Py_None) return Tensor();
+  if (THPVariable_Check(o)) {
+    const Tensor& t = THPVariable_Unpack(o);
+    if (t.scalar_type() == ScalarType::Float && t.is_contiguous()) return t;
+    return t.reshape({-1}).contiguous().to(ScalarType::Float);
+  }
+  const double v = PyFloat_AsDouble(o);
+  if (v == -1.0 && PyErr_Occurred()) throw PyFailure{};
+  return at::full({1}, v, at::TensorOptions().dtype(ScalarType::Float).device(dev));
+}
+
+int64_t count(const Tensor& t) { return t.defined() ? t.numel() : 0; }
+
+ScalarType epilogue_type(int64_t epilogue) {
+  switch (epilogue) {
+    case DQ8_EPI_ACC_S32: return ScalarType::Int;
+    case DQ8_EPI_REQUANT_CPU:
+    case DQ8_EPI_REQUANT_GPU:
+    case DQ8_EPI_REQUANT_FIXEDPOINT: return ScalarType::Char;
+    case DQ8_EPI_DEQUANT_F32:
+    case DQ8_EPI_REQUANT_CPU_DEQUANT_F32:
+    case DQ8_EPI_REQUANT_GPU_DEQUANT_F32: return ScalarType::Float;
+  }
+  raise(PyExc_KeyError, "unknown epilogue");
+}
+
+int bias_kind(const Tensor& b) {
+  if (!b.defined()) return DQ8_BIAS_NONE;
+  switch (b.scalar_type()) {
+    case ScalarType::Int: return DQ8_BIAS_S32;
+    case ScalarType::Float: return DQ8_BIAS_F32;
+    case ScalarType::Char: return DQ8_BIAS_S8;
+    default: raise(PyExc_KeyError, "bias type");
+  }
+}
+
+// [outer, channels, inner] of a shape along an axis (None: one channel)
+struct View3 {
+  int64_t outer = 1, nch = 1, inner = 1;
+  View3(const Tensor& x, PyObject* axis) {
+    if (axis == Py_None) {
+      inner = x.numel();
+      return;
+    }
+    int64_t a = integer(axis);
+    if (a < 0) a += x.dim();
+    if (a < 0 || a >= x.dim()) raise(PyExc_IndexError, "axis out of range");
+    for (int64_t i = 0; i < a; ++i) outer *= x.size(i);
+    nch = x.size(a);
+    for (int64_t i = a + 1; i < x.dim(); ++i) inner *= x.size(i);
+  }
+};
+
+// The dq8_postops_t inside a ctypes structure (None: null); the buffer is held while in use.
+struct Post {
+  Py_buffer view{};
+  const dq8_postops_t* p = nullptr;
+  explicit Post(PyObject* o) {
+    if (o == Py_None) return;
+    if (PyObject_GetBuffer(o, &view, PyBUF_SIMPLE) != 0) throw PyFailure{};
+    if (view.len != (Py_ssize_t)sizeof(dq8_postops_t)) raise(PyExc_TypeError, "expected a PostOps structure");
+    p = static_cast<const dq8_postops_t*>(view.buf);
+  }
+  Post(const Post&) = delete;
+  ~Post() {
+    if (view.obj) PyBuffer_Release(&view);
+  }
+};
+
+PyObject* wrap(PyObject* given, const Tensor& t) {
+  if (given != Py_None) {
+    Py_INCREF(given);
+    return given;
+  }
+  return THPVariable_Wrap(t);
+}
+
+void arguments(const char* name, Py_ssize_t n, Py_ssize_t want) {
+  if (n == want) return;
+  PyErr_Format(PyExc_TypeError, "%s takes %zd arguments (%zd given)", name, want, n);
+  throw PyFailure{};
+}
+
+template <typename F>
+PyObject* guarded(F&& f) {
+  HANDLE_TH_ERRORS
+  try {
+    return f();
+  } catch (const PyFailure&) {
+    return nullptr;
+  }
+  END_HANDLE_TH_ERRORS
+}
+
+int float_kind(const Tensor& x, const char* refusal) {
+  if (x.scalar_type() == ScalarType::Float) return DQ8_DTYPE_F32;
+  if (x.scalar_type() == ScalarType::Half) return DQ8_DTYPE_F16;
+  raise(PyExc_TypeError, refusal);
+}
+
+// quantize(x, scale, zero_point, axis, qmin, qmax, round_mode, kind, store_dtype, out)
+PyObject* py_quantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    arguments("quantize", n, 10);
+    const Tensor x = dense(device_tensor(a[0]));
+    const Tensor &s = device_tensor(a[1]), &z = device_tensor(a[2]);
+    const int xk = float_kind(x, "quantize takes f32 or f16 input");
+    const View3 v(x, a[3]);
+    const int64_t qmin = integer(a[4]), qmax = integer(a[5]);
+    const int round_mode = (int)integer(a[6]), kind = (int)integer(a[7]);
+    const Tensor out = a[9] != Py_None
+                           ? tensor(a[9])
+                           : empty(x.sizes(), reinterpret_cast<THPDtype*>(a[8])->scalar_type, x.device());
+    const int64_t n_q = a[3] != Py_None ? s.numel() : 1;
+    void* st = stream();
+    launch("dq8_quantize", [&] {
+      return dq8_quantize_ex(ptr(x), xk, ptr(out), kind, v.outer, v.nch, v.inner, (const float*)ptr(s),
+                             (const int32_t*)ptr(z), n_q, qmin, qmax, round_mode, st);
+    });
+    return wrap(a[9], out);
+  });
+}
+
+// dequantize(q, scale, zero_point, axis, kind, out)
+PyObject* py_dequantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    arguments("dequantize", n, 6);
+    const Tensor q = dense(device_tensor(a[0]));
+    const Tensor &s = device_tensor(a[1]), &z = device_tensor(a[2]);
+    const View3 v(q, a[3]);
+    const int kind = (int)integer(a[4]);
+    const Tensor out = a[5] != Py_None ? tensor(a[5]) : empty(q.sizes(), ScalarType::Float, q.device());
+    const int64_t n_q = a[3] != Py_None ? s.numel() : 1;
+    void* st = stream();
+    launch("dq8_dequantize", [&] {
+      return dq8_dequantize_ex(ptr(q), kind, (float*)ptr(out), v.outer, v.nch, v.inner,
+                               (const float*)ptr(s), (const int32_t*)ptr(z), n_q, st);
+    });
+    return wrap(a[5], out);
+  });
+}
+
+// fake_quant(x, scale, zero_point, axis, qmin, qmax, round_mode, out)
+PyObject* py_fake_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    arguments("fake_quant", n, 8);
+    const Tensor &x0 = device_tensor(a[0]), &s = device_tensor(a[1]), &z = device_tensor(a[2]);
+    if (x0.scalar_type() != ScalarType::Float) raise(PyExc_TypeError, "fake_quant takes float32 tensors");
+    const Tensor x = dense(x0);
+    const View3 v(x, a[3]);
+    const int qmin = (int)integer(a[4]), qmax = (int)integer(a[5]), round_mode = (int)integer(a[6]);
+    const Tensor out = a[7] != Py_None ? tensor(a[7]) : empty(x.sizes(), ScalarType::Float, x.device());
+    const int64_t n_q = a[3] != Py_None ? s.numel() : 1;
+    void* st = stream();
+    launch("dq8_fake_quant", [&] {
+      return dq8_fake_quant((const float*)ptr(x), (float*)ptr(out), v.outer, v.nch, v.inner,
+                            (const float*)ptr(s), (const int32_t*)ptr(z), n_q, qmin, qmax, round_mode, st);
+    });
+    return wrap(a[7], out);
+  });
+}
+
+// minmax(x, min_io, max_io, axis, workspace)
+PyObject* py_minmax(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    arguments("minmax", n, 5);
+    const Tensor &x0 = device_tensor(a[0]), &lo = device_tensor(a[1]), &hi = device_tensor(a[2]);
+    if (x0.scalar_type() != ScalarType::Float || lo.scalar_type() != ScalarType::Float ||
+        hi.scalar_type() != ScalarType::Float)
+      raise(PyExc_TypeError, "minmax takes float32 tensors");
+    const Tensor x = dense(x0);
+    const View3 v(x, a[3]);
+    if (lo.numel() != v.nch || hi.numel() != v.nch) {
+      PyErr_Format(PyExc_ValueError, "min / max state must have one entry per channel (%lld)",
+                   (long long)v.nch);
+      throw PyFailure{};
+    }
+    const size_t need = dq8_minmax_workspace_bytes(v.outer, v.nch, v.inner);
+    Tensor ws;
+    if (a[4] != Py_None) ws = tensor(a[4]);
+    if (!ws.defined() || (size_t)ws.nbytes() < need)
+      ws = empty({(int64_t)(need > 0 ? need : 1)}, ScalarType::Byte, x.device());
+    void* st = stream();
+    launch("dq8_minmax", [&] {
+      return dq8_minmax((const float*)ptr(x), v.outer, v.nch, v.inner, (float*)ptr(lo), (float*)ptr(hi),
+                        ptr(ws), ws.nbytes(), st);
+    });
+    Py_RETURN_NONE;
+  });
+}
+
+// lut8(q, table, out)
+PyObject* py_lut8(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    arguments("lut8", n, 3);
+    const Tensor &q0 = device_tensor(a[0]), &table = device_tensor(a[1]);
+    if (q0.element_size() != 1 || table.element_size() != 1 || table.numel() != 256)
+      raise(PyExc_TypeError, "lut8 takes 8-bit tensors and a 256-entry table");
+    const Tensor q = dense(q0);
+    const Tensor out = a[2] != Py_None ? tensor(a[2]) : empty(q.sizes(), table.scalar_type(), q.device());
+    void* st = stream();
+    launch("dq8_lut8", [&] { return dq8_lut8(ptr(q), ptr(out), q.numel(), ptr(table), st); });
+    return wrap(a[2], out);
+  });
+}
+
+// weight_only_qgemm(x, w, scale, zero_points, bias, tp_b, out, workspace)
+PyObject* py_weight_only(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    arguments("weight_only_qgemm", n, 8);
+    Tensor x = device_tensor(a[0]);
+    Tensor w = device_tensor(a[1]);
+    Tensor s = device_tensor(a[2]);
+    Tensor zp = optional_device_tensor(a[3]), bias = optional_device_tensor(a[4]);
+    const int xk = float_kind(x, "weight_only_qgemm takes f32 or f16 activations");
+    const ScalarType xt = x.scalar_type();
+    const bool w_signed = w.scalar_type() == ScalarType::Char;
+    if ((!w_signed && w.scalar_type() != ScalarType::Byte) || w.dim() != 2)
+      raise(PyExc_TypeError, "weight_only_qgemm takes a uint8 / int8 weight matrix");
+    if (x.dim() != 2 || x.stride(1) != 1) x = x.reshape({-1, x.size(-1)}).contiguous();
+    w = dense(w);
+    const bool tp_b = truth(a[5]);
+    const int64_t N = tp_b ? w.size(0) : w.size(1), K = tp_b ? w.size(1) : w.size(0), M = x.size(0);
+    if (x.size(1) != K) raise(PyExc_ValueError, "contraction dimensions differ");
+    auto as = [](const Tensor& t, ScalarType want) {
+      return t.scalar_type() == want ? dense(t) : t.to(want).contiguous();
+    };
+    s = as(s, xt);
+    if (bias.defined()) bias = as(bias, xt);
+    if (zp.defined()) zp = as(zp, ScalarType::Int);
+    const Tensor out = a[6] != Py_None ? tensor(a[6]) : empty({M, N}, xt, x.device());
+    Tensor ws;
+    if (THPVariable_Check(a[7])) {
+      ws = THPVariable_Unpack(a[7]);
+    } else if (truth(a[7])) {
+      const size_t need = dq8_weight_only_qgemm_workspace_bytes_ex(M, N, K, tp_b, xk);
+      if (need) ws = empty({(int64_t)need}, ScalarType::Byte, x.device());
+    }
+    const size_t ws_bytes = ws.defined() ? ws.nbytes() : 0;
+    void* st = stream();
+    launch("dq8_weight_only_qgemm", [&] {
+      return dq8_weight_only_qgemm(ptr(x), xk, x.stride(0), ptr(w), w_signed, w.stride(0), tp_b, ptr(s),
+                                   (const int32_t*)ptr(zp), ptr(bias), ptr(out), out.stride(0), M, N, K,
+                                   ptr(ws), ws_bytes, st);
+    });
+    return wrap(a[6], out);
+  });
+}
+
+// An operand matrix whose rows may be strided but whose elements are dense.
+Tensor matrix(const Tensor& t) { return t.dim() != 2 || t.stride(1) != 1 ? t.contiguous() : t; }
+
+int64_t leading(const Tensor& t) { return std::max(t.stride(0), t.size(1)); }
+
+// qgemm(a, w, epilogue, sx, sw, so, bias, tp_a, tp_b, zx, zw, zo, out, post)
+PyObject* py_qgemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    arguments("qgemm", n, 14);
+    const Tensor x = matrix(device_tensor(a[0])), w = matrix(device_tensor(a[1]));
+    const Tensor bias = optional_device_tensor(a[6]);
+    if (x.dim() != 2 || w.dim() != 2) raise(PyExc_ValueError, "qgemm takes matrices");
+    const int64_t epilogue = integer(a[2]);
+    const bool tp_a = truth(a[7]), tp_b = truth(a[8]);
+    const int64_t M = x.size(tp_a ? 1 : 0), K = x.size(tp_a ? 0 : 1);
+    const int64_t N = w.size(tp_b ? 0 : 1);
+    if (K != w.size(tp_b ? 1 : 0)) raise(PyExc_ValueError, "mismatch contraction dim");
+    const int zx = (int)integer(a[9]), zw = (int)integer(a[10]), zo = (int)integer(a[11]);
+    const at::Device dev = x.device();
+    const Tensor out = a[12] != Py_None ? tensor(a[12]) : empty({M, N}, epilogue_type(epilogue), dev);
+    const Tensor sx = scale(a[3], dev), sw = scale(a[4], dev), so = scale(a[5], dev);
+    const int kind = bias_kind(bias);
+    const Post post(a[13]);
+    const size_t need = dq8_qgemm_workspace_bytes_zp(M, N, K, tp_a, tp_b, zx, zw);
+    Tensor ws;
+    if (need) ws = empty({(int64_t)need}, ScalarType::Byte, dev);
+    void* st = stream();
+    launch("dq8_qgemm", [&] {
+      return dq8_qgemm_fused((const int8_t*)ptr(x), leading(x), (const int8_t*)ptr(w), leading(w), ptr(out),
+                             M ? out.stride(0) : N, M, N, K, tp_a, tp_b, (int)epilogue, ptr(bias), kind,
+                             (const float*)ptr(sx), count(sx), (const float*)ptr(sw), count(sw),
+                             (const float*)ptr(so), count(so), zx, zw, zo, ptr(ws), need, post.p, st);
+    });
+    return wrap(a[12], out);
+  });
+}
+
+// qlinear_f32(x, w, epilogue, sx, sw, so, bias, zo, round_mode, out)
+PyObject* py_qlinear_f32(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    arguments("qlinear_f32", n, 10);
+    Tensor x = device_tensor(a[0]);
+    const Tensor w = matrix(device_tensor(a[1]));
+    const Tensor bias = optional_device_tensor(a[6]);
+    const int64_t epilogue = integer(a[2]);
+    if (x.dim() != 2 || x.stride(1) != 1) x = x.reshape({-1, x.size(-1)}).contiguous();
+    if (w.dim() != 2) raise(PyExc_ValueError, "qlinear_f32 takes a weight matrix");
+    const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+    if (w.size(1) != K) raise(PyExc_ValueError, "mismatch contraction dim");
+    const at::Device dev = x.device();
+    const Tensor out = a[9] != Py_None ? tensor(a[9]) : empty({M, N}, epilogue_type(epilogue), dev);
+    const Tensor sx = scale(a[3], dev), sw = scale(a[4], dev), so = scale(a[5], dev);
+    const int kind = bias_kind(bias);
+    const int zo = (int)integer(a[7]), round_mode = (int)integer(a[8]);
+    void* st = stream();
+    launch("dq8_qlinear_f32", [&] {
+      return dq8_qlinear_f32((const float*)ptr(x), leading(x), (const int8_t*)ptr(w), leading(w), ptr(out),
+                             M ? out.stride(0) : N, M, N, K, (int)epilogue, ptr(bias), kind,
+                             (const float*)ptr(sx), (const float*)ptr(sw), count(sw),
+                             (const float*)ptr(so), count(so), zo, round_mode, st);
+    });
+    return wrap(a[9], out);
+  });
+}
+
+template <typename T, int N>
+struct Numbers {
+  T v[N];
+  explicit Numbers(PyObject* o) {
+    PyObject* s = PySequence_Fast(o, "expected a sequence of integers");
+    if (!s) throw PyFailure{};
+    const Py_ssize_t n = PySequence_Fast_GET_SIZE(s);
+    bool bad = n > N;
+    for (int i = 0; i < N; ++i) v[i] = 0;
+    for (Py_ssize_t i = 0; i < n && !bad; ++i) {
+      const int64_t x = PyLong_AsLongLong(PySequence_Fast_GET_ITEM(s, i));
+      bad = x == -1 && PyErr_Occurred();
+      v[i] = (T)x;
+    }
+    Py_DECREF(s);
+    if (bad) {
+      if (!PyErr_Occurred()) PyErr_SetString(PyExc_IndexError, "too many values");
+      throw PyFailure{};
+    }
+  }
+};
+
+// qconv2d(x, w, padding, metadata, out_shape, epilogue, sx, sw, so, bias, zo, out, workspace, post)
+PyObject* py_qconv2d(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    arguments("qconv2d", n, 14);
+    const Tensor x = dense(device_tensor(a[0])), w = dense(device_tensor(a[1]));
+    const Tensor bias = optional_device_tensor(a[9]);
+    if (x.dim() != 4 || w.dim() != 4) raise(PyExc_ValueError, "qconv2d takes tensors of rank 4");
+    const Numbers<int32_t, 4> padding(a[2]);
+    const Numbers<int32_t, 17> md(a[3]);
+    const Numbers<int64_t, 4> os(a[4]);
+    const int64_t epilogue = integer(a[5]);
+    const at::Device dev = x.device();
+    const Tensor out = a[11] != Py_None ? tensor(a[11])
+                                        : empty(at::IntArrayRef(os.v, 4), epilogue_type(epilogue), dev);
+    const Tensor sx = scale(a[6], dev), sw = scale(a[7], dev), so = scale(a[8], dev);
+    const int kind = bias_kind(bias), zo = (int)integer(a[10]);
+    const Post post(a[13]);
+    const int64_t *is = x.sizes().data(), *ws_ = w.sizes().data();
+    const size_t need = truth(a[12]) ? dq8_qconv2d_workspace_bytes_ex(is, ws_, os.v, md.v) : 0;
+    Tensor ws;
+    if (need) ws = empty({(int64_t)need}, ScalarType::Byte, dev);
+    void* st = stream();
+    launch("dq8_qconv2d", [&] {
+      return dq8_qconv2d_fused((const int8_t*)ptr(x), is, (const int8_t*)ptr(w), ws_, padding.v, md.v,
+                               ptr(out), os.v, (int)epilogue, ptr(bias), kind, (const float*)ptr(sx),
+                               (const float*)ptr(sw), count(sw), (const float*)ptr(so), zo, ptr(ws), need,
+                               post.p, st);
+    });
+    return wrap(a[11], out);
+  });
+}
+
+PyMethodDef kMethods[] = {
+#define DQ8_METHOD(name, fn) {name, (PyCFunction)(void (*)(void))fn, METH_FASTCALL, nullptr}
+    DQ8_METHOD("quantize", py_quantize),
+    DQ8_METHOD("dequantize", py_dequantize),
+    DQ8_METHOD("fake_quant", py_fake_quant),
+    DQ8_METHOD("minmax", py_minmax),
+    DQ8_METHOD("lut8", py_lut8),
+    DQ8_METHOD("weight_only_qgemm", py_weight_only),
+    DQ8_METHOD("qgemm", py_qgemm),
+    DQ8_METHOD("qlinear_f32", py_qlinear_f32),
+    DQ8_METHOD("qconv2d", py_qconv2d),
+#undef DQ8_METHOD
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_torch_calls", nullptr, -1, kMethods,
+                       nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__torch_calls(void) { return PyModule_Create(&kModule); }

@@ -1,7 +1,9 @@
 """torch-tensor front-end of the raw kernel C ABI (include/disc_q8.h).
 
 PyTorch only supplies device memory and the current stream here; every function
-launches the hand-written HIP kernels in libdisc_q8_ral.so.
+launches the hand-written HIP kernels in libdisc_q8_ral.so.  The operators go through
+csrc_torch/torch_calls.cc, which reads the tensors and makes the call in native code; ctypes is
+left for what is called once per program (and for kernel variants that a test forces).
 """
 import ctypes as C
 
@@ -22,6 +24,14 @@ _OUT_DTYPE = {EPI_ACC_S32: torch.int32, EPI_REQUANT_CPU: torch.int8,
               EPI_REQUANT_CPU_DEQUANT_F32: torch.float32,
               EPI_REQUANT_GPU_DEQUANT_F32: torch.float32,
               EPI_REQUANT_FIXEDPOINT: torch.int8}
+
+
+def _native():
+    """The native callers; replaces itself by the loaded module's accessor on first use."""
+    global _native
+    mod = _lib.torch_calls()
+    _native = lambda: mod  # noqa: E731
+    return mod
 
 
 def _ptr(t):
@@ -70,12 +80,9 @@ QUANT_KINDS = {"int8": (0, torch.int8), "uint8": (1, torch.uint8), "int16": (2, 
                "uint16": (3, torch.int16), "int32": (4, torch.int32), "uint32": (5, torch.int32)}
 
 
-def _quant_kind(dtype):
-    if isinstance(dtype, str):
-        return QUANT_KINDS[dtype]
-    name = str(dtype).replace("torch.", "")
-    kind, _ = QUANT_KINDS[name]
-    return kind, dtype
+# (by torch dtype as well: a dict lookup per call)
+_KINDS = {**QUANT_KINDS, **{getattr(torch, name): (kind, getattr(torch, name))
+                            for name, (kind, _) in QUANT_KINDS.items() if hasattr(torch, name)}}
 
 
 def quantize(x, scale, zero_point, axis=None, qmin=-128, qmax=127,
@@ -83,74 +90,30 @@ def quantize(x, scale, zero_point, axis=None, qmin=-128, qmax=127,
     """mhlo_disc.quantize on the GPU.  scale/zero_point: device tensors (f32 / i32); x: f32 or
     f16.  dtype: a torch dtype or one of the names in QUANT_KINDS -- the unsigned 16 / 32 bit
     types are returned in the signed torch dtype of the same width (same bits)."""
-    _need_cuda(x, scale, zero_point)
-    if x.dtype not in (torch.float32, torch.float16):
-        raise TypeError("quantize takes f32 or f16 input")
-    x = x.contiguous()
-    outer, nch, inner = _view3(tuple(x.shape), axis)
     if out is not None and not isinstance(dtype, str):
         dtype = out.dtype
-    kind, store = _quant_kind(dtype)
-    if out is None:
-        out = torch.empty(x.shape, dtype=store, device=x.device)
-    n_q = scale.numel() if axis is not None else 1
-    st = _lib.lib().dq8_quantize_ex(_ptr(x), 0 if x.dtype == torch.float32 else 1, _ptr(out), kind,
-                                    outer, nch, inner, _ptr(scale), _ptr(zero_point), n_q,
-                                    int(qmin), int(qmax), round_mode, _stream())
-    _lib.check(st, "dq8_quantize")
-    return out
+    kind, store = _KINDS[dtype]
+    return _native().quantize(x, scale, zero_point, axis, qmin, qmax, round_mode, kind, store, out)
 
 
 def fake_quant(x, scale, zero_point, axis=None, qmin=-128, qmax=127,
                round_mode=ROUND_HALF_TO_EVEN, out=None):
     """dequantize(quantize(x)) in one pass: f32 -> f32, the same bits as the two calls."""
-    _need_cuda(x, scale, zero_point)
-    if x.dtype != torch.float32:
-        raise TypeError("fake_quant takes float32 tensors")
-    x = x.contiguous()
-    outer, nch, inner = _view3(tuple(x.shape), axis)
-    if out is None:
-        out = torch.empty_like(x)
-    n_q = scale.numel() if axis is not None else 1
-    st = _lib.lib().dq8_fake_quant(_ptr(x), _ptr(out), outer, nch, inner, _ptr(scale),
-                                   _ptr(zero_point), n_q, qmin, qmax, round_mode, _stream())
-    _lib.check(st, "dq8_fake_quant")
-    return out
+    return _native().fake_quant(x, scale, zero_point, axis, qmin, qmax, round_mode, out)
 
 
 def minmax(x, min_io, max_io, axis=None, workspace=None):
     """Folds the minimum and maximum of `x` (device f32), per tensor (axis None) or per
     slice along `axis`, into the running values min_io / max_io (device f32, one entry or
     one per channel).  Returns (min_io, max_io)."""
-    _need_cuda(x, min_io, max_io)
-    if x.dtype != torch.float32 or min_io.dtype != torch.float32 or max_io.dtype != torch.float32:
-        raise TypeError("minmax takes float32 tensors")
-    x = x.contiguous()
-    outer, nch, inner = _view3(tuple(x.shape), axis)
-    if min_io.numel() != nch or max_io.numel() != nch:
-        raise ValueError("min / max state must have one entry per channel (%d)" % nch)
-    L = _lib.lib()
-    need = L.dq8_minmax_workspace_bytes(outer, nch, inner)
-    if workspace is None or workspace.numel() * workspace.element_size() < need:
-        workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
-    st = L.dq8_minmax(_ptr(x), outer, nch, inner, _ptr(min_io), _ptr(max_io), _ptr(workspace),
-                      workspace.numel() * workspace.element_size(), _stream())
-    _lib.check(st, "dq8_minmax")
+    _native().minmax(x, min_io, max_io, axis, workspace)
     return min_io, max_io
 
 
 def lut8(q, table, out=None):
     """out[i] = table[bit pattern of q[i]] for an int8 / uint8 device tensor; `table` is a
     256-entry device tensor of the output's 8-bit type."""
-    _need_cuda(q, table)
-    if q.element_size() != 1 or table.element_size() != 1 or table.numel() != 256:
-        raise TypeError("lut8 takes 8-bit tensors and a 256-entry table")
-    q = q.contiguous()
-    if out is None:
-        out = torch.empty(q.shape, dtype=table.dtype, device=q.device)
-    st = _lib.lib().dq8_lut8(_ptr(q), _ptr(out), q.numel(), _ptr(table), _stream())
-    _lib.check(st, "dq8_lut8")
-    return out
+    return _native().lut8(q, table, out)
 
 
 def weight_only_qgemm(x, w, scale, zero_points=None, bias=None, tp_b=True, out=None,
@@ -160,36 +123,7 @@ def weight_only_qgemm(x, w, scale, zero_points=None, bias=None, tp_b=True, out=N
     bias have x's dtype, zero_points is int32.  workspace=False withholds the scratch that
     [K,N] weights are transposed into and that a launch split over k keeps its partial sums
     in; a uint8 tensor is used as that scratch."""
-    _need_cuda(x, w, scale, zero_points, bias)
-    if x.dtype not in (torch.float32, torch.float16):
-        raise TypeError("weight_only_qgemm takes f32 or f16 activations")
-    if w.dtype not in (torch.uint8, torch.int8) or w.dim() != 2:
-        raise TypeError("weight_only_qgemm takes a uint8 / int8 weight matrix")
-    if x.dim() != 2 or x.stride(1) != 1:
-        x = x.reshape(-1, x.shape[-1]).contiguous()
-    w = w.contiguous()
-    n, k = (w.shape if tp_b else (w.shape[1], w.shape[0]))
-    m = x.shape[0]
-    if x.shape[1] != k:
-        raise ValueError("contraction dimensions differ")
-    scale = scale.to(x.dtype).contiguous()
-    bias = bias.to(x.dtype).contiguous() if bias is not None else None
-    zero_points = zero_points.to(torch.int32).contiguous() if zero_points is not None else None
-    if out is None:
-        out = torch.empty((m, n), dtype=x.dtype, device=x.device)
-    L = _lib.lib()
-    if isinstance(workspace, torch.Tensor):
-        ws, ws_bytes = workspace, workspace.numel() * workspace.element_size()
-    else:
-        ws_bytes = L.dq8_weight_only_qgemm_workspace_bytes_ex(
-            m, n, k, int(tp_b), 0 if x.dtype == torch.float32 else 1) if workspace else 0
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
-    st = L.dq8_weight_only_qgemm(_ptr(x), 0 if x.dtype == torch.float32 else 1, x.stride(0),
-                                 _ptr(w), int(w.dtype == torch.int8), w.stride(0), int(tp_b),
-                                 _ptr(scale), _ptr(zero_points), _ptr(bias), _ptr(out),
-                                 out.stride(0), m, n, k, _ptr(ws), ws_bytes, _stream())
-    _lib.check(st, "dq8_weight_only_qgemm")
-    return out
+    return _native().weight_only_qgemm(x, w, scale, zero_points, bias, tp_b, out, workspace)
 
 
 def weight_only_undo_compiler_layout(reordered_kn):
@@ -223,17 +157,8 @@ def activation_table(fn, s_in, z_in, s_out, z_out, in_dtype=torch.int8, out_dtyp
 def dequantize(q, scale, zero_point, axis=None, out=None, dtype=None):
     """mhlo_disc.dequantize on the GPU; dtype names the quantized type where q's torch dtype
     does not (the unsigned 16 / 32 bit types, see QUANT_KINDS)."""
-    _need_cuda(q, scale, zero_point)
-    q = q.contiguous()
-    outer, nch, inner = _view3(tuple(q.shape), axis)
-    if out is None:
-        out = torch.empty(q.shape, dtype=torch.float32, device=q.device)
-    kind, _ = _quant_kind(dtype if dtype is not None else q.dtype)
-    n_q = scale.numel() if axis is not None else 1
-    st = _lib.lib().dq8_dequantize_ex(_ptr(q), kind, _ptr(out), outer, nch, inner, _ptr(scale),
-                                      _ptr(zero_point), n_q, _stream())
-    _lib.check(st, "dq8_dequantize")
-    return out
+    kind, _ = _KINDS[dtype if dtype is not None else q.dtype]
+    return _native().dequantize(q, scale, zero_point, axis, kind, out)
 
 
 def make_postops(residual=None, residual_scale=None, residual_zp=0, relu=False, out_scale=None,
@@ -272,8 +197,15 @@ def qgemm(a, w, epilogue, sx=None, sw=None, so=None, bias=None, tp_a=False, tp_b
           zx=0, zw=0, zo=0, variant=-1, out=None, post=None):
     """int8 GEMM with a fused epilogue.  a: [M,K] ([K,M] if tp_a); w: [N,K] if tp_b
     else [K,N]; scales are device f32 tensors with 1 or N entries."""
+    if post is not None:
+        if variant != -1:
+            raise ValueError("fused operators go with the library's own choice of kernel")
+        post = post[0] if isinstance(post, tuple) else post
+    if variant == -1:
+        return _native().qgemm(a, w, epilogue, sx, sw, so, bias, tp_a, tp_b, zx, zw, zo, out, post)
+    # a forced kernel variant: the tests' entry point, in the test-hooks library
     _need_cuda(a, w, bias)
-    L = _lib.lib()
+    L = _lib.hooks()
     # rows may be strided (leading dimension > row length); elements must be dense
     if a.dim() != 2 or a.stride(1) != 1:
         a = a.contiguous()
@@ -291,28 +223,14 @@ def qgemm(a, w, epilogue, sx=None, sw=None, so=None, bias=None, tp_a=False, tp_b
     sw = _scale(sw, dev) if sw is not None else None
     so = _scale(so, dev) if so is not None else None
     bias_kind = BIAS_NONE if bias is None else _BIAS_KIND[bias.dtype]
-    # with zero points and the heuristic this includes the two correction vectors of the
-    # MFMA path; a forced generic variant (0) needs none of it
-    ws_bytes = (L.dq8_qgemm_workspace_bytes_zp(m, n, k, int(tp_a), int(tp_b), zx, zw)
-                if variant == -1 else L.dq8_qgemm_workspace_bytes(m, n, k, int(tp_a), int(tp_b)))
+    ws_bytes = L.dq8_qgemm_workspace_bytes(m, n, k, int(tp_a), int(tp_b))
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-    args = (_ptr(a), max(a.stride(0), a.shape[1]), _ptr(w), max(w.stride(0), w.shape[1]),
-            _ptr(out), out.stride(0) if m else n,
-            m, n, k, int(tp_a), int(tp_b), epilogue, _ptr(bias), bias_kind,
-            _ptr(sx), sx.numel() if sx is not None else 0,
-            _ptr(sw), sw.numel() if sw is not None else 0,
-            _ptr(so), so.numel() if so is not None else 0,
-            zx, zw, zo, _ptr(ws), ws_bytes)
-    if post is not None:
-        if variant != -1:
-            raise ValueError("fused operators go with the library's own choice of kernel")
-        po, keep = post if isinstance(post, tuple) else (post, None)
-        st = L.dq8_qgemm_fused(*args, C.byref(po), _stream())
-    elif variant == -1:
-        st = L.dq8_qgemm(*args, _stream())
-    else:       # a forced kernel variant: the tests' entry point, in the test-hooks library
-        L = _lib.hooks()
-        st = L.dq8_qgemm_variant(variant, *args, _stream())
+    st = L.dq8_qgemm_variant(
+        variant, _ptr(a), max(a.stride(0), a.shape[1]), _ptr(w), max(w.stride(0), w.shape[1]),
+        _ptr(out), out.stride(0) if m else n, m, n, k, int(tp_a), int(tp_b), epilogue, _ptr(bias),
+        bias_kind, _ptr(sx), sx.numel() if sx is not None else 0,
+        _ptr(sw), sw.numel() if sw is not None else 0,
+        _ptr(so), so.numel() if so is not None else 0, zx, zw, zo, _ptr(ws), ws_bytes, _stream())
     _lib.check(st, "dq8_qgemm", L)
     return out
 
@@ -325,29 +243,7 @@ def qlinear_f32(x, w, epilogue, sx, sw=None, so=None, bias=None, zo=0,
                 round_mode=ROUND_HALF_TO_EVEN, out=None):
     """quantize(x; sx, zero point 0) -> qgemm(., w [N,K]) with the given epilogue, one launch,
     for a few rows of f32 activations x [M,K]; the same bits as quantize followed by qgemm."""
-    _need_cuda(x, w, bias)
-    L = _lib.lib()
-    if x.dim() != 2 or x.stride(1) != 1:
-        x = x.reshape(-1, x.shape[-1]).contiguous()
-    if w.dim() != 2 or w.stride(1) != 1:
-        w = w.contiguous()
-    m, k = x.shape
-    n = w.shape[0]
-    if w.shape[1] != k:
-        raise ValueError("mismatch contraction dim")
-    dev = x.device
-    if out is None:
-        out = torch.empty((m, n), dtype=_OUT_DTYPE[epilogue], device=dev)
-    sx = _scale(sx, dev)
-    sw = _scale(sw, dev) if sw is not None else None
-    so = _scale(so, dev) if so is not None else None
-    bias_kind = BIAS_NONE if bias is None else _BIAS_KIND[bias.dtype]
-    st = L.dq8_qlinear_f32(_ptr(x), max(x.stride(0), k), _ptr(w), max(w.stride(0), k), _ptr(out),
-                           out.stride(0) if m else n, m, n, k, epilogue, _ptr(bias), bias_kind,
-                           _ptr(sx), _ptr(sw), sw.numel() if sw is not None else 0,
-                           _ptr(so), so.numel() if so is not None else 0, zo, round_mode, _stream())
-    _lib.check(st, "dq8_qlinear_f32")
-    return out
+    return _native().qlinear_f32(x, w, epilogue, sx, sw, so, bias, zo, round_mode, out)
 
 
 NHWC_OHWI = (0, 3, 1, 2, 3, 0, 1, 2, 0, 3, 1, 2)
@@ -358,8 +254,16 @@ def qconv2d(x, w, padding, metadata, out_shape, epilogue, sx=None, sw=None, so=N
     """int8 convolution; layouts/strides/dilations from the 17-entry ral_qconv
     metadata, padding = (top, bottom, left, right).  workspace=False withholds the scratch
     that keeps channel counts off a multiple of 16 on the MFMA kernels."""
+    if post is not None:
+        if variant != -1:
+            raise ValueError("fused operators go with the library's own choice of kernel")
+        post = post[0] if isinstance(post, tuple) else post
+    if variant == -1:
+        return _native().qconv2d(x, w, padding, metadata, out_shape, epilogue, sx, sw, so, bias, zo,
+                                 out, workspace, post)
+    # a forced kernel variant: the tests' entry point, in the test-hooks library
     _need_cuda(x, w, bias)
-    L = _lib.lib()
+    L = _lib.hooks()
     x = x.contiguous()
     w = w.contiguous()
     dev = x.device
@@ -373,20 +277,10 @@ def qconv2d(x, w, padding, metadata, out_shape, epilogue, sx=None, sw=None, so=N
     md = (C.c_int32 * 17)(*metadata)
     ws_bytes = L.dq8_qconv2d_workspace_bytes_ex(i64x4(*x.shape), i64x4(*w.shape), i64x4(*out_shape), md) if workspace else 0
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-    args = (_ptr(x), i64x4(*x.shape), _ptr(w), i64x4(*w.shape),
-            (C.c_int32 * 4)(*padding), md, _ptr(out),
-            i64x4(*out_shape), epilogue, _ptr(bias), bias_kind, _ptr(sx), _ptr(sw),
-            sw.numel() if sw is not None else 0, _ptr(so), zo, _ptr(ws), ws_bytes)
-    if post is not None:
-        if variant != -1:
-            raise ValueError("fused operators go with the library's own choice of kernel")
-        po, keep = post if isinstance(post, tuple) else (post, None)
-        st = L.dq8_qconv2d_fused(*args, C.byref(po), _stream())
-    elif variant == -1:
-        st = L.dq8_qconv2d_ws(*args, _stream())
-    else:       # a forced kernel variant: the tests' entry point, in the test-hooks library
-        L = _lib.hooks()
-        st = L.dq8_qconv2d_variant(variant, *args, _stream())
+    st = L.dq8_qconv2d_variant(
+        variant, _ptr(x), i64x4(*x.shape), _ptr(w), i64x4(*w.shape), (C.c_int32 * 4)(*padding), md,
+        _ptr(out), i64x4(*out_shape), epilogue, _ptr(bias), bias_kind, _ptr(sx), _ptr(sw),
+        sw.numel() if sw is not None else 0, _ptr(so), zo, _ptr(ws), ws_bytes, _stream())
     _lib.check(st, "dq8_qconv2d", L)
     return out
 
