@@ -176,11 +176,56 @@ minmax_lastaxis(const float* __restrict__ x, int64_t rows, int nch, int rows_per
   }
 }
 
+// Scale and zero point of one channel from its running minimum and maximum, the observers'
+// arithmetic (R tools/torch_quant/torch_quant/observer.py:134-163): separately rounded f32
+// operations and true divisions.  `range` is (q_max - q_min) / 2 for the symmetric schemes and
+// q_max - q_min for the affine ones.
+struct QParamsOut {
+  float* scale;         // null: only the minimum and maximum are wanted
+  int32_t* zero_point;
+  int32_t* status;      // 1: min <= max in every channel, 2: not so (host-visible memory)
+  int symmetric;
+  float range;
+  int q_min, q_max;
+};
+__device__ __forceinline__ void qparams_one(const QParamsOut& q, int c, float lo, float hi) {
+  const float neg = lo < 0.0f ? lo : 0.0f, pos = hi > 0.0f ? hi : 0.0f;
+  const float eps = std::numeric_limits<float>::epsilon();
+  float s = (q.symmetric ? (-neg > pos ? -neg : pos) : pos - neg) / q.range;
+  s = s > eps ? s : eps;
+  int z = 0;
+  if (!q.symmetric) {
+    z = q.q_min - (int)rintf(neg / s);
+    z = z < q.q_min ? q.q_min : (z > q.q_max ? q.q_max : z);
+  }
+  q.scale[c] = s;
+  q.zero_point[c] = z;
+}
+__device__ __forceinline__ void signal(int32_t* status, bool ok) {
+  __hip_atomic_store(status, ok ? 1 : 2, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The same for many channels, behind pass 2: one workgroup, which also finds out whether every
+// channel's minimum is at most its maximum (not so after a NaN).
+__global__ void __launch_bounds__(1024)
+minmax_qparams(const float* __restrict__ lo, const float* __restrict__ hi, int channels,
+               const QParamsOut q) {
+  bool ok = true;
+  for (int c = threadIdx.x; c < channels; c += 1024) {
+    const float a = lo[c], b = hi[c];
+    ok = ok && a <= b;
+    qparams_one(q, c, a, b);
+  }
+  const bool all = __syncthreads_and(ok);
+  if (threadIdx.x == 0) signal(q.status, all);
+}
+
 // ---- pass 2, rows layout: one workgroup per channel c; its pairs are
-// partial[(o * channels + c) * segs + s], o < outer, s < segs
+// partial[(o * channels + c) * segs + s], o < outer, s < segs.  With a single channel the
+// workgroup goes on to the channel's scale and zero point where they are wanted.
 __global__ void __launch_bounds__(kThreads)
 minmax_fold_rows(const float2* __restrict__ partial, int64_t outer, int channels, int segs,
-                 float* __restrict__ min_io, float* __restrict__ max_io) {
+                 float* __restrict__ min_io, float* __restrict__ max_io, const QParamsOut q) {
   const int c = blockIdx.x;
   MinMax m = identity();
   for (int64_t o = 0; o < outer; ++o) {
@@ -204,6 +249,10 @@ minmax_fold_rows(const float2* __restrict__ partial, int64_t outer, int channels
     fold(m, MinMax{min_io[c], max_io[c]});
     min_io[c] = m.lo;
     max_io[c] = m.hi;
+    if (q.scale) {
+      qparams_one(q, c, m.lo, m.hi);
+      signal(q.status, m.lo <= m.hi);
+    }
   }
 }
 
@@ -311,11 +360,12 @@ extern "C" size_t dq8_minmax_workspace_bytes(int64_t outer, int64_t channels, in
 
 namespace {
 
-// Shared by the two entry points: both passes with the (min, max) pairs in `partial`.  Pass 1
+// Shared by the entry points: both passes with the (min, max) pairs in `partial`.  Pass 1
 // writes every pair pass 2 reads, so the scratch needs no particular contents beforehand.
+// `q`: of a single channel (null where scale and zero point are not wanted).
 int run_minmax(const float* x, int64_t outer, int64_t channels, int64_t inner,
                float* min_io, float* max_io, float2* partial, const Plan& p, bool vec,
-               hipStream_t st) {
+               hipStream_t st, const QParamsOut* q = nullptr) {
   if (p.last_axis) {
     const dim3 grid((unsigned)p.gx, (unsigned)p.gy), block((unsigned)p.bx, (unsigned)p.by);
     if (vec)
@@ -341,7 +391,7 @@ int run_minmax(const float* x, int64_t outer, int64_t channels, int64_t inner,
                        dim3(kThreads), 0, st, partial, outer, (int)channels, p.segs, min_io, max_io);
   else
     hipLaunchKernelGGL(minmax_fold_rows, dim3((unsigned)channels), dim3(kThreads), 0, st, partial,
-                       outer, (int)channels, p.segs, min_io, max_io);
+                       outer, (int)channels, p.segs, min_io, max_io, q ? *q : QParamsOut{});
   return check_hip(hipGetLastError(), "minmax_fold_rows launch");
 }
 
@@ -363,6 +413,35 @@ extern "C" int dq8_minmax(const float* x, int64_t outer, int64_t channels, int64
               "dq8_minmax: workspace too small (see dq8_minmax_workspace_bytes)");
   return run_minmax(x, outer, channels, inner, min_io, max_io,
                     static_cast<float2*>(workspace), p, vec, (hipStream_t)stream);
+}
+
+// A whole observation step: the running minimum and maximum, then scale and zero point from
+// them, with nothing read back in between.
+extern "C" int dq8_observe(const float* x, int64_t outer, int64_t channels, int64_t inner,
+                           float* min_io, float* max_io, int symmetric, int32_t q_min,
+                           int32_t q_max, float* scale, int32_t* zero_point, int32_t* status,
+                           void* workspace, size_t workspace_bytes, void* stream) {
+  clear_error();
+  DQ8_REQUIRE(outer > 0 && channels > 0 && inner > 0, "dq8_observe: empty tensor");
+  DQ8_REQUIRE(x && min_io && max_io && scale && zero_point && status, "dq8_observe: null pointer");
+  DQ8_REQUIRE(channels < (1LL << 31), "dq8_observe: too many channels");
+  DQ8_REQUIRE(q_min < q_max && q_min >= -32768 && q_max <= 65535,
+              "dq8_observe: quant_min/quant_max outside the 8- and 16-bit ranges");
+  const bool last_axis = inner == 1 && channels > 1;
+  const bool vec = aligned(x, 16) && (last_axis ? channels % 4 == 0 : inner % 4 == 0);
+  Plan p;
+  DQ8_REQUIRE(make_plan(outer, channels, inner, vec, &p), "dq8_observe: tensor too large");
+  DQ8_REQUIRE(workspace && workspace_bytes >= (size_t)p.pairs * sizeof(float2),
+              "dq8_observe: workspace too small (see dq8_minmax_workspace_bytes)");
+  const float full = (float)(q_max - q_min);
+  const QParamsOut q = {scale, zero_point, status, symmetric, symmetric ? full / 2 : full, q_min, q_max};
+  if (int s = run_minmax(x, outer, channels, inner, min_io, max_io, static_cast<float2*>(workspace),
+                         p, vec, (hipStream_t)stream, channels == 1 ? &q : nullptr))
+    return s;
+  if (channels == 1) return 0;
+  hipLaunchKernelGGL(minmax_qparams, dim3(1), dim3(1024), 0, (hipStream_t)stream, min_io, max_io,
+                     (int)channels, q);
+  return check_hip(hipGetLastError(), "minmax_qparams launch");
 }
 
 // ---- the same with the pairs in memory the library brings along -------------------------

@@ -18,7 +18,12 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <atomic>
+#include <chrono>
+#include <exception>
+#include <mutex>
 #include <string>
+#include <vector>
 
 #include "disc_q8.h"
 
@@ -281,6 +286,135 @@ PyObject* py_minmax(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// Pinned words that kernels report to the host through; a call borrows one while it waits.
+class StatusWords {
+ public:
+  // null when all are in use (then the caller takes one of its own)
+  static StatusWords& get() {
+    static StatusWords* words = new StatusWords;   // (for the process: torch may be gone at its end)
+    return *words;
+  }
+  volatile int32_t* borrow() {
+    std::lock_guard<std::mutex> guard(mu_);
+    if (free_.empty()) return nullptr;
+    volatile int32_t* w = free_.back();
+    free_.pop_back();
+    return w;
+  }
+  void give_back(volatile int32_t* w) {
+    std::lock_guard<std::mutex> guard(mu_);
+    free_.push_back(w);
+  }
+
+ private:
+  static constexpr int kWords = 64, kStride = 32;   // a 128-byte line each
+  StatusWords() {
+    page_ = at::empty({kWords * kStride}, at::TensorOptions().dtype(ScalarType::Int).pinned_memory(true));
+    for (int i = 0; i < kWords; ++i) free_.push_back(page_.data_ptr<int32_t>() + i * kStride);
+  }
+  Tensor page_;
+  std::mutex mu_;
+  std::vector<volatile int32_t*> free_;
+};
+
+struct StatusWord {
+  volatile int32_t* w = StatusWords::get().borrow();
+  Tensor own;
+  StatusWord() {
+    if (!w) {
+      own = at::empty({1}, at::TensorOptions().dtype(ScalarType::Int).pinned_memory(true));
+      w = own.data_ptr<int32_t>();
+    }
+    *w = 0;
+  }
+  StatusWord(const StatusWord&) = delete;
+  ~StatusWord() {
+    if (!own.defined()) StatusWords::get().give_back(w);
+  }
+  // Waits for the device's answer: reading the word costs a microsecond, a stream
+  // synchronisation ten.  After a while (a long queue in front, or a stream that cannot
+  // answer, such as one under capture) it is left to the synchronisation, which reports errors.
+  int32_t wait(const c10::hip::HIPStream& stream) const {
+    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(5);
+    for (int i = 0;; ++i) {
+      const int32_t v = *w;
+      if (v != 0) {
+        std::atomic_thread_fence(std::memory_order_acquire);
+        return v;
+      }
+      __builtin_ia32_pause();
+      if ((i & 255) == 255 && std::chrono::steady_clock::now() > until) break;
+    }
+    stream.synchronize();
+    return *w;
+  }
+};
+
+// observe(x, min_io, max_io, axis, symmetric, q_min, q_max, fake_quant)
+//   -> (min <= max everywhere, scale, zero_point, fake-quantized x or None)
+// One step of an observer: four kernels at most, the last of them the fake quantization, and one
+// wait for the answer whether the observed range is sound.
+PyObject* py_observe(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    arguments("observe", n, 8);
+    const Tensor &x0 = device_tensor(a[0]), &lo = device_tensor(a[1]), &hi = device_tensor(a[2]);
+    if (x0.scalar_type() != ScalarType::Float || lo.scalar_type() != ScalarType::Float ||
+        hi.scalar_type() != ScalarType::Float || !lo.is_contiguous() || !hi.is_contiguous())
+      raise(PyExc_TypeError, "observe takes float32 tensors");
+    const Tensor x = dense(x0);
+    const View3 v(x, a[3]);
+    if (lo.numel() != v.nch || hi.numel() != v.nch) {
+      PyErr_Format(PyExc_ValueError, "min / max state must have one entry per channel (%lld)",
+                   (long long)v.nch);
+      throw PyFailure{};
+    }
+    const bool symmetric = truth(a[4]), fake = truth(a[7]);
+    const int q_min = (int)integer(a[5]), q_max = (int)integer(a[6]);
+    const size_t need = dq8_minmax_workspace_bytes(v.outer, v.nch, v.inner);
+    const Tensor ws = empty({(int64_t)need}, ScalarType::Byte, x.device());
+    const Tensor s = empty(lo.sizes(), ScalarType::Float, x.device());
+    const Tensor z = empty(lo.sizes(), ScalarType::Int, x.device());
+    Tensor y;
+    if (fake) y = empty(x.sizes(), ScalarType::Float, x.device());
+    const StatusWord status;
+    const c10::hip::HIPStream st = c10::hip::getCurrentHIPStream();
+    int32_t answer = 0;
+    launch("dq8_observe", [&] {
+      if (int e = dq8_observe((const float*)ptr(x), v.outer, v.nch, v.inner, (float*)ptr(lo), (float*)ptr(hi),
+                              symmetric, q_min, q_max, (float*)ptr(s), (int32_t*)ptr(z),
+                              const_cast<int32_t*>(status.w), ptr(ws), need, (void*)st.stream()))
+        return e;
+      if (fake)
+        if (int e = dq8_fake_quant((const float*)ptr(x), (float*)ptr(y), v.outer, v.nch, v.inner,
+                                   (const float*)ptr(s), (const int32_t*)ptr(z), v.nch, q_min, q_max,
+                                   DQ8_ROUND_HALF_TO_EVEN, (void*)st.stream()))
+          return e;
+      return 0;
+    });
+    std::exception_ptr failed;
+    Py_BEGIN_ALLOW_THREADS
+    try {
+      answer = status.wait(st);
+    } catch (...) {
+      failed = std::current_exception();
+    }
+    Py_END_ALLOW_THREADS
+    if (failed) std::rethrow_exception(failed);
+    PyObject* r = PyTuple_New(4);
+    if (!r) throw PyFailure{};
+    PyTuple_SET_ITEM(r, 0, PyBool_FromLong(answer == 1));
+    PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(s));
+    PyTuple_SET_ITEM(r, 2, THPVariable_Wrap(z));
+    if (fake) {
+      PyTuple_SET_ITEM(r, 3, THPVariable_Wrap(y));
+    } else {
+      Py_INCREF(Py_None);
+      PyTuple_SET_ITEM(r, 3, Py_None);
+    }
+    return r;
+  });
+}
+
 // lut8(q, table, out)
 PyObject* py_lut8(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
@@ -464,6 +598,7 @@ PyMethodDef kMethods[] = {
     DQ8_METHOD("dequantize", py_dequantize),
     DQ8_METHOD("fake_quant", py_fake_quant),
     DQ8_METHOD("minmax", py_minmax),
+    DQ8_METHOD("observe", py_observe),
     DQ8_METHOD("lut8", py_lut8),
     DQ8_METHOD("weight_only_qgemm", py_weight_only),
     DQ8_METHOD("qgemm", py_qgemm),

@@ -110,6 +110,14 @@ def minmax(x, min_io, max_io, axis=None, workspace=None):
     return min_io, max_io
 
 
+def observe(x, min_io, max_io, symmetric, q_min, q_max, axis=None, fake_quant=False):
+    """One observation step: minmax(x, min_io, max_io, axis), then the 8-bit scale and zero point
+    of every channel from the running values and, if asked for, fake_quant(x) with them.  Returns
+    (sound, scale, zero_point, fake-quantized x or None); `sound` is False when a channel's
+    minimum is not at most its maximum (a NaN was observed).  x must not be empty."""
+    return _native().observe(x, min_io, max_io, axis, symmetric, q_min, q_max, fake_quant)
+
+
 def lut8(q, table, out=None):
     """out[i] = table[bit pattern of q[i]] for an int8 / uint8 device tensor; `table` is a
     256-entry device tensor of the output's 8-bit type."""

@@ -121,6 +121,20 @@ class Observer:
             zero_point = torch.clamp(zero_point, q_min, q_max)
         return scale, zero_point
 
+    def _observe(self, x, axis):
+        """Running min / max, scale and zero point, and the fake quantization of x in this mode,
+        for 8-bit types: what _calculate_qparams and _fake_quant do, on the device without a
+        round trip per step.  Returns the observer's result for x."""
+        fake = self.fake_quant and x.dtype == torch.float32
+        sound, scale, zero_point, y = K.observe(
+            x.detach().float(), self.min_val, self.max_val, self.symmetric, self.q_min,
+            self.q_max, axis=axis, fake_quant=fake)
+        assert sound, "min {} should be less than max {}".format(self.min_val, self.max_val)
+        self.scale, self.zero_point = scale, zero_point
+        if fake:
+            return y
+        return self._fake_quant(x, scale, zero_point) if self.fake_quant else x
+
     def _fake_quant(self, x, scale, zero_point):
         """quantize -> dequantize with the observer's qparams in one GPU kernel (8-bit
         types); the int32 bias grid is evaluated with the same formula in torch."""
@@ -146,6 +160,8 @@ class MinMaxObserver(Observer):
         self.max_val = torch.tensor(float("-inf"), device=self.device)
 
     def __call__(self, x):
+        if self.observe and self.bit == 8 and x.numel() > 0:
+            return self._observe(x, None)
         if self.observe:
             K.minmax(x.detach().float(), self.min_val.reshape(1), self.max_val.reshape(1))
             self.scale, self.zero_point = self._calculate_qparams(self.min_val, self.max_val)
@@ -175,6 +191,8 @@ class PerChannelMinMaxObserver(Observer):
             if self.min_val.numel() == 0 or self.max_val.numel() == 0:
                 self.min_val = torch.full((nch,), float("inf"), device=self.device)
                 self.max_val = torch.full((nch,), float("-inf"), device=self.device)
+            if self.bit == 8:
+                return self._observe(x, self.ch_axis)
             K.minmax(x.detach().float(), self.min_val, self.max_val, axis=self.ch_axis)
             self.scale, self.zero_point = self._calculate_qparams(self.min_val, self.max_val)
         if self.fake_quant:

@@ -137,6 +137,21 @@ size_t dq8_minmax_static_max_bytes(void);
 int dq8_minmax_static(const float* x, int64_t outer, int64_t channels, int64_t inner,
                       float* min_io, float* max_io, void* stream);
 
+/* One observation step of a calibration observer (R tools/torch_quant/torch_quant/observer.py
+ * :134-163, 236-241): dq8_minmax, then scale and zero point of every channel from its running
+ * values, on the device and without reading anything back:
+ *   symmetric: scale = max(max(-min', max') / ((q_max - q_min) / 2), eps), zero point 0
+ *   affine:    scale = max((max' - min') / (q_max - q_min), eps),
+ *              zero point = clamp(q_min - rne(min' / scale), q_min, q_max)
+ * with min' = min(min, 0), max' = max(max, 0), eps = 2^-23.  scale / zero_point: device,
+ * `channels` entries.  status: one int32 that device and host can reach (pinned host memory),
+ * set to 1 when all of this has been written and every channel has min <= max, to 2 when one has
+ * not (a NaN was observed).  The tensor must not be empty; workspace as for dq8_minmax. */
+int dq8_observe(const float* x, int64_t outer, int64_t channels, int64_t inner, float* min_io,
+                float* max_io, int symmetric, int32_t q_min, int32_t q_max, float* scale,
+                int32_t* zero_point, int32_t* status, void* workspace, size_t workspace_bytes,
+                void* stream);
+
 /* ---- quantize / dequantize -------------------------------------------- */
 
 /* x (device, f32) is viewed as [outer, nch, inner]; scale (device f32) and zp

@@ -179,3 +179,41 @@ def test_per_channel_and_bias_observers(K):
     np.testing.assert_array_equal(b_ob.scale.cpu().numpy(), bs)
     want_b = (np.clip(np.rint(bias / bs), -2.0 ** 31, 2.0 ** 31 - 1) * bs).astype(np.float32)
     np.testing.assert_array_equal(got_b, want_b)
+
+
+@pytest.mark.parametrize("shape,axis", [((1,), None), ((4097,), None), ((2000, 4100), None),
+                                        ((3, 5), 1), ((70, 1032), 1), ((1030, 33), 0), ((2, 5, 64), 1)])
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_observation_step_on_the_device(K, shape, axis, symmetric):
+    """min / max, scale, zero point and fake quantization of one step against the oracle, folded
+    into what an earlier step has seen; a NaN anywhere refuses the step, as before."""
+    from bladedisc_amd import observer as ob
+    rng = np.random.default_rng(sum(shape))
+    x = (rng.standard_normal(shape) * 2 + 0.5).astype(np.float32)
+    y = (x * np.float32(0.75) - np.float32(1)).astype(np.float32)
+    dtype = torch.qint8 if symmetric else torch.quint8
+    lim = (-128, 127) if symmetric else (0, 255)
+    if axis is None:
+        o = ob.MinMaxObserver(dtype=dtype, qscheme=torch.per_tensor_symmetric if symmetric
+                              else torch.per_tensor_affine)
+    else:
+        o = ob.PerChannelMinMaxObserver(axis, dtype=dtype, qscheme=torch.per_channel_symmetric
+                                        if symmetric else torch.per_channel_affine)
+    o(dev(x))
+    got = o(dev(y)).cpu().numpy()
+    lo, hi = OB.running_min_max([x, y], ch_axis=axis)
+    s, z = OB.calculate_qparams(lo, hi, *lim, symmetric=symmetric)
+    np.testing.assert_array_equal(o.scale.cpu().numpy(), s)
+    np.testing.assert_array_equal(o.zero_point.cpu().numpy(), z)
+    assert o.scale.dim() == o.zero_point.dim() == (0 if axis is None else 1)
+    s, z = np.asarray(s, np.float32), np.asarray(z, np.int32)
+    q = O.quantize(y, s if axis is not None else s.reshape(1), z.reshape(-1), axis=axis, qmin=lim[0],
+                   qmax=lim[1], dtype=np.int8 if symmetric else np.uint8)
+    want = O.dequantize(q, s if axis is not None else s.reshape(1), z.reshape(-1), axis=axis)
+    np.testing.assert_array_equal(got, want)
+    kept = o.scale
+    bad = y.copy()
+    bad.reshape(-1)[-1] = np.nan
+    with pytest.raises(AssertionError):
+        o(dev(bad))
+    assert o.scale is kept
