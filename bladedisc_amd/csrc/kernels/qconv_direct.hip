@@ -125,13 +125,21 @@ bool stream_conv_plan(DirectConvParams* p) {
   // MFMAs of 32 cycles per 32 channels plus the part of their requantisation that does not
   // run under another wave's MFMAs, plus the time of loading and of the last epilogue: three
   // blocks of a 3 x 3 filter, which is the measure for the short blocks of a 1 x 1 filter too).
+  // (a tile's results and residual are addressed with 31-bit offsets)
+  const int64_t reach = std::max(p->epi.ldo, p->epi.resid_kind == 2 ? p->epi.ldr : 0);
   const int64_t nf = ns / 32;
   const int64_t block_clk = (K / 32) * nf * 32 + nf * 230;
   const int64_t fixed_clk = p->Kh * p->Kw > 1 ? 3 * block_clk : 3 * (18 * 2 * 32 + 2 * 230);
   int64_t best_cost = -1, best_tpi = 0, best_patch = 0;
-  for (int64_t tpi = 1; tpi <= ceil_div(hw, 32); ++tpi) {
+  // One step per distinct tile size, from the largest down, until the rounds alone cost more than
+  // the best tiling found: the planner is called per launch, and a 1 x 1 filter's "image" is all
+  // pixels (walked tile count by tile count, 32 x 56 x 56 took 12 us of the host's time).
+  const int64_t most_1x1 = fixed / 1024 * 1024 / p->Ci / 32 * 32;      // (pixels that fit the LDS)
+  if (fixed < 1024 || most_1x1 < 32) return false;
+  for (int64_t tpi = p->Kh * p->Kw == 1 ? ceil_div(hw, most_1x1) : 1, next; tpi <= ceil_div(hw, 32); tpi = next) {
     const int64_t tile = ceil_div(hw, tpi);
-    if (ceil_div(hw, tile) != tpi) continue;               // the same tiling as a smaller tpi
+    next = tile > 1 ? ceil_div(hw, tile - 1) : hw + 1;
+    if (best_cost >= 0 && ceil_div((int64_t)p->NB * tpi * tiles_n, cus) * (block_clk + fixed_clk) > best_cost) break;
     // image rows a tile of `tile` consecutive pixels can span, wherever it starts in a row (an
     // upper bound for this tiling, in closed form: the planner is called per launch)
     const int64_t span = std::min<int64_t>((tile + p->Wo - 2) / p->Wo + 1, p->Ho);
@@ -139,7 +147,7 @@ bool stream_conv_plan(DirectConvParams* p) {
     const int64_t patch = p->Kh * p->Kw == 1
                               ? (ceil_div(tile, 32) * 32 * p->Ci + 1023) / 1024 * 1024
                               : ((span + p->Kh - 1) * pitch * p->Ci + 1023) / 1024 * 1024;
-    if (patch > fixed) continue;
+    if (patch > fixed || tile * reach >= (1LL << 31)) continue;
     const int64_t blocks = ceil_div(tile, 32);
     const int64_t simd0 = ceil_div(blocks, 8) + (blocks > 4 ? ceil_div(blocks - 4, 8) : 0);
     const int64_t wgs = (int64_t)p->NB * tpi * tiles_n;
@@ -168,7 +176,7 @@ bool stream_conv_plan(DirectConvParams* p) {
 }
 
 namespace {
-template <int KH, int KW, int CI, int NS, int EPI, bool POST>
+template <int KH, int KW, int CI, int NS, int EPI, int POST>
 int launch_stream_t(const DirectConvParams& p, hipStream_t st) {
   const int lds = p.patch_bytes + stream_conv_weight_lds(KH * KW * CI, NS) + stream_conv_cp_bytes(NS);
   auto kern = qconv_stream_kernel<KH, KW, CI, NS, EPI, POST>;
@@ -182,9 +190,9 @@ int launch_stream_t(const DirectConvParams& p, hipStream_t st) {
 
 template <int KH, int KW, int CI, int NS, int EPI>
 int launch_stream_post(const DirectConvParams& p, hipStream_t st) {
-  const bool post = p.epi.table != nullptr || p.epi.resid_kind != 0;
-  return post ? launch_stream_t<KH, KW, CI, NS, EPI, true>(p, st)
-              : launch_stream_t<KH, KW, CI, NS, EPI, false>(p, st);
+  return p.epi.table       ? launch_stream_t<KH, KW, CI, NS, EPI, 1>(p, st)
+         : p.epi.resid_kind ? launch_stream_t<KH, KW, CI, NS, EPI, 2>(p, st)
+                            : launch_stream_t<KH, KW, CI, NS, EPI, 0>(p, st);
 }
 
 template <int EPI>
@@ -196,10 +204,7 @@ int launch_stream_epi(const DirectConvParams& p, hipStream_t st) {
   if (taps == 1 && p.Ci == 64 && p.slice_n == 128) return launch_stream_post<1, 1, 64, 128, EPI>(p, st);
   if (taps == 1 && p.Ci == 64 && p.slice_n == 64) return launch_stream_post<1, 1, 64, 64, EPI>(p, st);
   if (taps == 1 && p.Ci == 128 && p.slice_n == 128) return launch_stream_post<1, 1, 128, 128, EPI>(p, st);
-  // (256 channels: without fused operators only -- with them the kernel would spill)
-  if (taps == 1 && p.Ci == 256 && !(p.epi.table != nullptr || p.epi.resid_kind != 0)) {
-    if (p.slice_n == 64) return launch_stream_t<1, 1, 256, 64, EPI, false>(p, st);
-  }
+  if (taps == 1 && p.Ci == 256 && p.slice_n == 64) return launch_stream_post<1, 1, 256, 64, EPI>(p, st);
   return fail("the streaming convolution kernel has no instance for this filter");
 }
 }  // namespace

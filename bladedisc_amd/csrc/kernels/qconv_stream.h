@@ -45,6 +45,8 @@
 
 namespace dq8 {
 
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+
 // LDS bytes the kernel needs on top of the patch: the padded weight slice (rows of K + 16
 // bytes, rounded up to the 8 KiB the eight waves' equal shares of load instructions cover) and
 // the per-channel (scale, addend) pairs.
@@ -55,9 +57,13 @@ constexpr int stream_conv_weight_lds(int K, int NS) {
 // tile per wave)
 constexpr int stream_conv_cp_bytes(int NS) { return NS * 8 + 256 + (NS >= 64 ? 8 * 32 * NS : 0); }
 
-// POST: the launch has operators fused behind the convolution (their code and registers are kept
-// out of the plain form).
-template <int KH, int KW, int CI, int NS, int EPI, bool POST>
+// POST: the operators fused behind the convolution -- 0 none, 1 a table, 2 a residual (their code
+// and registers are kept out of each other's forms).  A table that only clamps costs nothing
+// (table_clamp).  The int8 residual of a block is fetched a block ahead, in row order, and meets
+// the results in the wave's result tile in LDS; fetched where it is used, every fragment waited
+// for a trip to memory (32 x 56 x 56 x 64 -> 256, 1 x 1, int8 residual + ReLU + quantize: 30 us,
+// of which 7 were arithmetic).
+template <int KH, int KW, int CI, int NS, int EPI, int POST>
 __global__ void __launch_bounds__(512) qconv_stream_kernel(const DirectConvParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   static_assert(EPI == DQ8_EPI_REQUANT_CPU || EPI == DQ8_EPI_REQUANT_GPU, "int8 results only");
@@ -82,15 +88,15 @@ __global__ void __launch_bounds__(512) qconv_stream_kernel(const DirectConvParam
   // instruction covers whole 64- or 128-byte pieces, which can be written through the L2 (see
   // st_through: an ordinary store's dirty lines are written back after the kernel's last wave,
   // 25 MB of results in about 2.5 us; 32-byte pieces written through are slower than that).
-  // Not where the fused operators come on top of a filter slice of 144 registers: no room.
-  constexpr bool STAGE = NS >= 64 && !(POST && KS * NF * 4 + NF * 16 > 170);
+  constexpr bool STAGE = NS >= 64;
   constexpr int LPR = NS / 16;                // lanes (16-byte chunks) per row of that tile
   // The factors of a lane's channels (16 scales and 16 addends per 32-channel fragment) stay in
   // registers over all blocks where the filter slice leaves room for them; otherwise they are
   // read from LDS per fragment, all reads of a fragment ahead of its arithmetic (read one by one
   // as they are needed, each read exposes the LDS latency under the other waves' fragment reads).
-  constexpr bool HOIST_OS = KS * NF * 4 + NF * 16 + NF * 16 + 60 <= 240;
-  constexpr bool HOIST_B = KS * NF * 4 + NF * 16 + NF * 32 + 60 <= 240;
+  // (With a residual its registers and the arithmetic on it take that room.)
+  constexpr bool HOIST_OS = POST != 2 && KS * NF * 4 + NF * 16 + NF * 16 + 60 <= 240;
+  constexpr bool HOIST_B = POST != 2 && KS * NF * 4 + NF * 16 + NF * 32 + 60 <= 240;
   static_assert(W_PER_WAVE * NW * 1024 <= W_LDS, "weight area");
   static_assert(NS % 32 == 0 && K % 32 == 0 && KS * NF * 4 <= 160, "the filter slice must fit the registers");
 
@@ -133,12 +139,44 @@ __global__ void __launch_bounds__(512) qconv_stream_kernel(const DirectConvParam
   const unsigned lds_base =
       (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(size_t)(lds_void_t*)smem);
 
+  // Results and residual of the tile through buffer descriptors that begin at its first pixel and
+  // channel: a lane with nothing to store (or fetch) gives an out-of-range offset, so that every
+  // wave issues the same number of memory instructions per block and can count what is in flight.
+  const int64_t tile0 = (int64_t)img * hw + p0;
+  const __amdgpu_buffer_rsrc_t out_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      static_cast<int8_t*>(e.out) + tile0 * e.ldo + n0, 0, 0x7fffffff, kBufferRsrcWord3);
+  const bool resid_s8 = POST == 2 && e.resid_kind == 2 && e.resid_vec && e.N % 16 == 0;
+  const __amdgpu_buffer_rsrc_t res_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<int8_t*>(static_cast<const int8_t*>(e.resid)) + (resid_s8 ? tile0 * e.ldr + n0 : 0), 0,
+      0x7fffffff, kBufferRsrcWord3);
+  // chunk u (64 lanes per instruction) of a block's 32 x NS tile in LDS: row, and channels 16 c
+  auto tile_row = [&](int u) { return u / LPR; };
+  auto tile_chunk = [&](int u) { return (u % LPR) ^ (NS == 64 ? (u / LPR >> 2) & 3 : (u / LPR >> 1) & (LPR - 1)); };
+  v4i res[NF];                       // the residual of the wave's next block
+  auto load_resid = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < NF; ++i) {
+      int row, c;
+      if constexpr (STAGE) {
+        row = tile_row(i * 64 + lane);
+        c = tile_chunk(i * 64 + lane);
+      } else {                       // in fragment order: the lane's pixel, 16 channels of fragment i
+        row = lane & 31;
+        c = 2 * i + (lane >> 5);
+      }
+      const bool ok = p0 + b * 32 + row < p_end && n0 + c * 16 < e.N;
+      res[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(
+          res_rsrc, ok ? (int)((b * 32 + row) * e.ldr) + c * 16 : kOutOfRange, 0, 0));
+    }
+  };
+  if (POST == 2 && resid_s8) load_resid(wave);
+
   // ---- per-channel factors: the loads go out first and are used last
   ColRaw raw = {1.0f, 1.0f, 1.0f, 0};
   if (tid < NS) raw = col_fetch<EPI>(e, n0 + tid < e.N ? n0 + tid : e.N - 1);
   uint32_t tab_word = 0;
-  if (POST && e.table && tid >= 64 && tid < 128)      // (a fused table: 256 bytes, fetched by wave 1)
-    tab_word = reinterpret_cast<const uint32_t*>(e.table)[tid - 64];
+  if (POST == 1)                                      // (a fused table: 256 bytes, four to a lane)
+    tab_word = reinterpret_cast<const uint32_t*>(e.table)[lane];
 
   // ---- the weight slice: LDS rows of ROWC chunks, chunk g = 64 j + lane of instruction j
 #pragma unroll
@@ -251,7 +289,11 @@ __global__ void __launch_bounds__(512) qconv_stream_kernel(const DirectConvParam
     cp_os[tid] = c.os;
     cp_b[tid] = c.b;
   }
-  if (POST && e.table && tid >= 64 && tid < 128) reinterpret_cast<uint32_t*>(tab)[tid - 64] = tab_word;
+  ClampTable ct = {true, -128.0f, 127.0f};
+  if (POST == 1) {
+    ct = table_clamp(tab_word);
+    if (!ct.clamps && tid < 64) reinterpret_cast<uint32_t*>(tab)[tid] = tab_word;
+  }
   int later = 0;                     // (1 x 1) load instructions of this wave's blocks after the current one
   if constexpr (POINT) {
     for (int b = wave + NW; b < nblocks; b += NW) {
@@ -264,6 +306,8 @@ __global__ void __launch_bounds__(512) qconv_stream_kernel(const DirectConvParam
   DQ8_TRACE_WAVE(3);
 
   const bool plain = e.bias_kind == DQ8_BIAS_NONE && e.zo == 0;
+  ResidTail rt = {};
+  if (POST == 2 && resid_s8) rt = resid_tail(e);
   int8_t* out = static_cast<int8_t*>(e.out);
   const int c0 = lane >> 5;
   const int pitch_bytes = PWp << LOG2_CI;
@@ -293,8 +337,16 @@ __global__ void __launch_bounds__(512) qconv_stream_kernel(const DirectConvParam
     int hq;
     if constexpr (POINT) {
       hq = b * 32 + (lane & 31);
-      wait_patch_loads(later);        // the block's pixels have landed (later blocks' may be on their way)
-      later -= IPB;
+      // The block's pixels have landed: for the wave's first block while those of the others may
+      // be on their way; from the second on they have had a block's time to, and what may be in
+      // flight behind them are the stores of the block before (and the residual of this one).
+      constexpr int kYounger = (STAGE ? NF : 0) + (POST == 2 ? NF : 0);
+      if (b == wave)
+        wait_patch_loads(later);
+      else if (POST != 2 || resid_s8)
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(kYounger));
+      else
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
     } else {
       const int px = px_raw < p_end ? px_raw : p_end - 1;
       const int y = (int)__umulhi((unsigned)px, p.wo_inv), x = px - y * p.Wo;
@@ -361,8 +413,19 @@ __global__ void __launch_bounds__(512) qconv_stream_kernel(const DirectConvParam
     // pixel lane % 32 and the channel quads 8 g + 4 (lane / 32) .. + 3; two half-wave swaps
     // leave it with 16 consecutive channels, one 16-byte store
     const int64_t m = (int64_t)img * hw + px_raw;
+    if (POST == 2 && resid_s8) {
+      // the block's residual into the wave's result tile (its previous results have been read:
+      // LDS serves a wave in order), and the next block's on its way
+      if constexpr (STAGE) {
+#pragma unroll
+        for (int i = 0; i < NF; ++i) *reinterpret_cast<v4i*>(stg + (i * 64 + lane) * 16) = res[i];
+        load_resid(b + NW);
+      }
+    }
+    // MODE 0: with bias and zero point, 1: without; 2 / 3: int8 residual without / with zero points
     auto finish = [&](auto mode_c) {
-      constexpr bool PLAIN = decltype(mode_c)::value == 1;
+      constexpr int MODE = decltype(mode_c)::value;
+      constexpr bool PLAIN = MODE == 1;
       static_for<NF>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
         const int cl0 = j * 32 + 4 * c0;
@@ -380,14 +443,30 @@ __global__ void __launch_bounds__(512) qconv_stream_kernel(const DirectConvParam
         };
         // all LDS reads of the fragment ahead of its arithmetic (the instantiations with fused
         // operators have no registers to spare for that and read as they go)
-        constexpr bool kAhead = !POST && (!HOIST_OS || (!PLAIN && !HOIST_B));
+        constexpr bool kAhead = POST == 0 && (!HOIST_OS || (!PLAIN && !HOIST_B));
         v4f os4[kAhead ? 4 : 1], b4[kAhead ? 4 : 1];
         if constexpr (kAhead) {
 #pragma unroll
           for (int g = 0; g < 4; ++g) factors(g, os4[g], b4[g]);
           __builtin_amdgcn_sched_barrier(0);
         }
-        uint32_t w[4];
+        const int r = lane & 31;
+        const int slot = STAGE ? (2 * j + c0) ^ (NS == 64 ? (r >> 2) & 3 : (r >> 1) & (LPR - 1)) : 0;
+        uint32_t w[4], rw[4];
+        if constexpr (MODE >= 2) {
+          v4i rv;
+          if constexpr (STAGE)
+            rv = *reinterpret_cast<const v4i*>(stg + r * NS + slot * 16);
+          else
+            rv = res[j];
+          // (the swaps below, undone: two words of four channels each, per half-wave)
+          const auto r01 = __builtin_amdgcn_permlane32_swap(rv[0], rv[1], false, false);
+          const auto r23 = __builtin_amdgcn_permlane32_swap(rv[2], rv[3], false, false);
+          rw[0] = r01[0];
+          rw[2] = r01[1];
+          rw[1] = r23[0];
+          rw[3] = r23[1];
+        }
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           v4f os, b;
@@ -398,20 +477,24 @@ __global__ void __launch_bounds__(512) qconv_stream_kernel(const DirectConvParam
             factors(g, os, b);
           }
           const ColParams c[4] = {{os[0], b[0], 0}, {os[1], b[1], 0}, {os[2], b[2], 0}, {os[3], b[3], 0}};
-          w[g] = requant_pack4<EPI, PLAIN>(e, c, acc[j][4 * g + 0], acc[j][4 * g + 1],
-                                           acc[j][4 * g + 2], acc[j][4 * g + 3]);
+          if constexpr (MODE >= 2)
+            w[g] = resid_pack4<EPI, MODE == 2>(e, rt, c, acc[j][4 * g + 0], acc[j][4 * g + 1],
+                                               acc[j][4 * g + 2], acc[j][4 * g + 3], rw[g]);
+          else
+            w[g] = requant_pack4<EPI, PLAIN>(e, c, acc[j][4 * g + 0], acc[j][4 * g + 1],
+                                             acc[j][4 * g + 2], acc[j][4 * g + 3], ct.lo, ct.hi);
         }
         const auto s02 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
         const auto s13 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
         v4i v = {(int)s02[0], (int)s02[1], (int)s13[0], (int)s13[1]};
         const int n = n0 + j * 32 + 16 * c0;
-        // (operators fused behind the convolution: a table, or + residual [, ReLU] and quantize)
-        if (POST && (e.table || e.resid_kind)) fused_tail16(e, tab, m, n, px_raw < p_end, v);
+        // (a table to look up, or a residual of the general form; staged results meet theirs on
+        // the way out, when the accumulators' registers are free)
+        if (!STAGE && ((POST == 1 && !ct.clamps) || (POST == 2 && MODE < 2)))
+          fused_tail16<true>(e, tab, m, n, px_raw < p_end, v);
         if constexpr (STAGE) {
           // chunk c of tile row r in slot c ^ f(r), f such that the 16 lanes of a write phase
           // (16 consecutive rows, the same chunk) cover all banks
-          const int r = lane & 31;
-          const int slot = (2 * j + c0) ^ (NS == 64 ? (r >> 2) & 3 : (r >> 1) & (LPR - 1));
           *reinterpret_cast<v4i*>(stg + r * NS + slot * 16) = v;
         } else if (px_raw < p_end && n < e.N) {
           int8_t* dst = out + m * e.ldo + n;
@@ -425,21 +508,28 @@ __global__ void __launch_bounds__(512) qconv_stream_kernel(const DirectConvParam
         }
       });
     };
-    if (plain)
+    if (POST == 2 && rt.fast && rt.zero)
+      finish(IntC<POST == 2 ? 2 : 0>());
+    else if (POST == 2 && rt.fast)
+      finish(IntC<POST == 2 ? 3 : 0>());
+    else if (plain)
       finish(IntC<1>());
     else
       finish(IntC<0>());
+    if (POST == 2 && resid_s8 && !STAGE) load_resid(b + NW);
     if constexpr (STAGE) {
       // (the wave's own writes, in order: no barrier)
 #pragma unroll
       for (int i = 0; i < NF; ++i) {
         const int u = i * 64 + lane;
-        const int r = u / LPR;
-        const int c = (u % LPR) ^ (NS == 64 ? (r >> 2) & 3 : (r >> 1) & (LPR - 1));
-        const v4i v = *reinterpret_cast<const v4i*>(stg + u * 16);
-        const int px2 = p0 + b * 32 + r;
-        if (px2 < p_end && n0 + c * 16 < e.N)
-          st_through(out + ((int64_t)img * hw + px2) * e.ldo + n0 + c * 16, v);
+        const int row = tile_row(u), c = tile_chunk(u);
+        v4i v = *reinterpret_cast<const v4i*>(stg + u * 16);
+        const bool ok = p0 + b * 32 + row < p_end && n0 + c * 16 < e.N;
+        if ((POST == 1 && !ct.clamps) || (POST == 2 && !rt.fast))
+          fused_tail16<true>(e, tab, tile0 + b * 32 + row, n0 + c * 16, p0 + b * 32 + row < p_end, v);
+        // (sc0 sc1: written through the L2, as st_through)
+        __builtin_amdgcn_raw_buffer_store_b128(
+            __builtin_bit_cast(v4u, v), out_rsrc, ok ? (int)((b * 32 + row) * e.ldo) + c * 16 : kOutOfRange, 0, 17);
       }
     }
     DQ8_TRACE_WAVE(5 + 2 * ((b - wave) / NW));

@@ -1283,11 +1283,11 @@ int qconv2d_impl(int variant, const int8_t* in, const int64_t in_sizes[4], const
       sp.NB = (int)NB; sp.H = sp.Ho = (int)Ho; sp.Wd = sp.Wo = (int)Wo;
     }
     sp.epi = e;
-    const bool ok = stream_out && Ci <= 256 && (Ci <= 128 || !fused) && stream_conv_has_instance(1, 1, (int)Ci) &&
+    const bool ok = stream_out && Ci <= 256 && stream_conv_has_instance(1, 1, (int)Ci) &&
                     stream_conv_plan(&sp);
     if (!auto_pick)
       DQ8_REQUIRE(ok, "dq8_qconv2d: the streaming variant needs a 3 x 3 or 1 x 1 filter on 64 or "
-                      "128 input channels (1 x 1 without fused operators also on 256), stride and "
+                      "128 input channels (1 x 1 also on 256), stride and "
                       "dilation 1, an int8 result (float output stage) and 16-byte aligned output "
                       "rows");
     // Against the GEMM kernels, whose k tile of 128 is half empty at 64 channels and whose

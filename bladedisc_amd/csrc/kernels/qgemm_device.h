@@ -279,9 +279,11 @@ __device__ __forceinline__ void st_through(void* p, const v4i& v) {
 // PLAIN: the launch has no bias and no output zero point, so the additive terms are +0.0f and
 // are left out.  Adding +0.0f changes nothing but the sign of a zero, and a zero of either
 // sign gives the byte 0 below, so the result is the same bit for bit.
+// lo, hi: integers in [-128, 127], the bounds of the int8 range or a fused clamp's (table_clamp).
 template <int EPI, bool PLAIN = false>
 __device__ __forceinline__ uint32_t requant_pack4(const EpiParams& p, const ColParams (&c)[4],
-                                                  int a0, int a1, int a2, int a3) {
+                                                  int a0, int a1, int a2, int a3,
+                                                  float lo = -128.0f, float hi = 127.0f) {
   const int acc[4] = {a0, a1, a2, a3};
   float clamped[4];
 #pragma unroll
@@ -297,7 +299,7 @@ __device__ __forceinline__ uint32_t requant_pack4(const EpiParams& p, const ColP
     }
     // v_med3_f32: one instruction for the clamp; with a NaN operand it returns the
     // minimum of the other two, so NaN -> -128 like the CPU path
-    clamped[e] = __builtin_amdgcn_fmed3f(d, -128.0f, 127.0f);
+    clamped[e] = __builtin_amdgcn_fmed3f(d, lo, hi);
   }
   // Rounding, conversion and packing in one instruction per result: adding 1.5 * 2^23 rounds
   // the clamped value to an integer (nearest even) and leaves its two's-complement int8 in
@@ -519,11 +521,108 @@ __device__ __forceinline__ void tile_coords(int bid, int nblocks, int tiles_m, i
   tn = in_panel / rows;
 }
 
+// A fused table that only clamps -- ReLU, ReLU6 or a hard tanh between tensors of one scale --
+// needs no lookup: clamp(clamp(q, -128, 127), lo, hi) of an integer q is the clamp the
+// requantisation ends with, with other bounds, and costs nothing.  Looked up, a table costs 16
+// LDS byte reads and about 50 vector instructions per 16 results (32 x 56 x 56 x 64 -> 64, 3 x 3:
+// 11.1 us with a lookup, 7.0 without a table).  Called by whole waves; `word`: the lane's four
+// entries 4 lane .. 4 lane + 3 (by bit pattern).
+struct ClampTable {
+  bool clamps;
+  float lo, hi;   // the bounds of the requantisation: the table's, or the int8 range
+};
+__device__ __forceinline__ ClampTable table_clamp(uint32_t word) {
+  const int lo = (int)(int8_t)(__builtin_amdgcn_readlane((int)word, 32) & 0xff);   // entry of -128
+  const int hi = __builtin_amdgcn_readlane((int)word, 31) >> 24;                   // entry of 127
+  const int q0 = (int)(int8_t)(4 * (threadIdx.x & 63));
+  bool same = lo <= hi;
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const int q = q0 + b;
+    same = same && (int)(int8_t)(word >> (8 * b)) == (q < lo ? lo : (q > hi ? hi : q));
+  }
+  const bool clamps = __builtin_amdgcn_ballot_w64(same) == ~0ull;
+  return {clamps, clamps ? (float)lo : -128.0f, clamps ? (float)hi : 127.0f};
+}
+
+// The int8 residual form (dequantize, + residual, [ReLU], quantize) on accumulators.  Behind the
+// requantisation its arithmetic is carried on in f32 registers instead of packing the int8
+// result, unpacking it again and testing every step's special cases: 14 to 19 vector
+// instructions per result, requantisation included, where the general form below takes about 30.
+// With all three scales between 2^-40 and 2^40 every intermediate is finite, so that
+//  * q - zo is (c + magic) - (magic + zo): both steps exact (c is clamped to [-128, 127]);
+//  * the exact quotient by the reciprocal (elementwise::div4_by_constant) needs no probe;
+//  * ReLU before a quantize with a positive scale is a lower bound z2 of the final clamp:
+//    t < 0 gives t / s2 + z2 <= z2, t >= 0 gives >= z2, the same in every rounding.
+struct ResidTail {
+  bool fast;        // this form applies (uniform over the launch)
+  bool zero;        // no zero point anywhere: the additions of zo, -zr and z2 are left out
+  float so, rs, s2, y2, zr, z2, lo, mzo;
+};
+__device__ __forceinline__ ResidTail resid_tail(const EpiParams& e) {
+  ResidTail t = {};
+  if (e.resid_kind != 2) return t;
+  t.so = e.so[0];
+  t.rs = e.resid_scale[0];
+  t.s2 = e.out_scale[0];
+  t.y2 = 1.0f / t.s2;
+  t.zr = (float)e.resid_zp;
+  t.z2 = (float)e.out_zp;
+  t.mzo = 12582912.0f + (float)e.zo;
+  t.lo = e.relu ? fminf(fmaxf(-128.0f, t.z2), 127.0f) : -128.0f;
+  auto small = [](int z) { return z >= -65536 && z <= 65536; };
+  t.fast = e.resid_vec && e.N % 16 == 0 && !e.fixedpoint && t.s2 > 0.0f &&
+           elementwise::divisor_in_fast_range(t.so) && elementwise::divisor_in_fast_range(t.rs) &&
+           elementwise::divisor_in_fast_range(t.s2) && small(e.zo) && small(e.resid_zp) && small(e.out_zp);
+  t.zero = e.zo == 0 && e.resid_zp == 0 && e.out_zp == 0;
+  return t;
+}
+// r: the residual's four int8 of the same channels
+template <int EPI, bool ZERO>
+__device__ __forceinline__ uint32_t resid_pack4(const EpiParams& p, const ResidTail& t,
+                                                const ColParams (&c)[4], int a0, int a1, int a2,
+                                                int a3, uint32_t r) {
+  const int acc[4] = {a0, a1, a2, a3};
+  const float magic = 12582912.0f;
+  float v[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float d = (float)acc[e];
+    if (EPI == DQ8_EPI_REQUANT_CPU) {
+      d = d + c[e].b;
+      d = d * c[e].os;
+      if (!ZERO) d = d + (float)p.zo;
+    } else {
+      d = c[e].os * d;
+      d = d + c[e].b;
+    }
+    d = (__builtin_amdgcn_fmed3f(d, -128.0f, 127.0f) + magic) - (ZERO ? magic : t.mzo);
+    float f = (float)(int)(int8_t)(r >> (8 * e));
+    if (!ZERO) f = f - t.zr;
+    const float x = d * t.so + f * t.rs;      // (separate roundings: the file has contraction off)
+    const float q0 = x * t.y2;
+    float q = __builtin_fmaf(__builtin_fmaf(-q0, t.s2, x), t.y2, q0);
+    if (!ZERO) q = q + t.z2;
+    v[e] = __builtin_amdgcn_fmed3f(q, t.lo, 127.0f);
+  }
+  uint32_t word = __float_as_uint(v[0] + magic);
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm("v_add_f32_sdwa %0, %1, %2 dst_sel:BYTE_1 dst_unused:UNUSED_PRESERVE src0_sel:DWORD src1_sel:DWORD"
+      : "+v"(word) : "v"(v[1]), "v"(magic));
+  asm("v_add_f32_sdwa %0, %1, %2 dst_sel:BYTE_2 dst_unused:UNUSED_PRESERVE src0_sel:DWORD src1_sel:DWORD"
+      : "+v"(word) : "v"(v[2]), "v"(magic));
+  asm("v_add_f32_sdwa %0, %1, %2 dst_sel:BYTE_3 dst_unused:UNUSED_PRESERVE src0_sel:DWORD src1_sel:DWORD"
+      : "+v"(word) : "v"(v[3]), "v"(magic));
+#endif
+  return word;
+}
+
 // Operators fused behind the quantized result of an int8 epilogue.  `v` holds the 16 consecutive
 // channels n .. n + 15 of output row m (which is also how the residual is read); `tab` is the
 // 256-entry table in LDS when e.table is set; `row_ok`: the row exists.  Table:
 // v = table[(uint8) v]; residual: v = quantize(resid_add(dequantize(v), r)) with the arithmetic
-// of the separate library calls.
+// of the separate library calls.  TIGHT: word by word, for a kernel that has few registers left.
+template <bool TIGHT = false>
 __device__ __forceinline__ void fused_tail16(const EpiParams& e, const uint8_t* tab, int64_t m,
                                              int n, bool row_ok, v4i& v) {
   if (e.table) {
@@ -532,6 +631,7 @@ __device__ __forceinline__ void fused_tail16(const EpiParams& e, const uint8_t* 
       const uint32_t x = (uint32_t)v[d];
       v[d] = (int)((uint32_t)tab[x & 0xff] | ((uint32_t)tab[(x >> 8) & 0xff] << 8) |
                    ((uint32_t)tab[(x >> 16) & 0xff] << 16) | ((uint32_t)tab[x >> 24] << 24));
+      if (TIGHT) __builtin_amdgcn_sched_barrier(0);
     });
   } else if (row_ok && n < e.N) {
     const float so_v = e.so[0], s2 = e.out_scale[0], z2 = (float)e.out_zp;
@@ -590,6 +690,7 @@ __device__ __forceinline__ void fused_tail16(const EpiParams& e, const uint8_t* 
         });
         v[d] = (int)w2;
       }
+      if (TIGHT) __builtin_amdgcn_sched_barrier(0);
     });
   }
 }
@@ -908,7 +1009,29 @@ __device__ __forceinline__ void mfma_epilogue(v16i (&acc)[FM][FN], const EpiPara
         }
       }
     };
-    // MODE 0: float stage with its additive terms, 1: without them, 2: fixed-point stage
+    // a fused table that clamps becomes the bounds of the requantisation's clamp
+    bool lookup = BeforeStores::kPostOps && e.table;
+    float clamp_lo = -128.0f, clamp_hi = 127.0f;
+    if (BeforeStores::kPostOps && e.table && !fixedpoint) {
+      const ClampTable ct = table_clamp(reinterpret_cast<const uint32_t*>(tab)[lane]);
+      lookup = !ct.clamps;
+      clamp_lo = ct.lo;
+      clamp_hi = ct.hi;
+    }
+    const ResidTail rt = BeforeStores::kPostOps && FM * FN <= 8 ? resid_tail(e) : ResidTail{};
+    // the residual of the wave's next fragment, in flight while the current one is worked on
+    // (16 consecutive channels of the lane's row, as they are stored; N % 16 == 0, so a chunk is
+    // inside the row or past it; rows and chunks past the end read some other part)
+    auto load_resid = [&](int i, int j) {
+      const int m = m_wave0 + i * 32 + (lane & 31), n = n_wave0 + j * 32 + 16 * (lane >> 5);
+      return *reinterpret_cast<const v4i*>(static_cast<const int8_t*>(e.resid) +
+                                           (int64_t)(m < m_end ? m : m_end - 1) * e.ldr +
+                                           (n < e.N ? n : e.N - 16));
+    };
+    v4i res = {0, 0, 0, 0};
+    if (BeforeStores::kPostOps && rt.fast) res = load_resid(0, 0);
+    // MODE 0: float stage with its additive terms, 1: without them, 2: fixed-point stage, 3 / 4:
+    // float stage and an int8 residual without / with zero points
     auto store_all = [&](auto mode_c) {
       constexpr int MODE = decltype(mode_c)::value;
       // (static_for: with 16 fragments a loop this size is past what "#pragma unroll" unrolls,
@@ -930,10 +1053,24 @@ __device__ __forceinline__ void mfma_epilogue(v16i (&acc)[FM][FN], const EpiPara
         }
         static_for<FM>([&](auto ic) {
           constexpr int i = decltype(ic)::value;
-          uint32_t w[4];
+          uint32_t w[4], rw[4];
+          if constexpr (MODE >= 3) {
+            // (the swaps below, undone: two words of four channels each, per half-wave)
+            const auto r01 = __builtin_amdgcn_permlane32_swap(res[0], res[1], false, false);
+            const auto r23 = __builtin_amdgcn_permlane32_swap(res[2], res[3], false, false);
+            rw[0] = r01[0];
+            rw[2] = r01[1];
+            rw[1] = r23[0];
+            rw[3] = r23[1];
+            constexpr int next = j * FM + i + 1;
+            if constexpr (next < FM * FN) res = load_resid(next % FM, next / FM);
+          }
 #pragma unroll
           for (int g = 0; g < 4; ++g) {
-            if (MODE == 2) {
+            if constexpr (MODE >= 3) {
+              w[g] = resid_pack4<EPI, MODE == 3>(e, rt, c[g], acc[i][j][4 * g + 0], acc[i][j][4 * g + 1],
+                                                 acc[i][j][4 * g + 2], acc[i][j][4 * g + 3], rw[g]);
+            } else if (MODE == 2) {
               w[g] = 0;
 #pragma unroll
               for (int q = 0; q < 4; ++q)
@@ -943,14 +1080,15 @@ __device__ __forceinline__ void mfma_epilogue(v16i (&acc)[FM][FN], const EpiPara
                         << (8 * q);
             } else {
               w[g] = requant_pack4<EPI, MODE == 1>(e, c[g], acc[i][j][4 * g + 0], acc[i][j][4 * g + 1],
-                                                   acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
+                                                   acc[i][j][4 * g + 2], acc[i][j][4 * g + 3],
+                                                   clamp_lo, clamp_hi);
             }
           }
           // swap(a, b): the upper half of a trades places with the lower half of b
           const auto s02 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
           const auto s13 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
           v4i v = {(int)s02[0], (int)s02[1], (int)s13[0], (int)s13[1]};
-          if (BeforeStores::kPostOps && (e.table || e.resid_kind)) {
+          if (BeforeStores::kPostOps && MODE < 3 && (lookup || e.resid_kind)) {
             const int n = n_wave0 + j * 32 + 16 * (lane >> 5);
             const int64_t m = m_wave0 + i * 32 + (lane & 31);
             fused_tail16(e, tab, m, n, m < m_end, v);
@@ -962,8 +1100,14 @@ __device__ __forceinline__ void mfma_epilogue(v16i (&acc)[FM][FN], const EpiPara
         });
       });
     };
+    // (not in the four-wave 256 x 256 cross-check variant, whose 16 fragments leave no registers)
+    constexpr bool kResid = BeforeStores::kPostOps && FM * FN <= 8;
     if (fixedpoint)
       store_all(IntC<2>());
+    else if (kResid && rt.fast && rt.zero)
+      store_all(IntC<kResid ? 3 : 0>());
+    else if (kResid && rt.fast)
+      store_all(IntC<kResid ? 4 : 0>());
     else if (plain)
       store_all(IntC<1>());
     else

@@ -2084,3 +2084,49 @@ def test_conv_dispatch_sweep_agrees_with_the_generic_kernel(K):
         got = K.qconv2d(x, wt, padding, md, osh, K.EPI_REQUANT_CPU, **sc, post=K.make_postops(table=table))
         assert torch.equal(got, K.lut8(q, table)), (nb, h, w_, ci, co, k, stride, pad, dil)
     assert cases >= 80
+
+
+@pytest.mark.parametrize("nb,h,ci,co,k", [(1, 9, 64, 64, 3), (5, 31, 64, 64, 3), (3, 17, 128, 48, 3),
+                                          (2, 56, 64, 256, 1), (40, 33, 64, 48, 1), (8, 33, 128, 512, 1),
+                                          (9, 28, 256, 64, 1), (9, 28, 256, 128, 1), (2, 14, 512, 2048, 1),
+                                          (3, 28, 16, 64, 4), (1, 7, 512, 192, 3)])
+def test_clamping_tables_and_int8_residuals_equal_the_separate_operators(K, nb, h, ci, co, k):
+    """A fused table that clamps (ReLU, ReLU6) is taken as bounds, an int8 residual runs on the
+    accumulators where the scales allow it: the bits of the separate calls, with and without
+    zero points, with scales and tables on either side of those conditions."""
+    rng = np.random.default_rng(h * ci + co)
+    pad = [k // 2, (k - 1) // 2] * 2
+    x = dev(rng.integers(-128, 128, (nb, h, h, ci), dtype=np.int8))
+    wt = dev(rng.integers(-128, 128, (co, k, k, ci), dtype=np.int8))
+    md = list(O.NHWC_OHWI_METADATA) + [1, 1, 1, 1, 1]
+    osh = [nb, h, h, co]
+    s_acc = float(np.sqrt(k * k * ci) * 74 * 74)
+    so = np.float32(0.043)
+    sc = dict(sx=dev(np.array([0.02], np.float32)), so=dev(np.array([so])),
+              sw=dev((rng.uniform(0.7, 1.3, co) * (50 * 0.043 / 0.02 / s_acc)).astype(np.float32)))
+    bias = dev((rng.standard_normal(co) * 20 * so).astype(np.float32))
+    zi = lambda v: torch.full((1,), v, dtype=torch.int32, device="cuda")  # noqa: E731
+    rq = dev(rng.integers(-128, 128, osh, dtype=np.int8))
+    entries = np.arange(256).astype(np.uint8).view(np.int8)
+    almost = np.clip(entries, 0, 127)
+    almost[200] += 1
+    for epi, zo in ((K.EPI_REQUANT_CPU, 0), (K.EPI_REQUANT_CPU, 3), (K.EPI_REQUANT_GPU, 0)):
+        kw = dict(bias=bias if epi == K.EPI_REQUANT_CPU else dev(rng.standard_normal(co).astype(np.float32) * 20),
+                  zo=zo, **sc)
+        q = K.qconv2d(x, wt, pad, md, osh, epi, **kw)
+        for table in (np.clip(entries, 0, 127), np.clip(entries, -7, 90), entries, almost,
+                      np.full(256, 5, np.int8), np.clip(entries, -128, -1)):
+            t = dev(np.ascontiguousarray(table.astype(np.int8)))
+            got = K.qconv2d(x, wt, pad, md, osh, epi, post=K.make_postops(table=t), **kw)
+            assert torch.equal(got, K.lut8(q, t))
+        y = K.dequantize(q, sc["so"], zi(zo))
+        for rz, z2, s2, relu in ((0, 0, 0.05, True), (0, 0, 0.05, False), (-5, -128, 0.037, True),
+                                 (4, 130, 0.05, True), (0, -140, 0.05, True), (0, 0, -0.05, True),
+                                 (0, 7, 2e12, False)):
+            rs, ds2 = dev(np.array([0.031], np.float32)), dev(np.array([s2], np.float32))
+            t = y + K.dequantize(rq, rs, zi(rz))
+            t = torch.where(t < 0, torch.zeros_like(t), t) if relu else t
+            want = K.quantize(t, ds2, zi(z2))
+            got = K.qconv2d(x, wt, pad, md, osh, epi, post=K.make_postops(
+                residual=rq, residual_scale=rs, residual_zp=rz, relu=relu, out_scale=ds2, out_zp=z2), **kw)
+            assert torch.equal(got, want), (epi, zo, rz, z2, s2, relu)
