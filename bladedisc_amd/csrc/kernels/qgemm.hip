@@ -249,27 +249,51 @@ pad_rows_s8_kernel(const int8_t* __restrict__ src, int64_t ld, int8_t* __restric
   }
 }
 
-// out[r] = mul * sum_k X[r, k] + add for an int8 matrix whose rows are 16-byte aligned and a
-// multiple of 16 long: the zero-point corrections of a GEMM.  One wave per row.
-__global__ void __launch_bounds__(256)
-rowsum_s8_kernel(const int8_t* __restrict__ X, int64_t ld, int rows, int K, int mul, int add,
-                 int32_t* __restrict__ out) {
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+// What a GEMM wants of an operand before it starts, for both operands in one launch: rows of any
+// length and alignment copied to 16-byte aligned rows of ldd bytes (zero-filled past K), and the
+// row's share of the zero-point correction, corr[r] = mul * sum_k src[r, k] + add.  Either part
+// may be absent (dst or corr null).  One wave per row, 16 bytes per lane and step: read as aligned
+// words and shifted into place, since a row may start at any byte (a byte at a time, the copy of
+// 1501 x 1000 took 4.8 us; this launch does that, the 777 rows of the other operand and the
+// sums in 3.5).
+struct RowsJob {
+  const int8_t* src;
+  int64_t ld;
+  int8_t* dst;
+  int32_t* corr;
+  int rows, K, ldd, mul, add;
+};
+__global__ void __launch_bounds__(256) prepare_rows_kernel(const RowsJob ja, const RowsJob jb) {
+  int row = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool first = row < ja.rows;
+  const RowsJob& j = first ? ja : jb;
+  row -= first ? 0 : ja.rows;
+  if (row >= j.rows) return;
   const int lane = threadIdx.x & 63;
-  if (row >= rows) return;
-  const v4i* p = reinterpret_cast<const v4i*>(X + (int64_t)row * ld);
-  int s = 0;
-  for (int c = lane; c < K / 16; c += 64) {
-    const v4i v = p[c];
+  const int8_t* s = j.src + (int64_t)row * j.ld;
+  const int a = (int)(reinterpret_cast<uintptr_t>(s) & 3);            // (the same for the whole row)
+  const uint32_t* w = reinterpret_cast<const uint32_t*>(s - a);
+  const int last = (a + j.K - 1) >> 2;                                // the last word with a byte of the row
+  int sum = 0;
+  for (int c = lane * 16; c < (j.dst ? j.ldd : j.K); c += 64 * 16) {
+    uint32_t x[5];
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const int x = v[w];
-      s += (int)(int8_t)x + (int)(int8_t)(x >> 8) + (int)(int8_t)(x >> 16) + (x >> 24);
+    for (int i = 0; i < 5; ++i) x[i] = w[min((c >> 2) + i, last)];
+    v4i v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint32_t t = __builtin_amdgcn_alignbyte(x[i + 1], x[i], a);
+      const int left = j.K - c - 4 * i;                               // bytes of the row in this word
+      t = left >= 4 ? t : (left <= 0 ? 0u : t & (0xffffffffu >> (8 * (4 - left))));
+      v[i] = (int)t;
+      sum = __builtin_amdgcn_sdot4((int)t, 0x01010101, sum, false);
     }
+    if (j.dst) *reinterpret_cast<v4i*>(j.dst + (int64_t)row * j.ldd + c) = v;
   }
+  if (!j.corr) return;
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  if (lane == 0) out[row] = mul * s + add;
+  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+  if (lane == 0) j.corr[row] = j.mul * sum + j.add;
 }
 
 #ifdef DQ8_TEST_HOOKS
@@ -619,11 +643,13 @@ extern "C" const char* dq8_qgemm_variant_name(int variant) {
 
 extern "C" size_t dq8_qgemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int tp_a,
                                             int tp_b) {
-  // an operand that is not k-contiguous, or whose K is not a multiple of 16, is rewritten
-  // as [rows, K rounded up to 16] (zero filled) for the MFMA kernels
+  // an operand that is not k-contiguous, or whose K is not a multiple of 16, is rewritten as
+  // [rows, K rounded up to 16] (zero filled) for the MFMA kernels, rows a multiple of 128 bytes
+  // apart: their loads cover 8 rows x 128 bytes, which is 8 cache lines if the rows begin at one
+  // and 16 otherwise (777 x 1504, 1008 of k: 6.8 us, 1024 of k: 6.2)
   size_t bytes = 0;
   auto pad = [](int64_t v) { return (size_t)((v + 255) / 256 * 256); };
-  const int64_t kp = (K + 15) / 16 * 16;
+  const int64_t kp = (K + 127) / 128 * 128;
   if (tp_a || K % 16 != 0) bytes += pad(M * kp);
   if (!tp_b || K % 16 != 0) bytes += pad(N * kp);
   return bytes;
@@ -724,10 +750,29 @@ int qgemm_impl(int variant, const int8_t* A, int64_t lda, const int8_t* W, int64
   // zero points itself.
   const bool has_zp = zx != 0 || zw != 0;
   const bool auto_pick = variant == -1;
-  // The MFMA kernels want A [M, K'] and W [N, K'], k-contiguous, rows 16-byte aligned, K' a
+  // The tiled MFMA kernels want A [M, K'] and W [N, K'], k-contiguous, rows 16-byte aligned, K' a
   // multiple of 16: operands in another layout, or with a ragged K, are rewritten into the
   // workspace (zero-filled up to K'; zeros add nothing to the sums).
-  const int64_t Kp = (K + 15) / 16 * 16;
+  const int64_t Kp = (K + 15) / 16 * 16, pitch = (K + 127) / 128 * 128;
+  // A few rows against rows of any length or alignment: the small-M kernel takes them as they are.
+  if (auto_pick && !tp_a && tp_b && K >= 64 &&
+      (K % 16 != 0 || !aligned(A, 16) || !aligned(W, 16) || lda % 16 != 0 || ldw % 16 != 0) &&
+      pick_any(M, N, Kp, true, es) == kSkinnyVariant) {
+    MainParams p = {};
+    p.A = A;
+    p.W = W;
+    p.lda = lda;
+    p.ldw = ldw;
+    p.M = (int)M;
+    p.N = (int)N;
+    p.K = (int)K;
+    p.epi = e;
+    p.ragged = 1;
+    p.zx = zx;
+    p.zw = zw;
+    p.kzz = (int)((uint32_t)K * (uint32_t)zx * (uint32_t)zw);
+    return launch_epi<false>(kSkinnyVariant, p, epilogue, st);
+  }
   const bool repack_a = K > 0 && (tp_a || K % 16 != 0);
   const bool repack_w = K > 0 && (!tp_b || K % 16 != 0);
   const bool have_ws = workspace != nullptr && aligned(workspace, 256) &&
@@ -739,10 +784,7 @@ int qgemm_impl(int variant, const int8_t* A, int64_t lda, const int8_t* W, int64
       aligned(workspace, 256) &&
       workspace_bytes >= dq8_qgemm_workspace_bytes_zp(M, N, K, tp_a, tp_b, zx, zw);
   if (auto_pick && has_zp && !zp_mfma) variant = 0;
-  // fused operators are implemented on the vector store paths of the MFMA kernels (and in
-  // the generic kernel): output rows that are not 16-byte aligned take the generic kernel
   const bool fused = e.table != nullptr || e.resid_kind != 0;
-  if (fused && !(es == 1 ? e.vec_store16 : e.vec_store)) variant = 0;
   // (a ragged K without the scratch to pad it, or unaligned operands: the generic kernel
   // takes any strides; a transposed operand without scratch stays an error below)
   if (variant != 0 && !mfma_operands && !((tp_a || !tp_b) && !have_ws)) variant = 0;
@@ -773,26 +815,28 @@ int qgemm_impl(int variant, const int8_t* A, int64_t lda, const int8_t* W, int64
   int64_t lda_use = lda, ldw_use = ldw;
   size_t ws_off = 0;
   auto pad = [](int64_t v) { return (size_t)((v + 255) / 256 * 256); };
-  auto repack = [&](const int8_t* src, int64_t ld, bool transposed, int64_t rows) {
+  // Where the operands go: a transposed one through the transpose kernel, one with ragged rows
+  // through prepare_rows_kernel, which also forms the zero-point corrections.
+  RowsJob job_w = {}, job_a = {};
+  auto place = [&](const int8_t* src, int64_t ld, bool transposed, int64_t rows, RowsJob* job) {
     int8_t* dst = (int8_t*)workspace + ws_off;
-    if (transposed)   // src is [K, rows]
+    ws_off += pad(rows * pitch);
+    if (transposed) {   // src is [K, rows]
       hipLaunchKernelGGL(transpose_s8_kernel,
-                         dim3((unsigned)ceil_div(rows, 64), (unsigned)ceil_div(Kp, 64)), dim3(256),
-                         0, st, src, ld, dst, (int)K, (int)rows, (int)Kp);
-    else
-      hipLaunchKernelGGL(pad_rows_s8_kernel,
-                         dim3((unsigned)std::min<int64_t>(ceil_div(rows * (Kp / 16), 256), 1 << 20)),
-                         dim3(256), 0, st, src, ld, dst, rows, (int)K, (int)Kp);
-    ws_off += pad(rows * Kp);
+                         dim3((unsigned)ceil_div(rows, 64), (unsigned)ceil_div(pitch, 64)), dim3(256),
+                         0, st, src, ld, dst, (int)K, (int)rows, (int)pitch);
+    } else {
+      *job = {src, ld, dst, nullptr, (int)rows, (int)K, (int)pitch, 0, 0};
+    }
     return dst;
   };
   if (repack_a) {
-    a_use = repack(A, lda, tp_a != 0, M);
-    lda_use = Kp;
+    a_use = place(A, lda, tp_a != 0, M, &job_a);
+    lda_use = pitch;
   }
   if (repack_w) {
-    w_use = repack(W, ldw, tp_b == 0, N);
-    ldw_use = Kp;
+    w_use = place(W, ldw, tp_b == 0, N, &job_w);
+    ldw_use = pitch;
   }
   if (repack_a || repack_w) DQ8_HIP(hipGetLastError());
   const int64_t K_true = K;
@@ -809,17 +853,52 @@ int qgemm_impl(int variant, const int8_t* A, int64_t lda, const int8_t* W, int64
   p.epi = e;
   if (auto_pick)
     variant = pick_any(M, N, K, pipe_ok(256, 256, p, false), es);
-  if (fused || e.fixedpoint) {   // the persistent forms carry neither
-    DQ8_REQUIRE(auto_pick || (variant != kPersist256 && variant != kPersist256x192 && variant != kPersist128),
+  const bool rows_aligned = es == 1 ? e.vec_store16 : e.vec_store;
+  if (fused || e.fixedpoint || !rows_aligned) {   // the persistent forms carry none of these
+    DQ8_REQUIRE(auto_pick || (!fused && !e.fixedpoint) ||
+                    (variant != kPersist256 && variant != kPersist256x192 && variant != kPersist128),
                 "dq8_qgemm: the persistent variants take neither fused operators nor the fixed-point stage");
     if (variant == kPersist256) variant = kPipe256w8;
     if (variant == kPersist256x192) variant = kPipe256x192;
     if (variant == kPersist128) variant = kPipe128w8;
   }
-  if (!zp_mfma) return launch_epi<false>(variant, p, epilogue, st);
+  // The small-M kernel forms the row sums next to its products; the tiled kernels start from them.
+  const bool zp_skinny = zp_mfma && variant == kSkinnyVariant;
+  if (zp_mfma && !zp_skinny && !is_pipe_variant(variant)) variant = kPipe64;   // (tiles the others cannot address)
 
-  // ---- zero points: row sums -> corrections -> a pipelined kernel that starts from them
-  if (!is_pipe_variant(variant)) variant = kPipe64;   // (small M, or tiles the others cannot address)
+  // Zero points: the row sums of the weights, and of the activations where the weights have one
+  // (wrapping int32 arithmetic on purpose, as in the kernels).
+  int32_t* corr_n = nullptr;
+  int32_t* corr_m = nullptr;
+  const int kzz = (int)((uint32_t)K_true * (uint32_t)zx * (uint32_t)zw);
+  if (zp_mfma && !zp_skinny) {
+    corr_n = reinterpret_cast<int32_t*>((int8_t*)workspace + ws_off);
+    auto sums = [&](RowsJob* job, const int8_t* use, int64_t ld, int64_t rows, int32_t* corr, int mul, int add) {
+      if (!job->src) *job = {use, ld, nullptr, nullptr, (int)rows, (int)K_true, 0, 0, 0};
+      job->corr = corr;
+      job->mul = mul;
+      job->add = add;
+    };
+    sums(&job_w, w_use, ldw_use, N, corr_n, -zx, kzz);
+    if (zw != 0) {
+      corr_m = reinterpret_cast<int32_t*>((int8_t*)corr_n + pad(N * 4));
+      sums(&job_a, a_use, lda_use, M, corr_m, -zw, 0);
+    }
+  }
+  if (job_a.rows + (int64_t)job_w.rows > 0) {
+    DQ8_REQUIRE(job_a.rows + (int64_t)job_w.rows < (1LL << 31) - 4, "dq8_qgemm: too many rows to re-lay out");
+    hipLaunchKernelGGL(prepare_rows_kernel, dim3((unsigned)ceil_div((int64_t)job_a.rows + job_w.rows, 4)),
+                       dim3(256), 0, st, job_a, job_w);
+    DQ8_HIP(hipGetLastError());
+  }
+  if (zp_skinny) {
+    p.zx = zx;
+    p.zw = zw;
+    p.kzz = kzz;
+  }
+  if (!zp_mfma || zp_skinny) return launch_epi<false>(variant, p, epilogue, st);
+
+  // ---- zero points: a pipelined kernel that starts from the corrections
   if (!pipe_ok(kVariants[variant].bm, kVariants[variant].bn, p, false)) {
     GenericParams g;
     g.A = a_use;
@@ -837,18 +916,8 @@ int qgemm_impl(int variant, const int8_t* A, int64_t lda, const int8_t* W, int64
         qgemm_generic_kernel<DQ8_EPI_REQUANT_GPU>, qgemm_generic_kernel<DQ8_EPI_DEQUANT_F32>,
         epilogue, g, M * N, st);
   }
-  int32_t* corr_n = reinterpret_cast<int32_t*>((int8_t*)workspace + ws_off);
-  int32_t* corr_m = reinterpret_cast<int32_t*>((int8_t*)corr_n + pad(N * 4));
-  // (wrapping int32 arithmetic on purpose, as in the kernels)
-  const int kzz = (int)((uint32_t)K_true * (uint32_t)zx * (uint32_t)zw);
-  hipLaunchKernelGGL(rowsum_s8_kernel, dim3((unsigned)ceil_div(N, 4)), dim3(256), 0, st, w_use,
-                     ldw_use, (int)N, (int)K, -zx, kzz, corr_n);
-  if (zw != 0)
-    hipLaunchKernelGGL(rowsum_s8_kernel, dim3((unsigned)ceil_div(M, 4)), dim3(256), 0, st, a_use,
-                       lda_use, (int)M, (int)K, -zw, 0, corr_m);
-  DQ8_HIP(hipGetLastError());
   p.corr_n = corr_n;
-  p.corr_m = zw != 0 ? corr_m : nullptr;
+  p.corr_m = corr_m;
   return launch_epi<false>(variant, p, epilogue, st);
 }
 }  // namespace
@@ -1207,12 +1276,9 @@ int qconv2d_impl(int variant, const int8_t* in, const int64_t in_sizes[4], const
   // Channel counts that are not a multiple of 16 (an RGB first layer): with scratch, input
   // and weights are rewritten with the channels zero-filled up to the next multiple; the
   // added channels contribute nothing and the MFMA kernels run on the padded tensors.
-  // (fused operators with an output the 16-byte stores cannot take run on the generic kernel,
-  // which reads the tensors as they were passed)
   const bool fused = e.table != nullptr || e.resid_kind != 0;
-  const bool fused_ok = !fused || (es == 1 ? e.vec_store16 : e.vec_store);
   const int64_t Cip = (Ci + 15) / 16 * 16;
-  if (nhwc_ohwi && Ci % 16 != 0 && variant != 0 && fused_ok && workspace != nullptr &&
+  if (nhwc_ohwi && Ci % 16 != 0 && variant != 0 && workspace != nullptr &&
       aligned(workspace, 256) &&
       workspace_bytes >= pad256(NB * H * Wd * Cip) + pad256(Co * Kh * Kw * Cip) &&
       NB * H * Wd * Cip < (1LL << 40) && Kh * Kw * Cip < (1LL << 31)) {
@@ -1231,7 +1297,7 @@ int qconv2d_impl(int variant, const int8_t* in, const int64_t in_sizes[4], const
     Ci = Cip;
     Kg = Kh * Kw * Ci;
   }
-  const bool fast_ok = nhwc_ohwi && Ci % 16 == 0 && aligned(in, 16) && aligned(w, 16) && fused_ok;
+  const bool fast_ok = nhwc_ohwi && Ci % 16 == 0 && aligned(in, 16) && aligned(w, 16);
   if (auto_pick && !fast_ok) variant = 0;
   if (variant != 0)
     DQ8_REQUIRE(fast_ok, "dq8_qconv2d: the MFMA variants need NHWC x OHWI, Ci % 16 == 0 and "
@@ -1323,7 +1389,7 @@ int qconv2d_impl(int variant, const int8_t* in, const int64_t in_sizes[4], const
     g.K = (int)Ci;
     g.epi = e;
     int v = pick_any(Mg, Co, Ci, pipe_ok(256, 256, g, false), es);
-    if (fused || e.fixedpoint) {   // the persistent forms carry neither
+    if (fused || e.fixedpoint || !(es == 1 ? e.vec_store16 : e.vec_store)) {   // (not in the persistent forms)
       if (v == kPersist256) v = kPipe256w8;
       if (v == kPersist256x192) v = kPipe256x192;
       if (v == kPersist128) v = kPipe128w8;

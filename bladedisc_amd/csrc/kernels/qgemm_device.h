@@ -87,6 +87,9 @@ struct MainParams {
   // output (m, n) starts at corr_n[n] + corr_m[m] instead of 0.
   const int32_t* corr_n;
   const int32_t* corr_m;
+  // The small-M kernel's form of the same (all zero = none): zero points, and K zx zw.
+  int zx, zw, kzz;
+  int ragged;           // (small-M kernel) rows of any alignment, any K
   // f32 activations quantized on their way into the matrix cores (qgemm_skinny_f32a_kernel):
   // A then points to floats, lda counts floats, and a row is quantized per tensor with
   // a_scale[0] (device), zero point 0, to [-128, 127] with the given rounding
@@ -265,7 +268,11 @@ __device__ __forceinline__ int requant_one(const EpiParams& p, const ColParams& 
 // twice as long as ordinary ones.
 __device__ __forceinline__ void st_through(void* p, const v4i& v) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" : : "v"(p), "v"(v) : "memory");
+  // A store of more than 8 bytes reads its data registers after it has been issued: two wait
+  // states have to pass before a vector instruction may write them again.  The compiler sees to
+  // that behind the stores it knows, not behind this one (without the s_nop the third word of the
+  // lanes 12-15, 28-31, 44-47, 60-63 now and then came out as the next fragment's).
+  asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
 #else
   *reinterpret_cast<v4i*>(p) = v;
 #endif
@@ -437,61 +444,6 @@ __device__ __forceinline__ float dequant_one_any(const EpiParams& p, const ColPa
   float r = 0.0f;
   dispatch_f32_form(p, [&](auto form) { r = dequant_one<decltype(form)::value>(p, c, acc, so_val); });
   return r;
-}
-
-// Stores the results for row m, columns n .. n+3 (n % 4 == 0).
-template <int EPI>
-__device__ __forceinline__ void store_group4(const EpiParams& p, int m, int n,
-                                             const ColParams (&c)[4], int a0, int a1,
-                                             int a2, int a3) {
-  const int acc[4] = {a0, a1, a2, a3};
-  const int64_t off = (int64_t)m * p.ldo + n;
-  const bool full = n + 3 < p.N;
-  if (EPI == DQ8_EPI_REQUANT_CPU || EPI == DQ8_EPI_REQUANT_GPU) {
-    int8_t* out = (int8_t*)p.out;
-    uint32_t w;
-    // (launches with fused operators never come here: without 16-byte aligned output rows
-    // they run on the generic kernel)
-    if (EPI == DQ8_EPI_REQUANT_CPU && p.fixedpoint) {
-      w = 0;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        w |= ((uint32_t)requant_one<EPI>(p, c[e], acc[e]) & 0xffu) << (8 * e);
-    } else {
-      w = requant_pack4<EPI>(p, c, a0, a1, a2, a3);
-    }
-    if (full && p.vec_store) {
-      *(uint32_t*)(out + off) = w;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (n + e < p.N) out[off + e] = (int8_t)(w >> (8 * e));
-    }
-  } else if (EPI == DQ8_EPI_ACC_S32) {
-    int32_t* out = (int32_t*)p.out;
-    if (full && p.vec_store) {
-      v4i w = {a0, a1, a2, a3};
-      *(v4i*)(out + off) = w;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (n + e < p.N) out[off + e] = acc[e];
-    }
-  } else {
-    float* out = (float*)p.out;
-    float f[4];
-    const float so_val = dequant_so(p);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) f[e] = dequant_one_any(p, c[e], acc[e], so_val);
-    if (full && p.vec_store) {
-      v4f w = {f[0], f[1], f[2], f[3]};
-      *(v4f*)(out + off) = w;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (n + e < p.N) out[off + e] = f[e];
-    }
-  }
 }
 
 // ----------------------------------------------------------------- main loop
@@ -695,8 +647,45 @@ __device__ __forceinline__ void fused_tail16(const EpiParams& e, const uint8_t* 
   }
 }
 
+// Stores int8 result rows that begin at any byte: `rows` rows of W bytes, of which the first
+// N - n_first exist, from LDS to out + m * ldo + n_first, by the threads t = 0 .. nt - 1.
+// `at(row, byte)`: where a byte of a row lies in LDS, 4-byte pieces of a row being contiguous.
+// Each row is written as the 4-byte words that lie inside it in memory and up to three single
+// bytes at either end.  (Byte by byte straight from the registers, 64 lanes on 32 rows, the
+// stores of 777 x 1501 took as long as the rest of the kernel.)
+template <int W, typename At>
+__device__ __forceinline__ void store_ragged_rows(int8_t* out, int64_t ldo, int rows, int m_first,
+                                                  int m_end, int n_first, int N, int t, int nt,
+                                                  At at) {
+  constexpr int LPR = W / 4;
+  const int valid = N - n_first < W ? N - n_first : W;
+  for (int u = t; u < rows * LPR; u += nt) {
+    const int row = u / LPR, i = u - row * LPR;
+    const int m = m_first + row;
+    if (m >= m_end) continue;
+    int8_t* dst = out + (int64_t)m * ldo + n_first;
+    const int s = (int)(-reinterpret_cast<intptr_t>(dst) & 3);         // bytes in front of the first whole word
+    const int o = 4 * i + s;
+    if (o + 4 <= valid) {
+      const uint32_t lo = *reinterpret_cast<const uint32_t*>(at(row, 4 * i));
+      const uint32_t hi = s ? *reinterpret_cast<const uint32_t*>(at(row, 4 * i + 4)) : 0u;
+      *reinterpret_cast<uint32_t*>(dst + o) = __builtin_amdgcn_alignbyte(hi, lo, s);
+    } else {
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        if (o + b < valid) dst[o + b] = *at(row, o + b);
+    }
+    if (i == 0) {
+#pragma unroll
+      for (int b = 0; b < 3; ++b)
+        if (b < s && b < valid) dst[b] = *at(row, b);
+    }
+  }
+}
+
 // Hook of mfma_epilogue: called once, after the int8 results have been computed into
 // registers and before the first of them is stored (the default does nothing).
+// A kernel with a hook of its own takes 16-byte aligned result rows only (its registers are full).
 // kPostOps: whether the epilogue carries the code of the fused operators (residual, table) and
 // of the fixed-point output stage; a kernel that is short of registers leaves them out and is
 // not chosen for such launches.
@@ -954,7 +943,8 @@ __device__ __forceinline__ void mfma_epilogue(v16i (&acc)[FM][FN], const EpiPara
   if (!active) return;
 
   constexpr bool kInt8Out = EPI == DQ8_EPI_REQUANT_CPU || EPI == DQ8_EPI_REQUANT_GPU;
-  if (kInt8Out && e.vec_store16) {
+  constexpr bool kRagged = __is_same(BeforeStores, NoHook);   // rows need not be 16-byte aligned
+  if constexpr (kInt8Out) {
     // int8 results straight from the registers.  Of a 32 x 32 fragment a lane holds row
     // lane % 32 and the four channel quads 8 g + 4 (lane / 32) .. + 3, g = 0 .. 3, one packed
     // word each.  Two half-wave swaps (v_permlane32_swap) trade quads between lane l and
@@ -992,6 +982,19 @@ __device__ __forceinline__ void mfma_epilogue(v16i (&acc)[FM][FN], const EpiPara
           const int c = ((wn_off + j * 32) >> 4) + (lane >> 5);
           *reinterpret_cast<v4i*>(tile + (row_wave0 + i * 32 + r) * BN + ((c ^ swz(r)) << 4)) = v;
         }
+        return;
+      }
+      if (kRagged && !e.vec_store16) {
+        // rows that begin at any byte: the fragment through a KiB of the wave's staging, 32 bytes
+        // a row
+        int8_t* stg = smem + CP_BYTES + BN * 4 + 256 + wave * 4096;
+        const int r = lane & 31;
+        *reinterpret_cast<v4i*>(stg + r * 32 + (((lane >> 5) ^ ((r >> 3) & 1)) << 4)) = v;
+        if (n_wave0 + j * 32 < e.N)
+          store_ragged_rows<32>(out, e.ldo, 32, m_wave0 + i * 32, m_end, n_wave0 + j * 32, e.N, lane, 64,
+                                [&](int row, int byte) {
+                                  return stg + row * 32 + ((((byte >> 4) ^ (row >> 3)) & 1) << 4) + (byte & 15);
+                                });
         return;
       }
       const int n = n_wave0 + j * 32 + 16 * (lane >> 5);
@@ -1154,7 +1157,15 @@ __device__ __forceinline__ void mfma_epilogue(v16i (&acc)[FM][FN], const EpiPara
           for (int i = 0; i < FM; ++i) store_frag(held[kHook ? i : 0][kHook ? j : 0], i, j);
       }
     }
-    if constexpr (BLOCK_STAGE && kWavePrivate) {
+    if (BLOCK_STAGE && kWavePrivate && !e.vec_store16) {
+      before_stores();
+      const int8_t* mine = tile + wave * (FM * 32 * 64);
+      if (n_wave0 < e.N)
+        store_ragged_rows<64>(out, e.ldo, FM * 32, m_wave0, m_end, n_wave0, e.N, lane, 64,
+                              [&](int row, int byte) {
+                                return mine + row * 64 + (((byte >> 4) ^ ((row >> 2) & 3)) << 4) + (byte & 15);
+                              });
+    } else if constexpr (BLOCK_STAGE && kWavePrivate) {
       before_stores();
       const int8_t* mine = tile + wave * (FM * 32 * 64);
 #pragma unroll
@@ -1180,6 +1191,12 @@ __device__ __forceinline__ void mfma_epilogue(v16i (&acc)[FM][FN], const EpiPara
       __syncthreads();
       before_stores();
       const int m_blk0 = m_wave0 - row_wave0;
+      if (!e.vec_store16) {
+        store_ragged_rows<BN>(out, e.ldo, kBM, m_blk0, m_end, n_blk0, e.N, tid, NT, [&](int row, int byte) {
+          return tile + row * BN + (((byte >> 4) ^ swz(row & 31)) << 4) + (byte & 15);
+        });
+        return;
+      }
 #pragma unroll
       for (int k = 0; k < kBM * kChunks / NT; ++k) {
         const int u = tid + k * NT;
@@ -1204,7 +1221,7 @@ __device__ __forceinline__ void mfma_epilogue(v16i (&acc)[FM][FN], const EpiPara
   }
   before_stores();
 
-  if (!kInt8Out && e.vec_store) {
+  if constexpr (!kInt8Out) {
     // int32 / f32 results: one 32 x 32 fragment (4 KiB) at a time through a per-wave LDS
     // tile, 128-byte rows with the 16-byte chunks swizzled by the row, then out as full
     // 128-byte row segments (8 lanes per row) instead of 32-byte pieces of 32 rows.
@@ -1234,6 +1251,22 @@ __device__ __forceinline__ void mfma_epilogue(v16i (&acc)[FM][FN], const EpiPara
               w[q] = __float_as_int(dequant_one<FORM>(e, c[q], acc[i][j][4 * g + q], so_val));
           }
           *reinterpret_cast<v4i*>(stage + r * 128 + ((chunk ^ (r & 7)) << 4)) = w;
+        }
+        if (kRagged && !e.vec_store) {
+          // (rows that are not 16-byte aligned: a lane per element, two 128-byte row segments
+          // per instruction)
+#pragma unroll 4
+          for (int it = 0; it < 16; ++it) {
+            const int row = it * 2 + (lane >> 5), col = lane & 31;
+            const int m = m_wave0 + i * 32 + row, n = n_wave0 + j * 32 + col;
+            int v = *reinterpret_cast<const int*>(stage + row * 128 + (((col >> 2) ^ (row & 7)) << 4) + (col & 3) * 4);
+            if (m < m_end && n < e.N) {
+              if (BeforeStores::kPostOps && EPI == DQ8_EPI_DEQUANT_F32 && e.resid_kind)
+                v = __float_as_int(finish_f32(e, __int_as_float(v), m, n));
+              static_cast<int32_t*>(e.out)[(int64_t)m * e.ldo + n] = v;
+            }
+          }
+          continue;
         }
 #pragma unroll
         for (int it = 0; it < 4; ++it) {
@@ -1282,30 +1315,6 @@ __device__ __forceinline__ void mfma_epilogue(v16i (&acc)[FM][FN], const EpiPara
       store_all(IntC<kF32Plain>());
     return;
   }
-
-  // direct stores: 4 consecutive channels of one row per accumulator quad
-  static_for<FN>([&](auto jc) {
-    constexpr int j = decltype(jc)::value;
-    static_for<4>([&](auto gc) {
-      constexpr int g = decltype(gc)::value;
-      const int cl = wn_off + j * 32 + 8 * g + 4 * (lane >> 5);
-      const int n = n_blk0 + cl;
-      if (n >= e.N) return;
-      const v4f p01 = *reinterpret_cast<const v4f*>(&cp[cl]);
-      const v4f p23 = *reinterpret_cast<const v4f*>(&cp[cl + 2]);
-      v4i sh = {0, 0, 0, 0};
-      if (fixedpoint) sh = *reinterpret_cast<const v4i*>(&cps[cl]);
-      const ColParams c[4] = {{p01[0], p01[1], sh[0]}, {p01[2], p01[3], sh[1]},
-                              {p23[0], p23[1], sh[2]}, {p23[2], p23[3], sh[3]}};
-      static_for<FM>([&](auto ic) {
-        constexpr int i = decltype(ic)::value;
-        const int m = m_wave0 + i * 32 + (lane & 31);
-        if (m < m_end)
-          store_group4<EPI>(e, m, n, c, acc[i][j][4 * g + 0], acc[i][j][4 * g + 1],
-                            acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
-      });
-    });
-  });
 }
 
 }  // namespace dq8

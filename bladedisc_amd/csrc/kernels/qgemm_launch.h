@@ -154,7 +154,10 @@ template <int NW, int MT, int EPI, int U = 4>
 int launch_skinny_t(const MainParams& p, hipStream_t st) {
   const dim3 grid((unsigned)ceil_div(p.N, 16), (unsigned)ceil_div(p.M, 16 * MT));
   DQ8_REQUIRE(grid.y <= 65535, "small-M qgemm: M too large for this variant");
-  hipLaunchKernelGGL((qgemm_skinny_kernel<NW, MT, EPI, U>), grid, dim3(NW * 64), 0, st, p);
+  const bool zp = p.zx != 0 || p.zw != 0;
+  auto kern = p.ragged ? (zp ? qgemm_skinny_kernel<NW, MT, EPI, U, true, true> : qgemm_skinny_kernel<NW, MT, EPI, U, false, true>)
+                       : (zp ? qgemm_skinny_kernel<NW, MT, EPI, U, true, false> : qgemm_skinny_kernel<NW, MT, EPI, U, false, false>);
+  hipLaunchKernelGGL(kern, grid, dim3(NW * 64), 0, st, p);
   return check_hip(hipGetLastError(), "qgemm_skinny launch");
 }
 
@@ -173,7 +176,7 @@ int launch_skinny(const MainParams& p, hipStream_t st) {
   // one or two rows against rows of at least 2048 of k (two steps of a wave): the
   // row-streaming kernel (M = 1, 3072 -> 768: 3.1 against 4.0 us; 4096^2: 3.8 against 5.0;
   // 8192^2: 12.7 against 14.2 us, 5.3 TB/s; at 768 of k, and from three rows on, it is slower)
-  if (p.M <= 2 && p.K >= 2048 && (int64_t)2 * p.K <= 64 * 1024) {
+  if (p.M <= 2 && p.K >= 2048 && (int64_t)2 * p.K <= 64 * 1024 && p.zx == 0 && p.zw == 0 && !p.ragged) {
     const bool deep8 = p.K > 4096;
     if (p.M == 1) return deep8 ? launch_gemv_t<1, 8, EPI>(p, st) : launch_gemv_t<1, 4, EPI>(p, st);
     return deep8 ? launch_gemv_t<2, 8, EPI>(p, st) : launch_gemv_t<2, 4, EPI>(p, st);
@@ -251,9 +254,17 @@ int launch_variant(int variant, MainParams& p, hipStream_t st) {
   }
   if constexpr (!CONV) {   // GEMM only: the small-M kernel and the persistent forms
     if (variant == kSkinnyVariant) return launch_skinny<EPI>(p, st);
-    if (variant == kPersist256) return launch_persist<256, 256, 2, 4, false, EPI>(p, 1, st);
     if (variant == kPersist128) return launch_persist<128, 128, 2, 4, false, EPI>(p, 2, st);
-    if (variant == kPersist256x192) return launch_persist<256, 192, 4, 2, false, EPI>(p, 1, st);
+    // (the 256-row persistent forms write int8; 4-byte results take the one-tile kernels)
+    constexpr bool kInt8 = EPI == DQ8_EPI_REQUANT_CPU || EPI == DQ8_EPI_REQUANT_GPU;
+    if (variant == kPersist256) {
+      if constexpr (kInt8) return launch_persist<256, 256, 2, 4, false, EPI>(p, 1, st);
+      else return launch_pipe<256, 256, 2, 4, 1, false, EPI>(p, st);
+    }
+    if (variant == kPersist256x192) {
+      if constexpr (kInt8) return launch_persist<256, 192, 4, 2, false, EPI>(p, 1, st);
+      else return launch_pipe<256, 192, 4, 2, 1, false, EPI>(p, st);
+    }
   }
   return fail("unknown or unsupported qgemm variant for this operation");
 }

@@ -9,7 +9,8 @@
 //  * operands go straight from global memory into v_mfma_i32_16x16x64_i8 operand
 //    layout (lane l: row l % 16, 16 k-bytes of group l / 16); W is the row operand, so
 //    the 4 accumulator registers of a lane are 4 consecutive output channels.
-// Needs K % 16 == 0 and 16-byte aligned, k-contiguous rows, like the other MFMA kernels.
+// The row-streaming and f32-activation kernels need K % 16 == 0 and 16-byte aligned rows; the
+// small-M kernel takes k-contiguous rows of any length and alignment (RAGGED).
 #ifndef DQ8_QGEMM_SKINNY_H_
 #define DQ8_QGEMM_SKINNY_H_
 
@@ -19,7 +20,24 @@
 namespace dq8 {
 
 // U: k-steps a wave has in flight
-template <int NW, int MT, int EPI, int U = 4>
+// ZP: sum (a - zx)(w - zw) = sum a w - zx sum w - zw sum a + K zx zw, the two sums by an MFMA each
+// with an operand of ones next to the products -- they come out in the products' own layout, the
+// matrix pipe has room, and the launch of a row-sum kernel in front (2.4 us, as long as the whole
+// of this kernel) is gone: M = 16, 768 -> 3072 with a zero point 7.4 -> 3.5 us.
+// RAGGED: rows of any alignment, K not a multiple of 16.  The operands pass through registers here,
+// so that an unaligned row is an unaligned load; the chunk that holds the end of a row is read byte
+// by byte by the lanes that have it.  (Copied to aligned rows first, as the tiled kernels need it,
+// the copy's launch and the trip through memory were 4-6 us in front of a kernel of 3.)
+typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
+__device__ __forceinline__ v4i row_tail(const int8_t* p, int bytes) {   // 0 < bytes < 16
+  uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int b = 0; b < 15; ++b)
+    if (b < bytes) w[b >> 2] |= (uint32_t)(uint8_t)p[b] << (8 * (b & 3));
+  return (v4i){(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+}
+
+template <int NW, int MT, int EPI, int U = 4, bool ZP = false, bool RAGGED = false>
 __global__ void __launch_bounds__(NW * 64) qgemm_skinny_kernel(const MainParams p) {
   __shared__ int red[NW][MT][256];
   // per wave: one k-step of weights and of each row tile ([16 rows][64 k], 1 KiB each) on its
@@ -52,6 +70,10 @@ __global__ void __launch_bounds__(NW * 64) qgemm_skinny_kernel(const MainParams 
   for (int t = 0; t < MT; ++t) acc[t] = (v4i){0, 0, 0, 0};
 
   const v4i zero = {0, 0, 0, 0};
+  const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
+  v4i sum_w = zero, sum_a[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) sum_a[t] = zero;
   for (int ks0 = wave; ks0 < KS; ks0 += NW * U) {
     // unconditional loads (a branch around each would serialise them): a chunk past K
     // (K % 16 == 0: entirely inside or outside) or of a row past M / N is read from the
@@ -61,11 +83,27 @@ __global__ void __launch_bounds__(NW * 64) qgemm_skinny_kernel(const MainParams 
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int k = (ks0 + u * NW) * 64;
-      in[u] = k + lchunk * 16 < p.K;
-      const int kk = in[u] ? k : 0;
-      wf[u] = *(const v4i*)(wp + kk);
+      if constexpr (RAGGED) {
+        in[u] = k + lchunk * 16 + 16 <= p.K;
+        // (a chunk that is not whole: from the start of the row, which K >= 80 makes whole)
+        const int kk = in[u] ? k : 0;
+        wf[u] = *(const v4i_any*)(wp + kk);
 #pragma unroll
-      for (int t = 0; t < MT; ++t) af[u][t] = *(const v4i*)(ap[t] + kk);
+        for (int t = 0; t < MT; ++t) af[u][t] = *(const v4i_any*)(ap[t] + kk);
+        const int tail = p.K - k - lchunk * 16;
+        if (tail > 0 && tail < 16) {
+          wf[u] = row_tail(wp + k, tail);
+#pragma unroll
+          for (int t = 0; t < MT; ++t) af[u][t] = row_tail(ap[t] + k, tail);
+          in[u] = true;
+        }
+      } else {
+        in[u] = k + lchunk * 16 < p.K;
+        const int kk = in[u] ? k : 0;
+        wf[u] = *(const v4i*)(wp + kk);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) af[u][t] = *(const v4i*)(ap[t] + kk);
+      }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -76,10 +114,12 @@ __global__ void __launch_bounds__(NW * 64) qgemm_skinny_kernel(const MainParams 
       for (int t = 0; t < MT; ++t)
         *(v4i*)&stage[wave][1 + t][lane * 4] = (in[u] && a_ok[t]) ? af[u][t] : zero;
       const v4i wfrag = *(const v4i*)&stage[wave][0][r * 16 + g * 4];
+      if (ZP) sum_w = __builtin_amdgcn_mfma_i32_16x16x64_i8(wfrag, ones, sum_w, 0, 0, 0);
 #pragma unroll
       for (int t = 0; t < MT; ++t) {
         const v4i afrag = *(const v4i*)&stage[wave][1 + t][r * 16 + g * 4];
         acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wfrag, afrag, acc[t], 0, 0, 0);
+        if (ZP) sum_a[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, afrag, sum_a[t], 0, 0, 0);
       }
     }
   }
@@ -88,14 +128,18 @@ __global__ void __launch_bounds__(NW * 64) qgemm_skinny_kernel(const MainParams 
 #pragma unroll
   for (int t = 0; t < MT; ++t)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) red[wave][t][r * 16 + 4 * g + v] = acc[t][v];
+    for (int v = 0; v < 4; ++v) {
+      // (wrapping, like the sums themselves)
+      const unsigned corr = ZP ? (unsigned)p.zx * (unsigned)sum_w[v] + (unsigned)p.zw * (unsigned)sum_a[t][v] : 0u;
+      red[wave][t][r * 16 + 4 * g + v] = (int)((unsigned)acc[t][v] - corr);
+    }
   __syncthreads();
 
   for (int idx = threadIdx.x; idx < MT * 256; idx += NW * 64) {
     const int t = idx >> 8, e = idx & 255;
     const int m = m0 + t * 16 + (e >> 4), n = n0 + (e & 15);
     if (m >= p.M || n >= p.N) continue;
-    int sum = 0;
+    int sum = ZP ? p.kzz : 0;
 #pragma unroll
     for (int w = 0; w < NW; ++w) sum += red[w][t][e];
     const EpiParams& ep = p.epi;

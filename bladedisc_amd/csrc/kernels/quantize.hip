@@ -6,13 +6,15 @@
 // division is a true IEEE division, so this file is compiled with
 // -ffp-contract=off.
 //
-// Three access patterns, all without per-element integer division:
-//   per tensor            1-D grid-stride over float4 / packed-4 elements
+// Access patterns:
+//   per tensor            1-D sweep over float4 / packed-4 elements
 //   per channel, inner==1 (channel is the last axis) 2-D tiles [rows, 4*threads];
 //                         each thread keeps its four scales / zero points in
 //                         registers while it walks down the rows
 //   per channel, inner%4==0 one (outer, channel) row per blockIdx.y
-// Anything else (odd sizes, unaligned pointers) takes the scalar kernel.
+// for f32 and the 8-bit types at sizes that are multiples of four; every other type, size and
+// alignment runs the two general kernels (quantize_lastaxis_any, quantize_flat and their
+// dequantize forms), four elements per thread as well.
 #include <algorithm>
 
 #include <cstdlib>
@@ -59,10 +61,16 @@ __device__ __forceinline__ uint32_t quant4_by_constants(const float4& v, const f
 template <int ROUND>
 __global__ void __launch_bounds__(kThreads)
 quantize_tensor_v4(const float4* __restrict__ x, uint32_t* __restrict__ out,
-                   int64_t n4, const float* __restrict__ scale,
+                   int64_t n, const float* __restrict__ scale,
                    const int32_t* __restrict__ zp, float lo, float hi) {
+  const int64_t n4 = n >> 2;
   const int64_t stride = (int64_t)gridDim.x * kThreads;
   int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {        // the elements behind the last four
+    const int64_t e = 4 * n4 + threadIdx.x;
+    reinterpret_cast<uint8_t*>(out)[e] = (uint8_t)quant_one<ROUND>(
+        reinterpret_cast<const float*>(x)[e], scale[0], (float)zp[0], lo, hi);
+  }
   if (i >= n4) return;
   // The data load goes out first: a wave has one load to make, and behind the scalar loads of
   // the parameters and the reciprocal it would start a cache miss later.
@@ -109,10 +117,16 @@ __device__ __forceinline__ float4 dequant_word4(uint32_t w, const int4& z, const
 template <bool SIGNED>
 __global__ void __launch_bounds__(kThreads)
 dequantize_tensor_v4x2(const uint32_t* __restrict__ q, float4* __restrict__ out,
-                       int64_t n4, const float* __restrict__ scale,
+                       int64_t n, const float* __restrict__ scale,
                        const int32_t* __restrict__ zp) {
   const float s = scale[0];
   const int z = zp[0];
+  const int64_t n4 = n >> 2;
+  if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {        // the elements behind the last word
+    const int64_t e = 4 * n4 + threadIdx.x;
+    const uint8_t b = reinterpret_cast<const uint8_t*>(q)[e];
+    reinterpret_cast<float*>(out)[e] = (float)((SIGNED ? (int)(int8_t)b : (int)b) - z) * s;
+  }
   const int64_t stride = (int64_t)gridDim.x * (2 * kThreads);
   for (int64_t i = (int64_t)blockIdx.x * (2 * kThreads) + threadIdx.x; i < n4; i += stride) {
     const bool two = i + kThreads < n4;
@@ -273,11 +287,17 @@ __device__ __forceinline__ float4 fake4_by_constant(const float4& v, float s, fl
 
 template <int ROUND>
 __global__ void __launch_bounds__(kThreads)
-fake_quant_tensor_v4(const float4* __restrict__ x, float4* __restrict__ out, int64_t n4,
+fake_quant_tensor_v4(const float4* __restrict__ x, float4* __restrict__ out, int64_t n,
                      const float* __restrict__ scale, const int32_t* __restrict__ zp, float lo,
                      float hi) {
+  const int64_t n4 = n >> 2;
   const int64_t stride = (int64_t)gridDim.x * kThreads;
   int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {        // the elements behind the last four
+    const int64_t e = 4 * n4 + threadIdx.x;
+    reinterpret_cast<float*>(out)[e] =
+        fake_one<ROUND>(reinterpret_cast<const float*>(x)[e], scale[0], zp[0], lo, hi);
+  }
   if (i >= n4) return;
   float4 v = x[i];                        // (the data load first, as in quantize_tensor_v4)
   __builtin_amdgcn_sched_barrier(0);
@@ -344,49 +364,9 @@ fake_quant_rows_v4(const float4* __restrict__ x, float4* __restrict__ out, unsig
                              fake_one<ROUND>(v.z, s, z, lo, hi), fake_one<ROUND>(v.w, s, z, lo, hi)));
 }
 
-template <int ROUND>
-__global__ void __launch_bounds__(kThreads)
-fake_quant_scalar(const float* __restrict__ x, float* __restrict__ out, int64_t begin, int64_t n,
-                  int64_t nch, int64_t inner, int per_channel, const float* __restrict__ scale,
-                  const int32_t* __restrict__ zp, float lo, float hi) {
-  for (int64_t i = begin + (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * kThreads) {
-    const int64_t c = per_channel ? (i / inner) % nch : 0;
-    out[i] = fake_one<ROUND>(x[i], scale[c], zp[c], lo, hi);
-  }
-}
-
-// ------------------------------------------------------------ scalar fallback
-template <int ROUND>
-__global__ void __launch_bounds__(kThreads)
-quantize_scalar(const float* __restrict__ x, uint8_t* __restrict__ out,
-                int64_t begin, int64_t n, int64_t nch, int64_t inner,
-                int per_channel, const float* __restrict__ scale,
-                const int32_t* __restrict__ zp, float lo, float hi) {
-  for (int64_t i = begin + (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * kThreads) {
-    int64_t c = per_channel ? (i / inner) % nch : 0;
-    out[i] = (uint8_t)(quant_one<ROUND>(x[i], scale[c], (float)zp[c], lo, hi) & 0xff);
-  }
-}
-
-__global__ void __launch_bounds__(kThreads)
-dequantize_scalar(const uint8_t* __restrict__ q, float* __restrict__ out,
-                  int64_t begin, int64_t n, int64_t nch, int64_t inner,
-                  int per_channel, const float* __restrict__ scale,
-                  const int32_t* __restrict__ zp, int is_signed) {
-  for (int64_t i = begin + (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * kThreads) {
-    int64_t c = per_channel ? (i / inner) % nch : 0;
-    int v = is_signed ? (int)(int8_t)q[i] : (int)q[i];
-    out[i] = (float)(v - zp[c]) * scale[c];
-  }
-}
-
-// ------------------------------------------------- wide outputs, f16 inputs
-// 16- and 32-bit quantized types and half-precision inputs: one element per thread, the same
-// separately rounded f32 steps.  The conversion of the clamped f32 value saturates: the f32
-// images of 2^31 - 1 and 2^32 - 1 are 2^31 and 2^32, one past the integer range.
+// ------------------------------------------------- any type, size and alignment
+// The conversion of the clamped f32 value saturates: the f32 images of 2^31 - 1 and 2^32 - 1 are
+// 2^31 and 2^32, one past the integer range.
 template <typename QT>
 __device__ __forceinline__ QT convert_clamped(float t) {
   return (QT)(int)t;
@@ -404,66 +384,263 @@ __device__ __forceinline__ uint16_t convert_clamped<uint16_t>(float t) {
   return (uint16_t)(unsigned)t;
 }
 
-template <typename XT, typename QT, int ROUND>
-__global__ void __launch_bounds__(kThreads)
-quantize_wide(const XT* __restrict__ x, QT* __restrict__ out, int64_t n, int64_t nch,
-              int64_t inner, int per_channel, const float* __restrict__ scale,
-              const int32_t* __restrict__ zp, float lo, float hi) {
-  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * kThreads) {
-    const int64_t c = per_channel ? (i / inner) % nch : 0;
-    const float t0 = (float)x[i] / scale[c];
-    const float t1 = t0 + (float)zp[c];
-    const float t2 = ROUND == DQ8_ROUND_HALF_TO_EVEN ? rintf(t1) : roundf(t1);
-    out[i] = convert_clamped<QT>(fminf(fmaxf(t2, lo), hi));
+// Four elements of a type as one memory operation.
+template <typename T>
+struct alignas(4 * sizeof(T)) Four {
+  T v[4];
+};
+template <typename T>
+__device__ __forceinline__ void st_stream_four(T* p, const Four<T>& f) {
+  if constexpr (sizeof(T) == 1) {
+    dq8::st_stream(reinterpret_cast<uint32_t*>(p), __builtin_bit_cast(uint32_t, f));
+  } else if constexpr (sizeof(T) == 2) {
+    __builtin_nontemporal_store(__builtin_bit_cast(uint64_t, f), reinterpret_cast<uint64_t*>(p));
+  } else {
+    dq8::st_stream(reinterpret_cast<float4*>(p), __builtin_bit_cast(float4, f));
   }
 }
 
-template <typename QT>
-__global__ void __launch_bounds__(kThreads)
-dequantize_wide(const QT* __restrict__ q, float* __restrict__ out, int64_t n, int64_t nch,
-                int64_t inner, int per_channel, const float* __restrict__ scale,
-                const int32_t* __restrict__ zp) {
-  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * kThreads) {
-    const int64_t c = per_channel ? (i / inner) % nch : 0;
-    // the input is converted to the zero point's type (i32) before the subtraction
-    out[i] = (float)((int32_t)q[i] - zp[c]) * scale[c];
+// What the general kernels do to one element: XT -> QT quantizes, QT -> float dequantizes,
+// float -> float fake-quantizes.
+template <int ROUND>
+struct Quantize {
+  float lo, hi;
+  template <typename XT, typename QT>
+  __device__ __forceinline__ void operator()(const XT& x, float s, int z, QT& q) const {
+    const float t1 = (float)x / s + (float)z;
+    const float t2 = ROUND == DQ8_ROUND_HALF_TO_EVEN ? rintf(t1) : roundf(t1);
+    q = convert_clamped<QT>(fminf(fmaxf(t2, lo), hi));
   }
+  // four at a time, divided through the reciprocals where the divisors allow it (the quotients'
+  // bits are those of the division, see div4_by_constant)
+  template <typename XT, typename QT>
+  __device__ __forceinline__ void four(const Four<XT>& x, const float4& s, const float4& y, bool fast,
+                                       const int4& z, Four<QT>& q) const {
+    if (!fast) {
+      (*this)(x.v[0], s.x, z.x, q.v[0]);
+      (*this)(x.v[1], s.y, z.y, q.v[1]);
+      (*this)(x.v[2], s.z, z.z, q.v[2]);
+      (*this)(x.v[3], s.w, z.w, q.v[3]);
+      return;
+    }
+    const float4 d = div4_by_constants(
+        make_float4((float)x.v[0], (float)x.v[1], (float)x.v[2], (float)x.v[3]), s, y);
+    const float t[4] = {d.x + (float)z.x, d.y + (float)z.y, d.z + (float)z.z, d.w + (float)z.w};
+    if constexpr (sizeof(QT) == 1 && ROUND == DQ8_ROUND_HALF_TO_EVEN) {
+      q = __builtin_bit_cast(Four<QT>, quant4_pack_rne(make_float4(t[0], t[1], t[2], t[3]), lo, hi));
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float r = ROUND == DQ8_ROUND_HALF_TO_EVEN ? rintf(t[i]) : roundf(t[i]);
+        q.v[i] = convert_clamped<QT>(fminf(fmaxf(r, lo), hi));
+      }
+    }
+  }
+};
+struct Dequantize {
+  template <typename QT>
+  __device__ __forceinline__ void operator()(const QT& q, float s, int z, float& y) const {
+    // (the input is converted to the zero point's type, i32, before the subtraction)
+    y = (float)((int32_t)q - z) * s;
+  }
+  template <typename QT>
+  __device__ __forceinline__ void four(const Four<QT>& q, const float4& s, const float4&, bool,
+                                       const int4& z, Four<float>& y) const {
+    (*this)(q.v[0], s.x, z.x, y.v[0]);
+    (*this)(q.v[1], s.y, z.y, y.v[1]);
+    (*this)(q.v[2], s.z, z.z, y.v[2]);
+    (*this)(q.v[3], s.w, z.w, y.v[3]);
+  }
+};
+template <int ROUND>
+struct FakeQuantize {
+  float lo, hi;
+  __device__ __forceinline__ void operator()(float x, float s, int z, float& y) const {
+    y = fake_one<ROUND>(x, s, z, lo, hi);
+  }
+  __device__ __forceinline__ void four(const Four<float>& x, const float4& s, const float4&, bool,
+                                       const int4& z, Four<float>& y) const {
+    (*this)(x.v[0], s.x, z.x, y.v[0]);
+    (*this)(x.v[1], s.y, z.y, y.v[1]);
+    (*this)(x.v[2], s.z, z.z, y.v[2]);
+    (*this)(x.v[3], s.w, z.w, y.v[3]);
+  }
+};
+
+__device__ __forceinline__ bool divisors_in_fast_range(const float4& s) {
+  return divisor_in_fast_range(s.x) && divisor_in_fast_range(s.y) && divisor_in_fast_range(s.z) &&
+         divisor_in_fast_range(s.w);
+}
+
+// Per channel on the last axis, any number of channels.  Four rows of nch elements are nch groups
+// of four, and group u of every such block of rows belongs to the same four channels (4 u mod nch
+// and the next three, cyclically), whatever nch: the threads of the [rows, channels] pattern, with
+// their scales and zero points in registers, on a tensor whose rows start anywhere.  1000 x 3073
+// to uint8: 8.2 us an element at a time with two 64-bit divisions each, 5.2 this way.
+template <typename IN, typename OUT, typename OP>
+__global__ void __launch_bounds__(kThreads)
+lastaxis_any(const IN* __restrict__ in, OUT* __restrict__ out, int64_t n, int nch, int blocks4,
+             int per_thread_block, const float* __restrict__ scale, const int32_t* __restrict__ zp,
+             const OP op) {
+  const int u = blockIdx.x * blockDim.x + threadIdx.x;
+  if (u >= nch) return;
+  const int64_t n4 = n >> 2;
+  const int step = blockDim.y;
+  const int r_end = min((int)(blockIdx.y + 1) * per_thread_block, blocks4);
+  int r = blockIdx.y * per_thread_block + threadIdx.y;
+  // two groups in flight per thread, the first two ahead of the parameters
+  Four<IN> x[2];
+  auto fetch = [&](int r0) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int64_t g = (int64_t)(r0 + k * step) * nch + u;
+      if (r0 + k * step < r_end && g < n4) x[k] = *reinterpret_cast<const Four<IN>*>(in + 4 * g);
+    }
+  };
+  fetch(r);
+  int c[4];
+  c[0] = 4 * u;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) c[0] -= c[0] >= nch ? nch : 0;
+#pragma unroll
+  for (int i = 1; i < 4; ++i) c[i] = c[i - 1] + 1 == nch ? 0 : c[i - 1] + 1;
+  const float4 s = make_float4(scale[c[0]], scale[c[1]], scale[c[2]], scale[c[3]]);
+  const int4 z = make_int4(zp[c[0]], zp[c[1]], zp[c[2]], zp[c[3]]);
+  const float4 y = make_float4(1.0f / s.x, 1.0f / s.y, 1.0f / s.z, 1.0f / s.w);
+  const bool fast = divisors_in_fast_range(s);
+  for (; r < r_end; r += 2 * step) {
+    Four<IN> v[2] = {x[0], x[1]};
+    fetch(r + 2 * step);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int64_t g = (int64_t)(r + k * step) * nch + u;
+      if (r + k * step >= r_end) break;
+      if (g < n4) {
+        Four<OUT> o;
+        op.four(v[k], s, y, fast, z, o);
+        st_stream_four(out + 4 * g, o);
+      } else if (g == n4) {                 // the up to three elements behind the last four
+        const float st[3] = {s.x, s.y, s.z};
+        const int zt[3] = {z.x, z.y, z.z};
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+          if (4 * n4 + i < n) op(in[4 * n4 + i], st[i], zt[i], out[4 * n4 + i]);
+      }
+    }
+  }
+}
+
+// Any axis (or per tensor): four consecutive elements per thread, whose channels follow from the
+// first one's by counting on.  VEC: the four are one memory operation.  INDEX: wide enough for n.
+template <typename IN, typename OUT, typename OP, bool VEC, typename INDEX>
+__global__ void __launch_bounds__(kThreads)
+flat_any(const IN* __restrict__ in, OUT* __restrict__ out, int64_t n, int64_t nch, int64_t inner,
+         int per_channel, const float* __restrict__ scale, const int32_t* __restrict__ zp, const OP op) {
+  const int64_t first = 4 * ((int64_t)blockIdx.x * kThreads + threadIdx.x);
+  if (first >= n) return;
+  const int left = n - first < 4 ? (int)(n - first) : 4;
+  Four<IN> x;
+  if (VEC && left == 4) {
+    x = *reinterpret_cast<const Four<IN>*>(in + first);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i < left) x.v[i] = in[first + i];
+  }
+  // (the parameters after the data load has been issued)
+  float sv[4];
+  int zv[4];
+  if (!per_channel) {
+    sv[0] = sv[1] = sv[2] = sv[3] = scale[0];
+    zv[0] = zv[1] = zv[2] = zv[3] = zp[0];
+  } else {
+    const INDEX row = (INDEX)first / (INDEX)inner;
+    INDEX at = (INDEX)first - row * (INDEX)inner, c = row % (INDEX)nch;
+    sv[0] = scale[c];
+    zv[0] = zp[c];
+#pragma unroll
+    for (int i = 1; i < 4; ++i) {
+      sv[i] = sv[i - 1];
+      zv[i] = zv[i - 1];
+      if (++at == (INDEX)inner && i < left) {
+        at = 0;
+        c = c + 1 == (INDEX)nch ? 0 : c + 1;
+        sv[i] = scale[c];
+        zv[i] = zp[c];
+      }
+    }
+  }
+  if (VEC && left == 4) {
+    const float4 s = make_float4(sv[0], sv[1], sv[2], sv[3]);
+    Four<OUT> o;
+    op.four(x, s, make_float4(1.0f / s.x, 1.0f / s.y, 1.0f / s.z, 1.0f / s.w), divisors_in_fast_range(s),
+            make_int4(zv[0], zv[1], zv[2], zv[3]), o);
+    st_stream_four(out + first, o);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i < left) op(x.v[i], sv[i], zv[i], out[first + i]);
+  }
+}
+
+template <typename IN, typename OUT, typename OP>
+int launch_any(const IN* in, OUT* out, int64_t outer, int64_t nch, int64_t inner, bool per_channel,
+               const float* scale, const int32_t* zp, const OP& op, hipStream_t st) {
+  const int64_t n = outer * nch * inner;
+  const bool vec = dq8::aligned(in, sizeof(Four<IN>)) && dq8::aligned(out, sizeof(Four<OUT>));
+  if (vec && per_channel && inner == 1 && outer >= 4 && nch < (1 << 28)) {
+    const int64_t blocks4 = dq8::ceil_div(outer, 4);          // four rows each, the last perhaps fewer
+    int bx = kThreads;
+    if (nch < kThreads)
+      for (bx = 1; bx < nch;) bx *= 2;
+    const int by = kThreads / bx;
+    // two groups of four per thread at least, about 64 Ki workgroups at most
+    const int64_t gx = dq8::ceil_div(nch, bx);
+    int64_t per = std::max<int64_t>(2 * by, dq8::ceil_div(blocks4 * gx, 65536));
+    per = dq8::ceil_div(per, by) * by;
+    if (dq8::ceil_div(blocks4, per) > 65535) per = dq8::ceil_div(dq8::ceil_div(blocks4, 65535), by) * by;
+    if (blocks4 < (1LL << 30)) {
+      hipLaunchKernelGGL((lastaxis_any<IN, OUT, OP>), dim3((unsigned)gx, (unsigned)dq8::ceil_div(blocks4, per)),
+                         dim3(bx, by), 0, st, in, out, n, (int)nch, (int)blocks4, (int)per, scale, zp, op);
+      return dq8::check_hip(hipGetLastError(), "quantize / dequantize launch");
+    }
+  }
+  const int64_t groups = dq8::ceil_div(n, 4 * (int64_t)kThreads);
+  DQ8_REQUIRE(groups < (1LL << 31), "quantize / dequantize: tensor too large for one launch");
+  auto kern = n < (1LL << 32) - 4 ? (vec ? flat_any<IN, OUT, OP, true, uint32_t> : flat_any<IN, OUT, OP, false, uint32_t>)
+                                  : (vec ? flat_any<IN, OUT, OP, true, uint64_t> : flat_any<IN, OUT, OP, false, uint64_t>);
+  hipLaunchKernelGGL(kern, dim3((unsigned)groups), dim3(kThreads), 0, st, in, out, n, nch, inner,
+                     (int)per_channel, scale, zp, op);
+  return dq8::check_hip(hipGetLastError(), "quantize / dequantize launch");
 }
 
 template <typename XT, typename QT>
-void launch_quantize_wide(bool rne, const void* x, void* out, int64_t n, int64_t nch,
-                          int64_t inner, int per_channel, const float* scale, const int32_t* zp,
-                          float lo, float hi, hipStream_t st) {
-  const dim3 grid(grid_for(n, 1)), block(kThreads);
-  if (rne)
-    hipLaunchKernelGGL((quantize_wide<XT, QT, DQ8_ROUND_HALF_TO_EVEN>), grid, block, 0, st,
-                       (const XT*)x, (QT*)out, n, nch, inner, per_channel, scale, zp, lo, hi);
-  else
-    hipLaunchKernelGGL((quantize_wide<XT, QT, DQ8_ROUND_HALF_AWAY_FROM_ZERO>), grid, block, 0, st,
-                       (const XT*)x, (QT*)out, n, nch, inner, per_channel, scale, zp, lo, hi);
+int launch_quantize_any(bool rne, const XT* x, void* out, int64_t outer, int64_t nch, int64_t inner,
+                        bool per_channel, const float* scale, const int32_t* zp, float lo, float hi,
+                        hipStream_t st) {
+  return rne ? launch_any(x, static_cast<QT*>(out), outer, nch, inner, per_channel, scale, zp,
+                          Quantize<DQ8_ROUND_HALF_TO_EVEN>{lo, hi}, st)
+             : launch_any(x, static_cast<QT*>(out), outer, nch, inner, per_channel, scale, zp,
+                          Quantize<DQ8_ROUND_HALF_AWAY_FROM_ZERO>{lo, hi}, st);
 }
 
 template <typename XT>
-bool launch_quantize_kind(int out_kind, bool rne, const void* x, void* out, int64_t n,
-                          int64_t nch, int64_t inner, int per_channel, const float* scale,
-                          const int32_t* zp, float lo, float hi, hipStream_t st) {
-#define DQ8_WIDE_CASE(KIND, QT)                                                              \
-  case KIND:                                                                                 \
-    launch_quantize_wide<XT, QT>(rne, x, out, n, nch, inner, per_channel, scale, zp, lo, hi, \
-                                 st);                                                        \
-    return true;
+int launch_quantize_kind(int out_kind, bool rne, const XT* x, void* out, int64_t outer, int64_t nch,
+                         int64_t inner, bool per_channel, const float* scale, const int32_t* zp,
+                         float lo, float hi, hipStream_t st) {
+#define DQ8_KIND_CASE(KIND, QT) \
+  case KIND:                    \
+    return launch_quantize_any<XT, QT>(rne, x, out, outer, nch, inner, per_channel, scale, zp, lo, hi, st);
   switch (out_kind) {
-    DQ8_WIDE_CASE(DQ8_I8, int8_t)
-    DQ8_WIDE_CASE(DQ8_U8, uint8_t)
-    DQ8_WIDE_CASE(DQ8_I16, int16_t)
-    DQ8_WIDE_CASE(DQ8_U16, uint16_t)
-    DQ8_WIDE_CASE(DQ8_I32, int32_t)
-    DQ8_WIDE_CASE(DQ8_U32, uint32_t)
+    DQ8_KIND_CASE(DQ8_I8, int8_t)
+    DQ8_KIND_CASE(DQ8_U8, uint8_t)
+    DQ8_KIND_CASE(DQ8_I16, int16_t)
+    DQ8_KIND_CASE(DQ8_U16, uint16_t)
+    DQ8_KIND_CASE(DQ8_I32, int32_t)
+    DQ8_KIND_CASE(DQ8_U32, uint32_t)
   }
-#undef DQ8_WIDE_CASE
-  return false;
+#undef DQ8_KIND_CASE
+  return dq8::fail("quantize: unknown out_kind");
 }
 
 }  // namespace
@@ -506,22 +683,17 @@ extern "C" int dq8_quantize(const float* x, void* out, int out_kind,
                          st, __VA_ARGS__);                                          \
   } while (0)
 
-  if (!per_channel) {
-    const int64_t n4 = vec_ok ? n / 4 : 0;
-    if (n4 > 0)
-      LAUNCH_RND(quantize_tensor_v4, dim3(sweep_grid(n4)), dim3(kThreads),
-                 (const float4*)x, (uint32_t*)out, n4, scale, zp, lo, hi);
-    if (n4 * 4 < n)
-      LAUNCH_RND(quantize_scalar, dim3(grid_for(n - n4 * 4, 1)), dim3(kThreads), x,
-                 (uint8_t*)out, n4 * 4, n, (int64_t)1, (int64_t)1, 0, scale, zp, lo, hi);
-  } else if (vec_ok && inner == 1 && nch % 4 == 0 && nch / 4 < (1 << 30) &&
+  if (!per_channel && vec_ok) {
+    LAUNCH_RND(quantize_tensor_v4, dim3(sweep_grid(n / 4)), dim3(kThreads),
+               (const float4*)x, (uint32_t*)out, n, scale, zp, lo, hi);
+  } else if (per_channel && vec_ok && inner == 1 && nch % 4 == 0 && nch / 4 < (1 << 30) &&
              dq8::aligned(scale, 16) && dq8::aligned(zp, 16)) {
     const int nch4 = (int)(nch / 4);
     const LastAxisPlan lp = plan_last_axis(outer, nch4);
     LAUNCH_RND(quantize_lastaxis_v4, dim3(lp.gx, lp.gy), dim3(lp.bx, lp.by), (const float4*)x,
                (uint32_t*)out, outer, nch4, lp.rows_per_block, (const float4*)scale,
                (const int4*)zp, lo, hi);
-  } else if (vec_ok && inner % 4 == 0 && outer * nch < (1LL << 31)) {
+  } else if (per_channel && vec_ok && inner % 4 == 0 && outer * nch < (1LL << 31)) {
     const int64_t rows = outer * nch;
     const int64_t inner4 = inner / 4;
     DQ8_REQUIRE(inner4 < (1LL << 38), "dq8_quantize: rows too long for one launch");
@@ -533,8 +705,8 @@ extern "C" int dq8_quantize(const float* x, void* out, int out_kind,
                (const float4*)x, (uint32_t*)out, (unsigned)rows, inner4, (unsigned)nch, scale,
                zp, lo, hi);
   } else {
-    LAUNCH_RND(quantize_scalar, dim3(grid_for(n, 1)), dim3(kThreads), x,
-               (uint8_t*)out, (int64_t)0, n, nch, inner, 1, scale, zp, lo, hi);
+    return launch_quantize_kind<float>(out_kind, rne, x, out, outer, nch, inner, per_channel, scale,
+                                       zp, lo, hi, st);
   }
 #undef LAUNCH_RND
   return dq8::check_hip(hipGetLastError(), "dq8_quantize launch");
@@ -557,18 +729,11 @@ extern "C" int dq8_dequantize(const void* q, int in_kind, float* out,
   const bool per_channel = n_q > 1;
   const bool vec_ok = dq8::aligned(q, 4) && dq8::aligned(out, 16);
 
-  if (!per_channel) {
-    const int64_t n4 = vec_ok ? n / 4 : 0;
-    if (n4 > 0) {
-      auto k = is_signed ? dequantize_tensor_v4x2<true> : dequantize_tensor_v4x2<false>;
-      hipLaunchKernelGGL(k, dim3(sweep_grid(dq8::ceil_div(n4, 2))), dim3(kThreads), 0, st,
-                         (const uint32_t*)q, (float4*)out, n4, scale, zp);
-    }
-    if (n4 * 4 < n)
-      hipLaunchKernelGGL(dequantize_scalar, dim3(grid_for(n - n4 * 4, 1)),
-                         dim3(kThreads), 0, st, (const uint8_t*)q, out, n4 * 4, n,
-                         (int64_t)1, (int64_t)1, 0, scale, zp, is_signed);
-  } else if (vec_ok && inner == 1 && nch % 4 == 0 && nch / 4 < (1 << 30) &&
+  if (!per_channel && vec_ok) {
+    auto k = is_signed ? dequantize_tensor_v4x2<true> : dequantize_tensor_v4x2<false>;
+    hipLaunchKernelGGL(k, dim3(sweep_grid(dq8::ceil_div(n / 4, 2))), dim3(kThreads), 0, st,
+                       (const uint32_t*)q, (float4*)out, n, scale, zp);
+  } else if (per_channel && vec_ok && inner == 1 && nch % 4 == 0 && nch / 4 < (1 << 30) &&
              dq8::aligned(scale, 16) && dq8::aligned(zp, 16)) {
     const int nch4 = (int)(nch / 4);
     const LastAxisPlan lp = plan_last_axis(outer, nch4);
@@ -576,7 +741,7 @@ extern "C" int dq8_dequantize(const void* q, int in_kind, float* out,
     hipLaunchKernelGGL(k, dim3(lp.gx, lp.gy), dim3(lp.bx, lp.by), 0, st, (const uint32_t*)q,
                        (float4*)out, outer, nch4, lp.rows_per_block, (const float4*)scale,
                        (const int4*)zp);
-  } else if (vec_ok && inner % 4 == 0 && outer * nch < (1LL << 31)) {
+  } else if (per_channel && vec_ok && inner % 4 == 0 && outer * nch < (1LL << 31)) {
     const int64_t rows = outer * nch;
     const bool v8 = inner >= 2048;     // two words per thread once a row is several workgroups
     const int64_t units = inner / 4;
@@ -590,9 +755,10 @@ extern "C" int dq8_dequantize(const void* q, int in_kind, float* out,
                        (const uint32_t*)q, (float4*)out, (unsigned)rows, units, (unsigned)nch,
                        scale, zp);
   } else {
-    hipLaunchKernelGGL(dequantize_scalar, dim3(grid_for(n, 1)), dim3(kThreads), 0,
-                       st, (const uint8_t*)q, out, (int64_t)0, n, nch, inner, 1,
-                       scale, zp, is_signed);
+    return is_signed ? launch_any((const int8_t*)q, out, outer, nch, inner, per_channel, scale, zp,
+                                  Dequantize{}, st)
+                     : launch_any((const uint8_t*)q, out, outer, nch, inner, per_channel, scale, zp,
+                                  Dequantize{}, st);
   }
   return dq8::check_hip(hipGetLastError(), "dq8_dequantize launch");
 }
@@ -627,22 +793,17 @@ extern "C" int dq8_fake_quant(const float* x, float* out, int64_t outer, int64_t
                          st, __VA_ARGS__);                                          \
   } while (0)
 
-  if (!per_channel) {
-    const int64_t n4 = vec_ok ? n / 4 : 0;
-    if (n4 > 0)
-      LAUNCH_RND(fake_quant_tensor_v4, dim3(sweep_grid(n4)), dim3(kThreads), (const float4*)x,
-                 (float4*)out, n4, scale, zp, lo, hi);
-    if (n4 * 4 < n)
-      LAUNCH_RND(fake_quant_scalar, dim3(grid_for(n - n4 * 4, 1)), dim3(kThreads), x, out,
-                 n4 * 4, n, (int64_t)1, (int64_t)1, 0, scale, zp, lo, hi);
-  } else if (vec_ok && inner == 1 && nch % 4 == 0 && nch / 4 < (1 << 30) &&
+  if (!per_channel && vec_ok) {
+    LAUNCH_RND(fake_quant_tensor_v4, dim3(sweep_grid(n / 4)), dim3(kThreads), (const float4*)x,
+               (float4*)out, n, scale, zp, lo, hi);
+  } else if (per_channel && vec_ok && inner == 1 && nch % 4 == 0 && nch / 4 < (1 << 30) &&
              dq8::aligned(scale, 16) && dq8::aligned(zp, 16)) {
     const int nch4 = (int)(nch / 4);
     const LastAxisPlan lp = plan_last_axis(outer, nch4);
     LAUNCH_RND(fake_quant_lastaxis_v4, dim3(lp.gx, lp.gy), dim3(lp.bx, lp.by), (const float4*)x,
                (float4*)out, outer, nch4, lp.rows_per_block, (const float4*)scale,
                (const int4*)zp, lo, hi);
-  } else if (vec_ok && inner % 4 == 0 && outer * nch < (1LL << 31) &&
+  } else if (per_channel && vec_ok && inner % 4 == 0 && outer * nch < (1LL << 31) &&
              inner / 4 < (1LL << 38) && dq8::ceil_div(outer * nch, 32768) <= 65535) {
     const int64_t rows = outer * nch;
     const int64_t inner4 = inner / 4;
@@ -652,8 +813,10 @@ extern "C" int dq8_fake_quant(const float* x, float* out, int64_t outer, int64_t
     LAUNCH_RND(fake_quant_rows_v4, dim3(gx, gy, (unsigned)gz), dim3(kThreads), (const float4*)x,
                (float4*)out, (unsigned)rows, inner4, (unsigned)nch, scale, zp, lo, hi);
   } else {
-    LAUNCH_RND(fake_quant_scalar, dim3(grid_for(n, 1)), dim3(kThreads), x, out, (int64_t)0, n,
-               nch, inner, 1, scale, zp, lo, hi);
+    return rne ? launch_any(x, out, outer, nch, inner, per_channel, scale, zp,
+                            FakeQuantize<DQ8_ROUND_HALF_TO_EVEN>{lo, hi}, st)
+               : launch_any(x, out, outer, nch, inner, per_channel, scale, zp,
+                            FakeQuantize<DQ8_ROUND_HALF_AWAY_FROM_ZERO>{lo, hi}, st);
   }
 #undef LAUNCH_RND
   return dq8::check_hip(hipGetLastError(), "dq8_fake_quant launch");
@@ -699,13 +862,11 @@ extern "C" int dq8_quantize_ex(const void* x, int x_dtype, void* out, int out_ki
   const bool rne = round_mode == DQ8_ROUND_HALF_TO_EVEN;
   const float lo = (float)qmin, hi = (float)qmax;
   hipStream_t st = (hipStream_t)stream;
-  if (x_dtype == DQ8_DTYPE_F32)
-    launch_quantize_kind<float>(out_kind, rne, x, out, n, nch, inner, n_q > 1, scale, zp, lo, hi,
-                                st);
-  else
-    launch_quantize_kind<_Float16>(out_kind, rne, x, out, n, nch, inner, n_q > 1, scale, zp, lo,
-                                   hi, st);
-  return dq8::check_hip(hipGetLastError(), "dq8_quantize_ex launch");
+  return x_dtype == DQ8_DTYPE_F32
+             ? launch_quantize_kind(out_kind, rne, static_cast<const float*>(x), out, outer, nch, inner,
+                                    n_q > 1, scale, zp, lo, hi, st)
+             : launch_quantize_kind(out_kind, rne, static_cast<const _Float16*>(x), out, outer, nch,
+                                    inner, n_q > 1, scale, zp, lo, hi, st);
 }
 
 extern "C" int dq8_dequantize_ex(const void* q, int in_kind, float* out, int64_t outer,
@@ -721,17 +882,13 @@ extern "C" int dq8_dequantize_ex(const void* q, int in_kind, float* out, int64_t
   if (n == 0) return 0;
   DQ8_REQUIRE(q && out && scale && zp, "dq8_dequantize_ex: null pointer");
   hipStream_t st = (hipStream_t)stream;
-  const dim3 grid(grid_for(n, 1)), block(kThreads);
-  const int pc = n_q > 1;
-#define DQ8_WIDE_CASE(QT)                                                                   \
-  hipLaunchKernelGGL(dequantize_wide<QT>, grid, block, 0, st, (const QT*)q, out, n, nch, inner, \
-                     pc, scale, zp)
+#define DQ8_KIND_CASE(QT) \
+  launch_any(static_cast<const QT*>(q), out, outer, nch, inner, n_q > 1, scale, zp, Dequantize{}, st)
   switch (in_kind) {
-    case DQ8_I16: DQ8_WIDE_CASE(int16_t); break;
-    case DQ8_U16: DQ8_WIDE_CASE(uint16_t); break;
-    case DQ8_I32: DQ8_WIDE_CASE(int32_t); break;
-    default: DQ8_WIDE_CASE(uint32_t); break;
+    case DQ8_I16: return DQ8_KIND_CASE(int16_t);
+    case DQ8_U16: return DQ8_KIND_CASE(uint16_t);
+    case DQ8_I32: return DQ8_KIND_CASE(int32_t);
+    default: return DQ8_KIND_CASE(uint32_t);
   }
-#undef DQ8_WIDE_CASE
-  return dq8::check_hip(hipGetLastError(), "dq8_dequantize_ex launch");
+#undef DQ8_KIND_CASE
 }

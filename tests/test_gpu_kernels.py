@@ -2130,3 +2130,67 @@ def test_clamping_tables_and_int8_residuals_equal_the_separate_operators(K, nb, 
             got = K.qconv2d(x, wt, pad, md, osh, epi, post=K.make_postops(
                 residual=rq, residual_scale=rs, residual_zp=rz, relu=relu, out_scale=ds2, out_zp=z2), **kw)
             assert torch.equal(got, want), (epi, zo, rz, z2, s2, relu)
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 64, 17), (3, 65, 1), (16, 79, 33), (17, 1000, 130), (32, 2049, 515), (200, 127, 70),
+                                   (256, 260, 129), (65, 1001, 1501), (300, 100, 257), (513, 333, 64), (777, 1000, 1501),
+                                   (1030, 4097, 260), (2100, 200, 3001), (4200, 72, 2100)])
+def test_qgemm_ragged_rows_and_results(K, m, k, n):
+    """k, n, alignments and row strides that are multiples of nothing, with and without zero points
+    and fused operators: small-M kernel on the rows as they are, tiled kernels on copied rows,
+    results stored from rows that begin at any byte -- bit-exact against the scalar kernel."""
+    rng = np.random.default_rng(m + 3 * k + 7 * n)
+    gen = 0
+    wide_a = dev(rng.integers(-128, 128, (m, k + 5), dtype=np.int8))
+    wide_w = dev(rng.integers(-128, 128, (n, k + 3), dtype=np.int8))
+    out8 = torch.empty((m, n + 3), dtype=torch.int8, device="cuda")
+    out32 = torch.empty((m, n + 1), dtype=torch.int32, device="cuda")
+    so = np.float32(0.02 * 0.025 * 74.0 * 74.0 * np.sqrt(k) / 40.0)
+    sc = dict(sx=dev(np.array([0.02], np.float32)), so=dev(np.array([so])),
+              sw=dev(rng.uniform(0.001, 0.05, n).astype(np.float32)))
+    bias = dev((rng.standard_normal(n) * 20 * so).astype(np.float32))
+    for a, w in ((wide_a[:, :k].contiguous(), wide_w[:, :k].contiguous()), (wide_a[:, 3:3 + k], wide_w[:, 1:1 + k])):
+        for zx, zw in ((0, 0), (-11, 0), (5, -3)):
+            kw = dict(zx=zx, zw=zw)
+            acc = K.qgemm(a, w, K.EPI_ACC_S32, variant=gen, **kw)
+            assert torch.equal(K.qgemm(a, w, K.EPI_ACC_S32, **kw), acc)
+            got = K.qgemm(a, w, K.EPI_ACC_S32, out=out32[:, 1:], **kw)
+            assert torch.equal(got, acc)
+            q = K.qgemm(a, w, K.EPI_REQUANT_CPU, bias=bias, zo=2, variant=gen, **sc, **kw)
+            assert torch.equal(K.qgemm(a, w, K.EPI_REQUANT_CPU, bias=bias, zo=2, **sc, **kw), q)
+            assert torch.equal(K.qgemm(a, w, K.EPI_REQUANT_CPU, bias=bias, zo=2, out=out8[:, 1:n + 1], **sc, **kw), q)
+            y = K.qgemm(a, w, K.EPI_REQUANT_CPU_DEQUANT_F32, bias=bias, **sc, **kw)
+            want = K.qgemm(a, w, K.EPI_REQUANT_CPU_DEQUANT_F32, bias=bias, variant=gen, **sc, **kw)
+            assert torch.equal(y.view(torch.int32), want.view(torch.int32))
+    table = dev(rng.integers(-128, 128, 256, dtype=np.int8))
+    got = K.qgemm(a, w, K.EPI_REQUANT_CPU, bias=bias, zo=2, post=K.make_postops(table=table), **sc, **kw)
+    assert torch.equal(got, K.lut8(q, table))
+    res = dev((rng.standard_normal((m, n)) * 40 * so).astype(np.float32))
+    got = K.qgemm(a, w, K.EPI_REQUANT_CPU_DEQUANT_F32, bias=bias, post=K.make_postops(residual=res), **sc, **kw)
+    assert torch.equal(got.view(torch.int32), (y + res).view(torch.int32))
+
+
+@pytest.mark.parametrize("shape,axis", [((1,), None), ((7,), None), ((1027,), None), ((3, 5), 1), ((4, 1), 1), ((9, 3), 1),
+                                        ((1000, 3073), 1), ((5, 259), 1), ((6, 258), 1), ((7, 1025), 0), ((33, 5), 0),
+                                        ((3, 6, 7), 1), ((2, 5, 1, 3), 2), ((1001, 33), 0)])
+def test_quantize_any_size_type_and_alignment(K, shape, axis):
+    """Sizes that are multiples of nothing, every quantized type, f16 input, bases at any element:
+    the oracle's bits, both ways and fake-quantized."""
+    rng = np.random.default_rng(sum(shape))
+    n = 1 if axis is None else shape[axis]
+    x = (rng.standard_normal(shape) * 50).astype(np.float32)
+    for name, lo, hi in (("int8", -128, 127), ("uint8", 0, 255), ("int16", -32768, 32767), ("int32", -2**31, 2**31 - 1)):
+        scale = rng.uniform(0.5, 1.5, n).astype(np.float32) * np.float32(2e-3 if name == "int16" else 1.0)
+        zp = rng.integers(-5, 6, n).astype(np.int32) + (128 if name == "uint8" else 0)
+        for xin in (x, x.astype(np.float16)):
+            want = O.quantize(xin.astype(np.float32), scale, zp, axis=axis, qmin=lo, qmax=hi, dtype=np.dtype(name).type)
+            base = torch.empty(x.size + 1, dtype=dev(xin).dtype, device="cuda")
+            for dx in (dev(xin), base[1:].view(shape)):
+                dx.copy_(dev(xin))
+                got = K.quantize(dx, dev(scale), dev(zp), axis=axis, qmin=lo, qmax=hi, dtype=getattr(torch, name))
+                np.testing.assert_array_equal(host(got), want)
+        want_f = O.dequantize(want, scale, zp, axis=axis)
+        np.testing.assert_array_equal(host(K.dequantize(got, dev(scale), dev(zp), axis=axis)), want_f)
+        if name in ("int8", "uint8"):
+            xf = dev(xin.astype(np.float32))
+            np.testing.assert_array_equal(host(K.fake_quant(xf, dev(scale), dev(zp), axis=axis, qmin=lo, qmax=hi)), want_f)
