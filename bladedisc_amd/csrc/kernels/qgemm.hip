@@ -344,6 +344,10 @@ DQ8_DECLARE_LAUNCH(true, DQ8_EPI_REQUANT_CPU)
 DQ8_DECLARE_LAUNCH(true, DQ8_EPI_REQUANT_GPU)
 DQ8_DECLARE_LAUNCH(true, DQ8_EPI_DEQUANT_F32)
 #undef DQ8_DECLARE_LAUNCH
+extern template int launch_zp_ragged<DQ8_EPI_ACC_S32>(int, MainParams&, hipStream_t);
+extern template int launch_zp_ragged<DQ8_EPI_REQUANT_CPU>(int, MainParams&, hipStream_t);
+extern template int launch_zp_ragged<DQ8_EPI_REQUANT_GPU>(int, MainParams&, hipStream_t);
+extern template int launch_zp_ragged<DQ8_EPI_DEQUANT_F32>(int, MainParams&, hipStream_t);
 
 int compute_units() {
   static std::atomic<int> cached{0};
@@ -369,6 +373,16 @@ int launch_epi(int variant, MainParams& p, int epilogue, hipStream_t st) {
     case DQ8_EPI_REQUANT_CPU: return launch_variant<CONV, DQ8_EPI_REQUANT_CPU>(variant, p, st);
     case DQ8_EPI_REQUANT_GPU: return launch_variant<CONV, DQ8_EPI_REQUANT_GPU>(variant, p, st);
     case DQ8_EPI_DEQUANT_F32: return launch_variant<CONV, DQ8_EPI_DEQUANT_F32>(variant, p, st);
+  }
+  return fail("unknown epilogue");
+}
+
+int launch_zp_ragged_epi(int variant, MainParams& p, int epilogue, hipStream_t st) {
+  switch (epilogue) {
+    case DQ8_EPI_ACC_S32: return launch_zp_ragged<DQ8_EPI_ACC_S32>(variant, p, st);
+    case DQ8_EPI_REQUANT_CPU: return launch_zp_ragged<DQ8_EPI_REQUANT_CPU>(variant, p, st);
+    case DQ8_EPI_REQUANT_GPU: return launch_zp_ragged<DQ8_EPI_REQUANT_GPU>(variant, p, st);
+    case DQ8_EPI_DEQUANT_F32: return launch_zp_ragged<DQ8_EPI_DEQUANT_F32>(variant, p, st);
   }
   return fail("unknown epilogue");
 }
@@ -754,10 +768,10 @@ int qgemm_impl(int variant, const int8_t* A, int64_t lda, const int8_t* W, int64
   // multiple of 16: operands in another layout, or with a ragged K, are rewritten into the
   // workspace (zero-filled up to K'; zeros add nothing to the sums).
   const int64_t Kp = (K + 15) / 16 * 16, pitch = (K + 127) / 128 * 128;
-  // A few rows against rows of any length or alignment: the small-M kernel takes them as they are.
+  // Rows of any length or alignment where the copy to aligned ones would cost as much as the
+  // product: the small-M kernel and the 64 x 64 tiles take them as they are.
   if (auto_pick && !tp_a && tp_b && K >= 64 &&
-      (K % 16 != 0 || !aligned(A, 16) || !aligned(W, 16) || lda % 16 != 0 || ldw % 16 != 0) &&
-      pick_any(M, N, Kp, true, es) == kSkinnyVariant) {
+      (K % 16 != 0 || !aligned(A, 16) || !aligned(W, 16) || lda % 16 != 0 || ldw % 16 != 0)) {
     MainParams p = {};
     p.A = A;
     p.W = W;
@@ -771,7 +785,14 @@ int qgemm_impl(int variant, const int8_t* A, int64_t lda, const int8_t* W, int64
     p.zx = zx;
     p.zw = zw;
     p.kzz = (int)((uint32_t)K * (uint32_t)zx * (uint32_t)zw);
-    return launch_epi<false>(kSkinnyVariant, p, epilogue, st);
+    const int v = pick_any(M, N, Kp, ragged_ok(p), es);
+    if (v == kSkinnyVariant) return launch_epi<false>(v, p, epilogue, st);
+    // (rows at odd bytes: each load is served in pieces, about 0.25 us per k tile -- 777 x 1504, 1000
+    // of k at any multiple of four 8.3 us, at odd bytes 11.5, copied first 12; 1000 x 768 with 3073
+    // of k 13.8, copied 12.7)
+    const bool words = aligned(A, 4) && aligned(W, 4) && lda % 4 == 0 && ldw % 4 == 0;
+    if (ragged_has_variant(v) && ragged_ok(p) && zw == 0 && (words || K <= 2048))
+      return launch_zp_ragged_epi(v, p, epilogue, st);
   }
   const bool repack_a = K > 0 && (tp_a || K % 16 != 0);
   const bool repack_w = K > 0 && (!tp_b || K % 16 != 0);
@@ -865,13 +886,16 @@ int qgemm_impl(int variant, const int8_t* A, int64_t lda, const int8_t* W, int64
   // The small-M kernel forms the row sums next to its products; the tiled kernels start from them.
   const bool zp_skinny = zp_mfma && variant == kSkinnyVariant;
   if (zp_mfma && !zp_skinny && !is_pipe_variant(variant)) variant = kPipe64;   // (tiles the others cannot address)
+  // (an input zero point alone: the one-tile kernels sum the weights up as they multiply them)
+  const bool zp_loop = zp_mfma && !zp_skinny && zw == 0 && zp_has_variant(variant) &&
+                       pipe_ok(kVariants[variant].bm, kVariants[variant].bn, p, false);
 
   // Zero points: the row sums of the weights, and of the activations where the weights have one
   // (wrapping int32 arithmetic on purpose, as in the kernels).
   int32_t* corr_n = nullptr;
   int32_t* corr_m = nullptr;
   const int kzz = (int)((uint32_t)K_true * (uint32_t)zx * (uint32_t)zw);
-  if (zp_mfma && !zp_skinny) {
+  if (zp_mfma && !zp_skinny && !zp_loop) {
     corr_n = reinterpret_cast<int32_t*>((int8_t*)workspace + ws_off);
     auto sums = [&](RowsJob* job, const int8_t* use, int64_t ld, int64_t rows, int32_t* corr, int mul, int add) {
       if (!job->src) *job = {use, ld, nullptr, nullptr, (int)rows, (int)K_true, 0, 0, 0};
@@ -891,11 +915,12 @@ int qgemm_impl(int variant, const int8_t* A, int64_t lda, const int8_t* W, int64
                        dim3(256), 0, st, job_a, job_w);
     DQ8_HIP(hipGetLastError());
   }
-  if (zp_skinny) {
+  if (zp_skinny || zp_loop) {
     p.zx = zx;
     p.zw = zw;
     p.kzz = kzz;
   }
+  if (zp_loop) return launch_zp_ragged_epi(variant, p, epilogue, st);
   if (!zp_mfma || zp_skinny) return launch_epi<false>(variant, p, epilogue, st);
 
   // ---- zero points: a pipelined kernel that starts from the corrections

@@ -5,6 +5,7 @@
 #ifndef DQ8_QGEMM_LAUNCH_H_
 #define DQ8_QGEMM_LAUNCH_H_
 
+#include <algorithm>
 #include <cstdlib>
 
 #include "dq8_common.h"
@@ -119,13 +120,19 @@ inline bool pipe_ok(int bm, int bn, const MainParams& p, bool conv) {
   return (int64_t)bm * p.lda + p.K + 2 * BK < (1LL << 31);
 }
 
-template <int BM, int BN, int WM, int WN, int KSPLIT, bool CONV, int EPI, bool ROWMAP = false>
+// What the RAGGED form of a 64 x 64 tile asks of the operands.
+inline bool ragged_ok(const MainParams& p) {
+  return p.K >= 16 && 64 * std::max(p.lda, p.ldw) + p.K + 512 < (1LL << 31);
+}
+
+template <int BM, int BN, int WM, int WN, int KSPLIT, bool CONV, int EPI, bool ROWMAP = false,
+          bool ZP = false, bool RAGGED = false>
 int launch_pipe(const MainParams& p, hipStream_t st) {
   constexpr int BK = 128;
   constexpr int lds = KSPLIT * 2 * (BM + BN) * BK;
-  DQ8_REQUIRE(pipe_ok(BM, BN, p, CONV) && (!ROWMAP || p.conv_bytes < (1LL << 31)),
+  DQ8_REQUIRE(RAGGED ? ragged_ok(p) : pipe_ok(BM, BN, p, CONV) && (!ROWMAP || p.conv_bytes < (1LL << 31)),
               "pipelined qgemm needs K % 16 == 0 and operands that fit 32-bit buffer offsets");
-  auto kern = qgemm_pipe_kernel<BM, BN, WM, WN, KSPLIT, CONV, EPI, ROWMAP>;
+  auto kern = qgemm_pipe_kernel<BM, BN, WM, WN, KSPLIT, CONV, EPI, ROWMAP, ZP, RAGGED>;
   static std::atomic<uint64_t> lds_allowed{0};
   if (int s = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds, &lds_allowed)) return s;
   hipLaunchKernelGGL(kern, dim3(p.tiles_m * p.tiles_n), dim3(WM * WN * KSPLIT * 64), lds, st, p);
@@ -269,6 +276,42 @@ int launch_variant(int variant, MainParams& p, hipStream_t st) {
   return fail("unknown or unsupported qgemm variant for this operation");
 }
 
+// Tiles with an input zero point summed up in the k loop, and the 64 x 64 ones on operand rows of
+// any length and alignment (qgemm_launch_zp_*.hip).
+inline bool zp_has_variant(int variant) {
+  return variant == kPipe64 || variant == kPipe64k2 || variant == kPipe64k4 || variant == kPipe128 ||
+         variant == kPipe128w8 || variant == kPipe256w8 || variant == kPipe256x192;
+}
+inline bool ragged_has_variant(int variant) {
+  return variant == kPipe64 || variant == kPipe64k2 || variant == kPipe64k4;
+}
+template <int EPI>
+int launch_zp_ragged(int variant, MainParams& p, hipStream_t st) {
+  const Variant& v = kVariants[variant];
+  p.tiles_m = (int)ceil_div(p.M, v.bm);
+  p.tiles_n = (int)ceil_div(p.N, v.bn);
+  if (p.ragged) {
+    switch (variant) {
+      case kPipe64: return p.zx ? launch_pipe<64, 64, 2, 2, 1, false, EPI, false, true, true>(p, st)
+                                : launch_pipe<64, 64, 2, 2, 1, false, EPI, false, false, true>(p, st);
+      case kPipe64k2: return p.zx ? launch_pipe<64, 64, 2, 2, 2, false, EPI, false, true, true>(p, st)
+                                  : launch_pipe<64, 64, 2, 2, 2, false, EPI, false, false, true>(p, st);
+      case kPipe64k4: return p.zx ? launch_pipe<64, 64, 2, 2, 4, false, EPI, false, true, true>(p, st)
+                                  : launch_pipe<64, 64, 2, 2, 4, false, EPI, false, false, true>(p, st);
+    }
+  }
+  switch (variant) {
+    case kPipe64: return launch_pipe<64, 64, 2, 2, 1, false, EPI, false, true>(p, st);
+    case kPipe64k2: return launch_pipe<64, 64, 2, 2, 2, false, EPI, false, true>(p, st);
+    case kPipe64k4: return launch_pipe<64, 64, 2, 2, 4, false, EPI, false, true>(p, st);
+    case kPipe128: return launch_pipe<128, 128, 2, 2, 1, false, EPI, false, true>(p, st);
+    case kPipe128w8: return launch_pipe<128, 128, 2, 4, 1, false, EPI, false, true>(p, st);
+    case kPipe256w8: return launch_pipe<256, 256, 2, 4, 1, false, EPI, false, true>(p, st);
+    case kPipe256x192: return launch_pipe<256, 192, 4, 2, 1, false, EPI, false, true>(p, st);
+  }
+  return fail("no kernel with a zero point in the k loop for this variant");
+}
+
 // The tiles a strided 1 x 1 convolution runs on as a GEMM over the pixels it reads (instantiated
 // next to the convolution kernels: CONV true; the GEMM files carry a stub).
 inline bool rowmap_has_variant(int variant) {
@@ -301,6 +344,12 @@ int launch_rowmap(int variant, MainParams& p, hipStream_t st) {
   template int launch_variant<CONV, EPI>(int, MainParams&, hipStream_t); \
   template int launch_f32a<CONV, EPI>(const MainParams&, hipStream_t);   \
   template int launch_rowmap<CONV, EPI>(int, MainParams&, hipStream_t);  \
+  }
+
+// the body of one qgemm_launch_zp_*.hip
+#define DQ8_INSTANTIATE_LAUNCH_ZP(EPI) \
+  namespace dq8 {                       \
+  template int launch_zp_ragged<EPI>(int, MainParams&, hipStream_t); \
   }
 
 #endif  // DQ8_QGEMM_LAUNCH_H_

@@ -1,0 +1,4 @@
+// Launchers of the int8 GEMM tiles with a zero point in the k loop or on ragged rows, epilogue REQUANT_GPU.
+#include "qgemm_launch.h"
+
+DQ8_INSTANTIATE_LAUNCH_ZP(DQ8_EPI_REQUANT_GPU)

@@ -105,7 +105,20 @@ constexpr int waitcnt_vm_lgkm0(int n) { return (n & 0xf) | ((n >> 4) << 14) | (0
 // of A is input pixel (m / (Ho Wo), sh ((m / Wo) % Ho), sw_ (m % Wo)) of the NHWC image that H,
 // Wd, Ci, Ho, Wo, sh, sw_ and conv_bytes describe (lda is not used): found once, before the k
 // loop, which is the GEMM's -- half the instructions of the implicit GEMM's.
-template <int BM, int BN, int WM, int WN, int KSPLIT, bool CONV, int EPI, bool ROWMAP = false>
+//
+// ZP: an input zero point, sum (a - zx) w = sum a w - zx sum w: every wave adds up the weight
+// fragments it multiplies (four v_dot4 per fragment, under the MFMAs), and the accumulators get
+// -zx times that behind the k loop.  A row-sum kernel in front costs a launch and a trip through
+// memory instead (M = 1000, 3072 -> 768: 7.7 us without a zero point, 11.1 with that launch).
+//
+// RAGGED: operand rows of any length (K >= 16) and alignment.  The loads go through registers --
+// an unaligned global load, then ds_write into the place the direct load would have filled -- one
+// k tile further ahead, and the chunk that holds the end of a row is shifted into place and
+// filled up with zeros.  For the 64 x 64 tiles, where copying the operands to aligned rows first
+// costs as much as the product (777 x 1000 x 1501: 13.3 us with the copy, 9.6 without).
+typedef int v4i_any_t __attribute__((ext_vector_type(4), aligned(1)));
+template <int BM, int BN, int WM, int WN, int KSPLIT, bool CONV, int EPI, bool ROWMAP = false,
+          bool ZP = false, bool RAGGED = false>
 __global__ void __launch_bounds__(WM* WN* KSPLIT * 64) qgemm_pipe_kernel(const MainParams p) {
   // The inline assembly only assembles in the device compilation; the host pass
   // just needs the kernel's stub.
@@ -192,13 +205,16 @@ __global__ void __launch_bounds__(WM* WN* KSPLIT * 64) qgemm_pipe_kernel(const M
       const int ho = rem / p.Wo, wo = rem - ho * p.Wo;
       a_off[i] = ((n_img * p.H + ho * p.sh) * p.Wd + wo * p.sw_) * p.Ci + kc;
     } else {
-      a_off[i] = (q * 8 + lr) * (int)p.lda + kc;
+      // (RAGGED loads are not bounds-checked: rows past M read the last row again)
+      const int row = RAGGED ? min(q * 8 + lr, p.M - 1 - m0) : q * 8 + lr;
+      a_off[i] = row * (int)p.lda + (RAGGED ? 0 : kc);
     }
   }
 #pragma unroll
   for (int i = 0; i < B_LD; ++i) {
     const int q = wave + i * NW;
-    b_off[i] = (q * 8 + lr) * (int)p.ldw + kc;
+    const int row = RAGGED ? min(q * 8 + lr, p.N - 1 - n0) : q * 8 + lr;
+    b_off[i] = row * (int)p.ldw + (RAGGED ? 0 : kc);
     b_lds[i] = __builtin_amdgcn_readfirstlane(A_BYTES + q * 1024);
   }
 
@@ -272,6 +288,43 @@ __global__ void __launch_bounds__(WM* WN* KSPLIT * 64) qgemm_pipe_kernel(const M
                              b_off[i] + t_koff);
   };
 
+  // RAGGED: tile `kt` into registers, and from there into stage `st` (tiles past the group's last
+  // are read by no one)
+  v4i held[RAGGED ? LD : 1];
+  const int k_first = RAGGED ? __builtin_amdgcn_readfirstlane(kt0) * BK : 0;
+  auto fetch_tile = [&](int kt, v4i (&held)[RAGGED ? LD : 1]) {
+    if (kt >= KT) return;
+    const int k = k_first + kt * BK + kc;
+    const int kk = k + 16 <= p.K ? k : p.K - 16;           // (a chunk that is not whole: the row's last 16)
+#pragma unroll
+    for (int i = 0; i < A_LD; ++i) held[RAGGED ? i : 0] = *reinterpret_cast<const v4i_any_t*>(a_base + (unsigned)(a_off[i] + kk));
+#pragma unroll
+    for (int i = 0; i < B_LD; ++i) held[RAGGED ? A_LD + i : 0] = *reinterpret_cast<const v4i_any_t*>(w_base + (unsigned)(b_off[i] + kk));
+  };
+  auto commit_tile = [&](int kt, int st, v4i (&held)[RAGGED ? LD : 1]) {
+    if (kt >= KT) return;
+    int8_t* base = smem + st * STAGE + lane * 16;
+    if (k_first + (kt + 1) * BK > p.K) {                   // the tile with the end of the rows
+      const int left = p.K - (k_first + kt * BK + kc);     // bytes of the row from the lane's chunk on
+      const int drop = left >= 16 ? 0 : (left > 0 ? 16 - left : 16);
+      const int sh = 8 * (drop & 7);
+#pragma unroll
+      for (int l = 0; l < (RAGGED ? LD : 1); ++l) {        // byte b of the chunk is byte b + drop of what was read
+        uint64_t lo = (uint32_t)held[l][0] | ((uint64_t)(uint32_t)held[l][1] << 32);
+        uint64_t hi = (uint32_t)held[l][2] | ((uint64_t)(uint32_t)held[l][3] << 32);
+        lo = drop >= 16 ? 0 : (drop >= 8 ? hi : lo);
+        hi = drop >= 8 ? 0 : hi;
+        lo = (lo >> sh) | ((hi << 1) << (63 - sh));
+        hi >>= sh;
+        held[l] = (v4i){(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32), (int)(uint32_t)hi, (int)(uint32_t)(hi >> 32)};
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < A_LD; ++i) *reinterpret_cast<v4i*>(base + a_lds[i]) = held[RAGGED ? i : 0];
+#pragma unroll
+    for (int i = 0; i < B_LD; ++i) *reinterpret_cast<v4i*>(base + b_lds[i]) = held[RAGGED ? A_LD + i : 0];
+  };
+
   // ---- fragment addressing.  Operand row R = R0 + lane%32 sits in block R/8 at row
   // R%8; the k-chunk c = 2*ks + lane/32 of that row is in slot c ^ (R%8) ^ (block&1).
   // R0 is a multiple of 32, so the block parity is bit 3 of the lane.
@@ -338,21 +391,37 @@ __global__ void __launch_bounds__(WM* WN* KSPLIT * 64) qgemm_pipe_kernel(const M
   // tile 0 has landed was measured and loses: every CU then pulls 128 KiB before the
   // first MFMA, and at full occupancy that start-up burst costs more than the one
   // exposed latency it saves.)
-  tile_setup(0);
-#pragma unroll
-  for (int idx = 0; idx < LD; ++idx) issue_load(idx, 0);
   EarlyColParams<EPI, NT, BN> early;
-  early.fetch(p.epi, n0);
-  __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
-  __syncthreads();
-  DQ8_TRACE_POINT(1);
-  tile_setup(1);
+  if constexpr (RAGGED) {
+    v4i first[RAGGED ? LD : 1];
+    fetch_tile(0, first);
+    fetch_tile(1, held);
+    early.fetch(p.epi, n0);
+    commit_tile(0, 0, first);
+    commit_tile(1, 1, held);
+    fetch_tile(2, held);
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(63));
+    __syncthreads();
+  } else {
+    tile_setup(0);
 #pragma unroll
-  for (int idx = 0; idx < LD; ++idx) issue_load(idx, 1);
+    for (int idx = 0; idx < LD; ++idx) issue_load(idx, 0);
+    early.fetch(p.epi, n0);
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
+    __syncthreads();
+    DQ8_TRACE_POINT(1);
+    tile_setup(1);
+#pragma unroll
+    for (int idx = 0; idx < LD; ++idx) issue_load(idx, 1);
+  }
 #pragma unroll
   for (int i = 0; i < FM; ++i) load_frag_a(0, 0, 0, i);
 #pragma unroll
   for (int j = 0; j < FN; ++j) load_frag_b(0, 0, 0, j);
+
+  int w_sum[ZP ? FN : 1];            // of the weights this wave has multiplied: row lane % 32, its half of k
+#pragma unroll
+  for (int j = 0; j < (ZP ? FN : 1); ++j) w_sum[j] = 0;
 
   // One k tile out of stage `cur` (an int, or a compile-time constant: see below).
   auto k_tile = [&](auto cur_v, int kt) {
@@ -364,9 +433,15 @@ __global__ void __launch_bounds__(WM* WN* KSPLIT * 64) qgemm_pipe_kernel(const M
         // has, the stage can take tile kt+2
         __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(63));
         __syncthreads();
-        tile_setup(kt + 2);
+        if constexpr (RAGGED) {
+          // (the next reader of the stage is behind the next tile's barrier)
+          commit_tile(kt + 2, cur, held);
+          fetch_tile(kt + 3, held);
+        } else {
+          tile_setup(kt + 2);
+        }
       }
-      if (ks == 3) {
+      if (ks == 3 && !RAGGED) {
         // tile kt+1 (older than the LD_KS2 loads of tile kt+2 just issued) has landed
         // for this wave; after the barrier, for all of them
         __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(LD_KS2));
@@ -387,14 +462,27 @@ __global__ void __launch_bounds__(WM* WN* KSPLIT * 64) qgemm_pipe_kernel(const M
 #pragma unroll
           for (int j = i; j < FN; j += FM) load_frag_b(3, cur, 3, j);
         } else if (ks == 2) {
+          if constexpr (!RAGGED) {
 #pragma unroll
-          for (int l = 0; l < LPR; ++l) issue_load(i * LPR + l, cur);
+            for (int l = 0; l < LPR; ++l) issue_load(i * LPR + l, cur);
+          }
         } else {
           load_frag_a(0, nxt, 0, i);
 #pragma unroll
           for (int j = i; j < FN; j += FM) load_frag_b(0, nxt, 0, j);
+          if constexpr (!RAGGED) {
 #pragma unroll
-          for (int l = 0; l < LPR; ++l) issue_load((FM + i) * LPR + l, cur);
+            for (int l = 0; l < LPR; ++l) issue_load((FM + i) * LPR + l, cur);
+          }
+        }
+        if constexpr (ZP) {
+          // (the row of MFMAs i sums the fragments j = i, i + FM, ...; shared out over the WM waves
+          // that multiply the same fragments, a branch per k-step, the 256 x 192 tile took 31 us
+          // instead of 17 for M = 4096, 768 -> 3072)
+#pragma unroll
+          for (int j = i; j < FN; j += FM)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) w_sum[j] = __builtin_amdgcn_sdot4(fb[ks][j][c], 0x01010101, w_sum[j], false);
         }
 #pragma unroll
         for (int j = 0; j < FN; ++j)
@@ -421,6 +509,28 @@ __global__ void __launch_bounds__(WM* WN* KSPLIT * 64) qgemm_pipe_kernel(const M
   // nothing of this wave may still be writing LDS when the workgroup retires
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
   DQ8_TRACE_POINT(2);
+
+  if constexpr (ZP) {
+    // from a lane per channel to the accumulators' layout, through a piece of LDS that only this
+    // wave touches -- once every wave's last loads and writes into the stages have landed
+    __syncthreads();
+    int* mine = reinterpret_cast<int*>(smem) + wave * (FN * 32);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int s = w_sum[j] + __shfl_xor(w_sum[j], 32, 64);
+      mine[j * 32 + (lane & 31)] = (int)(0u - (unsigned)p.zx * (unsigned)s);
+    }
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const v4i c = *reinterpret_cast<const v4i*>(&mine[j * 32 + 8 * g + 4 * (lane >> 5)]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int i = 0; i < FM; ++i) acc[i][j][4 * g + q] += c[q];
+      }
+  }
 
   if (KSPLIT > 1) {
     // add the groups' partial sums: groups 1.. park their accumulators in LDS (lane-major,
