@@ -66,27 +66,28 @@ quantize_tensor_v4(const float4* __restrict__ x, uint32_t* __restrict__ out,
   const int64_t n4 = n >> 2;
   const int64_t stride = (int64_t)gridDim.x * kThreads;
   int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {        // the elements behind the last four
-    const int64_t e = 4 * n4 + threadIdx.x;
+  if (i < n4) {
+    // The data load goes out first: a wave has one load to make, and behind the scalar loads of
+    // the parameters and the reciprocal it would start a cache miss later.
+    float4 v = x[i];
+    __builtin_amdgcn_sched_barrier(0);
+    const float s = scale[0];
+    const float z = (float)zp[0];
+    const float y = 1.0f / s;
+    const bool fast = divisor_in_fast_range(s);
+    for (;;) {
+      out[i] = fast ? quant4_by_constant<ROUND>(v, s, y, z, lo, hi)
+                    : pack4(quant_one<ROUND>(v.x, s, z, lo, hi), quant_one<ROUND>(v.y, s, z, lo, hi),
+                            quant_one<ROUND>(v.z, s, z, lo, hi), quant_one<ROUND>(v.w, s, z, lo, hi));
+      i += stride;
+      if (i >= n4) break;
+      v = x[i];
+    }
+  }
+  if (i - n4 < (n & 3)) {                  // the up to three elements behind the last four
+    const int64_t e = i + 3 * n4;
     reinterpret_cast<uint8_t*>(out)[e] = (uint8_t)quant_one<ROUND>(
         reinterpret_cast<const float*>(x)[e], scale[0], (float)zp[0], lo, hi);
-  }
-  if (i >= n4) return;
-  // The data load goes out first: a wave has one load to make, and behind the scalar loads of
-  // the parameters and the reciprocal it would start a cache miss later.
-  float4 v = x[i];
-  __builtin_amdgcn_sched_barrier(0);
-  const float s = scale[0];
-  const float z = (float)zp[0];
-  const float y = 1.0f / s;
-  const bool fast = divisor_in_fast_range(s);
-  for (;;) {
-    out[i] = fast ? quant4_by_constant<ROUND>(v, s, y, z, lo, hi)
-                  : pack4(quant_one<ROUND>(v.x, s, z, lo, hi), quant_one<ROUND>(v.y, s, z, lo, hi),
-                          quant_one<ROUND>(v.z, s, z, lo, hi), quant_one<ROUND>(v.w, s, z, lo, hi));
-    i += stride;
-    if (i >= n4) break;
-    v = x[i];
   }
 }
 
@@ -122,11 +123,6 @@ dequantize_tensor_v4x2(const uint32_t* __restrict__ q, float4* __restrict__ out,
   const float s = scale[0];
   const int z = zp[0];
   const int64_t n4 = n >> 2;
-  if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {        // the elements behind the last word
-    const int64_t e = 4 * n4 + threadIdx.x;
-    const uint8_t b = reinterpret_cast<const uint8_t*>(q)[e];
-    reinterpret_cast<float*>(out)[e] = (float)((SIGNED ? (int)(int8_t)b : (int)b) - z) * s;
-  }
   const int64_t stride = (int64_t)gridDim.x * (2 * kThreads);
   for (int64_t i = (int64_t)blockIdx.x * (2 * kThreads) + threadIdx.x; i < n4; i += stride) {
     const bool two = i + kThreads < n4;
@@ -134,6 +130,11 @@ dequantize_tensor_v4x2(const uint32_t* __restrict__ q, float4* __restrict__ out,
     const uint32_t w1 = two ? q[i + kThreads] : 0u;
     dq8::st_stream(&out[i], dequant_word<SIGNED>(w0, z, s));
     if (two) dq8::st_stream(&out[i + kThreads], dequant_word<SIGNED>(w1, z, s));
+  }
+  if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {        // the elements behind the last word
+    const int64_t e = 4 * n4 + threadIdx.x;
+    const uint8_t b = reinterpret_cast<const uint8_t*>(q)[e];
+    reinterpret_cast<float*>(out)[e] = (float)((SIGNED ? (int)(int8_t)b : (int)b) - z) * s;
   }
 }
 
@@ -293,26 +294,27 @@ fake_quant_tensor_v4(const float4* __restrict__ x, float4* __restrict__ out, int
   const int64_t n4 = n >> 2;
   const int64_t stride = (int64_t)gridDim.x * kThreads;
   int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {        // the elements behind the last four
-    const int64_t e = 4 * n4 + threadIdx.x;
+  if (i < n4) {
+    float4 v = x[i];                       // (the data load first, as in quantize_tensor_v4)
+    __builtin_amdgcn_sched_barrier(0);
+    const float s = scale[0];
+    const int z = zp[0];
+    const float y = 1.0f / s;
+    const bool fast = divisor_in_fast_range(s);
+    for (;;) {
+      dq8::st_stream(&out[i],
+                     fast ? fake4_by_constant<ROUND>(v, s, y, z, lo, hi)
+                          : make_float4(fake_one<ROUND>(v.x, s, z, lo, hi), fake_one<ROUND>(v.y, s, z, lo, hi),
+                                        fake_one<ROUND>(v.z, s, z, lo, hi), fake_one<ROUND>(v.w, s, z, lo, hi)));
+      i += stride;
+      if (i >= n4) break;
+      v = x[i];
+    }
+  }
+  if (i - n4 < (n & 3)) {                  // the up to three elements behind the last four
+    const int64_t e = i + 3 * n4;
     reinterpret_cast<float*>(out)[e] =
         fake_one<ROUND>(reinterpret_cast<const float*>(x)[e], scale[0], zp[0], lo, hi);
-  }
-  if (i >= n4) return;
-  float4 v = x[i];                        // (the data load first, as in quantize_tensor_v4)
-  __builtin_amdgcn_sched_barrier(0);
-  const float s = scale[0];
-  const int z = zp[0];
-  const float y = 1.0f / s;
-  const bool fast = divisor_in_fast_range(s);
-  for (;;) {
-    dq8::st_stream(&out[i],
-                   fast ? fake4_by_constant<ROUND>(v, s, y, z, lo, hi)
-                        : make_float4(fake_one<ROUND>(v.x, s, z, lo, hi), fake_one<ROUND>(v.y, s, z, lo, hi),
-                                      fake_one<ROUND>(v.z, s, z, lo, hi), fake_one<ROUND>(v.w, s, z, lo, hi)));
-    i += stride;
-    if (i >= n4) break;
-    v = x[i];
   }
 }
 
@@ -684,7 +686,7 @@ extern "C" int dq8_quantize(const float* x, void* out, int out_kind,
   } while (0)
 
   if (!per_channel && vec_ok) {
-    LAUNCH_RND(quantize_tensor_v4, dim3(sweep_grid(n / 4)), dim3(kThreads),
+    LAUNCH_RND(quantize_tensor_v4, dim3(sweep_grid(n / 4 + n % 4)), dim3(kThreads),
                (const float4*)x, (uint32_t*)out, n, scale, zp, lo, hi);
   } else if (per_channel && vec_ok && inner == 1 && nch % 4 == 0 && nch / 4 < (1 << 30) &&
              dq8::aligned(scale, 16) && dq8::aligned(zp, 16)) {
@@ -794,7 +796,7 @@ extern "C" int dq8_fake_quant(const float* x, float* out, int64_t outer, int64_t
   } while (0)
 
   if (!per_channel && vec_ok) {
-    LAUNCH_RND(fake_quant_tensor_v4, dim3(sweep_grid(n / 4)), dim3(kThreads), (const float4*)x,
+    LAUNCH_RND(fake_quant_tensor_v4, dim3(sweep_grid(n / 4 + n % 4)), dim3(kThreads), (const float4*)x,
                (float4*)out, n, scale, zp, lo, hi);
   } else if (per_channel && vec_ok && inner == 1 && nch % 4 == 0 && nch / 4 < (1 << 30) &&
              dq8::aligned(scale, 16) && dq8::aligned(zp, 16)) {
