@@ -60,6 +60,8 @@ _PROTOS = {
     "dq8_weight_only_qgemm_workspace_bytes_ex": (C.c_size_t, [_I64, _I64, _I64, _INT, _INT]),
     "dq8_weight_only_qgemm": (_INT, [_VP, _INT, _I64, _VP, _INT, _I64, _INT, _VP, _VP, _VP, _VP,
                                      _I64, _I64, _I64, _I64, _VP, C.c_size_t, _VP]),
+    "dq8_attention_f32": (_INT, [_VP, _I64, _I64, _I64, _I64, _VP, _VP, _VP, _VP]),
+    "dq8_layernorm_f32": (_INT, [_VP, _I64, _I64, _VP, _VP, _F32, _VP, _VP, _VP, _VP]),
     "dq8_qlinear_f32_fused_max_rows": (_I64, [_I64, _I64]),
     "dq8_qlinear_f32": (_INT, [_VP, _I64, _VP, _I64, _VP, _I64, _I64, _I64, _I64, _INT, _VP, _INT,
                                _VP, _VP, _I64, _VP, _I64, _I32, _INT, _VP]),

@@ -5,7 +5,7 @@ for one encoder layer (examples/PyTorch/Quantization/bert_ptq.py, pytorch_blade/
 quantization): the four linears (merged QKV, attention output, FFN1, FFN2) run as
 int8 GEMMs with per-tensor activation scales, per-output-channel weight scales and a
 fused bias + requantisation; ``quantize`` / ``dequantize`` sit between them and the
-fp32 LayerNorm / softmax / GELU, which PyTorch computes.  Scales come from a min/max
+fp32 LayerNorm / softmax / GELU.  Scales come from a min/max
 calibration pass, as the reference's observers produce them.
 
 Two backends execute the quantized operators:
@@ -145,6 +145,24 @@ class QuantBertLayer:
         h = self.f["tok_emb"][t] + self.f["pos_emb"][pos][None]
         return _layer_norm(h, self.f["emb_ln_g"], self.f["emb_ln_b"])
 
+    def _native_ops(self, h):
+        """Whether the f32 operators between the linears run on this library's kernels (heads of
+        64 channels, a hidden size its layer norm takes)."""
+        return h == 64 * self.heads and h <= 2048
+
+    def _attention(self, qkv):
+        """attention() of the quantized layer: this library's kernel where it applies."""
+        if self._native_ops(qkv.shape[-1] // 3):
+            return K.attention(qkv, self.heads)
+        return self.attention(qkv)
+
+    def _norm(self, x, name):
+        """The layer norms of the quantized layer, likewise."""
+        g, b = self.f[name + "_g"], self.f[name + "_b"]
+        if self._native_ops(x.shape[-1]):
+            return K.layer_norm(x, g, b, 1e-12)
+        return _layer_norm(x, g, b)
+
     def attention(self, qkv):
         """softmax(q k^T / sqrt(d)) v in fp32, PyTorch's fused kernel.  qkv: [B, S, 3H] -> [B, S, H].
         (Written out as two batched products, a scale and a softmax the same arithmetic is nine
@@ -214,13 +232,33 @@ class QuantBertLayer:
         shape = x.shape
         x2 = x.reshape(-1, shape[-1])
         x_q = self.be.quantize(x2, self.s_in[name])
-        r2 = residual.reshape(-1, residual.shape[-1])
-        y = self.be.qlinear_dequantized_residual(x_q, self.w_q[name], self.bias[name],
-                                                 self.s_in[name], self.sw[name],
-                                                 self.s_out[name], r2)
+        y = self._residual_gemm(name, x_q, residual)
         if rec is not None:
             rec[name] = dict(x=x2, x_q=x_q, y_plus_residual=y)
         return y.reshape(*shape[:-1], y.shape[-1])
+
+    def _residual_gemm(self, name, x_q, residual):
+        return self.be.qlinear_dequantized_residual(
+            x_q, self.w_q[name], self.bias[name], self.s_in[name], self.sw[name],
+            self.s_out[name], residual.reshape(-1, residual.shape[-1]))
+
+    def _forward_fused(self, h):
+        """forward() with every operator in the pass of a neighbour: the quantize in front of a
+        linear in the kernel that produces its input, what follows a linear in its epilogue --
+        eight launches, the bits of the separate operators."""
+        f = self.f
+        b, s, c = h.shape
+        h2 = h.reshape(-1, c)
+        x_q = self.be.quantize(h2, self.s_in["qkv"])
+        qkv = self.be.qlinear_dequantized(x_q, self.w_q["qkv"], self.bias["qkv"], self.s_in["qkv"],
+                                          self.sw["qkv"], self.s_out["qkv"])
+        ctx_q = K.attention(qkv.reshape(b, s, 3 * c), self.heads, self.s_in["out"])
+        pre1 = self._residual_gemm("out", ctx_q.reshape(-1, c), h2)
+        h1, h1_q = K.layer_norm(pre1, f["ln1_g"], f["ln1_b"], 1e-12, self.s_in["ffn1"])
+        mid_q = self.be.qlinear_table(h1_q, self.w_q["ffn1"], self.bias["ffn1"], self.s_in["ffn1"],
+                                      self.sw["ffn1"], self.s_out["ffn1"], self.gelu_table)
+        pre2 = self._residual_gemm("ffn2", mid_q, h1)
+        return K.layer_norm(pre2, f["ln2_g"], f["ln2_b"], 1e-12).reshape(b, s, c)
 
     def _ffn_fused(self, h1, rec):
         """quantize -> ffn1 -> [table: dequantize, GELU, quantize] -> ffn2 -> dequantize."""
@@ -288,19 +326,21 @@ class QuantBertLayer:
     def forward(self, h, record=None):
         if not self.s_in:
             raise RuntimeError("calibrate() first")
+        if self.fuse_epilogue and record is None and self._native_ops(h.shape[-1]):
+            return self._forward_fused(h)
         qkv = self._qlinear("qkv", h, record)
-        ctx = self.attention(qkv)
+        ctx = self._attention(qkv)
         if self.fuse_epilogue:
             pre1 = self._qlinear_residual("out", ctx, h, record)
-            h1 = _layer_norm(pre1, self.f["ln1_g"], self.f["ln1_b"])
+            h1 = self._norm(pre1, "ln1")
             pre2 = self._ffn_fused(h1, record)       # h1 + ffn2(gelu(ffn1(h1)))
-            return _layer_norm(pre2, self.f["ln2_g"], self.f["ln2_b"])
+            return self._norm(pre2, "ln2")
         attn = self._qlinear("out", ctx, record)
-        h1 = _layer_norm(h + attn, self.f["ln1_g"], self.f["ln1_b"])
+        h1 = self._norm(h + attn, "ln1")
         if self.fuse_gelu:
             f2 = self._ffn_fused(h1, record)
         else:
             f1 = self._qlinear("ffn1", h1, record)
             g = torch.nn.functional.gelu(f1)
             f2 = self._qlinear("ffn2", g, record)
-        return _layer_norm(h1 + f2, self.f["ln2_g"], self.f["ln2_b"])
+        return self._norm(h1 + f2, "ln2")

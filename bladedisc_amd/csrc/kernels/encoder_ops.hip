@@ -1,0 +1,309 @@
+// The f32 operators between the quantized linears of a transformer encoder layer, each with the
+// quantize that follows it in the same pass: softmax(q k^T / sqrt(d)) v, and layer normalisation.
+#include "dq8_common.h"
+#include "disc_q8.h"
+#include "q8_elementwise.h"
+
+#pragma clang fp contract(off)
+
+namespace dq8 {
+namespace {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+// int8 of four values, dq8_quantize's bits (zero point 0, half to even)
+__device__ __forceinline__ uint32_t quantize4(const v4f& v, float s, float y, bool fast) {
+  using namespace elementwise;
+  const float4 x = make_float4(v[0], v[1], v[2], v[3]);
+  if (fast) return quant4_pack_rne(div4_by_constant(x, s, y));
+  return pack4(quant_one<1>(x.x, s, 0.f, -128.f, 127.f), quant_one<1>(x.y, s, 0.f, -128.f, 127.f),
+               quant_one<1>(x.z, s, 0.f, -128.f, 127.f), quant_one<1>(x.w, s, 0.f, -128.f, 127.f));
+}
+
+// ------------------------------------------------------------------ attention
+// Heads of 64 channels, f32 throughout, on v_mfma_f32_16x16x4_f32 (64 flops per clock and SIMD, the
+// bound: 8 x 128 x 12 heads are 0.4 Gflop = 2.6 us of the chip's f32 matrix rate).  A wave takes 16
+// query rows, a workgroup up to four waves (64 rows) of one head; keys and values pass through LDS
+// 64 at a time, the next 64 on their way in registers meanwhile.
+//  * S^T = K Q^T: the keys are the MFMA's row operand, so that a lane (r, g) = (lane % 16, lane / 16)
+//    holds the scores of query r with keys 4 g .. 4 g + 3 of a 16-key tile.  The 64 channels are
+//    summed in the order {s, 16 + s, 32 + s, 48 + s}, s = 0 .. 15: group g then needs channels
+//    16 g .. 16 g + 15 of its row, four 16-byte reads.
+//  * O^T = V^T P^T: that same lane's probabilities are, as they are, the column operand of the step
+//    over keys {v, 4 + v, 8 + v, 12 + v}; nothing is exchanged between lanes.  Channel 4 i + t is
+//    row i of output tile t, so that a row operand is read 16 bytes at a time and a lane ends up with
+//    16 consecutive channels of its query: one 16-byte store once quantized.
+//  * The softmax is the online form, a maximum and a sum per query over the four lanes that share
+//    it, once per 64 keys.
+// The heads of all sequences run fastest over the workgroups: those of one head then meet on one XCD
+// (workgroups go to the eight in turn, and the heads are most often a multiple of eight or four), and
+// its keys and values are read from memory into one L2.
+// LDS rows of keys are 272 bytes apart: 16 lanes reading the same channels of 16 keys then cover all
+// 64 banks.
+constexpr int kHead = 64, kBlock = 64;
+constexpr int kKeyPitch = kHead + 4;       // floats
+
+template <int WAVES, bool QUANT>
+__global__ void __launch_bounds__(WAVES * 64)
+attention_f32_kernel(const float* __restrict__ qkv, int S, uint32_t all_heads, int heads, float scale_log2,
+                     float* __restrict__ out, int8_t* __restrict__ out_q, const float* __restrict__ q_scale) {
+  __shared__ __attribute__((aligned(16))) float keys[kBlock * kKeyPitch];
+  __shared__ __attribute__((aligned(16))) float vals[kBlock * kHead];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const uint32_t bh = blockIdx.x % all_heads, tile = blockIdx.x / all_heads;
+  const int b = (int)(bh / heads), h = (int)(bh % heads);
+  const int64_t row3 = 3 * (int64_t)heads * kHead;           // floats between two tokens
+  const float* base = qkv + (int64_t)b * S * row3 + h * kHead;
+  const int q0 = ((int)tile * WAVES + wave) * 16;
+
+  // the wave's queries: lane (r, g) channels 16 g .. 16 g + 15 of row r, scaled by log2(e) / sqrt(d)
+  v4f q[4];
+  {
+    const int row = q0 + r < S ? q0 + r : S - 1;
+    const v4f* p = reinterpret_cast<const v4f*>(base + row * row3 + 16 * g);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q[i] = p[i];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q[i] *= scale_log2;
+  }
+
+  // 64 keys and values: 16 lanes per row
+  const int lrow = threadIdx.x >> 4, lcol = (threadIdx.x & 15) * 4;
+  constexpr int step = WAVES * 4;                            // rows a pass covers
+  constexpr int kPasses = (kBlock + step - 1) / step;
+  v4f kreg[kPasses], vreg[kPasses];
+  auto fetch = [&](int key0) {
+#pragma unroll
+    for (int i = 0; i < kPasses; ++i) {
+      const int row = lrow + i * step;
+      kreg[i] = vreg[i] = (v4f){0.f, 0.f, 0.f, 0.f};        // (past the sequence: a zero probability times this)
+      if (row < kBlock && key0 + i * step < S) {
+        const int key = key0 + row < S ? key0 + row : S - 1;
+        const float* p = base + key * row3 + (int64_t)heads * kHead + lcol;
+        kreg[i] = *reinterpret_cast<const v4f*>(p);
+        vreg[i] = *reinterpret_cast<const v4f*>(p + (int64_t)heads * kHead);
+      }
+    }
+  };
+  auto commit = [&]() {
+#pragma unroll
+    for (int i = 0; i < kPasses; ++i) {
+      const int row = lrow + i * step;
+      if (row < kBlock) {
+        *reinterpret_cast<v4f*>(&keys[row * kKeyPitch + lcol]) = kreg[i];
+        *reinterpret_cast<v4f*>(&vals[row * kHead + lcol]) = vreg[i];
+      }
+    }
+  };
+
+  v4f o[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) o[t] = (v4f){0.f, 0.f, 0.f, 0.f};
+  float m = -__builtin_inff(), l = 0.f;
+  fetch(0);
+  for (int key0 = 0; key0 < S; key0 += kBlock) {
+    __syncthreads();                       // the block before has been read
+    commit();
+    __syncthreads();
+    if (key0 + kBlock < S) fetch(key0 + kBlock);
+    // scores of 64 keys, 16 per lane (already in units of log2)
+    v4f s[4];
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) {
+      s[kt] = (v4f){0.f, 0.f, 0.f, 0.f};
+      if (key0 + kt * 16 >= S) continue;                    // (uniform: tiles past the sequence)
+      const v4f* kp = reinterpret_cast<const v4f*>(&keys[(kt * 16 + r) * kKeyPitch + 16 * g]);
+      v4f k[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) k[i] = kp[i];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) s[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i][c], q[i][c], s[kt], 0, 0, 0);
+    }
+    float top = m;
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        if (key0 + kt * 16 + 4 * g + v >= S) s[kt][v] = -__builtin_inff();
+        top = fmaxf(top, s[kt][v]);
+      }
+    top = fmaxf(top, __shfl_xor(top, 16, 64));
+    top = fmaxf(top, __shfl_xor(top, 32, 64));
+    const float keep = __builtin_amdgcn_exp2f(m - top);     // (m = -inf at first: 0)
+    m = top;
+    float sum = 0.f;
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        s[kt][v] = __builtin_amdgcn_exp2f(s[kt][v] - top);
+        sum += s[kt][v];
+      }
+    l = l * keep + sum;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) o[t] *= keep;
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) {
+      if (key0 + kt * 16 >= S) continue;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const v4f vv = *reinterpret_cast<const v4f*>(&vals[(kt * 16 + 4 * g + v) * kHead + 4 * r]);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[t], s[kt][v], o[t], 0, 0, 0);
+      }
+    }
+  }
+  // the four lanes of a query have each summed their own keys
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (q0 + r >= S) return;
+  const float inv = 1.0f / l;
+  // channel 16 g + 4 v + t is element v of tile t
+  v4f y[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) y[v][t] = o[t][v] * inv;
+  const int64_t at = ((int64_t)b * S + q0 + r) * heads * kHead + h * kHead + 16 * g;
+  if (QUANT) {
+    const float sc = q_scale[0];
+    const float rcp = 1.0f / sc;
+    const bool fast = elementwise::divisor_in_fast_range(sc);
+    uint32_t w[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) w[v] = quantize4(y[v], sc, rcp, fast);
+    *reinterpret_cast<uint4*>(out_q + at) = make_uint4(w[0], w[1], w[2], w[3]);
+  } else {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) *reinterpret_cast<v4f*>(out + at + 4 * v) = y[v];
+  }
+}
+
+// ------------------------------------------------------------------ layer normalisation
+// A wave per row, up to 2048 columns in its registers: mean, then the variance of the differences,
+// then (x - mean) * rstd * gamma + beta, written as f32, quantized, or both -- the row is read once
+// and the quantize that follows costs its one byte per element.  Bound by the launch at encoder
+// sizes (1024 x 768: 3 MB read).
+template <int N4, bool QUANT>
+__global__ void __launch_bounds__(256)
+layernorm_f32_kernel(const float* __restrict__ x, int64_t rows, int cols, const float* __restrict__ gamma,
+                     const float* __restrict__ beta, float eps, float* __restrict__ out,
+                     int8_t* __restrict__ out_q, const float* __restrict__ q_scale) {
+  const int lane = threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const v4f* p = reinterpret_cast<const v4f*>(x + row * cols);
+  const int n4 = cols >> 2;
+  v4f v[N4];
+#pragma unroll
+  for (int i = 0; i < N4; ++i) v[i] = lane + 64 * i < n4 ? p[lane + 64 * i] : (v4f){0.f, 0.f, 0.f, 0.f};
+  v4f ga[N4], be[N4];
+#pragma unroll
+  for (int i = 0; i < N4; ++i) {
+    const int c = lane + 64 * i < n4 ? lane + 64 * i : 0;
+    ga[i] = reinterpret_cast<const v4f*>(gamma)[c];
+    be[i] = reinterpret_cast<const v4f*>(beta)[c];
+  }
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < N4; ++i) sum += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+  const float mean = sum / (float)cols;
+  float sq = 0.f;
+#pragma unroll
+  for (int i = 0; i < N4; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float d = lane + 64 * i < n4 ? v[i][e] - mean : 0.f;
+      v[i][e] = d;
+      sq += d * d;
+    }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) sq += __shfl_xor(sq, off, 64);
+  const float rstd = 1.0f / __builtin_sqrtf(sq / (float)cols + eps);
+  float sc = 1.f, rcp = 1.f;
+  bool fast = true;
+  if (QUANT) {
+    sc = q_scale[0];
+    rcp = 1.0f / sc;
+    fast = elementwise::divisor_in_fast_range(sc);
+  }
+#pragma unroll
+  for (int i = 0; i < N4; ++i) {
+    if (lane + 64 * i >= n4) continue;
+    const v4f y = v[i] * rstd * ga[i] + be[i];
+    if (out) reinterpret_cast<v4f*>(out + row * cols)[lane + 64 * i] = y;
+    if (QUANT) reinterpret_cast<uint32_t*>(out_q + row * cols)[lane + 64 * i] = quantize4(y, sc, rcp, fast);
+  }
+}
+
+template <int N4>
+void launch_layernorm(const float* x, int64_t rows, int cols, const float* gamma, const float* beta, float eps,
+                      float* out, int8_t* out_q, const float* q_scale, hipStream_t st) {
+  const dim3 grid((unsigned)ceil_div(rows, 4)), block(256);
+  if (out_q)
+    hipLaunchKernelGGL((layernorm_f32_kernel<N4, true>), grid, block, 0, st, x, rows, cols, gamma, beta, eps, out,
+                       out_q, q_scale);
+  else
+    hipLaunchKernelGGL((layernorm_f32_kernel<N4, false>), grid, block, 0, st, x, rows, cols, gamma, beta, eps,
+                       out, out_q, q_scale);
+}
+
+}  // namespace
+}  // namespace dq8
+
+using namespace dq8;
+
+extern "C" int dq8_attention_f32(const float* qkv, int64_t batch, int64_t seq, int64_t heads,
+                                 int64_t head_dim, float* out, int8_t* out_q, const float* q_scale,
+                                 void* stream) {
+  clear_error();
+  DQ8_REQUIRE(batch >= 0 && seq >= 0 && heads >= 0, "dq8_attention_f32: negative size");
+  DQ8_REQUIRE(head_dim == kHead, "dq8_attention_f32: heads of 64 channels only");
+  if (batch == 0 || seq == 0 || heads == 0) return 0;
+  DQ8_REQUIRE(qkv && (out || out_q), "dq8_attention_f32: null pointer");
+  DQ8_REQUIRE(!(out && out_q) && (!out_q || q_scale), "dq8_attention_f32: an f32 result, or an int8 one and its scale");
+  DQ8_REQUIRE(aligned(qkv, 16) && aligned(out, 16) && aligned(out_q, 16), "dq8_attention_f32: 16-byte aligned tensors");
+  // waves of 16 queries: four to a workgroup, fewer for a short sequence
+  const int waves = (int)(seq >= 49 ? 4 : ceil_div(seq, 16));
+  const int64_t tiles = ceil_div(seq, 16 * waves);
+  DQ8_REQUIRE(seq < (1 << 24) && batch < (1 << 24) && heads < (1 << 24) && batch * heads < (1LL << 31) / tiles,
+              "dq8_attention_f32: too large");
+  const dim3 grid((unsigned)(batch * heads * tiles)), block(64 * waves);
+  const float scale_log2 = 1.4426950408889634f / 8.0f;      // log2(e) / sqrt(64)
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, block, 0, (hipStream_t)stream, qkv, (int)seq, (uint32_t)(batch * heads), (int)heads, scale_log2, out, out_q,
+                       q_scale);
+  };
+  switch (waves) {
+    case 1: launch(out_q ? attention_f32_kernel<1, true> : attention_f32_kernel<1, false>); break;
+    case 2: launch(out_q ? attention_f32_kernel<2, true> : attention_f32_kernel<2, false>); break;
+    case 3: launch(out_q ? attention_f32_kernel<3, true> : attention_f32_kernel<3, false>); break;
+    default: launch(out_q ? attention_f32_kernel<4, true> : attention_f32_kernel<4, false>); break;
+  }
+  return check_hip(hipGetLastError(), "dq8_attention_f32 launch");
+}
+
+extern "C" int dq8_layernorm_f32(const float* x, int64_t rows, int64_t cols, const float* gamma,
+                                 const float* beta, float eps, float* out, int8_t* out_q,
+                                 const float* q_scale, void* stream) {
+  clear_error();
+  DQ8_REQUIRE(rows >= 0 && cols >= 0, "dq8_layernorm_f32: negative size");
+  if (rows == 0 || cols == 0) return 0;
+  DQ8_REQUIRE(cols % 4 == 0 && cols <= 2048, "dq8_layernorm_f32: up to 2048 columns, a multiple of 4");
+  DQ8_REQUIRE(x && gamma && beta && (out || out_q) && (!out_q || q_scale), "dq8_layernorm_f32: null pointer");
+  DQ8_REQUIRE(aligned(x, 16) && aligned(gamma, 16) && aligned(beta, 16) && aligned(out, 16) && aligned(out_q, 4),
+              "dq8_layernorm_f32: 16-byte aligned tensors");
+  DQ8_REQUIRE(rows < (1LL << 32), "dq8_layernorm_f32: too many rows");
+  hipStream_t st = (hipStream_t)stream;
+  const int n = (int)ceil_div(cols, 256);
+  if (n <= 1) launch_layernorm<1>(x, rows, (int)cols, gamma, beta, eps, out, out_q, q_scale, st);
+  else if (n <= 3) launch_layernorm<3>(x, rows, (int)cols, gamma, beta, eps, out, out_q, q_scale, st);
+  else if (n == 4) launch_layernorm<4>(x, rows, (int)cols, gamma, beta, eps, out, out_q, q_scale, st);
+  else launch_layernorm<8>(x, rows, (int)cols, gamma, beta, eps, out, out_q, q_scale, st);
+  return check_hip(hipGetLastError(), "dq8_layernorm_f32 launch");
+}

@@ -592,6 +592,59 @@ PyObject* py_qconv2d(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// attention(qkv [.., seq, 3 heads 64], heads, scale or None): int8 result with a scale, else f32
+PyObject* py_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    arguments("attention", n, 3);
+    const Tensor x = dense(device_tensor(a[0]));
+    if (x.scalar_type() != ScalarType::Float || x.dim() != 3)
+      raise(PyExc_TypeError, "attention takes a float32 tensor of rank 3");
+    const int64_t heads = integer(a[1]), h3 = x.size(2);
+    if (heads <= 0 || h3 % (3 * heads) != 0) raise(PyExc_ValueError, "attention: heads do not divide the channels");
+    const Tensor s = optional_device_tensor(a[2]);
+    const Tensor out = empty({x.size(0), x.size(1), h3 / 3}, s.defined() ? ScalarType::Char : ScalarType::Float,
+                             x.device());
+    void* st = stream();
+    launch("dq8_attention_f32", [&] {
+      return dq8_attention_f32((const float*)ptr(x), x.size(0), x.size(1), heads, h3 / 3 / heads,
+                               s.defined() ? nullptr : (float*)ptr(out), s.defined() ? (int8_t*)ptr(out) : nullptr,
+                               (const float*)ptr(s), st);
+    });
+    return THPVariable_Wrap(out);
+  });
+}
+
+// layer_norm(x, gamma, beta, eps, scale or None): y, or (y, int8 of y) with a scale
+PyObject* py_layer_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    arguments("layer_norm", n, 5);
+    const Tensor x = dense(device_tensor(a[0]));
+    const Tensor &g = device_tensor(a[1]), &b = device_tensor(a[2]);
+    if (x.scalar_type() != ScalarType::Float || g.scalar_type() != ScalarType::Float ||
+        b.scalar_type() != ScalarType::Float || x.dim() < 1 || !g.is_contiguous() || !b.is_contiguous() ||
+        g.numel() != x.size(-1) || b.numel() != x.size(-1))
+      raise(PyExc_TypeError, "layer_norm takes float32 tensors, weight and bias of the last dimension");
+    const float eps = (float)PyFloat_AsDouble(a[3]);
+    if (PyErr_Occurred()) throw PyFailure{};
+    const Tensor s = optional_device_tensor(a[4]);
+    const int64_t cols = x.size(-1), rows = cols ? x.numel() / cols : 0;
+    const Tensor y = empty(x.sizes(), ScalarType::Float, x.device());
+    Tensor q;
+    if (s.defined()) q = empty(x.sizes(), ScalarType::Char, x.device());
+    void* st = stream();
+    launch("dq8_layernorm_f32", [&] {
+      return dq8_layernorm_f32((const float*)ptr(x), rows, cols, (const float*)ptr(g), (const float*)ptr(b), eps,
+                               (float*)ptr(y), (int8_t*)ptr(q), (const float*)ptr(s), st);
+    });
+    if (!s.defined()) return THPVariable_Wrap(y);
+    PyObject* r = PyTuple_New(2);
+    if (!r) throw PyFailure{};
+    PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(y));
+    PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(q));
+    return r;
+  });
+}
+
 PyMethodDef kMethods[] = {
 #define DQ8_METHOD(name, fn) {name, (PyCFunction)(void (*)(void))fn, METH_FASTCALL, nullptr}
     DQ8_METHOD("quantize", py_quantize),
@@ -604,6 +657,8 @@ PyMethodDef kMethods[] = {
     DQ8_METHOD("qgemm", py_qgemm),
     DQ8_METHOD("qlinear_f32", py_qlinear_f32),
     DQ8_METHOD("qconv2d", py_qconv2d),
+    DQ8_METHOD("attention", py_attention),
+    DQ8_METHOD("layer_norm", py_layer_norm),
 #undef DQ8_METHOD
     {nullptr, nullptr, 0, nullptr}};
 

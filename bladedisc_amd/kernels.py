@@ -254,6 +254,19 @@ def qlinear_f32(x, w, epilogue, sx, sw=None, so=None, bias=None, zo=0,
     return _native().qlinear_f32(x, w, epilogue, sx, sw, so, bias, zo, round_mode, out)
 
 
+def attention(qkv, heads, scale=None):
+    """softmax(q k^T / sqrt(64)) v of a merged f32 projection [B, S, 3 * heads * 64] -> [B, S,
+    heads * 64], f32 throughout; with a one-element device `scale` the result is quantized to int8
+    in the same pass (the bits of quantize(., scale, 0) behind it)."""
+    return _native().attention(qkv, heads, scale)
+
+
+def layer_norm(x, weight, bias, eps=1e-5, scale=None):
+    """Layer normalisation over the last dimension (f32, up to 2048 columns, a multiple of 4);
+    with a one-element device `scale` returns (y, quantize(y, scale, 0)) from one pass."""
+    return _native().layer_norm(x, weight, bias, eps, scale)
+
+
 NHWC_OHWI = (0, 3, 1, 2, 3, 0, 1, 2, 0, 3, 1, 2)
 
 

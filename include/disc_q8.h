@@ -398,6 +398,22 @@ int dq8_weight_only_qgemm(const void* x, int x_dtype, int64_t ldx, const void* w
 int dq8_weight_only_undo_compiler_layout(const uint8_t* reordered, uint8_t* w_nk, int64_t K,
                                          int64_t N, void* stream);
 
+/* ---- f32 operators between quantized linears ------------------------------ */
+
+/* softmax(q k^T / sqrt(head_dim)) v of qkv [batch, seq, 3 * heads * head_dim] (device f32, q, k and
+ * v next to each other as a merged projection leaves them) to [batch, seq, heads * head_dim]: either
+ * out (f32), or out_q = dq8_quantize of it with scale q_scale[0], zero point 0, half to even
+ * (mhlo_disc.quantize in front of the linear that follows, taken into the pass).  head_dim 64;
+ * f32 throughout. */
+int dq8_attention_f32(const float* qkv, int64_t batch, int64_t seq, int64_t heads, int64_t head_dim,
+                      float* out, int8_t* out_q, const float* q_scale, void* stream);
+
+/* (x - mean) / sqrt(var + eps) * gamma + beta over the rows of x [rows, cols] (device f32), to
+ * out (f32), to out_q = dq8_quantize of that, or to both.  Up to 2048 columns, a multiple of 4. */
+int dq8_layernorm_f32(const float* x, int64_t rows, int64_t cols, const float* gamma,
+                      const float* beta, float eps, float* out, int8_t* out_q, const float* q_scale,
+                      void* stream);
+
 /* ---- int8 convolution (rank 4) ---------------------------------------- */
 
 /* Implicit-GEMM convolution.  Layouts are described exactly as ral_qconv's

@@ -2194,3 +2194,30 @@ def test_quantize_any_size_type_and_alignment(K, shape, axis):
         if name in ("int8", "uint8"):
             xf = dev(xin.astype(np.float32))
             np.testing.assert_array_equal(host(K.fake_quant(xf, dev(scale), dev(zp), axis=axis, qmin=lo, qmax=hi)), want_f)
+
+
+@pytest.mark.parametrize("b,s,heads", [(1, 1, 1), (2, 8, 12), (3, 17, 2), (1, 49, 3), (2, 64, 1), (1, 65, 12), (2, 333, 5)])
+def test_attention_equals_softmax_of_the_scores(K, b, s, heads):
+    """Edges of the 16-query and 64-key tiles, against the same in f64; the fused quantize is the
+    quantize of the f32 result."""
+    qkv = torch.randn(b, s, 3 * heads * 64, generator=torch.Generator().manual_seed(s)) * 1.5
+    q, k, v = (t.double().reshape(b, s, heads, 64).transpose(1, 2) for t in qkv.chunk(3, dim=-1))
+    want = (torch.softmax(q @ k.transpose(2, 3) / 8.0, -1) @ v).transpose(1, 2).reshape(b, s, heads * 64)
+    got = K.attention(qkv.cuda(), heads)
+    torch.testing.assert_close(got.cpu().double(), want, rtol=1e-5, atol=1e-5)
+    scale = torch.full((1,), 0.02, device="cuda")
+    assert torch.equal(K.attention(qkv.cuda(), heads, scale), K.quantize(got, scale, torch.zeros(1, dtype=torch.int32, device="cuda")))
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 4), (5, 252), (3, 260), (9, 768), (1026, 1000), (7, 1028), (2, 2048)])
+def test_layer_norm_with_and_without_its_quantize(K, rows, cols):
+    g = torch.Generator().manual_seed(cols)
+    x = torch.randn(rows, cols, generator=g) * 3 + 1
+    gamma, beta = torch.randn(cols, generator=g), torch.randn(cols, generator=g)
+    want = torch.nn.functional.layer_norm(x.double(), (cols,), gamma.double(), beta.double(), 1e-12)
+    y = K.layer_norm(x.cuda(), gamma.cuda(), beta.cuda(), 1e-12)
+    torch.testing.assert_close(y.cpu().double(), want, rtol=1e-5, atol=2e-5)
+    scale = torch.full((1,), 0.03, device="cuda")
+    y2, q = K.layer_norm(x.cuda(), gamma.cuda(), beta.cuda(), 1e-12, scale)
+    assert torch.equal(y2, y)
+    assert torch.equal(q, K.quantize(y, scale, torch.zeros(1, dtype=torch.int32, device="cuda")))
