@@ -39,8 +39,9 @@
 //  * wo_skinny_kernel: M <= 128 rows against 32 output channels per workgroup, the k range dealt
 //    over the waves and the partial sums added through LDS (bound by the weight bytes: 1 byte
 //    per weight from HBM);
-//  * wo_generic_kernel: one output per thread, any layout and alignment (also weights left as
-//    [K, N]).
+//  * wo_exact_f32_kernel: f32 activations on rows off 16 bytes (f16 ones: the LDS kernels' RAGGED
+//    forms);
+//  * wo_generic_kernel: one output per thread, fewer than 16 of k or weights left as [K, N].
 #include <algorithm>
 
 #include "dq8_common.h"
@@ -75,7 +76,22 @@ struct WoParams {
   // and, when `partial` is set, leaves its f32 sums in partial[y][M][N] for the reduction kernel
   float* partial;
   int k_split;          // a multiple of 64; K when the k range is not split
+  bool ragged;          // rows that are not multiples of 16 bytes, 16-byte aligned
 };
+
+// RAGGED kernels: rows of any length from 16 on and any alignment.  A row's 16-element chunk that
+// is not whole is read as the row's last 16 elements, of both operands, and the activations that a
+// chunk before it holds already are made zero (the weights that meet them are finite).
+typedef unsigned u4_any __attribute__((ext_vector_type(4), aligned(1)));
+__device__ __forceinline__ u4 load_any(const uint8_t* base, unsigned off) {
+  return *reinterpret_cast<const u4_any*>(base + off);
+}
+// the first z of eight halves made zero
+__device__ __forceinline__ u4 zero_first(u4 q, int z) {
+#pragma unroll
+  for (int d = 0; d < 4; ++d) q[d] = z >= 2 * d + 2 ? 0u : z == 2 * d + 1 ? q[d] & 0xffff0000u : q[d];
+  return q;
+}
 
 template <typename T>
 __device__ __forceinline__ float to_f32(T v) {
@@ -274,10 +290,15 @@ __global__ void __launch_bounds__(256) wo_tile_kernel(const WoParams p) {
 // f32 activations (XT = float) are split on their way into LDS, x = hi + lo with hi = half(x)
 // and lo = half(x - hi), into two half tiles of the same layout; every weight fragment is
 // multiplied with both.
-template <typename XT, int WM, int FM, int FN, int SETS>
+//
+// RAGGED (f16): plain loads of any alignment in place of the buffer loads; only the k tile with the
+// end of the rows is handled differently (M = 512, 2047 -> 3001, one output per thread before:
+// 11.9 ms).
+template <typename XT, int WM, int FM, int FN, int SETS, bool RAGGED = false>
 __global__ void __launch_bounds__(WM * 128, (WM == 1 || sizeof(XT) == 4) ? 1 : 2)
     wo_lds_kernel(const WoParams p) {
   constexpr bool F32 = sizeof(XT) == 4;
+  static_assert(!RAGGED || !F32, "f32 activations: wo_exact_f32_kernel");
   constexpr int BM = WM * FM * 32, BN = 2 * FN * 32, BK = 64;
   constexpr int NT = WM * 128;                           // WM x 2 waves
   constexpr int XL = F32 ? 16 : 8;                       // lanes (16 bytes each) per activation row
@@ -328,7 +349,7 @@ __global__ void __launch_bounds__(WM * 128, (WM == 1 || sizeof(XT) == 4) ? 1 : 2
   for (int i = 0; i < XP; ++i) {
     const int row = tid / XL + (NT / XL) * i;
     const int sx = (row ^ (row >> 3)) & 7;
-    xo[i] = (int)((int64_t)min(row, mrows - 1) * p.ldx * sizeof(XT)) + 16 * xc;
+    xo[i] = (int)((int64_t)min(row, mrows - 1) * p.ldx * sizeof(XT)) + (RAGGED ? 0 : 16 * xc);
     // (four floats become four halves: half of the 16-byte chunk xc / 2)
     xl[i] = F32 ? row * 128 + (((xc >> 1) ^ sx) << 4) + 8 * (xc & 1)
                 : row * 128 + ((xc ^ sx) << 4);
@@ -339,13 +360,24 @@ __global__ void __launch_bounds__(WM * 128, (WM == 1 || sizeof(XT) == 4) ? 1 : 2
   for (int i = 0; i < WP; ++i) {
     const int row = (tid >> 2) + (NT / 4) * i;
     const int sw = (row ^ (row >> 3)) & 7;
-    wo[i] = (int)((int64_t)min(row, nrows - 1) * p.w_sn) + 16 * wc;
+    wo[i] = (int)((int64_t)min(row, nrows - 1) * p.w_sn) + (RAGGED ? 0 : 16 * wc);
     wl[i] = row * 128 + (((2 * wc) ^ sw) << 4);
     wl1[i] = row * 128 + (((2 * wc + 1) ^ sw) << 4);
     cpark[i] = centre(p, n0 + min(row, nrows - 1));
   }
   u4 xr[SETS][XP], wr[SETS][WP];
+  const uint8_t* xbase = reinterpret_cast<const uint8_t*>(static_cast<const XT*>(p.x) + (int64_t)m0 * p.ldx);
+  const uint8_t* wbase = p.w + (int64_t)n0 * p.w_sn;
   auto fetch = [&](u4* xq, u4* wq, int k0) {
+    if constexpr (RAGGED) {
+      const unsigned kx = min(kbeg + k0 + 16 * (xc >> 1), p.K - 16) + 8 * (xc & 1);
+      const unsigned kw = min(kbeg + k0 + 16 * wc, p.K - 16);
+#pragma unroll
+      for (int i = 0; i < XP; ++i) xq[i] = load_any(xbase, (unsigned)xo[i] + 2 * kx);
+#pragma unroll
+      for (int i = 0; i < WP; ++i) wq[i] = load_any(wbase, (unsigned)wo[i] + kw);
+      return;
+    }
     const bool xv = k0 + (F32 ? 4 : 8) * xc < klen, wv = k0 + 16 * wc < klen;   // K % 16 == 0
 #pragma unroll
     for (int i = 0; i < XP; ++i)
@@ -355,7 +387,13 @@ __global__ void __launch_bounds__(WM * 128, (WM == 1 || sizeof(XT) == 4) ? 1 : 2
     for (int i = 0; i < WP; ++i)
       wq[i] = __builtin_amdgcn_raw_buffer_load_b128(wrs, wv ? wo[i] + k0 : kPast, 0, 0);
   };
-  auto park = [&](const u4* xq, const u4* wq, int stage) {
+  auto park = [&](u4* xq, const u4* wq, int stage, int k0) {
+    if (RAGGED && k0 + BK > klen) {                        // (uniform) the end of the rows
+      const int c16 = kbeg + k0 + 16 * (xc >> 1);
+      const int z = c16 - min(c16, p.K - 16) - 8 * (xc & 1);
+#pragma unroll
+      for (int i = 0; i < XP; ++i) xq[i] = zero_first(xq[i], z);
+    }
 #pragma unroll
     for (int i = 0; i < XP; ++i) {
       if constexpr (F32) {
@@ -472,7 +510,7 @@ __global__ void __launch_bounds__(WM * 128, (WM == 1 || sizeof(XT) == 4) ? 1 : 2
     fetch(xr[u], wr[u], (t + SETS) * BK);
     multiply(u % 2);
     __builtin_amdgcn_sched_barrier(0);
-    park(xr[(u + 1) % SETS], wr[(u + 1) % SETS], (u + 1) % 2);
+    park(xr[(u + 1) % SETS], wr[(u + 1) % SETS], (u + 1) % 2, (t + 1) * BK);
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -480,7 +518,7 @@ __global__ void __launch_bounds__(WM * 128, (WM == 1 || sizeof(XT) == 4) ? 1 : 2
 #pragma unroll
   for (int d = 0; d < SETS; ++d) fetch(xr[d], wr[d], d * BK);
   __builtin_amdgcn_sched_barrier(0);
-  park(xr[0], wr[0], 0);
+  park(xr[0], wr[0], 0, 0);
   __syncthreads();
   __builtin_amdgcn_sched_barrier(0);
   int t = 0;
@@ -689,10 +727,12 @@ __global__ void __launch_bounds__(NW * 64) wo_gemv_kernel(const WoParams p) {
 // weights --, keeps three units in registers on their way from memory, and turns them into MFMA
 // fragments through a piece of LDS that only this wave touches (no barrier: the LDS executes a
 // wave's instructions in order).  f32 activations are split into hi and lo half tiles there.
-// MR: rows staged (16 or 32).
-template <typename XT, int NW, int MR>
+// MR: rows staged (16 or 32).  RAGGED (f16): as in wo_lds_kernel (M = 16, 3001 -> 4096, one output
+// per thread before: 567 us).
+template <typename XT, int NW, int MR, bool RAGGED = false>
 __global__ void __launch_bounds__(NW * 64) wo_skinny_lds_kernel(const WoParams p) {
   constexpr bool F32 = sizeof(XT) == 4;
+  static_assert(!RAGGED || !F32, "f32 activations: wo_exact_f32_kernel");
   constexpr int XL = F32 ? 16 : 8;                       // lanes per activation row of a unit
   constexpr int XP = MR * XL / 64;                       // activation loads per lane and unit
   constexpr int XBYTES = MR * 128 * (F32 ? 2 : 1);       // [hi, then lo] half tiles
@@ -725,7 +765,7 @@ __global__ void __launch_bounds__(NW * 64) wo_skinny_lds_kernel(const WoParams p
     const int row = lane / XL + (64 / XL) * i;
     const int sx = (row ^ (row >> 3)) & 7;
     xok[i] = row < mrows;                                // (rows past M are never stored)
-    xo[i] = (int)((int64_t)min(row, mrows - 1) * p.ldx * sizeof(XT)) + 16 * xc;
+    xo[i] = (int)((int64_t)min(row, mrows - 1) * p.ldx * sizeof(XT)) + (RAGGED ? 0 : 16 * xc);
     xl[i] = F32 ? row * 128 + (((xc >> 1) ^ sx) << 4) + 8 * (xc & 1)
                 : row * 128 + ((xc ^ sx) << 4);
   }
@@ -733,12 +773,23 @@ __global__ void __launch_bounds__(NW * 64) wo_skinny_lds_kernel(const WoParams p
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int row = (lane >> 2) + 16 * i;
-    wo[i] = (int)((int64_t)min(row, nrows - 1) * p.w_sn) + 16 * wc;
+    wo[i] = (int)((int64_t)min(row, nrows - 1) * p.w_sn) + (RAGGED ? 0 : 16 * wc);
     wl[i] = row * 64 + ((wc ^ ((row >> 2) & 3)) << 4);
   }
   const h2 c = centre(p, n0 + min(r, nrows - 1));
   u4 xr[D][XP], wr[D][2];
+  const uint8_t* xbase = static_cast<const uint8_t*>(p.x);
+  const uint8_t* wbase = p.w + (int64_t)n0 * p.w_sn;
   auto fetch = [&](u4* xq, u4* wq, int k0) {
+    if constexpr (RAGGED) {
+      const unsigned kx = min(k0 + 16 * (xc >> 1), p.K - 16) + 8 * (xc & 1);
+      const unsigned kw = min(k0 + 16 * wc, p.K - 16);
+#pragma unroll
+      for (int i = 0; i < XP; ++i) xq[i] = load_any(xbase, (unsigned)xo[i] + 2 * kx);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) wq[i] = load_any(wbase, (unsigned)wo[i] + kw);
+      return;
+    }
     const bool xv = k0 + (F32 ? 4 : 8) * xc < p.K, wv = k0 + 16 * wc < p.K;   // K % 16 == 0
 #pragma unroll
     for (int i = 0; i < XP; ++i)
@@ -748,7 +799,13 @@ __global__ void __launch_bounds__(NW * 64) wo_skinny_lds_kernel(const WoParams p
     for (int i = 0; i < 2; ++i)
       wq[i] = __builtin_amdgcn_raw_buffer_load_b128(wrs, wv ? wo[i] + k0 : kPast, 0, 0);
   };
-  auto park = [&](const u4* xq, const u4* wq) {
+  auto park = [&](u4* xq, const u4* wq, int k0) {
+    if (RAGGED && k0 + 64 > p.K) {                         // (uniform) the end of the rows
+      const int c16 = k0 + 16 * (xc >> 1);
+      const int z = c16 - min(c16, p.K - 16) - 8 * (xc & 1);
+#pragma unroll
+      for (int i = 0; i < XP; ++i) xq[i] = zero_first(xq[i], z);
+    }
 #pragma unroll
     for (int i = 0; i < XP; ++i) {
       if constexpr (F32) {
@@ -805,7 +862,7 @@ __global__ void __launch_bounds__(NW * 64) wo_skinny_lds_kernel(const WoParams p
   for (int k0 = w64; k0 < p.K; k0 += D * NW * 64) {
 #pragma unroll
     for (int u = 0; u < D; ++u) {
-      park(xr[u], wr[u]);
+      park(xr[u], wr[u], k0 + u * NW * 64);
       fetch(xr[u], wr[u], k0 + (D + u) * NW * 64);
       multiply();
       __builtin_amdgcn_sched_barrier(0);
@@ -895,6 +952,69 @@ __global__ void __launch_bounds__(NW * 64) wo_skinny16_kernel(const WoParams p) 
   }
 }
 
+// ---------------------------------------------------------------- f32, rows of any length
+// f32 activations on rows off 16 bytes, in f32 throughout (v_mfma_f32_32x32x2_f32): 32 rows x 32
+// channels per workgroup, k in units of 32 dealt over the waves, operands straight into registers
+// -- the 16 MFMAs of a unit take 1024 clocks, its five loads and sixteen conversions a third of
+// that.  (One output per thread before: M = 16, 3001 -> 4096 567 us, M = 512, 2047 -> 3001 11.9 ms.)
+template <int NW>
+__global__ void __launch_bounds__(NW * 64) wo_exact_f32_kernel(const WoParams p) {
+  __shared__ float red[NW - 1][16][64];
+  typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 31, g = lane >> 5;
+  const int tiles_m = (p.M + 31) / 32;
+  const int m0 = (int)(blockIdx.x % tiles_m) * 32, n0 = (int)(blockIdx.x / tiles_m) * 32;
+  const int n = min(n0 + r, p.N - 1);
+  const float* xrow = static_cast<const float*>(p.x) + (int64_t)min(m0 + r, p.M - 1) * p.ldx;
+  const uint8_t* wrow = p.w + (int64_t)n * p.w_sn;
+  const int zp = (p.zp ? p.zp[n] : 0) + (p.flip ? 128 : 0);
+  f16v acc;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+  f4 xq[2][4];
+  u4 wq[2];
+  auto fetch = [&](int set, int k0) {                      // lane group g: 16 of the unit's k
+    const int k = min(k0 + 16 * g, p.K - 16);
+    wq[set] = load_any(wrow, (unsigned)k);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) xq[set][i] = *reinterpret_cast<const f4_any*>(xrow + k + 4 * i);
+  };
+  auto multiply = [&](int set, int k0) {
+    if (k0 + 32 > p.K) {                                   // (uniform) the end of the rows
+      const int z = k0 + 16 * g - min(k0 + 16 * g, p.K - 16);
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        if (e < z) xq[set][e >> 2][e & 3] = 0.0f;
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int b = (int)(((wq[set][e >> 2] ^ p.flip) >> (8 * (e & 3))) & 0xffu);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xq[set][e >> 2][e & 3], (float)(b - zp), acc, 0, 0, 0);
+    }
+  };
+  const int w32 = __builtin_amdgcn_readfirstlane(wave) * 32;
+  fetch(0, w32);
+  for (int k0 = w32; k0 < p.K; k0 += 2 * NW * 32) {
+    fetch(1, k0 + NW * 32);
+    multiply(0, k0);
+    fetch(0, k0 + 2 * NW * 32);
+    if (k0 + NW * 32 < p.K) multiply(1, k0 + NW * 32);
+  }
+  if (wave > 0) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) red[wave - 1][v][lane] = acc[v];
+  }
+  __syncthreads();
+  if (wave == 0) {
+#pragma unroll
+    for (int w = 1; w < NW; ++w)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[v] += red[w - 1][v][lane];
+    store_frag<float>(p, acc, m0, n0 + r, lane);
+  }
+}
+
 // ---------------------------------------------------------------- any layout, any alignment
 template <typename XT>
 __global__ void __launch_bounds__(256) wo_generic_kernel(const WoParams p) {
@@ -915,11 +1035,11 @@ __global__ void __launch_bounds__(256) wo_generic_kernel(const WoParams p) {
   static_cast<XT*>(p.out)[(int64_t)m * p.ldo + n] = (XT)(acc * s + b);
 }
 
-template <typename XT, int WM, int FM, int FN, int SETS>
+template <typename XT, int WM, int FM, int FN, int SETS, bool RAGGED = false>
 int launch_lds(dim3 grid, const WoParams& p, hipStream_t st) {
   constexpr int lds = 2 * (WM * FM * 32 * (int)(sizeof(XT) / 2) + 2 * FN * 32) * 128;
   static_assert(lds <= 160 * 1024, "the stages fit the LDS");
-  auto kern = wo_lds_kernel<XT, WM, FM, FN, SETS>;
+  auto kern = wo_lds_kernel<XT, WM, FM, FN, SETS, RAGGED>;
   static std::atomic<uint64_t> lds_allowed{0};
   if (lds > 64 * 1024)
     if (int s = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds, &lds_allowed)) return s;
@@ -937,11 +1057,11 @@ int launch_gemv(const WoParams& p, hipStream_t st) {
   return check_hip(hipGetLastError(), "dq8_weight_only_qgemm launch");
 }
 
-template <typename XT, int MR>
+template <typename XT, int MR, bool RAGGED = false>
 int launch_skinny_lds(const WoParams& p, hipStream_t st) {
   constexpr int lds = 8 * (MR * 128 * (int)(sizeof(XT) / 2) + 32 * 64);
   static_assert(lds >= 7 * 16 * 64 * 4, "the partial sums of the waves fit");
-  auto kern = wo_skinny_lds_kernel<XT, 8, MR>;
+  auto kern = wo_skinny_lds_kernel<XT, 8, MR, RAGGED>;
   static std::atomic<uint64_t> lds_allowed{0};
   if (lds > 64 * 1024)
     if (int s = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds, &lds_allowed)) return s;
@@ -1040,8 +1160,10 @@ float big_tile_us(int64_t M, int64_t N, int64_t K) {
 // tiles: M = 32, 4096 -> 11008: 25.5 against 33.5 us; 4096^2: 15.7 against 17.9; 8192^2: 33.1
 // against 31.2) the kernels for few rows, and the 256-row tiles where they are estimated
 // cheaper.
-SplitPlan choose_small(int64_t M, int64_t N, int64_t K, int esz, bool may_split) {
+SplitPlan choose_small(int64_t M, int64_t N, int64_t K, int esz, bool ragged, bool may_split) {
   const SplitPlan none = {-1, 1, (int)K, 0.0f};
+  // (rows off 16 bytes: f16 has the small tiles and the staged small-M kernel, f32 its own kernel)
+  if (ragged) return esz == 4 || M <= 32 ? none : plan_split(M, N, K, esz, may_split);
   // (f32, between: 1536 x 1536 weights, M = 24: 10.0 against 11.2 us, M = 17: 9.5 against 9.2;
   // 768 -> 3072, M = 24: 8.7 against 7.6)
   if (M <= (esz == 4 && K >= 2048 ? 16 : esz == 4 && K >= 1280 ? 23 : 32)) return none;
@@ -1063,6 +1185,10 @@ int launch_form(int form, int splits, const WoParams& p, hipStream_t st) {
   constexpr int kSets = sizeof(XT) == 2 ? 4 : 2;         // (f32 rows are twice the registers)
   const dim3 grid((unsigned)(ceil_div(p.M, kForms[form].bm) * ceil_div(p.N, kForms[form].bn)),
                   (unsigned)splits);
+  if constexpr (sizeof(XT) == 2)
+    if (p.ragged)
+      return form == kForm128x128 ? launch_lds<XT, 2, 2, 2, kSets, true>(grid, p, st)
+                                  : launch_lds<XT, 2, 1, 1, kSets, true>(grid, p, st);
   switch (form) {
     case kForm64x64w2: return launch_lds<XT, 1, 2, 1, kSets>(grid, p, st);
     case kForm128x64: return launch_lds<XT, 2, 2, 1, kSets>(grid, p, st);
@@ -1084,9 +1210,9 @@ int launch(WoParams& p, bool fast, void* scratch, size_t scratch_bytes, hipStrea
                       256 * p.w_sn + (int64_t)p.K + 4096 < (1LL << 31);
   if (fast && lds_ok) {
     const bool have = scratch && aligned(scratch, 16);
-    SplitPlan s = choose_small(p.M, p.N, p.K, (int)sizeof(XT), have);
+    SplitPlan s = choose_small(p.M, p.N, p.K, (int)sizeof(XT), p.ragged, have);
     if (s.splits > 1 && scratch_bytes < split_bytes(s, p.M, p.N))
-      s = choose_small(p.M, p.N, p.K, (int)sizeof(XT), false);
+      s = choose_small(p.M, p.N, p.K, (int)sizeof(XT), p.ragged, false);
     if (s.form >= 0 && s.splits > 1) {
       const int sp = s.splits;
       p.partial = static_cast<float*>(scratch);
@@ -1105,6 +1231,27 @@ int launch(WoParams& p, bool fast, void* scratch, size_t scratch_bytes, hipStrea
     }
     if (s.form >= 0) return launch_form<XT>(s.form, 1, p, st);
   }
+  // (the staged kernel addresses activation and weight rows by 31-bit byte offsets)
+  const bool staged_ok =
+      ((int64_t)(p.M - 1) * p.ldx + p.K) * (int64_t)sizeof(XT) + 65536 < (1LL << 31) &&
+      32 * p.w_sn + (int64_t)p.K + 65536 < (1LL << 31);
+  if (fast && p.ragged) {
+    if constexpr (sizeof(XT) == 4) {
+      const int64_t tiles = ceil_div(p.M, 32) * ceil_div(p.N, 32);
+      // (few tiles: eight waves share the k range, so that most compute units' matrix cores run)
+      if (tiles <= 4 * compute_units()) {
+        hipLaunchKernelGGL(wo_exact_f32_kernel<8>, dim3((unsigned)tiles), dim3(512), 0, st, p);
+        return check_hip(hipGetLastError(), "dq8_weight_only_qgemm launch");
+      }
+      if (tiles < (1LL << 31)) {
+        hipLaunchKernelGGL(wo_exact_f32_kernel<4>, dim3((unsigned)tiles), dim3(256), 0, st, p);
+        return check_hip(hipGetLastError(), "dq8_weight_only_qgemm launch");
+      }
+    } else if (staged_ok && p.M <= 32) {
+      return p.M <= 16 ? launch_skinny_lds<XT, 16, true>(p, st) : launch_skinny_lds<XT, 32, true>(p, st);
+    }
+    fast = false;
+  }
   if (!fast) {
     const int64_t blocks = ceil_div((int64_t)p.M * p.N, 256);
     DQ8_REQUIRE(blocks < (1LL << 31), "dq8_weight_only_qgemm: problem too large");
@@ -1113,10 +1260,6 @@ int launch(WoParams& p, bool fast, void* scratch, size_t scratch_bytes, hipStrea
     const unsigned grid = (unsigned)ceil_div(p.N, 32);
     // (with more than 8 rows every workgroup re-reads the activations, which then outweigh
     // its weights: the narrow form only while the wide one would leave compute units idle)
-    // (the staged kernel addresses activation and weight rows by 31-bit byte offsets)
-    const bool staged_ok =
-        ((int64_t)(p.M - 1) * p.ldx + p.K) * (int64_t)sizeof(XT) + 65536 < (1LL << 31) &&
-        32 * p.w_sn + (int64_t)p.K + 65536 < (1LL << 31);
     // (it needs several 64-deep units per wave to run its pipeline: measured against the two
     // kernels below it wins from 12 rows on at 3072 and 4096 of k -- 4096^2 weights, f16, M = 32:
     // 10.7 against 14.9 us -- and from 5 rows on at 8192 -- M = 16: 16.8 against 22.5 us --, and
@@ -1218,9 +1361,9 @@ extern "C" size_t dq8_weight_only_qgemm_workspace_bytes_ex(int64_t M, int64_t N,
                                                            int tp_b, int x_dtype) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   size_t split = 0;
-  if ((x_dtype == DQ8_DTYPE_F16 || x_dtype == DQ8_DTYPE_F32) && K % 16 == 0 && M < (1LL << 31) &&
+  if ((x_dtype == DQ8_DTYPE_F16 || x_dtype == DQ8_DTYPE_F32) && K >= 16 && M < (1LL << 31) &&
       N < (1LL << 31) && K < (1LL << 31))
-    split = split_bytes(choose_small(M, N, K, x_dtype == DQ8_DTYPE_F32 ? 4 : 2, true), M, N);
+    split = split_bytes(choose_small(M, N, K, x_dtype == DQ8_DTYPE_F32 ? 4 : 2, K % 16 != 0, true), M, N);
   if (!split) return dq8_weight_only_qgemm_workspace_bytes(N, K, tp_b);
   return transposed_bytes(N, K, tp_b) + split;
 }
@@ -1278,10 +1421,10 @@ extern "C" int dq8_weight_only_qgemm(const void* x, int x_dtype, int64_t ldx, co
   p.N = (int)N;
   p.K = (int)K;
   p.flip = w_signed ? 0x80808080u : 0u;
-  // the MFMA kernels want k-contiguous 16-byte aligned rows of both operands; weights given
+  // the MFMA kernels want k-contiguous rows of both operands, of at least 16 elements; weights given
   // as [K, N] are transposed into the caller's scratch first (a runtime does that once per
   // constant weight and passes the result with tp_b = 1 from then on)
-  bool fast = K > 0 && K % 16 == 0 && aligned(x, 16) && (ldx * esz) % 16 == 0;
+  bool fast = K >= 16;
   // what the transposed weights leave of the scratch holds the partial sums of a split launch
   void* rest = workspace;
   size_t rest_bytes = workspace ? workspace_bytes : 0;
@@ -1300,7 +1443,8 @@ extern "C" int dq8_weight_only_qgemm(const void* x, int x_dtype, int64_t ldx, co
       fast = false;
     }
   }
-  fast = fast && aligned(p.w, 16) && p.w_sn % 16 == 0 && p.w_sk == 1;
+  fast = fast && p.w_sk == 1;
+  p.ragged = !(K % 16 == 0 && aligned(x, 16) && (ldx * esz) % 16 == 0 && aligned(p.w, 16) && p.w_sn % 16 == 0);
   return x_dtype == DQ8_DTYPE_F32 ? launch<float>(p, fast, rest, rest_bytes, st)
                                   : launch<_Float16>(p, fast, rest, rest_bytes, st);
 }

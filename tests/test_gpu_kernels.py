@@ -2221,3 +2221,23 @@ def test_layer_norm_with_and_without_its_quantize(K, rows, cols):
     y2, q = K.layer_norm(x.cuda(), gamma.cuda(), beta.cuda(), 1e-12, scale)
     assert torch.equal(y2, y)
     assert torch.equal(q, K.quantize(y, scale, torch.zeros(1, dtype=torch.int32, device="cuda")))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("m,k,n", [(1, 16, 1), (3, 17, 33), (16, 63, 40), (17, 65, 31), (32, 2047, 129), (33, 79, 65), (40, 1001, 300),
+                                   (100, 3009, 96), (129, 130, 700), (600, 2057, 130)])
+def test_weight_only_qgemm_rows_of_any_length_and_alignment(K, dtype, m, k, n):
+    """Row lengths that are multiples of nothing, and 16-byte lengths at odd bases, on either side
+    of the k tiles, of the row limits and of the tile sizes; one launch and split over k."""
+    rng = np.random.default_rng(m + k + n)
+    for signed in (False, True):
+        x, w, scale, zp, bias = _weight_only_case(rng, m, k, n, dtype, signed)
+        for ws in (True, False):
+            got = K.weight_only_qgemm(dev(x), dev(w), dev(scale), dev(zp), dev(bias), workspace=ws)
+            _weight_only_check(got, x, w, scale, zp, bias, dtype)
+        got = K.weight_only_qgemm(dev(x), dev(np.ascontiguousarray(w.T)), dev(scale), dev(zp), None, tp_b=False)
+        _weight_only_check(got, x, w, scale, zp, None, dtype)
+    x, w, scale, zp, bias = _weight_only_case(rng, m, (k + 15) // 16 * 16, n, dtype, False)
+    xb = torch.empty(x.size + 1, dtype=dtype, device="cuda")[1:].view(x.shape).copy_(dev(x))
+    wb = torch.empty(w.size + 3, dtype=torch.uint8, device="cuda")[3:].view(w.shape).copy_(dev(w))
+    _weight_only_check(K.weight_only_qgemm(xb, wb, dev(scale), dev(zp), dev(bias)), x, w, scale, zp, bias, dtype)
