@@ -23,22 +23,21 @@
 // layout: the order of the k values inside a fragment is free as long as both operands agree,
 // so lane (row, g) takes the 16 consecutive k values k0 + 16 g .. of its row -- 16 weight bytes
 // (one dwordx4), 16 activations -- and feeds two MFMAs with them.
-//  * wo_lds_kernel: tiles shared through LDS, everything above 32 rows (16 for f32): 64 x 64 or 128 x 128
-//    tiles while the problem is a few rounds of them -- with several workgroups per tile, each
-//    over a part of k, and wo_splitk_reduce_kernel behind them, where that is estimated
-//    cheaper --, 256 x 128 and 256 x 256 tiles beyond (1.06-1.16 PFLOP/s for f16 activations
-//    at 4096^2 .. 8192^2 weights, where the ROCm library's plain f16 GEMM reaches 1.16-1.49);
+//  * wo_lds_kernel: tiles shared through LDS, everything above 32 rows (16 for f32 against deep
+//    weights): 64 x 64 or 128 x 128 tiles while the problem is a few rounds of them -- with several
+//    workgroups per tile, each over a part of k, and wo_splitk_reduce_kernel behind them, where that
+//    is estimated cheaper --, 256 x 128 and 256 x 256 tiles beyond (1.06-1.16 PFLOP/s for f16
+//    activations at 4096^2 .. 8192^2 weights, where the ROCm library's plain f16 GEMM reaches
+//    1.16-1.49);
 //  * wo_tile_kernel: 2 x 2 waves, wave tile (32 FM) x (32 FN), operands straight into registers:
 //    operands too large for the LDS kernel's 31-bit offsets;
-//  * wo_skinny_lds_kernel: 5 .. 32 rows (16 for f32 activations) against deep or wide weights,
-//    32 output channels per workgroup, both operands loaded in row segments and turned into
-//    fragments through wave-private LDS;
+//  * wo_rows_kernel: 2 .. 32 rows, 16 .. 64 output channels per workgroup, both operands loaded in
+//    row segments and turned into fragments through wave-private LDS;
 //  * wo_gemv_kernel: one or two rows, a wave per output channel streaming its weight row on the
 //    vector ALUs;
-//  * wo_skinny16_kernel: M <= 16 rows against 16 output channels per workgroup (16x16x32 MFMA);
 //  * wo_skinny_kernel: M <= 128 rows against 32 output channels per workgroup, the k range dealt
-//    over the waves and the partial sums added through LDS (bound by the weight bytes: 1 byte
-//    per weight from HBM);
+//    over the waves and the partial sums added through LDS: operands too large for the two LDS
+//    kernels' 31-bit offsets;
 //  * wo_exact_f32_kernel: f32 activations on rows off 16 bytes (f16 ones: the LDS kernels' RAGGED
 //    forms);
 //  * wo_generic_kernel: one output per thread, fewer than 16 of k or weights left as [K, N].
@@ -718,32 +717,43 @@ __global__ void __launch_bounds__(NW * 64) wo_gemv_kernel(const WoParams p) {
   }
 }
 
-// ---------------------------------------------------------------- 8 < M <= 32, operands through LDS
-// 32 output channels per workgroup like wo_skinny_kernel<.., 1>, the k range dealt over the
-// waves in units of 64.  There every lane fetches its own activation row (32 rows x 32 bytes
-// per load instruction), and from nine rows on the compute unit's address path, not HBM, sets
-// the pace.  Here a wave loads each unit the way memory likes it -- eight lanes (sixteen for
-// f32) per 128-byte (256-byte) row segment of the activations, four per 64-byte segment of the
-// weights --, keeps three units in registers on their way from memory, and turns them into MFMA
-// fragments through a piece of LDS that only this wave touches (no barrier: the LDS executes a
-// wave's instructions in order).  f32 activations are split into hi and lo half tiles there.
-// MR: rows staged (16 or 32).  RAGGED (f16): as in wo_lds_kernel (M = 16, 3001 -> 4096, one output
-// per thread before: 567 us).
-template <typename XT, int NW, int MR, bool RAGGED = false>
-__global__ void __launch_bounds__(NW * 64) wo_skinny_lds_kernel(const WoParams p) {
+typedef float f4v __attribute__((ext_vector_type(4)));
+
+// ---------------------------------------------------------------- up to 32 rows, operands through LDS
+// 16 MT rows x 16 FN output channels per workgroup on v_mfma_f32_16x16x32_f16, the k range dealt
+// over the waves in units of 64.  Bound by the weight bytes from HBM.  When every lane fetches its
+// own activation row (wo_skinny_kernel: 32 rows x 32 bytes per load instruction), the compute
+// unit's address path, not HBM, sets the pace from nine rows on.  Here a wave loads each unit the
+// way memory likes it -- eight lanes (sixteen for f32) per 128-byte (256-byte) row segment of the
+// activations, four per 64-byte segment of the weights --, keeps D units in registers on their way
+// from memory, and turns them into MFMA fragments through a piece of LDS that only this wave touches
+// (no barrier: the LDS executes a wave's instructions in order).  f32 activations are split into hi
+// and lo half tiles there.
+// The width is what balances the chip: with 32 channels and 32 rows per workgroup in every case,
+// 11008 channels were 344 workgroups on 256 compute units, one at a time in 144 registers, and half
+// the multiplications met rows that were not there.  4096 -> 11008, M = 16: f16 14.6 -> 11.3 us (18.3 ->
+// 13.9 with weights from HBM, 3.2 TB/s), f32 21.5 -> 12.7; 8192 -> 2048 11.3 -> 7.9; M = 32, 4096 -> 11008
+// 18.8 -> 12.1.  More units in registers were slower (D = 4 in place of 2: M = 32 14.0, f32 14.5)
+// except for the narrowest form (4096 -> 8192 9.5 against 10.6).
+// RAGGED (f16): as in wo_lds_kernel (M = 16, 3001 -> 4096, one output per thread before: 567 us).
+constexpr int kRowsWaves = 8;
+
+template <typename XT, int MT, int FN, int D, bool RAGGED = false>
+__global__ void __launch_bounds__(kRowsWaves * 64) wo_rows_kernel(const WoParams p) {
   constexpr bool F32 = sizeof(XT) == 4;
   static_assert(!RAGGED || !F32, "f32 activations: wo_exact_f32_kernel");
+  constexpr int NW = kRowsWaves, MR = 16 * MT, BN = 16 * FN;
   constexpr int XL = F32 ? 16 : 8;                       // lanes per activation row of a unit
   constexpr int XP = MR * XL / 64;                       // activation loads per lane and unit
   constexpr int XBYTES = MR * 128 * (F32 ? 2 : 1);       // [hi, then lo] half tiles
-  constexpr int WBYTES = 32 * 64;
-  constexpr int D = 3;                                   // units in registers
-  static_assert(D * (XP + 2) <= 63, "vmcnt is a 6-bit counter");
+  constexpr int WBYTES = BN * 64;
+  static_assert(D * (XP + FN) <= 63, "vmcnt is a 6-bit counter");
+  static_assert(MT * FN <= NW && MT * FN * 1024 <= XBYTES + WBYTES, "the waves' partial sums fit the LDS");
   extern __shared__ __attribute__((aligned(16))) uint8_t wo_lds[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 31, g = lane >> 5;
-  const int n0 = blockIdx.x * 32;
-  const int nrows = min(32, p.N - n0), mrows = min(MR, p.M);
+  const int r = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * BN;
+  const int nrows = min(BN, p.N - n0), mrows = min(MR, p.M);
   uint8_t* const xs = wo_lds + wave * (XBYTES + WBYTES);
   uint8_t* const ws = xs + XBYTES;
   // descriptors over the activation rows and this workgroup's weight rows; the host has
@@ -769,15 +779,17 @@ __global__ void __launch_bounds__(NW * 64) wo_skinny_lds_kernel(const WoParams p
     xl[i] = F32 ? row * 128 + (((xc >> 1) ^ sx) << 4) + 8 * (xc & 1)
                 : row * 128 + ((xc ^ sx) << 4);
   }
-  int wo[2], wl[2];
+  int wo[FN], wl[FN];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < FN; ++i) {
     const int row = (lane >> 2) + 16 * i;
     wo[i] = (int)((int64_t)min(row, nrows - 1) * p.w_sn) + (RAGGED ? 0 : 16 * wc);
     wl[i] = row * 64 + ((wc ^ ((row >> 2) & 3)) << 4);
   }
-  const h2 c = centre(p, n0 + min(r, nrows - 1));
-  u4 xr[D][XP], wr[D][2];
+  h2 c[FN];
+#pragma unroll
+  for (int j = 0; j < FN; ++j) c[j] = centre(p, n0 + min(16 * j + r, nrows - 1));
+  u4 xr[D][XP], wr[D][FN];
   const uint8_t* xbase = static_cast<const uint8_t*>(p.x);
   const uint8_t* wbase = p.w + (int64_t)n0 * p.w_sn;
   auto fetch = [&](u4* xq, u4* wq, int k0) {
@@ -787,7 +799,7 @@ __global__ void __launch_bounds__(NW * 64) wo_skinny_lds_kernel(const WoParams p
 #pragma unroll
       for (int i = 0; i < XP; ++i) xq[i] = load_any(xbase, (unsigned)xo[i] + 2 * kx);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) wq[i] = load_any(wbase, (unsigned)wo[i] + kw);
+      for (int i = 0; i < FN; ++i) wq[i] = load_any(wbase, (unsigned)wo[i] + kw);
       return;
     }
     const bool xv = k0 + (F32 ? 4 : 8) * xc < p.K, wv = k0 + 16 * wc < p.K;   // K % 16 == 0
@@ -796,7 +808,7 @@ __global__ void __launch_bounds__(NW * 64) wo_skinny_lds_kernel(const WoParams p
       xq[i] = __builtin_amdgcn_raw_buffer_load_b128(
           xrs, xv && xok[i] ? xo[i] + (int)sizeof(XT) * k0 : kPast, 0, 0);
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < FN; ++i)
       wq[i] = __builtin_amdgcn_raw_buffer_load_b128(wrs, wv ? wo[i] + k0 : kPast, 0, 0);
   };
   auto park = [&](u4* xq, const u4* wq, int k0) {
@@ -823,33 +835,39 @@ __global__ void __launch_bounds__(NW * 64) wo_skinny_lds_kernel(const WoParams p
       }
     }
 #pragma unroll
-    for (int i = 0; i < 2; ++i) *reinterpret_cast<u4*>(&ws[wl[i]]) = wq[i];
+    for (int i = 0; i < FN; ++i) *reinterpret_cast<u4*>(&ws[wl[i]]) = wq[i];
   };
-  f16v acc;
+  f4v acc[MT][FN];
 #pragma unroll
-  for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
-  // this lane's fragment rows (activation rows past the staged ones re-read a staged one:
-  // their results are not stored)
-  const int xrow = r & (MR - 1), sxr = (xrow ^ (xrow >> 3)) & 7, swr = (r >> 2) & 3;
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = (f4v){0.f, 0.f, 0.f, 0.f};
+  // lane (r, g): the unit's k values 16 g .. 16 g + 15 of row r of a fragment, as two k steps
   auto multiply = [&]() {
+    h8 a[F32 ? 2 : 1][MT][2];
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {                          // the unit's two 32-deep chunks
-      const int cx = 4 * q + 2 * g;
-      const h8 a0 = *reinterpret_cast<const h8*>(&xs[xrow * 128 + ((cx ^ sxr) << 4)]);
-      const h8 a1 = *reinterpret_cast<const h8*>(&xs[xrow * 128 + (((cx + 1) ^ sxr) << 4)]);
-      const u4 wq = *reinterpret_cast<const u4*>(&ws[r * 64 + (((2 * q + g) ^ swr) << 4)]);
+    for (int part = 0; part < (F32 ? 2 : 1); ++part)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const int row = 16 * i + r, sx = (row ^ (row >> 3)) & 7;
+          a[part][i][s] = *reinterpret_cast<const h8*>(
+              &xs[part * MR * 128 + row * 128 + (((2 * g + s) ^ sx) << 4)]);
+        }
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int row = 16 * j + r;
+      const u4 wq = *reinterpret_cast<const u4*>(&ws[row * 64 + ((g ^ ((row >> 2) & 3)) << 4)]);
       h8 w0, w1;
-      widen16(wq, p.flip, c, w0, w1);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, w0, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, w1, acc, 0, 0, 0);
-      if constexpr (F32) {
-        const h8 l0 =
-            *reinterpret_cast<const h8*>(&xs[MR * 128 + xrow * 128 + ((cx ^ sxr) << 4)]);
-        const h8 l1 =
-            *reinterpret_cast<const h8*>(&xs[MR * 128 + xrow * 128 + (((cx + 1) ^ sxr) << 4)]);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(l0, w0, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(l1, w1, acc, 0, 0, 0);
-      }
+      widen16(wq, p.flip, c[j], w0, w1);
+#pragma unroll
+      for (int part = 0; part < (F32 ? 2 : 1); ++part)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[part][i][0], w0, acc[i][j], 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[part][i][1], w1, acc[i][j], 0, 0, 0);
+        }
     }
   };
   // units wave, wave + NW, ... of 64 of k; set u holds unit i + u on its way from memory
@@ -862,94 +880,37 @@ __global__ void __launch_bounds__(NW * 64) wo_skinny_lds_kernel(const WoParams p
   for (int k0 = w64; k0 < p.K; k0 += D * NW * 64) {
 #pragma unroll
     for (int u = 0; u < D; ++u) {
+      if (u > 0 && k0 + u * NW * 64 >= p.K) break;         // (uniform)
       park(xr[u], wr[u], k0 + u * NW * 64);
       fetch(xr[u], wr[u], k0 + (D + u) * NW * 64);
       multiply();
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  // partial sums of the waves through LDS (all waves are done with their pieces of it)
+  // partial sums of the waves through LDS (all waves are done with their pieces of it), a
+  // fragment to each of the first MT x FN waves
   __syncthreads();
-  float* const red = reinterpret_cast<float*>(wo_lds);   // [NW - 1][16][64]
-  if (wave > 0) {
+  float* const red = reinterpret_cast<float*>(wo_lds);   // [MT * FN][NW][4][64]
 #pragma unroll
-    for (int v = 0; v < 16; ++v) red[((wave - 1) * 16 + v) * 64 + lane] = acc[v];
-  }
+  for (int f = 0; f < MT * FN; ++f)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) red[((f * NW + wave) * 4 + v) * 64 + lane] = acc[f / FN][f % FN][v];
   __syncthreads();
-  if (wave == 0) {
+  if (wave >= MT * FN) return;
+  f4v sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int w = 1; w < NW; ++w)
+  for (int w = 0; w < NW; ++w)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[v] += red[((w - 1) * 16 + v) * 64 + lane];
-    store_frag<XT>(p, acc, 0, n0 + r, lane);
-  }
-}
-
-// ---------------------------------------------------------------- M <= 16
-// 16 output channels per workgroup on v_mfma_f32_16x16x32_f16: twice as many workgroups as the
-// 32-channel form for the same weights (a 4096 x 4096 weight gives 256 instead of 128), and a
-// lane (row, g) takes the 16 consecutive k values k0 + 16 g .. of a 64-deep chunk, so a wave's
-// load covers 64 contiguous bytes of each of its 16 weight rows.
-typedef float f4v __attribute__((ext_vector_type(4)));
-
-template <typename XT, int NW>
-__global__ void __launch_bounds__(NW * 64) wo_skinny16_kernel(const WoParams p) {
-  __shared__ float red[NW - 1][4][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16;
-  const int n = min(n0 + r, p.N - 1);
-  const XT* xrow = static_cast<const XT*>(p.x) + (int64_t)min(r, p.M - 1) * p.ldx + 16 * g;
-  const uint8_t* wrow = p.w + (int64_t)n * p.w_sn + 16 * g;
-  const h2 c = centre(p, n);
-  f4v acc = {0.f, 0.f, 0.f, 0.f};
-  const u4 zero = {0, 0, 0, 0};
-  constexpr int U = 4;
-  for (int k0 = wave * 64; k0 < p.K; k0 += U * NW * 64) {
-    XFrag<XT> xf[U];
-    u4 wf[U];
+    for (int v = 0; v < 4; ++v) sum[v] += red[((wave * NW + w) * 4 + v) * 64 + lane];
+  // D of the 16x16 MFMA: column n = lane % 16, rows 4 (lane / 16) + v
+  const int n = n0 + 16 * (wave % FN) + r, m0 = 16 * (wave / FN) + 4 * g;
+  if (n >= p.N) return;
+  const float sc = to_f32(static_cast<const XT*>(p.scale)[n]);
+  const float bi = p.bias ? to_f32(static_cast<const XT*>(p.bias)[n]) : 0.0f;
+  XT* out = static_cast<XT*>(p.out);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int kk = k0 + u * NW * 64;
-      const bool valid = kk + 16 * g < p.K;              // K % 16 == 0: whole 16-chunks
-      const int k = valid ? kk : 0;
-      wf[u] = valid ? *reinterpret_cast<const u4*>(wrow + k) : zero;
-      xf[u].load(xrow + k, valid);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      h8 w0, w1;
-      widen16(wf[u], p.flip, c, w0, w1);
-#pragma unroll
-      for (int part = 0; part < XFrag<XT>::kParts; ++part) {
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[u].step(part, 0), w0, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[u].step(part, 1), w1, acc, 0, 0, 0);
-      }
-    }
-  }
-  if (wave > 0) {
-#pragma unroll
-    for (int v = 0; v < 4; ++v) red[wave - 1][v][lane] = acc[v];
-  }
-  __syncthreads();
-  if (wave == 0) {
-#pragma unroll
-    for (int w = 1; w < NW; ++w)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) acc[v] += red[w - 1][v][lane];
-    // D of the 16x16 MFMA: column n = lane % 16, rows 4 (lane / 16) + v
-    const int nn = n0 + r;
-    if (nn < p.N) {
-      const float s = to_f32(static_cast<const XT*>(p.scale)[nn]);
-      const float b = p.bias ? to_f32(static_cast<const XT*>(p.bias)[nn]) : 0.0f;
-      XT* out = static_cast<XT*>(p.out);
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int m = 4 * g + v;
-        if (m < p.M) out[(int64_t)m * p.ldo + nn] = (XT)(acc[v] * s + b);
-      }
-    }
-  }
+  for (int v = 0; v < 4; ++v)
+    if (m0 + v < p.M) out[(int64_t)(m0 + v) * p.ldo + n] = (XT)(sum[v] * sc + bi);
 }
 
 // ---------------------------------------------------------------- f32, rows of any length
@@ -1057,16 +1018,47 @@ int launch_gemv(const WoParams& p, hipStream_t st) {
   return check_hip(hipGetLastError(), "dq8_weight_only_qgemm launch");
 }
 
-template <typename XT, int MR, bool RAGGED = false>
-int launch_skinny_lds(const WoParams& p, hipStream_t st) {
-  constexpr int lds = 8 * (MR * 128 * (int)(sizeof(XT) / 2) + 32 * 64);
-  static_assert(lds >= 7 * 16 * 64 * 4, "the partial sums of the waves fit");
-  auto kern = wo_skinny_lds_kernel<XT, 8, MR, RAGGED>;
+template <typename XT, int MT, int FN, bool RAGGED>
+int launch_rows_fn(const WoParams& p, hipStream_t st) {
+  constexpr int D = sizeof(XT) == 2 && MT == 1 && FN == 1 ? 4 : 2;
+  constexpr int lds = kRowsWaves * (MT * 2048 * (int)(sizeof(XT) / 2) + FN * 1024);
+  static_assert(lds <= 160 * 1024, "the units fit the LDS");
+  auto kern = wo_rows_kernel<XT, MT, FN, D, RAGGED>;
   static std::atomic<uint64_t> lds_allowed{0};
   if (lds > 64 * 1024)
     if (int s = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds, &lds_allowed)) return s;
-  hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(p.N, 32)), dim3(512), lds, st, p);
+  hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(p.N, 16 * FN)), dim3(kRowsWaves * 64), lds, st, p);
   return check_hip(hipGetLastError(), "dq8_weight_only_qgemm launch");
+}
+
+template <typename XT, int MT, bool RAGGED>
+int launch_rows_mt(const WoParams& p, hipStream_t st) {
+  // The workgroup's width: the fewest rounds of the chip, a round priced at the bytes a workgroup
+  // stages per unit (weights 16 x 64 a fragment, activations 16 MT x 64 elements).  4096 -> 11008,
+  // M = 16, weights from HBM: 16.5 / 16.5 / 13.9 / 15.4 us at 16 / 32 / 48 / 64 channels (three
+  // rounds, two, one, one); 4096^2 8.0 / 9.4 / 11.6 / 13.7; 6144^2 16.0 / 13.4 / 16.8 / 19.9.
+  const int64_t cus = compute_units(), tiles = ceil_div(p.N, 16);
+  int fn = 1;
+  int64_t least = INT64_MAX;
+  for (int f = 1; f <= 4; ++f) {
+    const int64_t t = ceil_div(ceil_div(tiles, f), cus) * (f + MT * (int)sizeof(XT));
+    if (t < least) least = t, fn = f;
+  }
+  // (two 16-channel workgroups share a compute unit: two whole rounds of them are one, and keep more
+  // in flight where the rows are deep: 8192^2, M = 16: 20.6 against 21.1 us from HBM, 16.7 against 20.5
+  // from the last-level cache; 4096 -> 8192 12.0 / 10.8)
+  if (MT == 1 && sizeof(XT) == 2 && p.K >= 8192 && 4 * tiles > 7 * cus && tiles <= 2 * cus) fn = 1;
+  switch (fn) {
+    case 1: return launch_rows_fn<XT, MT, 1, RAGGED>(p, st);
+    case 2: return launch_rows_fn<XT, MT, 2, RAGGED>(p, st);
+    case 3: return launch_rows_fn<XT, MT, 3, RAGGED>(p, st);
+    default: return launch_rows_fn<XT, MT, 4, RAGGED>(p, st);
+  }
+}
+
+template <typename XT, bool RAGGED = false>
+int launch_rows(const WoParams& p, hipStream_t st) {
+  return p.M <= 16 ? launch_rows_mt<XT, 1, RAGGED>(p, st) : launch_rows_mt<XT, 2, RAGGED>(p, st);
 }
 
 // The small tile forms of the LDS kernel, for problems whose tiles would leave most of the chip
@@ -1164,9 +1156,10 @@ SplitPlan choose_small(int64_t M, int64_t N, int64_t K, int esz, bool ragged, bo
   const SplitPlan none = {-1, 1, (int)K, 0.0f};
   // (rows off 16 bytes: f16 has the small tiles and the staged small-M kernel, f32 its own kernel)
   if (ragged) return esz == 4 || M <= 32 ? none : plan_split(M, N, K, esz, may_split);
-  // (f32, between: 1536 x 1536 weights, M = 24: 10.0 against 11.2 us, M = 17: 9.5 against 9.2;
-  // 768 -> 3072, M = 24: 8.7 against 7.6)
-  if (M <= (esz == 4 && K >= 2048 ? 16 : esz == 4 && K >= 1280 ? 23 : 32)) return none;
+  // (f32 from 17 rows on: the staged small-M kernel runs k as one chain per wave, the tiles split it: M =
+  // 24, 1024 -> 4096 7.4 against 8.9 us, 2048^2 10.3 / 11.2, 4096 -> 11008 21.8 / 25.6, but 3072 -> 768
+  // 13.0 / 11.9, 4096^2 16.4 / 16.3, 8192 -> 1024 27.4 / 17.0)
+  if (M <= (esz == 4 && K > 2048 && !(K <= 4096 && N >= 8192) ? 16 : 32)) return none;
   const SplitPlan s = plan_split(M, N, K, esz, may_split);
   if (esz == 2 && M > 128) {
     const float big = big_tile_us(M, N, K);
@@ -1234,7 +1227,7 @@ int launch(WoParams& p, bool fast, void* scratch, size_t scratch_bytes, hipStrea
   // (the staged kernel addresses activation and weight rows by 31-bit byte offsets)
   const bool staged_ok =
       ((int64_t)(p.M - 1) * p.ldx + p.K) * (int64_t)sizeof(XT) + 65536 < (1LL << 31) &&
-      32 * p.w_sn + (int64_t)p.K + 65536 < (1LL << 31);
+      64 * p.w_sn + (int64_t)p.K + 65536 < (1LL << 31);
   if (fast && p.ragged) {
     if constexpr (sizeof(XT) == 4) {
       const int64_t tiles = ceil_div(p.M, 32) * ceil_div(p.N, 32);
@@ -1248,7 +1241,7 @@ int launch(WoParams& p, bool fast, void* scratch, size_t scratch_bytes, hipStrea
         return check_hip(hipGetLastError(), "dq8_weight_only_qgemm launch");
       }
     } else if (staged_ok && p.M <= 32) {
-      return p.M <= 16 ? launch_skinny_lds<XT, 16, true>(p, st) : launch_skinny_lds<XT, 32, true>(p, st);
+      return launch_rows<XT, true>(p, st);
     }
     fast = false;
   }
@@ -1257,40 +1250,23 @@ int launch(WoParams& p, bool fast, void* scratch, size_t scratch_bytes, hipStrea
     DQ8_REQUIRE(blocks < (1LL << 31), "dq8_weight_only_qgemm: problem too large");
     hipLaunchKernelGGL(wo_generic_kernel<XT>, dim3((unsigned)blocks), dim3(256), 0, st, p);
   } else if (p.M <= 128) {
-    const unsigned grid = (unsigned)ceil_div(p.N, 32);
-    // (with more than 8 rows every workgroup re-reads the activations, which then outweigh
-    // its weights: the narrow form only while the wide one would leave compute units idle)
-    // (it needs several 64-deep units per wave to run its pipeline: measured against the two
-    // kernels below it wins from 12 rows on at 3072 and 4096 of k -- 4096^2 weights, f16, M = 32:
-    // 10.7 against 14.9 us -- and from 5 rows on at 8192 -- M = 16: 16.8 against 22.5 us --, and
-    // loses about a microsecond at 768 or 1040 of k)
-    // one row, or two where it was measured faster (f32 activations; f16 from 2048 to 8192 of
-    // k), while the rows fit 64 KiB of LDS: the row-streaming kernel on the vector ALUs (4096^2
-    // weights, M = 1: f16 4.3 against 5.8 us, f32 4.5 against 7.5; 8192^2: 13.5 against 15.2 us,
-    // 5.0 TB/s; three and four rows are slower that way than on the matrix cores)
-    if ((p.M == 1 || (p.M == 2 && (sizeof(XT) == 4 || (p.K >= 2048 && p.K <= 8192)))) &&
-        (int64_t)p.M * p.K * (int64_t)sizeof(XT) <= 64 * 1024) {
+    // One row, and two where it was measured faster, while the rows fit 64 KiB of LDS: the
+    // row-streaming kernel on the vector ALUs (4096^2 weights, M = 1: f16 4.3 us, f32 4.5; M = 2, weights
+    // from HBM, against the kernel below: 3072 -> 768 f16 5.1 / 5.3 us, f32 5.3 / 6.5; 8192 -> 1024 f32
+    // 8.8 / 12.0; 4096^2 f16 7.9 / 7.4, f32 8.5 / 8.7; 4096 -> 11008 f16 14.2 / 13.2, f32 15.3 / 14.1;
+    // 8192^2 from the last-level cache f32 20.0 / 20.9).
+    const bool two = sizeof(XT) == 4 ? p.N < 8192 || p.K > 4096 : p.N <= 1024 && p.K >= 2048 && p.K <= 8192;
+    if ((p.M == 1 || (p.M == 2 && two)) && (int64_t)p.M * p.K * (int64_t)sizeof(XT) <= 64 * 1024) {
       const bool deep = p.K > 4096;
       if (p.M == 1) return deep ? launch_gemv<XT, 1, 8>(p, st) : launch_gemv<XT, 1, 4>(p, st);
       return deep ? launch_gemv<XT, 2, 8>(p, st) : launch_gemv<XT, 2, 4>(p, st);
     }
-    // (and from 5 rows on against weights of at least 8192 channels, where its 32-channel
-    // workgroups fill the chip: 4096 -> 16384, M = 8: f16 17.7 against 19.6 us, f32 23.7
-    // against 30.5)
-    // (three and four rows that way only against narrow weights, where a workgroup per 16
-    // channels leaves most compute units idle: 3072 -> 768, M = 4: f16 5.3 against 5.5 us, f32
-    // 6.1 against 7.8; 8192 -> 1024: 8.0 against 9.5 and 10.2 against 13.0; at 4096 channels
-    // and more the matrix cores win)
-    if (p.M >= 3 && p.M <= 4 && p.N <= 1024 && p.K >= 2048 &&
-        (int64_t)4 * p.K * (int64_t)sizeof(XT) <= 128 * 1024)
-      return p.K > 4096 ? launch_gemv<XT, 4, 8>(p, st) : launch_gemv<XT, 4, 4>(p, st);
-    if (staged_ok && p.M <= 32 &&
-        ((p.K >= 2048 && p.M >= 12) || (p.M >= 5 && (p.K >= 6144 || (p.K >= 2048 && p.N >= 8192)))))
-      return p.M <= 16 ? launch_skinny_lds<XT, 16>(p, st) : launch_skinny_lds<XT, 32>(p, st);
-    if (p.M <= 8 || (p.M <= 16 && grid < 256))
-      hipLaunchKernelGGL((wo_skinny16_kernel<XT, 8>), dim3((unsigned)ceil_div(p.N, 16)), dim3(512),
-                         0, st, p);
-    else if (p.M <= 32)
+    // Up to 32 rows: the staged kernel (against kernels that gathered both operands lane by lane, weights
+    // from HBM, f16: 1024 -> 11008 M = 16 9.3 -> 6.3 us, 1536 -> 6144 M = 8 6.5 -> 5.8, M = 32 9.0 ->
+    // 7.2, 3072 -> 768 M = 4 6.4 -> 5.5; f32: 768 -> 3072 M = 16 5.7 -> 4.9, M = 32 8.9 -> 6.7).
+    if (staged_ok && p.M <= 32) return launch_rows<XT>(p, st);
+    const unsigned grid = (unsigned)ceil_div(p.N, 32);
+    if (p.M <= 32)
       hipLaunchKernelGGL((wo_skinny_kernel<XT, 8, 1>), dim3(grid), dim3(512), 0, st, p);
     else if (p.M <= 64)
       hipLaunchKernelGGL((wo_skinny_kernel<XT, 8, 2>), dim3(grid), dim3(512), 0, st, p);

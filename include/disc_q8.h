@@ -367,8 +367,9 @@ int dq8_transpose_s8(const int8_t* src, int64_t ld, int8_t* dst, int64_t rows,
  * the half 1024 + zp, + 128 for int8, which holds integers exactly only up to 2048; they are
  * device data and not checked).  [K,N] weights are transposed into `workspace`
  * (dq8_weight_only_qgemm_workspace_bytes) on every call; a runtime does that once per constant
- * weight with dq8_transpose_s8 and passes tp_b = 1.  Without the scratch, or with K % 16 != 0
- * or rows that are not 16-byte aligned, a slower kernel without alignment rules runs.
+ * weight with dq8_transpose_s8 and passes tp_b = 1.  Without the scratch, or with K < 16, a
+ * slower kernel with one output per thread runs; rows of other lengths and alignments than 16
+ * bytes have forms of their own.
  * Accumulation is f32; f32 activations enter the matrix cores as two halves: about 22
  * significant bits for |x| >= 1/8, an absolute 2^-25 per activation below (the low half is then
  * a subnormal half), and |x| must stay below 65504. */

@@ -2241,3 +2241,17 @@ def test_weight_only_qgemm_rows_of_any_length_and_alignment(K, dtype, m, k, n):
     xb = torch.empty(x.size + 1, dtype=dtype, device="cuda")[1:].view(x.shape).copy_(dev(x))
     wb = torch.empty(w.size + 3, dtype=torch.uint8, device="cuda")[3:].view(w.shape).copy_(dev(w))
     _weight_only_check(K.weight_only_qgemm(xb, wb, dev(scale), dev(zp), dev(bias)), x, w, scale, zp, bias, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("n", [1, 47, 4097, 8200, 12300])
+@pytest.mark.parametrize("m", [2, 16, 17, 32])
+def test_weight_only_qgemm_few_rows_at_every_workgroup_width(K, dtype, m, n):
+    """16, 32, 48 and 64 channels per workgroup (N up to 4096, 8192, 12288, 16384 on 256 compute units),
+    the last one partly filled; k of part of a unit, of an uneven number of units per wave, and past a
+    whole round of the waves; rows off 16 bytes."""
+    rng = np.random.default_rng(m + n)
+    for k in (16, 1040, 2112, 1043):
+        x, w, scale, zp, bias = _weight_only_case(rng, m, k, n, dtype, k == 1040)
+        _weight_only_check(K.weight_only_qgemm(dev(x), dev(w), dev(scale), dev(zp), dev(bias)), x, w, scale,
+                           zp, bias, dtype)
