@@ -294,7 +294,7 @@ __global__ void __launch_bounds__(256) wo_tile_kernel(const WoParams p) {
 // end of the rows is handled differently (M = 512, 2047 -> 3001, one output per thread before:
 // 11.9 ms).
 template <typename XT, int WM, int FM, int FN, int SETS, bool RAGGED = false>
-__global__ void __launch_bounds__(WM * 128, (WM == 1 || sizeof(XT) == 4) ? 1 : 2)
+__global__ void __launch_bounds__(WM * 128, sizeof(XT) == 4 ? 1 : 2)
     wo_lds_kernel(const WoParams p) {
   constexpr bool F32 = sizeof(XT) == 4;
   static_assert(!RAGGED || !F32, "f32 activations: wo_exact_f32_kernel");
@@ -504,11 +504,17 @@ __global__ void __launch_bounds__(WM * 128, (WM == 1 || sizeof(XT) == 4) ? 1 : 2
   // k tile t: set u = t % SETS has been handed to LDS stage t % 2 and takes tile t + SETS;
   // tile t + 1 (zeros past the last) is handed over behind the multiplication
   // (the scheduling barriers keep a later step's arithmetic on loaded registers -- the first
-  // instructions of widening -- from being moved up to where it would wait for their loads)
+  // instructions of widening -- from being moved up to where it would wait for their loads.  Between
+  // a multiplication and the hand-over behind it there is none: the tile handed over left memory
+  // SETS - 1 tiles ago, and its widening and writes fill the gaps between the MFMAs: M = 1024,
+  // 4096 -> 4096 46.3 -> 44.3 us, M = 2048 75.0 -> 71.4, 8192 -> 2048 85.0 -> 81.0.  With the hand-over
+  // in front of the multiplication the fragment reads queue behind its writes: 49.6, 8192 -> 2048 91.1.
+  // It stays for 256 x 256 tiles, which have no registers for both at once, and for f32 on 64 x 64
+  // tiles, where nothing was gained: M = 64, 4096 -> 4096 15.9 against 16.3 us without.)
   auto step = [&](int u, int t) {
     fetch(xr[u], wr[u], (t + SETS) * BK);
     multiply(u % 2);
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (FM * FN >= 8 || (F32 && FM * FN == 1)) __builtin_amdgcn_sched_barrier(0);
     park(xr[(u + 1) % SETS], wr[(u + 1) % SETS], (u + 1) % 2, (t + 1) * BK);
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
@@ -1066,9 +1072,9 @@ int launch_rows(const WoParams& p, hipStream_t st) {
 // reads, MFMAs, hand-over of the next tile, barrier): 0.4 us per k tile with two 32 x 32
 // fragments per wave, 0.27 us with one -- so below a few rounds of tiles the 64 x 64 tile on
 // four waves beats every larger one, although it moves the most bytes per MFMA.
-enum { kForm64x64w2 = 0, kForm128x64, kForm64x128w2, kForm128x128, kForm64x64, kNumForms };
+enum { kForm128x128 = 0, kForm64x64, kNumForms };
 struct TileForm { int bm, bn; };
-constexpr TileForm kForms[kNumForms] = {{64, 64}, {128, 64}, {64, 128}, {128, 128}, {64, 64}};
+constexpr TileForm kForms[kNumForms] = {{128, 128}, {64, 64}};
 
 // Plan: `splits` workgroups per tile of form `form`, each over k_split of the k range, and
 // (splits > 1) a reduction kernel behind them.  `us`: the estimate it was chosen by.
@@ -1180,15 +1186,14 @@ int launch_form(int form, int splits, const WoParams& p, hipStream_t st) {
                   (unsigned)splits);
   if constexpr (sizeof(XT) == 2)
     if (p.ragged)
-      return form == kForm128x128 ? launch_lds<XT, 2, 2, 2, kSets, true>(grid, p, st)
+      return form == kForm128x128 ? launch_lds<XT, 4, 1, 2, kSets, true>(grid, p, st)
                                   : launch_lds<XT, 2, 1, 1, kSets, true>(grid, p, st);
   switch (form) {
-    case kForm64x64w2: return launch_lds<XT, 1, 2, 1, kSets>(grid, p, st);
-    case kForm128x64: return launch_lds<XT, 2, 2, 1, kSets>(grid, p, st);
-    case kForm64x128w2: return launch_lds<XT, 1, 2, 2, kSets>(grid, p, st);
     case kForm128x128:
-      if constexpr (sizeof(XT) == 4) return launch_lds<XT, 4, 1, 2, kSets>(grid, p, st);
-      return launch_lds<XT, 2, 2, 2, kSets>(grid, p, st);
+      // (eight waves of two fragments: two waves per SIMD cover each other's reads and hand-overs, which
+      // is worth more than the LDS bytes that four waves of four fragments save -- M = 1024, 4096 -> 4096
+      // 42.9 against 44.3 us, M = 2048, 8192 -> 2048 78.9 / 81.0; unaligned rows, 4095 -> 4096 49.4 / 59.6)
+      return launch_lds<XT, 4, 1, 2, kSets>(grid, p, st);
     case kForm64x64: return launch_lds<XT, 2, 1, 1, kSets>(grid, p, st);
   }
   return fail("dq8_weight_only_qgemm: unknown tile form");
