@@ -2255,3 +2255,21 @@ def test_weight_only_qgemm_few_rows_at_every_workgroup_width(K, dtype, m, n):
         x, w, scale, zp, bias = _weight_only_case(rng, m, k, n, dtype, k == 1040)
         _weight_only_check(K.weight_only_qgemm(dev(x), dev(w), dev(scale), dev(zp), dev(bias)), x, w, scale,
                            zp, bias, dtype)
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 64, 3), (1, 64, 4), (33, 128, 37), (65, 64, 68), (130, 768, 66), (257, 3072, 132),
+                                   (1000, 256, 256)])
+def test_residual_behind_f32_results_at_the_edges_of_the_fragments(K, m, k, n):
+    """Rows and columns of a fragment past the result, N below and off a group of four, k in one and
+    in several wave groups: the bits of the dequantized result and a separate addition."""
+    g = torch.Generator().manual_seed(m + n)
+    a = torch.randint(-128, 128, (m, k), generator=g, dtype=torch.int8).cuda()
+    w = torch.randint(-128, 128, (n, k), generator=g, dtype=torch.int8).cuda()
+    sx, so = torch.tensor([0.02]).cuda(), torch.tensor([0.05 * k ** 0.5]).cuda()
+    sw = (torch.rand(n, generator=g) * 0.01 + 0.01).cuda()
+    run = lambda **kw: K.qgemm(a, w, K.EPI_REQUANT_CPU_DEQUANT_F32, sx=sx, sw=sw, so=so, **kw)  # noqa: E731
+    plain = run()
+    r = torch.randn(m, n, generator=g).cuda()
+    assert torch.equal(run(post=K.make_postops(residual=r)), plain + r)
+    q = torch.randint(-128, 128, (m, n), generator=g, dtype=torch.int8).cuda()
+    assert torch.equal(run(post=K.make_postops(residual=q, residual_scale=sx)), plain + q.float() * sx)
