@@ -111,7 +111,8 @@ def build_torch_calls(force=False):
     import sysconfig
 
     import torch
-    inputs = [TORCH_CALLS_SRC, os.path.join(ROOT, "include", "disc_q8.h")]
+    src = os.path.dirname(TORCH_CALLS_SRC)
+    inputs = [os.path.join(src, f) for f in os.listdir(src)] + [os.path.join(ROOT, "include", "disc_q8.h")]
     if (not force and os.path.exists(TORCH_CALLS)
             and os.path.getmtime(TORCH_CALLS) > max(map(os.path.getmtime, inputs))):
         return TORCH_CALLS

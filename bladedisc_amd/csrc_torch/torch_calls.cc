@@ -20,12 +20,12 @@
 
 #include <atomic>
 #include <chrono>
-#include <exception>
 #include <mutex>
 #include <string>
 #include <vector>
 
 #include "disc_q8.h"
+#include "unlocked.h"
 
 namespace {
 
@@ -47,14 +47,10 @@ void check(int status, const char* what) {
 
 void* stream() { return (void*)c10::hip::getCurrentHIPStream().stream(); }
 
-// The launch itself, without the interpreter lock.
-template <typename F>
-void launch(const char* what, F&& f) {
-  int status;
-  Py_BEGIN_ALLOW_THREADS
-  status = f();
-  Py_END_ALLOW_THREADS
-  check(status, what);
+// The launch itself, without the interpreter lock: f(args...), the arguments read before.
+template <typename... P, typename... A>
+void launch(const char* what, int (*f)(P...), A... args) {
+  check(dq8::call_unlocked(f, args...), what);
 }
 
 Tensor empty(at::IntArrayRef sizes, ScalarType t, const at::Device& dev) {
@@ -210,10 +206,8 @@ PyObject* py_quantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
                            : empty(x.sizes(), reinterpret_cast<THPDtype*>(a[8])->scalar_type, x.device());
     const int64_t n_q = a[3] != Py_None ? s.numel() : 1;
     void* st = stream();
-    launch("dq8_quantize", [&] {
-      return dq8_quantize_ex(ptr(x), xk, ptr(out), kind, v.outer, v.nch, v.inner, (const float*)ptr(s),
-                             (const int32_t*)ptr(z), n_q, qmin, qmax, round_mode, st);
-    });
+    launch("dq8_quantize", dq8_quantize_ex, ptr(x), xk, ptr(out), kind, v.outer, v.nch, v.inner,
+           (const float*)ptr(s), (const int32_t*)ptr(z), n_q, qmin, qmax, round_mode, st);
     return wrap(a[9], out);
   });
 }
@@ -229,10 +223,8 @@ PyObject* py_dequantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const Tensor out = a[5] != Py_None ? tensor(a[5]) : empty(q.sizes(), ScalarType::Float, q.device());
     const int64_t n_q = a[3] != Py_None ? s.numel() : 1;
     void* st = stream();
-    launch("dq8_dequantize", [&] {
-      return dq8_dequantize_ex(ptr(q), kind, (float*)ptr(out), v.outer, v.nch, v.inner,
-                               (const float*)ptr(s), (const int32_t*)ptr(z), n_q, st);
-    });
+    launch("dq8_dequantize", dq8_dequantize_ex, ptr(q), kind, (float*)ptr(out), v.outer, v.nch, v.inner,
+           (const float*)ptr(s), (const int32_t*)ptr(z), n_q, st);
     return wrap(a[5], out);
   });
 }
@@ -249,10 +241,8 @@ PyObject* py_fake_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const Tensor out = a[7] != Py_None ? tensor(a[7]) : empty(x.sizes(), ScalarType::Float, x.device());
     const int64_t n_q = a[3] != Py_None ? s.numel() : 1;
     void* st = stream();
-    launch("dq8_fake_quant", [&] {
-      return dq8_fake_quant((const float*)ptr(x), (float*)ptr(out), v.outer, v.nch, v.inner,
-                            (const float*)ptr(s), (const int32_t*)ptr(z), n_q, qmin, qmax, round_mode, st);
-    });
+    launch("dq8_fake_quant", dq8_fake_quant, (const float*)ptr(x), (float*)ptr(out), v.outer, v.nch,
+           v.inner, (const float*)ptr(s), (const int32_t*)ptr(z), n_q, qmin, qmax, round_mode, st);
     return wrap(a[7], out);
   });
 }
@@ -278,10 +268,8 @@ PyObject* py_minmax(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!ws.defined() || (size_t)ws.nbytes() < need)
       ws = empty({(int64_t)(need > 0 ? need : 1)}, ScalarType::Byte, x.device());
     void* st = stream();
-    launch("dq8_minmax", [&] {
-      return dq8_minmax((const float*)ptr(x), v.outer, v.nch, v.inner, (float*)ptr(lo), (float*)ptr(hi),
-                        ptr(ws), ws.nbytes(), st);
-    });
+    launch("dq8_minmax", dq8_minmax, (const float*)ptr(x), v.outer, v.nch, v.inner, (float*)ptr(lo),
+           (float*)ptr(hi), ptr(ws), ws.nbytes(), st);
     Py_RETURN_NONE;
   });
 }
@@ -378,28 +366,18 @@ PyObject* py_observe(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (fake) y = empty(x.sizes(), ScalarType::Float, x.device());
     const StatusWord status;
     const c10::hip::HIPStream st = c10::hip::getCurrentHIPStream();
+    launch("dq8_observe", dq8_observe, (const float*)ptr(x), v.outer, v.nch, v.inner, (float*)ptr(lo),
+           (float*)ptr(hi), symmetric, q_min, q_max, (float*)ptr(s), (int32_t*)ptr(z),
+           const_cast<int32_t*>(status.w), ptr(ws), need, (void*)st.stream());
+    if (fake)
+      launch("dq8_fake_quant", dq8_fake_quant, (const float*)ptr(x), (float*)ptr(y), v.outer, v.nch, v.inner,
+             (const float*)ptr(s), (const int32_t*)ptr(z), v.nch, q_min, q_max, DQ8_ROUND_HALF_TO_EVEN,
+             (void*)st.stream());
     int32_t answer = 0;
-    launch("dq8_observe", [&] {
-      if (int e = dq8_observe((const float*)ptr(x), v.outer, v.nch, v.inner, (float*)ptr(lo), (float*)ptr(hi),
-                              symmetric, q_min, q_max, (float*)ptr(s), (int32_t*)ptr(z),
-                              const_cast<int32_t*>(status.w), ptr(ws), need, (void*)st.stream()))
-        return e;
-      if (fake)
-        if (int e = dq8_fake_quant((const float*)ptr(x), (float*)ptr(y), v.outer, v.nch, v.inner,
-                                   (const float*)ptr(s), (const int32_t*)ptr(z), v.nch, q_min, q_max,
-                                   DQ8_ROUND_HALF_TO_EVEN, (void*)st.stream()))
-          return e;
-      return 0;
-    });
-    std::exception_ptr failed;
-    Py_BEGIN_ALLOW_THREADS
-    try {
+    {
+      const dq8::Unlocked unlocked;
       answer = status.wait(st);
-    } catch (...) {
-      failed = std::current_exception();
     }
-    Py_END_ALLOW_THREADS
-    if (failed) std::rethrow_exception(failed);
     PyObject* r = PyTuple_New(4);
     if (!r) throw PyFailure{};
     PyTuple_SET_ITEM(r, 0, PyBool_FromLong(answer == 1));
@@ -425,7 +403,7 @@ PyObject* py_lut8(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const Tensor q = dense(q0);
     const Tensor out = a[2] != Py_None ? tensor(a[2]) : empty(q.sizes(), table.scalar_type(), q.device());
     void* st = stream();
-    launch("dq8_lut8", [&] { return dq8_lut8(ptr(q), ptr(out), q.numel(), ptr(table), st); });
+    launch("dq8_lut8", dq8_lut8, ptr(q), ptr(out), q.numel(), ptr(table), st);
     return wrap(a[2], out);
   });
 }
@@ -464,11 +442,9 @@ PyObject* py_weight_only(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     const size_t ws_bytes = ws.defined() ? ws.nbytes() : 0;
     void* st = stream();
-    launch("dq8_weight_only_qgemm", [&] {
-      return dq8_weight_only_qgemm(ptr(x), xk, x.stride(0), ptr(w), w_signed, w.stride(0), tp_b, ptr(s),
-                                   (const int32_t*)ptr(zp), ptr(bias), ptr(out), out.stride(0), M, N, K,
-                                   ptr(ws), ws_bytes, st);
-    });
+    launch("dq8_weight_only_qgemm", dq8_weight_only_qgemm, ptr(x), xk, x.stride(0), ptr(w), w_signed,
+           w.stride(0), tp_b, ptr(s), (const int32_t*)ptr(zp), ptr(bias), ptr(out), out.stride(0), M, N, K,
+           ptr(ws), ws_bytes, st);
     return wrap(a[6], out);
   });
 }
@@ -500,12 +476,10 @@ PyObject* py_qgemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Tensor ws;
     if (need) ws = empty({(int64_t)need}, ScalarType::Byte, dev);
     void* st = stream();
-    launch("dq8_qgemm", [&] {
-      return dq8_qgemm_fused((const int8_t*)ptr(x), leading(x), (const int8_t*)ptr(w), leading(w), ptr(out),
-                             M ? out.stride(0) : N, M, N, K, tp_a, tp_b, (int)epilogue, ptr(bias), kind,
-                             (const float*)ptr(sx), count(sx), (const float*)ptr(sw), count(sw),
-                             (const float*)ptr(so), count(so), zx, zw, zo, ptr(ws), need, post.p, st);
-    });
+    launch("dq8_qgemm", dq8_qgemm_fused, (const int8_t*)ptr(x), leading(x), (const int8_t*)ptr(w),
+           leading(w), ptr(out), M ? out.stride(0) : N, M, N, K, tp_a, tp_b, (int)epilogue, ptr(bias), kind,
+           (const float*)ptr(sx), count(sx), (const float*)ptr(sw), count(sw), (const float*)ptr(so),
+           count(so), zx, zw, zo, ptr(ws), need, post.p, st);
     return wrap(a[12], out);
   });
 }
@@ -528,12 +502,10 @@ PyObject* py_qlinear_f32(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int kind = bias_kind(bias);
     const int zo = (int)integer(a[7]), round_mode = (int)integer(a[8]);
     void* st = stream();
-    launch("dq8_qlinear_f32", [&] {
-      return dq8_qlinear_f32((const float*)ptr(x), leading(x), (const int8_t*)ptr(w), leading(w), ptr(out),
-                             M ? out.stride(0) : N, M, N, K, (int)epilogue, ptr(bias), kind,
-                             (const float*)ptr(sx), (const float*)ptr(sw), count(sw),
-                             (const float*)ptr(so), count(so), zo, round_mode, st);
-    });
+    launch("dq8_qlinear_f32", dq8_qlinear_f32, (const float*)ptr(x), leading(x), (const int8_t*)ptr(w),
+           leading(w), ptr(out), M ? out.stride(0) : N, M, N, K, (int)epilogue, ptr(bias), kind,
+           (const float*)ptr(sx), (const float*)ptr(sw), count(sw), (const float*)ptr(so), count(so), zo,
+           round_mode, st);
     return wrap(a[9], out);
   });
 }
@@ -582,12 +554,9 @@ PyObject* py_qconv2d(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Tensor ws;
     if (need) ws = empty({(int64_t)need}, ScalarType::Byte, dev);
     void* st = stream();
-    launch("dq8_qconv2d", [&] {
-      return dq8_qconv2d_fused((const int8_t*)ptr(x), is, (const int8_t*)ptr(w), ws_, padding.v, md.v,
-                               ptr(out), os.v, (int)epilogue, ptr(bias), kind, (const float*)ptr(sx),
-                               (const float*)ptr(sw), count(sw), (const float*)ptr(so), zo, ptr(ws), need,
-                               post.p, st);
-    });
+    launch("dq8_qconv2d", dq8_qconv2d_fused, (const int8_t*)ptr(x), is, (const int8_t*)ptr(w), ws_,
+           padding.v, md.v, ptr(out), os.v, (int)epilogue, ptr(bias), kind, (const float*)ptr(sx),
+           (const float*)ptr(sw), count(sw), (const float*)ptr(so), zo, ptr(ws), need, post.p, st);
     return wrap(a[11], out);
   });
 }
@@ -605,11 +574,9 @@ PyObject* py_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const Tensor out = empty({x.size(0), x.size(1), h3 / 3}, s.defined() ? ScalarType::Char : ScalarType::Float,
                              x.device());
     void* st = stream();
-    launch("dq8_attention_f32", [&] {
-      return dq8_attention_f32((const float*)ptr(x), x.size(0), x.size(1), heads, h3 / 3 / heads,
-                               s.defined() ? nullptr : (float*)ptr(out), s.defined() ? (int8_t*)ptr(out) : nullptr,
-                               (const float*)ptr(s), st);
-    });
+    launch("dq8_attention_f32", dq8_attention_f32, (const float*)ptr(x), x.size(0), x.size(1), heads,
+           h3 / 3 / heads, s.defined() ? nullptr : (float*)ptr(out),
+           s.defined() ? (int8_t*)ptr(out) : nullptr, (const float*)ptr(s), st);
     return THPVariable_Wrap(out);
   });
 }
@@ -632,10 +599,8 @@ PyObject* py_layer_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Tensor q;
     if (s.defined()) q = empty(x.sizes(), ScalarType::Char, x.device());
     void* st = stream();
-    launch("dq8_layernorm_f32", [&] {
-      return dq8_layernorm_f32((const float*)ptr(x), rows, cols, (const float*)ptr(g), (const float*)ptr(b), eps,
-                               (float*)ptr(y), (int8_t*)ptr(q), (const float*)ptr(s), st);
-    });
+    launch("dq8_layernorm_f32", dq8_layernorm_f32, (const float*)ptr(x), rows, cols, (const float*)ptr(g),
+           (const float*)ptr(b), eps, (float*)ptr(y), (int8_t*)ptr(q), (const float*)ptr(s), st);
     if (!s.defined()) return THPVariable_Wrap(y);
     PyObject* r = PyTuple_New(2);
     if (!r) throw PyFailure{};

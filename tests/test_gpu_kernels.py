@@ -2273,3 +2273,40 @@ def test_residual_behind_f32_results_at_the_edges_of_the_fragments(K, m, k, n):
     assert torch.equal(run(post=K.make_postops(residual=r)), plain + r)
     q = torch.randint(-128, 128, (m, n), generator=g, dtype=torch.int8).cuda()
     assert torch.equal(run(post=K.make_postops(residual=q, residual_scale=sx)), plain + q.float() * sx)
+
+
+def test_operators_on_tensors_without_storage_or_rows_raise(K):
+    """What cannot be launched on raises an ordinary exception before anything is launched: a result
+    of rank 0 where rows are written, a tensor under torch.vmap, a sparse bias."""
+    i8 = torch.zeros((4, 64), dtype=torch.int8, device="cuda")
+    f32 = torch.zeros((4, 64), device="cuda")
+    one, zero = torch.ones(1, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+    sc = dict(sx=one, sw=one, so=one)
+    table = torch.zeros(256, dtype=torch.int8, device="cuda")
+    refusals = (IndexError, RuntimeError, NotImplementedError)
+
+    def rank0(dtype):
+        return torch.zeros((), dtype=dtype, device="cuda")
+
+    for call in (lambda: K.qgemm(i8, i8, K.EPI_ACC_S32, out=rank0(torch.int32)),
+                 lambda: K.qlinear_f32(f32, i8, K.EPI_REQUANT_CPU, out=rank0(torch.int8), **sc),
+                 lambda: K.weight_only_qgemm(f32, i8, f32[:, 0], out=rank0(torch.float32)),
+                 lambda: K.qgemm(i8, i8, K.EPI_REQUANT_CPU, bias=f32[0, :4].to_sparse(), **sc)):
+        with pytest.raises(refusals):
+            call()
+    batch8, batch32 = i8.reshape(2, 2, 64), f32.reshape(2, 2, 64)
+    lo, hi = one.clone(), one.clone()
+    for fn, arg in ((lambda t: K.quantize(t, one, zero), batch32), (lambda t: K.fake_quant(t, one, zero), batch32),
+                    (lambda t: K.dequantize(t, one, zero), batch8), (lambda t: K.lut8(t, table), batch8),
+                    (lambda t: K.minmax(t, lo, hi)[0], batch32),
+                    (lambda t: K.observe(t, lo, hi, True, -128, 127, fake_quant=True)[3], batch32),
+                    (lambda t: K.qgemm(t, i8, K.EPI_ACC_S32), batch8),
+                    (lambda t: K.qlinear_f32(t, i8, K.EPI_REQUANT_CPU, **sc), batch32),
+                    (lambda t: K.weight_only_qgemm(t, i8, f32[:, 0]), batch32),
+                    (lambda t: K.layer_norm(t, f32[0], f32[0]), batch32),
+                    (lambda t: K.attention(t, 1), torch.zeros((2, 1, 2, 192), device="cuda")),
+                    (lambda t: K.qconv2d(t, i8.reshape(4, 1, 1, 64), [0] * 4, list(O.NHWC_OHWI_METADATA) + [1] * 5,
+                                         [1, 1, 2, 4], K.EPI_ACC_S32), batch8.reshape(2, 1, 1, 2, 64))):
+        with pytest.raises(refusals):
+            torch.vmap(fn)(arg)
+    assert torch.equal(K.lut8(i8, table), i8)       # (and the next call works)
