@@ -18,13 +18,10 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
-#include <atomic>
-#include <chrono>
-#include <mutex>
-#include <string>
-#include <vector>
+#include <algorithm>
 
 #include "disc_q8.h"
+#include "status_words.h"
 #include "unlocked.h"
 
 namespace {
@@ -274,69 +271,17 @@ PyObject* py_minmax(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
-// Pinned words that kernels report to the host through; a call borrows one while it waits.
-class StatusWords {
- public:
-  // null when all are in use (then the caller takes one of its own)
-  static StatusWords& get() {
-    static StatusWords* words = new StatusWords;   // (for the process: torch may be gone at its end)
-    return *words;
-  }
-  volatile int32_t* borrow() {
-    std::lock_guard<std::mutex> guard(mu_);
-    if (free_.empty()) return nullptr;
-    volatile int32_t* w = free_.back();
-    free_.pop_back();
-    return w;
-  }
-  void give_back(volatile int32_t* w) {
-    std::lock_guard<std::mutex> guard(mu_);
-    free_.push_back(w);
-  }
+Tensor pinned_words(int64_t n) {
+  return at::empty({n}, at::TensorOptions().dtype(ScalarType::Int).pinned_memory(true));
+}
 
- private:
-  static constexpr int kWords = 64, kStride = 32;   // a 128-byte line each
-  StatusWords() {
-    page_ = at::empty({kWords * kStride}, at::TensorOptions().dtype(ScalarType::Int).pinned_memory(true));
-    for (int i = 0; i < kWords; ++i) free_.push_back(page_.data_ptr<int32_t>() + i * kStride);
-  }
-  Tensor page_;
-  std::mutex mu_;
-  std::vector<volatile int32_t*> free_;
-};
-
-struct StatusWord {
-  volatile int32_t* w = StatusWords::get().borrow();
-  Tensor own;
-  StatusWord() {
-    if (!w) {
-      own = at::empty({1}, at::TensorOptions().dtype(ScalarType::Int).pinned_memory(true));
-      w = own.data_ptr<int32_t>();
-    }
-    *w = 0;
-  }
-  StatusWord(const StatusWord&) = delete;
-  ~StatusWord() {
-    if (!own.defined()) StatusWords::get().give_back(w);
-  }
-  // Waits for the device's answer: reading the word costs a microsecond, a stream
-  // synchronisation ten.  After a while (a long queue in front, or a stream that cannot
-  // answer, such as one under capture) it is left to the synchronisation, which reports errors.
-  int32_t wait(const c10::hip::HIPStream& stream) const {
-    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(5);
-    for (int i = 0;; ++i) {
-      const int32_t v = *w;
-      if (v != 0) {
-        std::atomic_thread_fence(std::memory_order_acquire);
-        return v;
-      }
-      __builtin_ia32_pause();
-      if ((i & 255) == 255 && std::chrono::steady_clock::now() > until) break;
-    }
-    stream.synchronize();
-    return *w;
-  }
-};
+// (for the process: torch may be gone at its end)
+dq8::StatusWords& status_words() {
+  static constexpr int kWords = 64;
+  static const Tensor* page = new Tensor(pinned_words(kWords * dq8::StatusWords::kStride));
+  static dq8::StatusWords* words = new dq8::StatusWords(page->data_ptr<int32_t>(), kWords);
+  return *words;
+}
 
 // observe(x, min_io, max_io, axis, symmetric, q_min, q_max, fake_quant)
 //   -> (min <= max everywhere, scale, zero_point, fake-quantized x or None)
@@ -364,20 +309,39 @@ PyObject* py_observe(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const Tensor z = empty(lo.sizes(), ScalarType::Int, x.device());
     Tensor y;
     if (fake) y = empty(x.sizes(), ScalarType::Float, x.device());
-    const StatusWord status;
+    const float *xp = (const float*)ptr(x), *sp = (const float*)ptr(s);
+    float *lop = (float*)ptr(lo), *hip = (float*)ptr(hi), *yp = (float*)ptr(y);
+    int32_t* zp = (int32_t*)ptr(z);
+    void* wsp = ptr(ws);
     const c10::hip::HIPStream st = c10::hip::getCurrentHIPStream();
-    launch("dq8_observe", dq8_observe, (const float*)ptr(x), v.outer, v.nch, v.inner, (float*)ptr(lo),
-           (float*)ptr(hi), symmetric, q_min, q_max, (float*)ptr(s), (int32_t*)ptr(z),
-           const_cast<int32_t*>(status.w), ptr(ws), need, (void*)st.stream());
-    if (fake)
-      launch("dq8_fake_quant", dq8_fake_quant, (const float*)ptr(x), (float*)ptr(y), v.outer, v.nch, v.inner,
-             (const float*)ptr(s), (const int32_t*)ptr(z), v.nch, q_min, q_max, DQ8_ROUND_HALF_TO_EVEN,
-             (void*)st.stream());
+    void* raw = (void*)st.stream();
+    dq8::StatusWord<Tensor> status(status_words(), [](Tensor* own) {
+      *own = pinned_words(1);
+      return own->data_ptr<int32_t>();
+    });
+    const char* what = "dq8_observe";
+    int failed;
     int32_t answer = 0;
     {
       const dq8::Unlocked unlocked;
-      answer = status.wait(st);
+      auto drain = [&] { st.synchronize(); };
+      failed = dq8_observe(xp, v.outer, v.nch, v.inner, lop, hip, symmetric, q_min, q_max,
+                           const_cast<float*>(sp), zp, status.hand_out(), wsp, need, raw);
+      if (!failed && fake) {
+        what = "dq8_fake_quant";
+        failed = dq8_fake_quant(xp, yp, v.outer, v.nch, v.inner, sp, zp, v.nch, q_min, q_max,
+                                DQ8_ROUND_HALF_TO_EVEN, raw);
+      }
+      if (!failed) {
+        answer = status.wait(drain);
+      } else {
+        try {
+          status.settle(drain);
+        } catch (...) {   // (the error of the launch is the one to report)
+        }
+      }
     }
+    check(failed, what);
     PyObject* r = PyTuple_New(4);
     if (!r) throw PyFailure{};
     PyTuple_SET_ITEM(r, 0, PyBool_FromLong(answer == 1));

@@ -217,3 +217,17 @@ def test_observation_step_on_the_device(K, shape, axis, symmetric):
     with pytest.raises(AssertionError):
         o(dev(bad))
     assert o.scale is kept
+
+
+def test_refused_steps_leave_the_next_one_its_answer(K):
+    """More refused steps than there are status words, then a sound step and one with a NaN."""
+    x = torch.randn((3, 65), device="cuda")
+    lo, hi = fresh(1)
+    for _ in range(70):
+        with pytest.raises(RuntimeError, match="quant_min/quant_max"):
+            K.observe(x, lo, hi, True, 5, 5, fake_quant=True)
+    sound, scale, zero_point, y = K.observe(x, lo, hi, True, -128, 127, fake_quant=True)
+    assert sound and zero_point.item() == 0 and lo.item() == x.min().item()
+    assert torch.equal(y, K.fake_quant(x, scale, zero_point))
+    x[2, 64] = float("nan")
+    assert not K.observe(x, lo, hi, True, -128, 127)[0]

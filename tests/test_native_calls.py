@@ -42,3 +42,10 @@ def test_the_interpreter_lock_is_held_again_after_an_exception(tmp_path):
     r = subprocess.run([sys.executable, "-c", script], cwd=str(tmp_path), capture_output=True,
                        text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.strip() == "ok", (r.returncode, r.stdout, r.stderr)
+
+
+def test_a_status_word_with_an_answer_outstanding_is_not_lent_again(tmp_path):
+    """An answer that comes after its call has failed must not reach the next borrower."""
+    exe = _compile(tmp_path, "status_words_check.cc", "status_words_check", "-pthread")
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout + r.stderr
