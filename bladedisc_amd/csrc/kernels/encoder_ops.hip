@@ -77,10 +77,11 @@ attention_f32_kernel(const float* __restrict__ qkv, int S, uint32_t all_heads, i
 #pragma unroll
     for (int i = 0; i < kPasses; ++i) {
       const int row = lrow + i * step;
-      kreg[i] = vreg[i] = (v4f){0.f, 0.f, 0.f, 0.f};        // (past the sequence: a zero probability times this)
-      if (row < kBlock && key0 + i * step < S) {
-        const int key = key0 + row < S ? key0 + row : S - 1;
-        const float* p = base + key * row3 + (int64_t)heads * kHead + lcol;
+      // (zeros past the sequence: what stands there is met by a probability of zero, and zero times a
+      // copy of a token with infinite values would be a NaN)
+      kreg[i] = vreg[i] = (v4f){0.f, 0.f, 0.f, 0.f};
+      if (row < kBlock && key0 + row < S) {
+        const float* p = base + (key0 + row) * row3 + (int64_t)heads * kHead + lcol;
         kreg[i] = *reinterpret_cast<const v4f*>(p);
         vreg[i] = *reinterpret_cast<const v4f*>(p + (int64_t)heads * kHead);
       }
@@ -132,14 +133,17 @@ attention_f32_kernel(const float* __restrict__ qkv, int S, uint32_t all_heads, i
       }
     top = fmaxf(top, __shfl_xor(top, 16, 64));
     top = fmaxf(top, __shfl_xor(top, 32, 64));
-    const float keep = __builtin_amdgcn_exp2f(m - top);     // (m = -inf at first: 0)
+    // (scores of -inf alone so far: their probabilities are zero, where -inf - -inf would be a NaN for
+    // the keys to come; nothing but -inf in the whole row divides zero by zero at the end)
+    const float ref = top == -__builtin_inff() ? 0.f : top;
+    const float keep = __builtin_amdgcn_exp2f(m - ref);     // (m = -inf at first: 0)
     m = top;
     float sum = 0.f;
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        s[kt][v] = __builtin_amdgcn_exp2f(s[kt][v] - top);
+        s[kt][v] = __builtin_amdgcn_exp2f(s[kt][v] - ref);
         sum += s[kt][v];
       }
     l = l * keep + sum;

@@ -2310,3 +2310,28 @@ def test_operators_on_tensors_without_storage_or_rows_raise(K):
         with pytest.raises(refusals):
             torch.vmap(fn)(arg)
     assert torch.equal(K.lut8(i8, table), i8)       # (and the next call works)
+
+
+@pytest.mark.parametrize("s", [17, 64, 65, 130, 200])
+def test_attention_with_infinite_scores_and_values(K, s):
+    """Scores of -inf for the first keys (all of the first 64 where there are more), for every key,
+    and of +inf; infinite values in the last token, next to the rows past the sequence: the f64
+    result, NaN where that is NaN."""
+    g = torch.Generator().manual_seed(s)
+    qkv = torch.randn(3, s, 3 * 64, generator=g)
+    q, k, v = qkv[..., :64], qkv[..., 64:128], qkv[..., 128:]
+    q[..., 0] = q[..., 0].abs() + 0.5
+    q[0, 1, 0] = -1.0                                # +inf scores: no probability is defined
+    k[0, :min(64, s - 1), 0] = -float("inf")         # (the keys behind them decide)
+    k[1, :, 0] = -float("inf")
+    v[2, -1, 3], v[2, -1, 40] = float("inf"), -float("inf")
+    qd, kd, vd = q.double(), k.double(), v.double()
+    want = torch.softmax(qd @ kd.transpose(1, 2) / 8.0, -1) @ vd
+    assert not want[0, 0].isnan().any() and want[0, 1].isnan().all() and want[1].isnan().all()
+    assert (want[2, :, 3] == float("inf")).all() and (want[2, :, 40] == -float("inf")).all()
+    got = K.attention(qkv.cuda(), 1)
+    torch.testing.assert_close(got.cpu().double(), want, rtol=1e-5, atol=1e-5, equal_nan=True)
+    scale = torch.full((1,), 0.02, device="cuda")
+    got_q = K.attention(qkv.cuda(), 1, scale)
+    assert torch.equal(got_q, K.quantize(got, scale, torch.zeros(1, dtype=torch.int32, device="cuda")))
+    assert (got_q[2, :, 3] == 127).all() and (got_q[2, :, 40] == -128).all()
