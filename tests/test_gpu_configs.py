@@ -275,6 +275,40 @@ def test_config5_bert_layer_operators_in_the_gemm_epilogues_are_bit_identical(C,
 
 
 @pytest.mark.parametrize("backend", ["raw", "ral"])
+@pytest.mark.parametrize("batch,seq", [(8, 32), (3, 17), (1, 1), (2, 384)])
+def test_config5_bert_layer_in_eight_launches_has_the_bits_of_the_separate_operators(C, batch, seq, backend, monkeypatch):
+    """forward() without a record runs the layer with every operator in a neighbour's pass; the
+    output is that of the layer whose operators all run by themselves, bit for bit."""
+    from bladedisc_amd import bert_layer as B
+    from bladedisc_amd import ral
+    ctx = ex = None
+    if backend == "ral":
+        ctx = ral.RalContext(stream=torch.cuda.current_stream().cuda_stream)
+        ex = ctx.execution()
+    try:
+        be = B.RalBackend(ex) if ex is not None else B.RawBackend()
+        layer = B.QuantBertLayer(C.config5_weights(), be)
+        h = layer.embed(C.config5_tokens(batch, seq))
+        layer.calibrate(h)
+        rec = {}
+        want = layer.forward(h, rec)
+        assert all(rec[name]["y_q"] is not None for name in B.LINEARS)       # (nothing was fused)
+        layer.fuse_epilogue = layer.fuse_gelu = layer.fuse_dequant = True
+        taken = []
+        fused = layer._forward_fused
+        monkeypatch.setattr(layer, "_forward_fused", lambda x: taken.append(1) or fused(x))
+        got = layer.forward(h)
+        torch.cuda.synchronize()
+        assert taken and got.shape == want.shape
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+    finally:
+        if ex is not None:
+            torch.cuda.synchronize()
+            ex.close()
+            ctx.close()
+
+
+@pytest.mark.parametrize("backend", ["raw", "ral"])
 @pytest.mark.parametrize("fused", [False, True, "epilogue"])
 def test_config5_bert_layer_graph_replays_match_eager(C, fused, backend):
     """The captured layer against eager execution: several replays, with eager work and
