@@ -655,28 +655,36 @@ extern "C" const char* dq8_qgemm_variant_name(int variant) {
 }
 #endif
 
+namespace {
+size_t pad256(int64_t v) { return (size_t)((v + 255) / 256 * 256); }
+
+// The scratch of a problem: an operand that is not k-contiguous, or whose K is not a multiple of
+// 16, is rewritten as [rows, K rounded up to 16] (zero filled) for the MFMA kernels, rows K rounded
+// up to `row_multiple` bytes apart; zero points add the per-column and per-row corrections.
+size_t qgemm_scratch(int64_t M, int64_t N, int64_t K, bool tp_a, bool tp_b, bool zp, int64_t row_multiple) {
+  const int64_t pitch = (K + row_multiple - 1) / row_multiple * row_multiple;
+  size_t bytes = 0;
+  if (tp_a || K % 16 != 0) bytes += pad256(M * pitch);
+  if (!tp_b || K % 16 != 0) bytes += pad256(N * pitch);
+  if (zp) bytes += pad256(N * 4) + pad256(M * 4);
+  return bytes;
+}
+
+// Rows a multiple of 128 bytes apart where the scratch has room for them: the kernels' loads cover
+// 8 rows x 128 bytes, which is 8 cache lines if the rows begin at one and 16 otherwise (777 x 1504,
+// 1008 of k: 6.8 us, 1024 of k: 6.2).  Scratch of a caller that counts rows of K rounded up to 16 is
+// taken as well.
+constexpr int64_t kRowMultiple = 128, kRowMultipleLeast = 16;
+}  // namespace
+
 extern "C" size_t dq8_qgemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int tp_a,
                                             int tp_b) {
-  // an operand that is not k-contiguous, or whose K is not a multiple of 16, is rewritten as
-  // [rows, K rounded up to 16] (zero filled) for the MFMA kernels, rows a multiple of 128 bytes
-  // apart: their loads cover 8 rows x 128 bytes, which is 8 cache lines if the rows begin at one
-  // and 16 otherwise (777 x 1504, 1008 of k: 6.8 us, 1024 of k: 6.2)
-  size_t bytes = 0;
-  auto pad = [](int64_t v) { return (size_t)((v + 255) / 256 * 256); };
-  const int64_t kp = (K + 127) / 128 * 128;
-  if (tp_a || K % 16 != 0) bytes += pad(M * kp);
-  if (!tp_b || K % 16 != 0) bytes += pad(N * kp);
-  return bytes;
+  return qgemm_scratch(M, N, K, tp_a != 0, tp_b != 0, false, kRowMultiple);
 }
 
 extern "C" size_t dq8_qgemm_workspace_bytes_zp(int64_t M, int64_t N, int64_t K, int tp_a,
                                                int tp_b, int32_t zx, int32_t zw) {
-  size_t bytes = dq8_qgemm_workspace_bytes(M, N, K, tp_a, tp_b);
-  if (zx != 0 || zw != 0) {   // the per-column and per-row corrections
-    auto pad = [](int64_t v) { return (size_t)((v + 255) / 256 * 256); };
-    bytes += pad(N * 4) + pad(M * 4);
-  }
-  return bytes;
+  return qgemm_scratch(M, N, K, tp_a != 0, tp_b != 0, zx != 0 || zw != 0, kRowMultiple);
 }
 
 extern "C" int dq8_transpose_s8(const int8_t* src, int64_t ld, int8_t* dst, int64_t rows,
@@ -767,7 +775,7 @@ int qgemm_impl(int variant, const int8_t* A, int64_t lda, const int8_t* W, int64
   // The tiled MFMA kernels want A [M, K'] and W [N, K'], k-contiguous, rows 16-byte aligned, K' a
   // multiple of 16: operands in another layout, or with a ragged K, are rewritten into the
   // workspace (zero-filled up to K'; zeros add nothing to the sums).
-  const int64_t Kp = (K + 15) / 16 * 16, pitch = (K + 127) / 128 * 128;
+  const int64_t Kp = (K + 15) / 16 * 16;
   // Rows of any length or alignment where the copy to aligned ones would cost as much as the
   // product: the small-M kernel and the 64 x 64 tiles take them as they are.
   if (auto_pick && !tp_a && tp_b && K >= 64 &&
@@ -796,14 +804,16 @@ int qgemm_impl(int variant, const int8_t* A, int64_t lda, const int8_t* W, int64
   }
   const bool repack_a = K > 0 && (tp_a || K % 16 != 0);
   const bool repack_w = K > 0 && (!tp_b || K % 16 != 0);
-  const bool have_ws = workspace != nullptr && aligned(workspace, 256) &&
-                       workspace_bytes >= dq8_qgemm_workspace_bytes(M, N, K, tp_a, tp_b);
+  auto scratch = [&](bool zp, int64_t row_multiple) {
+    return workspace != nullptr && aligned(workspace, 256) &&
+           workspace_bytes >= qgemm_scratch(M, N, K, tp_a != 0, tp_b != 0, zp, row_multiple);
+  };
+  const int64_t row_multiple = scratch(has_zp && auto_pick, kRowMultiple) ? kRowMultiple : kRowMultipleLeast;
+  const int64_t pitch = (K + row_multiple - 1) / row_multiple * row_multiple;
+  const bool have_ws = scratch(false, row_multiple);
   const bool mfma_operands = (repack_a ? have_ws : (aligned(A, 16) && lda % 16 == 0)) &&
                              (repack_w ? have_ws : (aligned(W, 16) && ldw % 16 == 0));
-  const bool zp_mfma =
-      has_zp && auto_pick && K > 0 && mfma_operands && workspace != nullptr &&
-      aligned(workspace, 256) &&
-      workspace_bytes >= dq8_qgemm_workspace_bytes_zp(M, N, K, tp_a, tp_b, zx, zw);
+  const bool zp_mfma = has_zp && auto_pick && K > 0 && mfma_operands && scratch(true, row_multiple);
   if (auto_pick && has_zp && !zp_mfma) variant = 0;
   const bool fused = e.table != nullptr || e.resid_kind != 0;
   // (a ragged K without the scratch to pad it, or unaligned operands: the generic kernel
@@ -835,13 +845,12 @@ int qgemm_impl(int variant, const int8_t* A, int64_t lda, const int8_t* W, int64
   const int8_t* w_use = W;
   int64_t lda_use = lda, ldw_use = ldw;
   size_t ws_off = 0;
-  auto pad = [](int64_t v) { return (size_t)((v + 255) / 256 * 256); };
   // Where the operands go: a transposed one through the transpose kernel, one with ragged rows
   // through prepare_rows_kernel, which also forms the zero-point corrections.
   RowsJob job_w = {}, job_a = {};
   auto place = [&](const int8_t* src, int64_t ld, bool transposed, int64_t rows, RowsJob* job) {
     int8_t* dst = (int8_t*)workspace + ws_off;
-    ws_off += pad(rows * pitch);
+    ws_off += pad256(rows * pitch);
     if (transposed) {   // src is [K, rows]
       hipLaunchKernelGGL(transpose_s8_kernel,
                          dim3((unsigned)ceil_div(rows, 64), (unsigned)ceil_div(pitch, 64)), dim3(256),
@@ -905,7 +914,7 @@ int qgemm_impl(int variant, const int8_t* A, int64_t lda, const int8_t* W, int64
     };
     sums(&job_w, w_use, ldw_use, N, corr_n, -zx, kzz);
     if (zw != 0) {
-      corr_m = reinterpret_cast<int32_t*>((int8_t*)corr_n + pad(N * 4));
+      corr_m = reinterpret_cast<int32_t*>((int8_t*)corr_n + pad256(N * 4));
       sums(&job_a, a_use, lda_use, M, corr_m, -zw, 0);
     }
   }
@@ -1102,7 +1111,6 @@ bool is_nchw_oihw(const int32_t md[17]) {
   return true;
 }
 
-size_t pad256(int64_t v) { return (size_t)((v + 255) / 256 * 256); }
 
 int out_elem_size(int epilogue) {
   return (epilogue == DQ8_EPI_ACC_S32 || epilogue == DQ8_EPI_DEQUANT_F32 ||

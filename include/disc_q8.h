@@ -239,9 +239,10 @@ int dq8_tf_dequantize(const void* q, int in_kind, float* out, int64_t outer, int
 
 /* Bytes of device scratch dq8_qgemm needs for this problem with zx == zw == 0 (0 when it
  * needs none: tp_a == 0, tp_b == 1 and K % 16 == 0).  Operands in the other layout, or with
- * a K that is not a multiple of 16, are rewritten there as [rows, K rounded up to 128].  A
- * ragged K without the scratch still gives the right result, from the generic kernel; a
- * transposed operand without it is an error. */
+ * a K that is not a multiple of 16, are rewritten there as [rows, K rounded up to 128], or,
+ * where a caller's scratch only has room for that, as [rows, K rounded up to 16].  A ragged K
+ * without the scratch still gives the right result, from the generic kernel; a transposed
+ * operand without it is an error. */
 size_t dq8_qgemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int tp_a,
                                  int tp_b);
 /* The same for given input / weight zero points: with a non-zero one it adds two correction

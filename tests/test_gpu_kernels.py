@@ -2335,3 +2335,28 @@ def test_attention_with_infinite_scores_and_values(K, s):
     got_q = K.attention(qkv.cuda(), 1, scale)
     assert torch.equal(got_q, K.quantize(got, scale, torch.zeros(1, dtype=torch.int32, device="cuda")))
     assert (got_q[2, :, 3] == 127).all() and (got_q[2, :, 40] == -128).all()
+
+
+@pytest.mark.parametrize("m,n,k,tp_a,tp_b", [(300, 260, 784, 0, 0), (300, 260, 272, 1, 0), (129, 70, 1041, 1, 1),
+                                             (1000, 768, 777, 0, 1), (17, 33, 16, 0, 0)])
+@pytest.mark.parametrize("zx,zw", [(0, 0), (-11, 0), (5, -3)])
+def test_qgemm_scratch_for_rows_of_k_rounded_up_to_16(K, m, n, k, tp_a, tp_b, zx, zw):
+    """Scratch counted with rows of K rounded up to 16 bytes, less than dq8_qgemm_workspace_bytes
+    asks for, is enough, with and without room for the zero-point corrections; nothing behind it
+    is written."""
+    rng = np.random.default_rng(m + n + k)
+    a = rng.integers(-128, 128, (k, m) if tp_a else (m, k), dtype=np.int8)
+    w = rng.integers(-128, 128, (n, k) if tp_b else (k, n), dtype=np.int8)
+    want = ((a.T if tp_a else a).astype(np.int64) - zx) @ ((w if tp_b else w.T).astype(np.int64) - zw).T
+    up = lambda v: (v + 255) // 256 * 256      # noqa: E731
+    k16 = (k + 15) // 16 * 16
+    rows = (up(m * k16) if tp_a or k % 16 else 0) + (up(n * k16) if not tp_b or k % 16 else 0)
+    L, da, dw = K._lib.lib(), dev(a), dev(w)
+    for size in {rows, rows + (up(4 * n) + up(4 * m) if zx or zw else 0)}:
+        ws = torch.full((size + 256,), 77, dtype=torch.uint8, device="cuda")
+        out = torch.empty((m, n), dtype=torch.int32, device="cuda")
+        st = L.dq8_qgemm(K._ptr(da), da.stride(0), K._ptr(dw), dw.stride(0), K._ptr(out), n, m, n, k, tp_a, tp_b,
+                         K.EPI_ACC_S32, None, 0, None, 0, None, 0, None, 0, zx, zw, 0, K._ptr(ws), size, K._stream())
+        K._lib.check(st, "dq8_qgemm")
+        np.testing.assert_array_equal(host(out), want)
+        assert (ws[size:] == 77).all()
