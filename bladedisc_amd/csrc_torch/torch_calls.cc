@@ -78,6 +78,17 @@ int64_t integer(PyObject* o) {
   return v;
 }
 
+// int(o): a float as well
+int64_t as_integer(PyObject* o) {
+  if (PyLong_Check(o)) return integer(o);
+  PyObject* made = PyNumber_Long(o);
+  if (!made) throw PyFailure{};
+  const int64_t v = PyLong_AsLongLong(made);
+  Py_DECREF(made);
+  if (v == -1 && PyErr_Occurred()) throw PyFailure{};
+  return v;
+}
+
 bool truth(PyObject* o) {
   const int v = PyObject_IsTrue(o);
   if (v < 0) throw PyFailure{};
@@ -86,7 +97,7 @@ bool truth(PyObject* o) {
 
 Tensor dense(const Tensor& t) { return t.is_contiguous() ? t : t.contiguous(); }
 
-// A scale operand: a flat f32 device tensor, or a number.
+// A scale operand: a flat f32 device tensor, a number, or a sequence or array of numbers.
 Tensor scale(PyObject* o, const at::Device& dev) {
   if (o == Py_None) return Tensor();
   if (THPVariable_Check(o)) {
@@ -94,9 +105,19 @@ Tensor scale(PyObject* o, const at::Device& dev) {
     if (t.scalar_type() == ScalarType::Float && t.is_contiguous()) return t;
     return t.reshape({-1}).contiguous().to(ScalarType::Float);
   }
-  const double v = PyFloat_AsDouble(o);
-  if (v == -1.0 && PyErr_Occurred()) throw PyFailure{};
-  return at::full({1}, v, at::TensorOptions().dtype(ScalarType::Float).device(dev));
+  if (PyFloat_Check(o) || (PyNumber_Check(o) && !PyObject_HasAttrString(o, "__len__"))) {
+    const double v = PyFloat_AsDouble(o);
+    if (v == -1.0 && PyErr_Occurred()) throw PyFailure{};
+    return at::full({1}, v, at::TensorOptions().dtype(ScalarType::Float).device(dev));
+  }
+  // whatever else torch.tensor takes: lists, numpy arrays
+  PyObject* mod = PyImport_ImportModule("torch");
+  PyObject* made = mod ? PyObject_CallMethod(mod, "tensor", "O", o) : nullptr;
+  Py_XDECREF(mod);
+  if (!made) throw PyFailure{};
+  const Tensor t = THPVariable_Unpack(made);
+  Py_DECREF(made);
+  return t.reshape({-1}).to(ScalarType::Float).to(dev).contiguous();
 }
 
 int64_t count(const Tensor& t) { return t.defined() ? t.numel() : 0; }
@@ -196,7 +217,7 @@ PyObject* py_quantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const Tensor &s = device_tensor(a[1]), &z = device_tensor(a[2]);
     const int xk = float_kind(x, "quantize takes f32 or f16 input");
     const View3 v(x, a[3]);
-    const int64_t qmin = integer(a[4]), qmax = integer(a[5]);
+    const int64_t qmin = as_integer(a[4]), qmax = as_integer(a[5]);
     const int round_mode = (int)integer(a[6]), kind = (int)integer(a[7]);
     const Tensor out = a[9] != Py_None
                            ? tensor(a[9])

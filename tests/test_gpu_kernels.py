@@ -2360,3 +2360,27 @@ def test_qgemm_scratch_for_rows_of_k_rounded_up_to_16(K, m, n, k, tp_a, tp_b, zx
         K._lib.check(st, "dq8_qgemm")
         np.testing.assert_array_equal(host(out), want)
         assert (ws[size:] == 77).all()
+
+
+def test_bounds_and_scales_in_every_form_python_has_for_them(K):
+    """quantize's bounds as floats, a GEMM's scales as a number, list, numpy array or tensor of any
+    float type: the results of integers and flat f32 device tensors."""
+    rng = np.random.default_rng(5)
+    x = dev(rng.standard_normal((6, 64)).astype(np.float32))
+    one, zero = torch.full((1,), 0.05, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+    q = K.quantize(x, one, zero, qmin=-7, qmax=100)
+    for lo, hi in ((-7.0, 100.0), (np.float32(-7), np.int64(100)), (np.float64(-7.9), 100.5)):
+        assert torch.equal(K.quantize(x, one, zero, qmin=lo, qmax=hi), q)
+    w = dev(rng.integers(-128, 128, (5, 64), dtype=np.int8))
+    s = rng.uniform(0.01, 0.02, 5).astype(np.float32)
+    sx, so = np.float32(0.05), np.float32(0.3)
+    want = K.qgemm(q, w, K.EPI_REQUANT_CPU, sx=dev(sx.reshape(1)), sw=dev(s), so=dev(so.reshape(1)))
+    assert want.abs().max() > 0
+    for a, b, c in ((float(sx), s.tolist(), float(so)), (sx, s, so), ([float(sx)], s.astype(np.float64), so.reshape(1, 1)),
+                    (dev(sx.reshape(1)), dev(s).double().reshape(5, 1), dev(np.stack([so, so]))[:1])):
+        assert torch.equal(K.qgemm(q, w, K.EPI_REQUANT_CPU, sx=a, sw=b, so=c), want)
+    want = K.qlinear_f32(x, w, K.EPI_REQUANT_CPU, sx=dev(sx.reshape(1)), sw=dev(s), so=dev(so.reshape(1)))
+    assert torch.equal(K.qlinear_f32(x, w, K.EPI_REQUANT_CPU, sx=float(sx), sw=s.tolist(), so=so), want)
+    for bad in ("0.05", {}, object()):
+        with pytest.raises((TypeError, ValueError, RuntimeError)):
+            K.qgemm(q, w, K.EPI_REQUANT_CPU, sx=bad, sw=s.tolist(), so=so)
