@@ -139,8 +139,8 @@ def torch_calls():
     lib()
     if not os.path.exists(TORCH_CALLS_PATH):
         raise RuntimeError(
-            "%s is missing: build it with `python -m bladedisc_amd.build` "
-            "(there is no fallback)" % TORCH_CALLS_PATH)
+            "%s is missing: build it with `python -m bladedisc_amd.build`, which needs Python's and "
+            "torch's headers for it (there is no fallback)" % TORCH_CALLS_PATH)
     from . import _torch_calls
     return _torch_calls
 

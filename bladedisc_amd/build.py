@@ -105,31 +105,47 @@ def _record_resources(obj, lines):
         json.dump(kernels, f, indent=0, sort_keys=True)
 
 
+def torch_calls_headers():
+    """Include folders of Python and torch; RuntimeError naming what is not installed."""
+    import sysconfig
+    python = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(python, "Python.h")):
+        raise RuntimeError("Python's headers are missing (%s/Python.h)" % python)
+    try:
+        import torch
+    except ImportError as e:
+        raise RuntimeError("torch is missing (%s)" % e)
+    include = os.path.join(os.path.dirname(torch.__file__), "include")
+    if not os.path.exists(os.path.join(include, "torch", "csrc", "python_headers.h")):
+        raise RuntimeError("torch's C++ headers are missing (%s)" % include)
+    return [python, include, os.path.join(include, "torch", "csrc", "api", "include")]
+
+
 def build_torch_calls(force=False):
     """csrc_torch/torch_calls.cc -> _torch_calls.so, linked against the product library next to
-    it and the torch libraries of the running interpreter (loaded by `import torch` before)."""
-    import sysconfig
-
+    it and the torch libraries of the running interpreter (loaded by `import torch` before).
+    Compiled by hipcc, as everything else here; the HIP runtime is torch's."""
+    headers = torch_calls_headers()
     import torch
     src = os.path.dirname(TORCH_CALLS_SRC)
     inputs = [os.path.join(src, f) for f in os.listdir(src)] + [os.path.join(ROOT, "include", "disc_q8.h")]
     if (not force and os.path.exists(TORCH_CALLS)
             and os.path.getmtime(TORCH_CALLS) > max(map(os.path.getmtime, inputs))):
         return TORCH_CALLS
-    t = os.path.dirname(torch.__file__)
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
-           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+    cmd = [HIPCC, "-no-hip-rt", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
-           "-I" + os.path.join(ROOT, "include"), "-isystem", sysconfig.get_paths()["include"],
-           "-isystem", os.path.join(t, "include"),
-           "-isystem", os.path.join(t, "include", "torch", "csrc", "api", "include"),
-           "-isystem", "/opt/rocm/include", TORCH_CALLS_SRC, "-o", TORCH_CALLS,
-           "-L" + PKG, "-l:" + os.path.basename(LIB), "-L" + os.path.join(t, "lib"),
-           "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python",
-           "-Wl,-rpath,$ORIGIN"]
+           "-I" + os.path.join(ROOT, "include")]
+    for h in headers + ["/opt/rocm/include"]:
+        cmd += ["-isystem", h]
+    cmd += ["-x", "c++", TORCH_CALLS_SRC, "-x", "none", "-o", TORCH_CALLS,
+            "-L" + PKG, "-l:" + os.path.basename(LIB),
+            "-L" + os.path.join(os.path.dirname(torch.__file__), "lib"),
+            "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python",
+            "-Wl,-rpath,$ORIGIN"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
-        raise RuntimeError("g++ failed for %s:\n%s" % (TORCH_CALLS_SRC, r.stdout + r.stderr))
+        raise RuntimeError("hipcc failed for %s:\n%s" % (TORCH_CALLS_SRC, r.stdout + r.stderr))
     return TORCH_CALLS
 
 
@@ -180,7 +196,14 @@ def build(force=False, verbose=False, jobs=8):
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError("link of the test-hooks library failed:\n" + r.stdout + r.stderr)
-    build_torch_calls(force)
+    # The libraries above need neither Python nor torch; where their headers are not installed the
+    # native callers are left out, and kernels.py says so when it is used.
+    try:
+        torch_calls_headers()
+    except RuntimeError as e:
+        print("not built: %s: %s" % (os.path.basename(TORCH_CALLS), e), file=sys.stderr)
+    else:
+        build_torch_calls(force)
     return LIB
 
 

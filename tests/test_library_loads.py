@@ -70,3 +70,26 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
         kernels.variant_names()
     with pytest.raises(RuntimeError, match="no CPU fallback"):
         kernels.qlinear_f32_fused_max_rows(768, 768)
+
+
+def test_the_libraries_build_without_python_headers(monkeypatch, tmp_path, capsys):
+    """A machine without Python's headers still gets the C ABI and RAL libraries; the native
+    callers are left out, by name, and nothing of an earlier build of them is touched."""
+    import sysconfig
+
+    import pytest
+    from bladedisc_amd import build as b
+    paths = dict(sysconfig.get_paths(), include=str(tmp_path))
+    monkeypatch.setattr(sysconfig, "get_paths", lambda *a, **k: paths)
+    with pytest.raises(RuntimeError, match="Python.h"):
+        b.build_torch_calls()
+    # (nothing to compile: the objects and libraries that are there pass for new ones)
+    monkeypatch.setattr(b, "_compile", lambda *a, **k: (b.EXPORTS, ""))
+    monkeypatch.setattr(b, "sources", lambda: [b.EXPORTS])
+    for name in ("LIB", "HOOKS_LIB"):
+        lib = tmp_path / name
+        lib.write_bytes(b"")
+        monkeypatch.setattr(b, name, str(lib))
+    monkeypatch.setattr(b, "OBJ", str(tmp_path / "build"))
+    assert b.build() == b.LIB
+    assert "Python.h" in capsys.readouterr().err
