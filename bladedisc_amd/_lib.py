@@ -11,8 +11,19 @@ LIB_PATH = os.path.join(_PKG, "libdisc_q8_ral.so")
 # selection and the MFMA layout probe, which the product library does not carry
 HOOKS_LIB_PATH = os.path.join(_PKG, "libdisc_q8_testhooks.so")
 
-# the native callers of kernels.py (csrc_torch/torch_calls.cc), a CPython module
-TORCH_CALLS_PATH = os.path.join(_PKG, "_torch_calls.so")
+
+
+def torch_calls_path():
+    """Where the native callers of kernels.py are (csrc_torch/torch_calls.cc), a CPython module on
+    torch's C++ ABI: the torch and the interpreter it was built for are part of its name, so that
+    a module built for others is never loaded."""
+    import sysconfig
+
+    import torch
+    return os.path.join(_PKG, "_torch_calls.torch-%s.%s.so" % (torch.__version__,
+                                                               sysconfig.get_config_var("SOABI")))
+
+
 
 _lib = None
 _hooks = None
@@ -136,13 +147,19 @@ def lib():
 
 def torch_calls():
     """The module of native callers (kernels.py); it links the product library."""
+    import importlib.machinery
+    import importlib.util
     lib()
-    if not os.path.exists(TORCH_CALLS_PATH):
+    path = torch_calls_path()
+    if not os.path.exists(path):
         raise RuntimeError(
-            "%s is missing: build it with `python -m bladedisc_amd.build`, which needs Python's and "
-            "torch's headers for it (there is no fallback)" % TORCH_CALLS_PATH)
-    from . import _torch_calls
-    return _torch_calls
+            "%s is missing: build it for this torch with `python -m bladedisc_amd.build`, which "
+            "needs Python's and torch's headers for it (there is no fallback)" % path)
+    name = __package__ + "._torch_calls"
+    loader = importlib.machinery.ExtensionFileLoader(name, path)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_file_location(name, path, loader=loader))
+    loader.exec_module(module)
+    return module
 
 
 def check(status, what, L=None):

@@ -1,5 +1,5 @@
 """Builds libdisc_q8_ral.so: the gfx950 kernels, their C ABI and the RAL runtime; and
-_torch_calls.so, the native callers behind kernels.py.
+_torch_calls.*.so, the native callers behind kernels.py.
 
 Everything is compiled in-tree with hipcc for gfx950 only (hipcc cross-compiles
 without a GPU).  Usage: ``python -m bladedisc_amd.build [--force]``.
@@ -23,7 +23,6 @@ EXPORTS = os.path.join(CSRC, "exports.map")
 
 # a CPython module on torch's C++ headers (host code only)
 TORCH_CALLS_SRC = os.path.join(PKG, "csrc_torch", "torch_calls.cc")
-TORCH_CALLS = os.path.join(PKG, "_torch_calls.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
@@ -122,23 +121,25 @@ def torch_calls_headers():
 
 
 def build_torch_calls(force=False):
-    """csrc_torch/torch_calls.cc -> _torch_calls.so, linked against the product library next to
+    """csrc_torch/torch_calls.cc -> _lib.torch_calls_path(), linked against the product library next to
     it and the torch libraries of the running interpreter (loaded by `import torch` before).
     Compiled by hipcc, as everything else here; the HIP runtime is torch's."""
     headers = torch_calls_headers()
     import torch
+    from ._lib import torch_calls_path
+    target = torch_calls_path()
     src = os.path.dirname(TORCH_CALLS_SRC)
     inputs = [os.path.join(src, f) for f in os.listdir(src)] + [os.path.join(ROOT, "include", "disc_q8.h")]
-    if (not force and os.path.exists(TORCH_CALLS)
-            and os.path.getmtime(TORCH_CALLS) > max(map(os.path.getmtime, inputs))):
-        return TORCH_CALLS
+    if (not force and os.path.exists(target)
+            and os.path.getmtime(target) > max(map(os.path.getmtime, inputs))):
+        return target
     cmd = [HIPCC, "-no-hip-rt", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
            "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
            "-I" + os.path.join(ROOT, "include")]
     for h in headers + ["/opt/rocm/include"]:
         cmd += ["-isystem", h]
-    cmd += ["-x", "c++", TORCH_CALLS_SRC, "-x", "none", "-o", TORCH_CALLS,
+    cmd += ["-x", "c++", TORCH_CALLS_SRC, "-x", "none", "-o", target,
             "-L" + PKG, "-l:" + os.path.basename(LIB),
             "-L" + os.path.join(os.path.dirname(torch.__file__), "lib"),
             "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python",
@@ -146,7 +147,7 @@ def build_torch_calls(force=False):
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("hipcc failed for %s:\n%s" % (TORCH_CALLS_SRC, r.stdout + r.stderr))
-    return TORCH_CALLS
+    return target
 
 
 def build_test_code_objects():
@@ -201,7 +202,7 @@ def build(force=False, verbose=False, jobs=8):
     try:
         torch_calls_headers()
     except RuntimeError as e:
-        print("not built: %s: %s" % (os.path.basename(TORCH_CALLS), e), file=sys.stderr)
+        print("not built: the native callers of kernels.py: %s" % e, file=sys.stderr)
     else:
         build_torch_calls(force)
     return LIB

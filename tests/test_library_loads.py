@@ -93,3 +93,16 @@ def test_the_libraries_build_without_python_headers(monkeypatch, tmp_path, capsy
     monkeypatch.setattr(b, "OBJ", str(tmp_path / "build"))
     assert b.build() == b.LIB
     assert "Python.h" in capsys.readouterr().err
+
+
+def test_native_callers_of_another_torch_are_not_loaded(monkeypatch):
+    """The module is on torch's C++ ABI: one that was built for another torch (or interpreter) is
+    not found, instead of being loaded and going wrong somewhere."""
+    import pytest
+    import torch
+    from bladedisc_amd import _lib
+    assert torch.__version__ in os.path.basename(_lib.torch_calls_path())
+    assert _lib.torch_calls().qgemm
+    monkeypatch.setattr(torch, "__version__", "9.9.9")
+    with pytest.raises(RuntimeError, match="9.9.9.*build it for this torch"):
+        _lib.torch_calls()
