@@ -70,7 +70,9 @@ Tensor optional_device_tensor(PyObject* o) {
   return o == Py_None ? Tensor() : device_tensor(o);
 }
 
-void* ptr(const Tensor& t) { return t.defined() ? const_cast<void*>(t.const_data_ptr()) : nullptr; }
+// what is read, and what is written (a lazy copy becomes a real one first)
+const void* in(const Tensor& t) { return t.defined() ? t.const_data_ptr() : nullptr; }
+void* inout(const Tensor& t) { return t.defined() ? t.mutable_data_ptr() : nullptr; }
 
 int64_t integer(PyObject* o) {
   const int64_t v = PyLong_AsLongLong(o);
@@ -224,8 +226,8 @@ PyObject* py_quantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
                            : empty(x.sizes(), reinterpret_cast<THPDtype*>(a[8])->scalar_type, x.device());
     const int64_t n_q = a[3] != Py_None ? s.numel() : 1;
     void* st = stream();
-    launch("dq8_quantize", dq8_quantize_ex, ptr(x), xk, ptr(out), kind, v.outer, v.nch, v.inner,
-           (const float*)ptr(s), (const int32_t*)ptr(z), n_q, qmin, qmax, round_mode, st);
+    launch("dq8_quantize", dq8_quantize_ex, in(x), xk, inout(out), kind, v.outer, v.nch, v.inner,
+           (const float*)in(s), (const int32_t*)in(z), n_q, qmin, qmax, round_mode, st);
     return wrap(a[9], out);
   });
 }
@@ -241,8 +243,8 @@ PyObject* py_dequantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const Tensor out = a[5] != Py_None ? tensor(a[5]) : empty(q.sizes(), ScalarType::Float, q.device());
     const int64_t n_q = a[3] != Py_None ? s.numel() : 1;
     void* st = stream();
-    launch("dq8_dequantize", dq8_dequantize_ex, ptr(q), kind, (float*)ptr(out), v.outer, v.nch, v.inner,
-           (const float*)ptr(s), (const int32_t*)ptr(z), n_q, st);
+    launch("dq8_dequantize", dq8_dequantize_ex, in(q), kind, (float*)inout(out), v.outer, v.nch, v.inner,
+           (const float*)in(s), (const int32_t*)in(z), n_q, st);
     return wrap(a[5], out);
   });
 }
@@ -259,8 +261,8 @@ PyObject* py_fake_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const Tensor out = a[7] != Py_None ? tensor(a[7]) : empty(x.sizes(), ScalarType::Float, x.device());
     const int64_t n_q = a[3] != Py_None ? s.numel() : 1;
     void* st = stream();
-    launch("dq8_fake_quant", dq8_fake_quant, (const float*)ptr(x), (float*)ptr(out), v.outer, v.nch,
-           v.inner, (const float*)ptr(s), (const int32_t*)ptr(z), n_q, qmin, qmax, round_mode, st);
+    launch("dq8_fake_quant", dq8_fake_quant, (const float*)in(x), (float*)inout(out), v.outer, v.nch,
+           v.inner, (const float*)in(s), (const int32_t*)in(z), n_q, qmin, qmax, round_mode, st);
     return wrap(a[7], out);
   });
 }
@@ -286,8 +288,8 @@ PyObject* py_minmax(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!ws.defined() || (size_t)ws.nbytes() < need)
       ws = empty({(int64_t)(need > 0 ? need : 1)}, ScalarType::Byte, x.device());
     void* st = stream();
-    launch("dq8_minmax", dq8_minmax, (const float*)ptr(x), v.outer, v.nch, v.inner, (float*)ptr(lo),
-           (float*)ptr(hi), ptr(ws), ws.nbytes(), st);
+    launch("dq8_minmax", dq8_minmax, (const float*)in(x), v.outer, v.nch, v.inner, (float*)inout(lo),
+           (float*)inout(hi), inout(ws), ws.nbytes(), st);
     Py_RETURN_NONE;
   });
 }
@@ -330,10 +332,11 @@ PyObject* py_observe(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const Tensor z = empty(lo.sizes(), ScalarType::Int, x.device());
     Tensor y;
     if (fake) y = empty(x.sizes(), ScalarType::Float, x.device());
-    const float *xp = (const float*)ptr(x), *sp = (const float*)ptr(s);
-    float *lop = (float*)ptr(lo), *hip = (float*)ptr(hi), *yp = (float*)ptr(y);
-    int32_t* zp = (int32_t*)ptr(z);
-    void* wsp = ptr(ws);
+    const float* xp = (const float*)in(x);
+    float *lop = (float*)inout(lo), *hip = (float*)inout(hi);
+    float *sp = (float*)inout(s), *yp = (float*)inout(y);
+    int32_t* zp = (int32_t*)inout(z);
+    void* wsp = inout(ws);
     const c10::hip::HIPStream st = c10::hip::getCurrentHIPStream();
     void* raw = (void*)st.stream();
     dq8::StatusWord<Tensor> status(status_words(), [](Tensor* own) {
@@ -347,7 +350,7 @@ PyObject* py_observe(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const dq8::Unlocked unlocked;
       auto drain = [&] { st.synchronize(); };
       failed = dq8_observe(xp, v.outer, v.nch, v.inner, lop, hip, symmetric, q_min, q_max,
-                           const_cast<float*>(sp), zp, status.hand_out(), wsp, need, raw);
+                           sp, zp, status.hand_out(), wsp, need, raw);
       if (!failed && fake) {
         what = "dq8_fake_quant";
         failed = dq8_fake_quant(xp, yp, v.outer, v.nch, v.inner, sp, zp, v.nch, q_min, q_max,
@@ -388,7 +391,7 @@ PyObject* py_lut8(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const Tensor q = dense(q0);
     const Tensor out = a[2] != Py_None ? tensor(a[2]) : empty(q.sizes(), table.scalar_type(), q.device());
     void* st = stream();
-    launch("dq8_lut8", dq8_lut8, ptr(q), ptr(out), q.numel(), ptr(table), st);
+    launch("dq8_lut8", dq8_lut8, in(q), inout(out), q.numel(), in(table), st);
     return wrap(a[2], out);
   });
 }
@@ -427,9 +430,9 @@ PyObject* py_weight_only(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     const size_t ws_bytes = ws.defined() ? ws.nbytes() : 0;
     void* st = stream();
-    launch("dq8_weight_only_qgemm", dq8_weight_only_qgemm, ptr(x), xk, x.stride(0), ptr(w), w_signed,
-           w.stride(0), tp_b, ptr(s), (const int32_t*)ptr(zp), ptr(bias), ptr(out), out.stride(0), M, N, K,
-           ptr(ws), ws_bytes, st);
+    launch("dq8_weight_only_qgemm", dq8_weight_only_qgemm, in(x), xk, x.stride(0), in(w), w_signed,
+           w.stride(0), tp_b, in(s), (const int32_t*)in(zp), in(bias), inout(out), out.stride(0), M, N, K,
+           inout(ws), ws_bytes, st);
     return wrap(a[6], out);
   });
 }
@@ -461,10 +464,10 @@ PyObject* py_qgemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Tensor ws;
     if (need) ws = empty({(int64_t)need}, ScalarType::Byte, dev);
     void* st = stream();
-    launch("dq8_qgemm", dq8_qgemm_fused, (const int8_t*)ptr(x), leading(x), (const int8_t*)ptr(w),
-           leading(w), ptr(out), M ? out.stride(0) : N, M, N, K, tp_a, tp_b, (int)epilogue, ptr(bias), kind,
-           (const float*)ptr(sx), count(sx), (const float*)ptr(sw), count(sw), (const float*)ptr(so),
-           count(so), zx, zw, zo, ptr(ws), need, post.p, st);
+    launch("dq8_qgemm", dq8_qgemm_fused, (const int8_t*)in(x), leading(x), (const int8_t*)in(w),
+           leading(w), inout(out), M ? out.stride(0) : N, M, N, K, tp_a, tp_b, (int)epilogue, in(bias), kind,
+           (const float*)in(sx), count(sx), (const float*)in(sw), count(sw), (const float*)in(so),
+           count(so), zx, zw, zo, inout(ws), need, post.p, st);
     return wrap(a[12], out);
   });
 }
@@ -487,9 +490,9 @@ PyObject* py_qlinear_f32(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int kind = bias_kind(bias);
     const int zo = (int)integer(a[7]), round_mode = (int)integer(a[8]);
     void* st = stream();
-    launch("dq8_qlinear_f32", dq8_qlinear_f32, (const float*)ptr(x), leading(x), (const int8_t*)ptr(w),
-           leading(w), ptr(out), M ? out.stride(0) : N, M, N, K, (int)epilogue, ptr(bias), kind,
-           (const float*)ptr(sx), (const float*)ptr(sw), count(sw), (const float*)ptr(so), count(so), zo,
+    launch("dq8_qlinear_f32", dq8_qlinear_f32, (const float*)in(x), leading(x), (const int8_t*)in(w),
+           leading(w), inout(out), M ? out.stride(0) : N, M, N, K, (int)epilogue, in(bias), kind,
+           (const float*)in(sx), (const float*)in(sw), count(sw), (const float*)in(so), count(so), zo,
            round_mode, st);
     return wrap(a[9], out);
   });
@@ -539,9 +542,9 @@ PyObject* py_qconv2d(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Tensor ws;
     if (need) ws = empty({(int64_t)need}, ScalarType::Byte, dev);
     void* st = stream();
-    launch("dq8_qconv2d", dq8_qconv2d_fused, (const int8_t*)ptr(x), is, (const int8_t*)ptr(w), ws_,
-           padding.v, md.v, ptr(out), os.v, (int)epilogue, ptr(bias), kind, (const float*)ptr(sx),
-           (const float*)ptr(sw), count(sw), (const float*)ptr(so), zo, ptr(ws), need, post.p, st);
+    launch("dq8_qconv2d", dq8_qconv2d_fused, (const int8_t*)in(x), is, (const int8_t*)in(w), ws_,
+           padding.v, md.v, inout(out), os.v, (int)epilogue, in(bias), kind, (const float*)in(sx),
+           (const float*)in(sw), count(sw), (const float*)in(so), zo, inout(ws), need, post.p, st);
     return wrap(a[11], out);
   });
 }
@@ -559,9 +562,9 @@ PyObject* py_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const Tensor out = empty({x.size(0), x.size(1), h3 / 3}, s.defined() ? ScalarType::Char : ScalarType::Float,
                              x.device());
     void* st = stream();
-    launch("dq8_attention_f32", dq8_attention_f32, (const float*)ptr(x), x.size(0), x.size(1), heads,
-           h3 / 3 / heads, s.defined() ? nullptr : (float*)ptr(out),
-           s.defined() ? (int8_t*)ptr(out) : nullptr, (const float*)ptr(s), st);
+    launch("dq8_attention_f32", dq8_attention_f32, (const float*)in(x), x.size(0), x.size(1), heads,
+           h3 / 3 / heads, s.defined() ? nullptr : (float*)inout(out),
+           s.defined() ? (int8_t*)inout(out) : nullptr, (const float*)in(s), st);
     return THPVariable_Wrap(out);
   });
 }
@@ -584,8 +587,8 @@ PyObject* py_layer_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Tensor q;
     if (s.defined()) q = empty(x.sizes(), ScalarType::Char, x.device());
     void* st = stream();
-    launch("dq8_layernorm_f32", dq8_layernorm_f32, (const float*)ptr(x), rows, cols, (const float*)ptr(g),
-           (const float*)ptr(b), eps, (float*)ptr(y), (int8_t*)ptr(q), (const float*)ptr(s), st);
+    launch("dq8_layernorm_f32", dq8_layernorm_f32, (const float*)in(x), rows, cols, (const float*)in(g),
+           (const float*)in(b), eps, (float*)inout(y), (int8_t*)inout(q), (const float*)in(s), st);
     if (!s.defined()) return THPVariable_Wrap(y);
     PyObject* r = PyTuple_New(2);
     if (!r) throw PyFailure{};

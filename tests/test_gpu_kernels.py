@@ -2384,3 +2384,29 @@ def test_bounds_and_scales_in_every_form_python_has_for_them(K):
     for bad in ("0.05", {}, object()):
         with pytest.raises((TypeError, ValueError, RuntimeError)):
             K.qgemm(q, w, K.EPI_REQUANT_CPU, sx=bad, sw=s.tolist(), so=so)
+
+
+def test_results_into_lazy_copies_leave_the_original_alone(K):
+    """A result tensor or a running state that shares its memory with another one until it is
+    written (copy on write)."""
+    f32 = torch.randn((4, 64), device="cuda")
+    i8 = torch.randint(-128, 128, (4, 64), dtype=torch.int8, device="cuda")
+    one, zero = torch.full((1,), 0.05, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+    table = torch.arange(256, device="cuda").to(torch.uint8).view(torch.int8)
+    md = list(O.NHWC_OHWI_METADATA) + [1] * 5
+    for run, shape, dtype in ((lambda o: K.quantize(f32, one, zero, out=o), (4, 64), torch.int8),
+                              (lambda o: K.dequantize(i8, one, zero, out=o), (4, 64), torch.float32),
+                              (lambda o: K.fake_quant(f32, one, zero, out=o), (4, 64), torch.float32),
+                              (lambda o: K.lut8(i8, table, out=o), (4, 64), torch.int8),
+                              (lambda o: K.qgemm(i8, i8, K.EPI_ACC_S32, out=o), (4, 4), torch.int32),
+                              (lambda o: K.weight_only_qgemm(f32, i8, one.expand(4), out=o), (4, 4), torch.float32),
+                              (lambda o: K.qlinear_f32(f32, i8, K.EPI_DEQUANT_F32, one, one, out=o), (4, 4), torch.float32),
+                              (lambda o: K.qconv2d(i8.reshape(1, 1, 4, 64), i8.reshape(4, 1, 1, 64), [0] * 4, md,
+                                                   [1, 1, 4, 4], K.EPI_ACC_S32, out=o), (1, 1, 4, 4), torch.int32),
+                              (lambda o: K.minmax(f32, o, one.clone()), (1,), torch.float32),
+                              (lambda o: K.observe(f32, o, one.clone(), True, -128, 127), (1,), torch.float32)):
+        original = torch.full(shape, 99, dtype=dtype, device="cuda")
+        copy = torch._lazy_clone(original)
+        run(copy)
+        assert (original == 99).all()
+        assert not torch.equal(copy, original)
