@@ -885,9 +885,9 @@ int qgemm_impl(int variant, const int8_t* A, int64_t lda, const int8_t* W, int64
     variant = pick_any(M, N, K, pipe_ok(256, 256, p, false), es);
   const bool rows_aligned = es == 1 ? e.vec_store16 : e.vec_store;
   if (fused || e.fixedpoint || !rows_aligned) {   // the persistent forms carry none of these
-    DQ8_REQUIRE(auto_pick || (!fused && !e.fixedpoint) ||
-                    (variant != kPersist256 && variant != kPersist256x192 && variant != kPersist128),
-                "dq8_qgemm: the persistent variants take neither fused operators nor the fixed-point stage");
+    DQ8_REQUIRE(auto_pick || (variant != kPersist256 && variant != kPersist256x192 && variant != kPersist128),
+                "dq8_qgemm: the persistent variants take neither fused operators nor the fixed-point stage nor "
+                "result rows off 16 bytes");
     if (variant == kPersist256) variant = kPipe256w8;
     if (variant == kPersist256x192) variant = kPipe256x192;
     if (variant == kPersist128) variant = kPipe128w8;

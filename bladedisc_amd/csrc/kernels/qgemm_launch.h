@@ -262,15 +262,12 @@ int launch_variant(int variant, MainParams& p, hipStream_t st) {
   if constexpr (!CONV) {   // GEMM only: the small-M kernel and the persistent forms
     if (variant == kSkinnyVariant) return launch_skinny<EPI>(p, st);
     if (variant == kPersist128) return launch_persist<128, 128, 2, 4, false, EPI>(p, 2, st);
-    // (the 256-row persistent forms write int8; 4-byte results take the one-tile kernels)
-    constexpr bool kInt8 = EPI == DQ8_EPI_REQUANT_CPU || EPI == DQ8_EPI_REQUANT_GPU;
-    if (variant == kPersist256) {
-      if constexpr (kInt8) return launch_persist<256, 256, 2, 4, false, EPI>(p, 1, st);
-      else return launch_pipe<256, 256, 2, 4, 1, false, EPI>(p, st);
-    }
-    if (variant == kPersist256x192) {
-      if constexpr (kInt8) return launch_persist<256, 192, 4, 2, false, EPI>(p, 1, st);
-      else return launch_pipe<256, 192, 4, 2, 1, false, EPI>(p, st);
+    // (the 256-row persistent forms write int8; 4-byte results are never given to them)
+    if constexpr (EPI == DQ8_EPI_REQUANT_CPU || EPI == DQ8_EPI_REQUANT_GPU) {
+      if (variant == kPersist256) return launch_persist<256, 256, 2, 4, false, EPI>(p, 1, st);
+      if (variant == kPersist256x192) return launch_persist<256, 192, 4, 2, false, EPI>(p, 1, st);
+    } else if (variant == kPersist256 || variant == kPersist256x192) {
+      return fail("the persistent variants of 256 rows write int8 results only");
     }
   }
   return fail("unknown or unsupported qgemm variant for this operation");

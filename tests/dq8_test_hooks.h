@@ -18,7 +18,8 @@ extern "C" {
  *  (dq8_qgemm_num_variants() of them, names from dq8_qgemm_variant_name()).  A problem
  *  an MFMA variant cannot take (unaligned rows; K % 16 != 0 without scratch) runs on the
  *  generic kernel whatever the variant; non-zero zx / zw with a forced MFMA variant is an error
- *  (they need the heuristic or the generic variant). */
+ *  (they need the heuristic or the generic variant), and so is a persistent variant with result
+ *  rows off 16 bytes or, of the 256-row ones, with 4-byte results. */
 int dq8_qgemm_variant(int variant, const int8_t* A, int64_t lda,
                       const int8_t* W, int64_t ldw, void* out, int64_t ldo,
                       int64_t M, int64_t N, int64_t K, int tp_a, int tp_b,

@@ -24,10 +24,18 @@ def host(t):
     return t.cpu().numpy()
 
 
-def gemm_variants(K, k):
-    """All variant ids of the GEMM."""
+def persistent_refuses(K, v, row, out_bytes):
+    """Whether variant v is a persistent kernel that has no form for result rows of `row` elements
+    of this size: they store 16 bytes at a time, the 256-row ones int8 alone."""
+    name = K.variant_names()[v] if v >= 0 else ""
+    return name.startswith("persist_") and (row * out_bytes % 16 != 0 or
+                                            (out_bytes == 4 and name.startswith("persist_256x")))
+
+
+def gemm_variants(K, k, row=16, out_bytes=1):
+    """All variant ids of the GEMM that take result rows of `row` elements of this size."""
     return [i for i, nm in enumerate(K.variant_names())
-            if not nm.startswith(("direct3x3_", "stream"))]
+            if not nm.startswith(("direct3x3_", "stream")) and not persistent_refuses(K, i, row, out_bytes)]
 
 
 def make_scales(rng, n, per_channel=True):
@@ -68,7 +76,7 @@ def test_qgemm_acc_s32_all_variants(K, m, n, k):
     w = rng.integers(-128, 128, (n, k), dtype=np.int8)
     want, _ = O.gemm_s32_fast(a, w)
     da, dw = dev(a), dev(w)
-    for v in gemm_variants(K, k):
+    for v in gemm_variants(K, k, n, 4):
         got = host(K.qgemm(da, dw, K.EPI_ACC_S32, variant=v))
         np.testing.assert_array_equal(got, want, err_msg=K.variant_names()[v])
     np.testing.assert_array_equal(host(K.qgemm(da, dw, K.EPI_ACC_S32)), want)
@@ -92,7 +100,7 @@ def test_qgemm_requant_cpu(K, m, n, k, bias):
         b32 = O.bias_f32_to_s32(bf, sx, sw)
         bias_t = dev(bf)
     want = O.requant_cpu(acc, sx, sw, so, b32=b32)
-    for v in [-1] + gemm_variants(K, k):
+    for v in [-1] + gemm_variants(K, k, n):
         got = host(K.qgemm(dev(a), dev(w), K.EPI_REQUANT_CPU, sx=dev(np.array([sx])), sw=dev(sw),
                            so=dev(np.array([so])), bias=bias_t, variant=v))
         np.testing.assert_array_equal(got, want, err_msg="variant %d" % v)
@@ -101,16 +109,18 @@ def test_qgemm_requant_cpu(K, m, n, k, bias):
 
 
 @pytest.mark.parametrize("m,n,k", [
-    (4133, 4109, 272),     # 17 x 17 tiles of 256 x 256: more tiles than compute units, not a multiple of 8
-    (4096, 4300, 144),     # 16 x 17 = 272 tiles: dealt per XCD; two k tiles, the second ragged
+    (4133, 4112, 272),     # 17 x 17 tiles of 256 x 256: more tiles than compute units, not a multiple of 8
+    (4133, 4109, 272),     # (result rows at any byte: no persistent form)
+    (4096, 4304, 144),     # 16 x 17 = 272 tiles: dealt per XCD; two k tiles, the second ragged
+    (4096, 4300, 144),     # (rows of 4-byte results alone on 16 bytes)
     (5000, 3840, 128),     # 20 x 20 tiles of 256 x 192 / 20 x 15 of 256 x 256; one k tile
     (16384, 1536, 400),    # three and four rounds of the two big tile shapes
 ])
 def test_qgemm_persistent_variants_walk_many_tiles(K, m, n, k):
     """The persistent kernels with several output tiles per workgroup: ragged last tiles in
     M, N and K, tile counts that do and do not divide over the XCDs, all epilogue families
-    (int8 with and without additive terms, int32, f32), and the heuristic's own pick at these
-    sizes -- bit-exact against the oracle."""
+    (int8 with and without additive terms; int32 and f32 from the 128-row form, which alone has
+    them), and the heuristic's own pick at these sizes -- bit-exact against the oracle."""
     rng = np.random.default_rng(m + 3 * n + 7 * k)
     a = rng.integers(-128, 128, (m, k), dtype=np.int8)
     w = rng.integers(-128, 128, (n, k), dtype=np.int8)
@@ -126,14 +136,19 @@ def test_qgemm_persistent_variants_walk_many_tiles(K, m, n, k):
     dsx, dsw, dso = dev(np.array([sx])), dev(sw), dev(np.array([so]))
     names = K.variant_names()
     persistent = [i for i, nm in enumerate(names) if nm.startswith("persist_")]
-    assert len(persistent) >= 2
+    assert len(persistent) == 3
     for v in [-1] + persistent:
         tag = names[v] if v >= 0 else "heuristic"
-        got = host(K.qgemm(da, dw, K.EPI_REQUANT_CPU, sx=dsx, sw=dsw, so=dso, variant=v))
-        np.testing.assert_array_equal(got, want_plain, err_msg=tag)
-        got = host(K.qgemm(da, dw, K.EPI_REQUANT_CPU, sx=dsx, sw=dsw, so=dso, bias=dev(bf), zo=3,
-                           variant=v))
-        np.testing.assert_array_equal(got, want_bias, err_msg=tag)
+        if not persistent_refuses(K, v, n, 1):
+            got = host(K.qgemm(da, dw, K.EPI_REQUANT_CPU, sx=dsx, sw=dsw, so=dso, variant=v))
+            np.testing.assert_array_equal(got, want_plain, err_msg=tag)
+            got = host(K.qgemm(da, dw, K.EPI_REQUANT_CPU, sx=dsx, sw=dsw, so=dso, bias=dev(bf), zo=3,
+                               variant=v))
+            np.testing.assert_array_equal(got, want_bias, err_msg=tag)
+            got = host(K.qgemm(da, dw, K.EPI_REQUANT_GPU, sx=dsx, sw=dsw, so=dso, bias=dev(bf), variant=v))
+            np.testing.assert_array_equal(got, O.requant_gpu(acc, sx, sw, so, bias_f32=bf), err_msg=tag)
+        if persistent_refuses(K, v, n, 4):
+            continue
         np.testing.assert_array_equal(host(K.qgemm(da, dw, K.EPI_ACC_S32, variant=v)), acc, err_msg=tag)
         got = host(K.qgemm(da, dw, K.EPI_DEQUANT_F32, sx=dsx, sw=dsw, bias=dev(bf), variant=v))
         assert np.array_equal(got.view(np.uint32), want_f32.view(np.uint32)), tag
@@ -142,8 +157,28 @@ def test_qgemm_persistent_variants_walk_many_tiles(K, m, n, k):
                            zo=3, variant=v))
         want = O.dequantize(want_bias, np.array([so], np.float32), np.array([3], np.int32))
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), tag
-        got = host(K.qgemm(da, dw, K.EPI_REQUANT_GPU, sx=dsx, sw=dsw, so=dso, bias=dev(bf), variant=v))
-        np.testing.assert_array_equal(got, O.requant_gpu(acc, sx, sw, so, bias_f32=bf), err_msg=tag)
+
+
+def test_forced_persistent_variants_refuse_what_they_have_no_form_for(K):
+    """A forced persistent kernel runs or says so: no other kernel in its place."""
+    one = torch.ones(1, device="cuda")
+    sc = dict(sx=one, sw=one, so=one)
+    a = torch.zeros((300, 64), dtype=torch.int8, device="cuda")
+    refused = 0
+    for v, name in enumerate(K.variant_names()):
+        if not name.startswith("persist_"):
+            continue
+        for n, epi, out_bytes in ((256, K.EPI_ACC_S32, 4), (256, K.EPI_DEQUANT_F32, 4), (256, K.EPI_REQUANT_CPU, 1),
+                                  (264, K.EPI_REQUANT_GPU, 1), (258, K.EPI_REQUANT_CPU_DEQUANT_F32, 4)):
+            w = torch.zeros((n, 64), dtype=torch.int8, device="cuda")
+            kw = {} if epi == K.EPI_ACC_S32 else sc
+            if persistent_refuses(K, v, n, out_bytes):
+                refused += 1
+                with pytest.raises(RuntimeError, match="persistent"):
+                    K.qgemm(a, w, epi, variant=v, **kw)
+            else:
+                assert not K.qgemm(a, w, epi, variant=v, **kw).any()
+    assert refused == 2 * 4 + 2
 
 
 @pytest.mark.parametrize("m,n,k", [(64, 768, 768), (1000, 768, 3072), (257, 130, 64), (5, 7, 48),
@@ -272,7 +307,7 @@ def test_qgemm_requant_gpu(K, per_channel, bias):
         bi = rng.integers(-128, 128, n).astype(np.int8)
         bias_t = dev(bi)
     want = O.requant_gpu(acc, sx, sw, so, bias_f32=bf, bias_i8=bi)
-    for v in [-1] + gemm_variants(K, k):
+    for v in [-1] + gemm_variants(K, k, n):
         got = host(K.qgemm(dev(a), dev(w), K.EPI_REQUANT_GPU, sx=dev(sx), sw=dev(sw), so=dev(so),
                            bias=bias_t, variant=v))
         np.testing.assert_array_equal(got, want, err_msg="variant %d" % v)
@@ -310,9 +345,10 @@ def test_qgemm_requant_then_dequantize_in_one_epilogue(K, m, n, k, form):
                                bias_i8=bi)
     want = O.dequantize(q_want, np.array([so], np.float32), np.array([zo], np.int32))
     sov, zov = t(so), dev(np.array([zo], np.int32))
-    for v in [-1] + gemm_variants(K, k):
+    for v in [-1] + gemm_variants(K, k, n):
+        f32_v = -1 if persistent_refuses(K, v, n, 4) else v
         got = K.qgemm(dev(a), dev(w), fused, sx=t(sx), sw=dev(sw), so=sov, bias=bias_t, zo=zo,
-                      variant=v)
+                      variant=f32_v)
         assert got.dtype == torch.float32
         two = K.dequantize(K.qgemm(dev(a), dev(w), epi, sx=t(sx), sw=dev(sw), so=sov, bias=bias_t,
                                    zo=zo, variant=v), sov, zov)
@@ -334,7 +370,7 @@ def test_qgemm_dequant_f32(K):
     bias = rng.standard_normal(n).astype(np.float32)
     want = O.dequant_acc(acc, sx, sw, bias)
     exact = acc.astype(np.float64) * (np.float64(sx) * sw.astype(np.float64)) + bias
-    for v in [-1] + gemm_variants(K, k):
+    for v in [-1] + gemm_variants(K, k, n, 4):
         got = host(K.qgemm(dev(a), dev(w), K.EPI_DEQUANT_F32, sx=dev(np.array([sx])), sw=dev(sw),
                            bias=dev(bias), variant=v))
         np.testing.assert_array_equal(got, want)
@@ -1437,7 +1473,7 @@ def test_qgemm_strided_rows_all_variants(K, m, n, k, pad):
     so = pick_so(acc, sx, sw)
     want = O.requant_cpu(acc, sx, sw, so)
     da, dw = dev(a_full)[:, :k], dev(w_full)[:, pad:pad + k]
-    for v in [-1] + gemm_variants(K, k):
+    for v in [-1] + gemm_variants(K, k, n + pad):
         out_full = torch.full((m, n + pad), 77, dtype=torch.int8, device="cuda")
         K.qgemm(da, dw, K.EPI_REQUANT_CPU, sx=dev(np.array([sx])), sw=dev(sw),
                 so=dev(np.array([so])), out=out_full[:, :n], variant=v)
@@ -1463,7 +1499,7 @@ def test_qgemm_ragged_channels_in_16_byte_aligned_rows(K, m, n, k, ldo):
     want2 = O.requant_gpu(acc, sx, sw, so, bias_f32=bias)
     da, dw = dev(a), dev(w)
     scales = dict(sx=dev(np.array([sx])), sw=dev(sw), so=dev(np.array([so])))
-    for v in [-1] + gemm_variants(K, k):
+    for v in [-1] + gemm_variants(K, k, ldo):
         for epi, want, b in ((K.EPI_REQUANT_CPU, want1, None), (K.EPI_REQUANT_GPU, want2, dev(bias))):
             out_full = torch.full((m, ldo), 77, dtype=torch.int8, device="cuda")
             K.qgemm(da, dw, epi, bias=b, out=out_full[:, :n], variant=v, **scales)
@@ -1488,6 +1524,8 @@ def test_qgemm_random_shapes_epilogues_variants(K):
         so = pick_so(acc, sx, np.broadcast_to(sw, (n,)))
         v = choices[int(rng.integers(0, len(choices)))]
         epi = int(rng.integers(0, 4))
+        if persistent_refuses(K, v, n, 4 if epi in (0, 3) else 1):
+            v = -1
         tag = "case %d: %dx%dx%d variant %d epilogue %d" % (case, m, n, k, v, epi)
         da, dw = dev(a), dev(w)
         dsx, dsw, dso = dev(np.array([sx])), dev(sw), dev(np.array([so]))
@@ -1540,7 +1578,7 @@ def test_requant_nan_and_inf_scales_saturate_like_the_oracle(K):
         want_gpu = O.requant_gpu(acc, sx, sw, so, bias_f32=bias)
         want_cpu = O.requant_cpu(acc, sx, sw, so)
     assert (want_gpu[:, 3] == -128).all()
-    for v in gemm_variants(K, k):
+    for v in gemm_variants(K, k, n):
         got = host(K.qgemm(dev(a), dev(w), K.EPI_REQUANT_GPU, sx=dev(np.array([sx])), sw=dev(sw),
                            so=dev(np.array([so])), bias=dev(bias), variant=v))
         np.testing.assert_array_equal(got, want_gpu, err_msg="variant %d" % v)
