@@ -2448,3 +2448,94 @@ def test_results_into_lazy_copies_leave_the_original_alone(K):
         run(copy)
         assert (original == 99).all()
         assert not torch.equal(copy, original)
+
+
+def _fused_forms_equal_the_separate_operators(K, a, w, zx, rng):
+    """Everything dq8_qgemm fuses behind a product with an input zero point, into results of their
+    own and into rows that begin at any byte, against the scalar kernel and the operators by
+    themselves."""
+    (m, k), n, gen = a.shape, w.shape[0], 0
+    so = np.float32(0.02 * 0.025 * 74.0 * 74.0 * np.sqrt(k) / 40.0)
+    dso, sr, s2 = (dev(np.array([v], np.float32)) for v in (so, so * 0.7, so * 1.4))
+    zi = lambda v: torch.full((1,), v, dtype=torch.int32, device="cuda")  # noqa: E731
+    sc = dict(sx=dev(np.array([0.02], np.float32)), so=dso, sw=dev(rng.uniform(0.001, 0.05, n).astype(np.float32)), zx=zx)
+    bias = dev((rng.standard_normal(n) * 20 * so).astype(np.float32))
+    b32 = dev(rng.integers(-20000, 20000, n).astype(np.int32))
+    q = K.qgemm(a, w, K.EPI_REQUANT_CPU, bias=bias, zo=2, variant=gen, **sc)
+    y = K.dequantize(q, dso, zi(2))
+    wide8, wide32 = torch.empty((m, n + 3), dtype=torch.int8, device="cuda"), torch.empty((m, n + 1), device="cuda")
+    res8 = dev(rng.integers(-128, 128, (m, n + 5), dtype=np.int8))
+    res32 = dev((rng.standard_normal((m, n + 3)) * 40 * so).astype(np.float32))
+    outs8, outs32 = (None, wide8[:, 1:n + 1]), (None, wide32[:, 1:])
+    table = dev(rng.integers(-128, 128, 256, dtype=np.int8))
+    clamp = dev(np.clip(np.arange(256).astype(np.uint8).view(np.int8), 0, 100).astype(np.int8))
+    for t in (table, clamp):
+        for out in outs8:
+            got = K.qgemm(a, w, K.EPI_REQUANT_CPU, bias=bias, zo=2, out=out, post=K.make_postops(table=t), **sc)
+            assert torch.equal(got, K.lut8(q, t))
+    for r8 in (res8[:, :n].contiguous(), res8[:, 2:n + 2]):
+        t = y + K.dequantize(r8.contiguous(), sr, zi(-4))
+        relu = torch.where(t < 0, torch.zeros_like(t), t)
+        for out in outs8:
+            got = K.qgemm(a, w, K.EPI_REQUANT_CPU, bias=bias, zo=2, out=out, post=K.make_postops(
+                residual=r8, residual_scale=sr, residual_zp=-4, relu=True, out_scale=s2, out_zp=-9), **sc)
+            assert torch.equal(got, K.quantize(relu, s2, zi(-9)))
+        for out in outs32:
+            got = K.qgemm(a, w, K.EPI_REQUANT_CPU_DEQUANT_F32, bias=bias, zo=2, out=out,
+                          post=K.make_postops(residual=r8, residual_scale=sr, residual_zp=-4), **sc)
+            assert torch.equal(got.contiguous().view(torch.int32), t.view(torch.int32))
+    for r32 in (res32[:, :n].contiguous(), res32[:, 1:n + 1]):
+        t = y + r32
+        for out in outs32:
+            got = K.qgemm(a, w, K.EPI_REQUANT_CPU_DEQUANT_F32, bias=bias, zo=2, out=out,
+                          post=K.make_postops(residual=r32), **sc)
+            assert torch.equal(got.contiguous().view(torch.int32), t.view(torch.int32))
+        for out in outs8:
+            got = K.qgemm(a, w, K.EPI_REQUANT_CPU, bias=bias, zo=2, out=out,
+                          post=K.make_postops(residual=r32, out_scale=s2), **sc)
+            assert torch.equal(got, K.quantize(t, s2, zi(0)))
+    fix = K.qgemm(a, w, K.EPI_REQUANT_FIXEDPOINT, bias=b32, zo=-3, variant=gen, **sc)
+    for out in outs8:
+        assert torch.equal(K.qgemm(a, w, K.EPI_REQUANT_FIXEDPOINT, bias=b32, zo=-3, out=out, **sc), fix)
+        got = K.qgemm(a, w, K.EPI_REQUANT_FIXEDPOINT, bias=b32, zo=-3, out=out, post=K.make_postops(table=table), **sc)
+        assert torch.equal(got, K.lut8(fix, table))
+    assert q.unique().numel() > 20
+
+
+# shapes of every tile that sums the zero point up in its k loop, and of the small-M kernel
+ZP_TILES = [((300, 261, 96), "pipe_64x64x128"), ((1100, 770, 2064), "pipe_64x64x128_k2"),
+            ((256, 512, 8192), "pipe_64x64x128_k4"), ((2048, 2048, 4096), "pipe_128x128x128"),
+            ((4097, 768, 272), "pipe_128x128x128_w8"), ((4096, 4096, 256), "pipe_256x256x128_w8"),
+            ((4000, 3070, 256), "pipe_256x192x128_w8"), ((33, 257, 80), "skinny_16")]
+
+
+@pytest.mark.parametrize("shape,kernel", ZP_TILES, ids=[t[1] for t in ZP_TILES])
+def test_fused_operators_behind_a_zero_point_in_the_k_loop(K, shape, kernel):
+    m, n, k = shape
+    assert K._lib.lib().dq8_qgemm_kernel_name(m, n, k, 1).decode() == kernel
+    rng = np.random.default_rng(m + n + k)
+    a, w = dev(rng.integers(-128, 128, (m, k), dtype=np.int8)), dev(rng.integers(-128, 128, (n, k), dtype=np.int8))
+    for zx in (-11, 100):
+        _fused_forms_equal_the_separate_operators(K, a, w, zx, rng)
+
+
+# the same for operand rows of any length and alignment; K rounded up to 16 names the tile
+RAGGED_TILES = [((300, 261, 90), "pipe_64x64x128"), ((260, 130, 1001), "pipe_64x64x128"),
+                ((1100, 770, 2058), "pipe_64x64x128_k2"), ((320, 513, 8204), "pipe_64x64x128_k4"),
+                ((33, 257, 79), "skinny_16")]
+
+
+@pytest.mark.parametrize("shape,kernel", RAGGED_TILES, ids=["%s-%d" % (t[1], t[0][2]) for t in RAGGED_TILES])
+def test_fused_operators_behind_rows_of_any_length(K, shape, kernel):
+    m, n, k = shape
+    assert K._lib.lib().dq8_qgemm_kernel_name(m, n, (k + 15) // 16 * 16, 1).decode() == kernel
+    rng = np.random.default_rng(m + n + k)
+    wide_a = dev(rng.integers(-128, 128, (m, (k + 11) // 4 * 4), dtype=np.int8))
+    wide_w = dev(rng.integers(-128, 128, (n, (k + 15) // 4 * 4), dtype=np.int8))
+    # (rows on four bytes at any k, at odd bytes up to 2048 of k: what the tiles take as they are)
+    forms = [(wide_a[:, 4:4 + k], wide_w[:, 8:8 + k])] + \
+        ([(wide_a[:, :k].contiguous(), wide_w[:, :k].contiguous()), (wide_a[:, 3:3 + k], wide_w[:, 1:1 + k])]
+         if k <= 2048 else [])
+    for a, w in forms:
+        for zx in (0, -11):
+            _fused_forms_equal_the_separate_operators(K, a, w, zx, rng)
