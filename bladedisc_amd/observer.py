@@ -13,7 +13,9 @@ modes (``observe`` / ``fake_quant``), state (``min_val``, ``max_val``, ``scale``
   multiplies by ``1 / scale`` and can differ from it in the last bit at ties).
 
 The qparams arithmetic itself (observer.py:134-163) is a handful of float32 operations on
-the min / max vectors; it is done with torch on the device that holds the state.
+the min / max vectors.  An 8-bit observation step does it, the statistic and the fake quantization
+in one call (``dq8_observe``, ``dq8_fake_quant``) with a single wait for the device;
+``_calculate_qparams`` is the same in torch, for the int32 types and for a state that is read back.
 """
 from typing import NamedTuple, Tuple
 
