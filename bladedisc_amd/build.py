@@ -126,7 +126,7 @@ def build_torch_calls(force=False):
     Compiled by hipcc, as everything else here; the HIP runtime is torch's."""
     headers = torch_calls_headers()
     import torch
-    from ._lib import torch_calls_path
+    from bladedisc_amd._lib import torch_calls_path
     target = torch_calls_path()
     src = os.path.dirname(TORCH_CALLS_SRC)
     inputs = [os.path.join(src, f) for f in os.listdir(src)] + [os.path.join(ROOT, "include", "disc_q8.h")]
@@ -209,6 +209,8 @@ def build(force=False, verbose=False, jobs=8):
 
 
 if __name__ == "__main__":
+    if ROOT not in sys.path:
+        sys.path.insert(0, ROOT)
     path = build(force="--force" in sys.argv, verbose=True)
     build_test_code_objects()
     print("built", path)

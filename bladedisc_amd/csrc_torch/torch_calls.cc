@@ -112,9 +112,9 @@ Tensor scale(PyObject* o, const at::Device& dev) {
     if (v == -1.0 && PyErr_Occurred()) throw PyFailure{};
     return at::full({1}, v, at::TensorOptions().dtype(ScalarType::Float).device(dev));
   }
-  // whatever else torch.tensor takes: lists, numpy arrays
+  // whatever else torch.tensor takes: lists, tuples, numpy arrays
   PyObject* mod = PyImport_ImportModule("torch");
-  PyObject* made = mod ? PyObject_CallMethod(mod, "tensor", "O", o) : nullptr;
+  PyObject* made = mod ? PyObject_CallMethod(mod, "tensor", "(O)", o) : nullptr;
   Py_XDECREF(mod);
   if (!made) throw PyFailure{};
   const Tensor t = THPVariable_Unpack(made);

@@ -2415,6 +2415,7 @@ def test_bounds_and_scales_in_every_form_python_has_for_them(K):
     want = K.qgemm(q, w, K.EPI_REQUANT_CPU, sx=dev(sx.reshape(1)), sw=dev(s), so=dev(so.reshape(1)))
     assert want.abs().max() > 0
     for a, b, c in ((float(sx), s.tolist(), float(so)), (sx, s, so), ([float(sx)], s.astype(np.float64), so.reshape(1, 1)),
+                    ((float(sx),), tuple(s.tolist()), so),
                     (dev(sx.reshape(1)), dev(s).double().reshape(5, 1), dev(np.stack([so, so]))[:1])):
         assert torch.equal(K.qgemm(q, w, K.EPI_REQUANT_CPU, sx=a, sw=b, so=c), want)
     want = K.qlinear_f32(x, w, K.EPI_REQUANT_CPU, sx=dev(sx.reshape(1)), sw=dev(s), so=dev(so.reshape(1)))
