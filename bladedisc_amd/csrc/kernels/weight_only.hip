@@ -23,12 +23,12 @@
 // layout: the order of the k values inside a fragment is free as long as both operands agree,
 // so lane (row, g) takes the 16 consecutive k values k0 + 16 g .. of its row -- 16 weight bytes
 // (one dwordx4), 16 activations -- and feeds two MFMAs with them.
-//  * wo_lds_kernel: tiles shared through LDS, everything above 32 rows (16 for f32 against deep
-//    weights): 64 x 64 or 128 x 128 tiles while the problem is a few rounds of them -- with several
-//    workgroups per tile, each over a part of k, and wo_splitk_reduce_kernel behind them, where that
-//    is estimated cheaper --, 256 x 128 and 256 x 256 tiles beyond (1.06-1.16 PFLOP/s for f16
-//    activations at 4096^2 .. 8192^2 weights, where the ROCm library's plain f16 GEMM reaches
+//  * wo_dma_kernel: tiles loaded straight into LDS, everything above 32 rows (16 for f32 against deep or
+//    wide weights): 32 x 64 to 128 x 256 tiles, with several workgroups per tile, each over a part of
+//    k, and wo_splitk_reduce_kernel behind them, where that is estimated cheaper (1.1-1.2 PFLOP/s for
+//    f16 activations at 4096^2 .. 8192^2 weights, where the ROCm library's plain f16 GEMM reaches
 //    1.16-1.49);
+//  * wo_ragged_kernel: the same for f16 rows that are not multiples of 16 bytes, through registers;
 //  * wo_tile_kernel: 2 x 2 waves, wave tile (32 FM) x (32 FN), operands straight into registers:
 //    operands too large for the LDS kernel's 31-bit offsets;
 //  * wo_rows_kernel: 2 .. 32 rows, 16 .. 64 output channels per workgroup, both operands loaded in
@@ -36,15 +36,18 @@
 //  * wo_gemv_kernel: one or two rows, a wave per output channel streaming its weight row on the
 //    vector ALUs;
 //  * wo_skinny_kernel: M <= 128 rows against 32 output channels per workgroup, the k range dealt
-//    over the waves and the partial sums added through LDS: operands too large for the two LDS
+//    over the waves and the partial sums added through LDS: operands too large for the LDS
 //    kernels' 31-bit offsets;
-//  * wo_exact_f32_kernel: f32 activations on rows off 16 bytes (f16 ones: the LDS kernels' RAGGED
-//    forms);
+//  * wo_exact_f32_kernel: f32 activations on rows off 16 bytes (f16 ones: wo_ragged_kernel, and
+//    wo_rows_kernel's RAGGED form up to 32 rows);
 //  * wo_generic_kernel: one output per thread, fewer than 16 of k or weights left as [K, N].
 #include <algorithm>
+#include <type_traits>
+#include <utility>
 
 #include "dq8_common.h"
 #include "disc_q8.h"
+#include "lds_direct.h"
 
 #pragma clang fp contract(off)
 
@@ -71,7 +74,7 @@ struct WoParams {
   int64_t ldx, ldo, w_sn, w_sk;
   int M, N, K;
   unsigned flip;        // 0x80808080 for signed weights (b ^ 0x80 = b + 128 as unsigned)
-  // split k (wo_lds_kernel): workgroup (tile, y) multiplies k in [y k_split, (y + 1) k_split)
+  // split k (wo_dma_kernel, wo_ragged_kernel): workgroup (tile, y) multiplies k in [y k_split, (y + 1) k_split)
   // and, when `partial` is set, leaves its f32 sums in partial[y][M][N] for the reduction kernel
   float* partial;
   int k_split;          // a multiple of 64; K when the k range is not split
@@ -92,6 +95,18 @@ __device__ __forceinline__ u4 zero_first(u4 q, int z) {
   return q;
 }
 
+// body(Int<0>()), ..., body(Int<N - 1>())
+template <int V>
+using Int = std::integral_constant<int, V>;
+template <typename Body, int... I>
+__device__ __forceinline__ void static_for_seq(Body&& body, std::integer_sequence<int, I...>) {
+  (body(Int<I>()), ...);
+}
+template <int N, typename Body>
+__device__ __forceinline__ void static_for_n(Body&& body) {
+  static_for_seq(body, std::make_integer_sequence<int, N>());
+}
+
 template <typename T>
 __device__ __forceinline__ float to_f32(T v) {
   return (float)v;
@@ -108,6 +123,32 @@ __device__ __forceinline__ void widen16(u4 q, unsigned flip, h2 c, h8& s0, h8& s
   const h2 b2 = pair(q.w, 0x05010400u), b3 = pair(q.w, 0x07030602u);
   s0 = (h8){a0.x, a0.y, a1.x, a1.y, a2.x, a2.y, a3.x, a3.y};
   s1 = (h8){b0.x, b0.y, b1.x, b1.y, b2.x, b2.y, b3.x, b3.y};
+}
+
+// eight of them: one k-step
+__device__ __forceinline__ h8 widen8(unsigned d0, unsigned d1, unsigned flip, h2 c) {
+  auto pair = [&](unsigned d, unsigned sel) {
+    return __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, d ^ flip, sel)) - c;
+  };
+  const h2 a0 = pair(d0, 0x05010400u), a1 = pair(d0, 0x07030602u);
+  const h2 a2 = pair(d1, 0x05010400u), a3 = pair(d1, 0x07030602u);
+  return (h8){a0.x, a0.y, a1.x, a1.y, a2.x, a2.y, a3.x, a3.y};
+}
+
+// x = hi + lo of two activations, hi = half(x), lo = half(x - hi).  x - hi is exact, as a difference
+// and as the fused multiply-add that reads the half where it is: four instructions for two values
+// in place of eight.
+__device__ __forceinline__ void split2(float x, float y, h2& hi, h2& lo) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  hi = __builtin_convertvector((f2){x, y}, h2);
+#if defined(__HIP_DEVICE_COMPILE__)
+  f2 d;
+  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(d.x) : "v"(hi), "v"(x));
+  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(d.y) : "v"(hi), "v"(y));
+#else
+  const f2 d = {x - (float)hi.x, y - (float)hi.y};
+#endif
+  lo = __builtin_convertvector(d, h2);
 }
 
 // The 16 activations of a lane for one 32-deep k chunk: two k-steps, and for f32 activations a
@@ -267,47 +308,31 @@ __global__ void __launch_bounds__(256) wo_tile_kernel(const WoParams p) {
       store_frag<XT>(p, acc[i][j], m0 + i * 32, n0 + j * 32 + r, lane);
 }
 
-// ---------------------------------------------------------------- tiled kernel through LDS (f16)
-// (64 WM) x 128 tile, WM x 2 waves (WM = 1, 2 or 4), k tiles of 64 in two LDS stages.  The
-// register kernel above makes every lane fetch its own row, 64 cache lines per load
-// instruction, and the compute unit's address path caps it at about 15 bytes per clock
-// (0.4 PFLOP/s whatever the shape); here eight lanes cover one 128-byte row segment of the
-// activations and four one 64-byte segment of the weights, the tile is shared through LDS
-// (16-byte chunks XOR-swizzled by the row so that the fragment reads spread over the banks),
-// and the fragments are read back as ds_read_b128.  The weights are widened to halves once,
-// on their way into LDS (128-byte rows like the activations'), not by every wave that reads
-// them.
+// ---------------------------------------------------------------- f16 rows of any length: tiles through registers and LDS
+// (32 WM) x (64 FN) tile, WM x 2 waves of 32 x (32 FN), k tiles of 64 in two LDS stages.  Eight lanes
+// cover one 128-byte row segment of the activations and four one 64-byte segment of the weights, by
+// loads of any alignment; the tile is shared through LDS (16-byte chunks XOR-swizzled by the row so
+// that the fragment reads spread over the banks) and the fragments are read back as ds_read_b128.
+// The weights are widened to halves once, on their way into LDS (128-byte rows like the
+// activations'), not by every wave that reads them.  Only the k tile with the end of the rows is
+// handled differently (M = 512, 2047 -> 3001, one output per thread before: 11.9 ms).
 //
 // Four register sets hold the k tiles t + 1 .. t + 4 on their way from memory while tile t is
-// multiplied.  The loads are buffer loads without a branch around them (a chunk past the k
-// range gets an offset past the descriptor and reads zeros) and the main loop is four k tiles
-// of straight-line code, so that the wait in front of a tile's hand-over to LDS counts the
-// loads issued after it instead of draining them all: with conditional loads in a loop of
-// guarded steps every k tile waited out a whole trip to memory (0.8 us per k tile on a
-// quiet chip, 1.5-2 us on a busy one).
-//
-// f32 activations (XT = float) are split on their way into LDS, x = hi + lo with hi = half(x)
-// and lo = half(x - hi), into two half tiles of the same layout; every weight fragment is
-// multiplied with both.
-//
-// RAGGED (f16): plain loads of any alignment in place of the buffer loads; only the k tile with the
-// end of the rows is handled differently (M = 512, 2047 -> 3001, one output per thread before:
-// 11.9 ms).
-template <typename XT, int WM, int FM, int FN, int SETS, bool RAGGED = false>
-__global__ void __launch_bounds__(WM * 128, sizeof(XT) == 4 ? 1 : 2)
-    wo_lds_kernel(const WoParams p) {
-  constexpr bool F32 = sizeof(XT) == 4;
-  static_assert(!RAGGED || !F32, "f32 activations: wo_exact_f32_kernel");
-  constexpr int BM = WM * FM * 32, BN = 2 * FN * 32, BK = 64;
+// multiplied.  The loads have no branch around them and the main loop is four k tiles of
+// straight-line code, so that the wait in front of a tile's hand-over to LDS counts the loads
+// issued after it instead of draining them all: with conditional loads in a loop of guarded steps
+// every k tile waited out a whole trip to memory (0.8 us per k tile on a quiet chip, 1.5-2 us on a
+// busy one).
+template <int WM, int FN>
+__global__ void __launch_bounds__(WM * 128, 2) wo_ragged_kernel(const WoParams p) {
+  constexpr int BM = WM * 32, BN = 2 * FN * 32, BK = 64, SETS = 4;
   constexpr int NT = WM * 128;                           // WM x 2 waves
-  constexpr int XL = F32 ? 16 : 8;                       // lanes (16 bytes each) per activation row
-  constexpr int XP = (BM * XL) / NT;                     // activation chunks per thread
+  constexpr int XP = (BM * 8) / NT;                      // activation chunks per thread
   constexpr int WP = (BN * 4) / NT;                      // weight chunks per thread
-  constexpr int XS = BM * 128 * (F32 ? 2 : 1);           // activation bytes of a stage
-  constexpr int kPast = (int)0x80000000;                 // an offset no descriptor covers
+  constexpr int XS = BM * 128;                           // activation bytes of a stage
   static_assert(SETS % 2 == 0 && SETS * (XP + WP) <= 63, "two LDS stages; vmcnt has 6 bits");
-  // two stages of (activation tile [hi, then lo], widened weight tile), 128 bytes per row
-  extern __shared__ __attribute__((aligned(16))) uint8_t wo_lds[];
+  // two stages of (activation tile, widened weight tile), 128 bytes per row
+  extern __shared__ __attribute__((aligned(1024))) uint8_t wo_lds[];
   uint8_t* const xs[2] = {wo_lds, wo_lds + XS};
   uint8_t* const ws[2] = {wo_lds + 2 * XS, wo_lds + 2 * XS + BN * 128};
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -316,7 +341,7 @@ __global__ void __launch_bounds__(WM * 128, sizeof(XT) == 4 ? 1 : 2)
   // Workgroups go to the 8 XCDs round-robin, and each XCD has its own L2.  Where the tile grid
   // divides, XCD x takes one compact patch of it (the grid cut 4 x 2: an activation row is
   // twice the bytes of a weight row), so that its L2 fetches the patch's operand rows instead
-  // of every activation row (measured at 4096^3: 295 MB fetched per launch without this).
+  // of every activation row.
   int tile = blockIdx.x;
   {
     const int tiles_m = gridDim.x / tiles_n;
@@ -331,27 +356,18 @@ __global__ void __launch_bounds__(WM * 128, sizeof(XT) == 4 ? 1 : 2)
   const int r = lane & 31, g = lane >> 5;
   const int kbeg = blockIdx.y * p.k_split;               // this workgroup's k range
   const int klen = min(p.K, kbeg + p.k_split) - kbeg;
-  // descriptors over the tile's rows from (first row, kbeg); the host has checked that the
-  // offsets below fit 31 bits
   const int mrows = min(BM, p.M - m0), nrows = min(BN, p.N - n0);
-  const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<XT*>(static_cast<const XT*>(p.x) + (int64_t)m0 * p.ldx + kbeg), 0,
-      (int)(((int64_t)(mrows - 1) * p.ldx + klen) * sizeof(XT)), kBufferWord3);
-  const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t*>(p.w + (int64_t)n0 * p.w_sn + kbeg), 0,
-      (int)((int64_t)(nrows - 1) * p.w_sn + klen), kBufferWord3);
 
-  // global -> LDS assignment (rows past the tile's last re-read that one)
-  const int xc = tid & (XL - 1), wc = tid & 3;           // 16-byte chunk of the row's k tile
+  // global -> LDS assignment (rows past the tile's last re-read that one; the host has checked that
+  // the offsets fit 31 bits)
+  const int xc = tid & 7, wc = tid & 3;                  // 16-byte chunk of the row's k tile
   int xo[XP], xl[XP];
 #pragma unroll
   for (int i = 0; i < XP; ++i) {
-    const int row = tid / XL + (NT / XL) * i;
+    const int row = tid / 8 + (NT / 8) * i;
     const int sx = (row ^ (row >> 3)) & 7;
-    xo[i] = (int)((int64_t)min(row, mrows - 1) * p.ldx * sizeof(XT)) + (RAGGED ? 0 : 16 * xc);
-    // (four floats become four halves: half of the 16-byte chunk xc / 2)
-    xl[i] = F32 ? row * 128 + (((xc >> 1) ^ sx) << 4) + 8 * (xc & 1)
-                : row * 128 + ((xc ^ sx) << 4);
+    xo[i] = (int)((int64_t)min(row, mrows - 1) * p.ldx * 2);
+    xl[i] = row * 128 + ((xc ^ sx) << 4);
   }
   int wo[WP], wl[WP], wl1[WP];
   h2 cpark[WP];
@@ -359,56 +375,31 @@ __global__ void __launch_bounds__(WM * 128, sizeof(XT) == 4 ? 1 : 2)
   for (int i = 0; i < WP; ++i) {
     const int row = (tid >> 2) + (NT / 4) * i;
     const int sw = (row ^ (row >> 3)) & 7;
-    wo[i] = (int)((int64_t)min(row, nrows - 1) * p.w_sn) + (RAGGED ? 0 : 16 * wc);
+    wo[i] = (int)((int64_t)min(row, nrows - 1) * p.w_sn);
     wl[i] = row * 128 + (((2 * wc) ^ sw) << 4);
     wl1[i] = row * 128 + (((2 * wc + 1) ^ sw) << 4);
     cpark[i] = centre(p, n0 + min(row, nrows - 1));
   }
   u4 xr[SETS][XP], wr[SETS][WP];
-  const uint8_t* xbase = reinterpret_cast<const uint8_t*>(static_cast<const XT*>(p.x) + (int64_t)m0 * p.ldx);
+  const uint8_t* xbase = reinterpret_cast<const uint8_t*>(static_cast<const _Float16*>(p.x) + (int64_t)m0 * p.ldx);
   const uint8_t* wbase = p.w + (int64_t)n0 * p.w_sn;
   auto fetch = [&](u4* xq, u4* wq, int k0) {
-    if constexpr (RAGGED) {
-      const unsigned kx = min(kbeg + k0 + 16 * (xc >> 1), p.K - 16) + 8 * (xc & 1);
-      const unsigned kw = min(kbeg + k0 + 16 * wc, p.K - 16);
+    const unsigned kx = min(kbeg + k0 + 16 * (xc >> 1), p.K - 16) + 8 * (xc & 1);
+    const unsigned kw = min(kbeg + k0 + 16 * wc, p.K - 16);
 #pragma unroll
-      for (int i = 0; i < XP; ++i) xq[i] = load_any(xbase, (unsigned)xo[i] + 2 * kx);
+    for (int i = 0; i < XP; ++i) xq[i] = load_any(xbase, (unsigned)xo[i] + 2 * kx);
 #pragma unroll
-      for (int i = 0; i < WP; ++i) wq[i] = load_any(wbase, (unsigned)wo[i] + kw);
-      return;
-    }
-    const bool xv = k0 + (F32 ? 4 : 8) * xc < klen, wv = k0 + 16 * wc < klen;   // K % 16 == 0
-#pragma unroll
-    for (int i = 0; i < XP; ++i)
-      xq[i] = __builtin_amdgcn_raw_buffer_load_b128(
-          xrs, xv ? xo[i] + (int)sizeof(XT) * k0 : kPast, 0, 0);
-#pragma unroll
-    for (int i = 0; i < WP; ++i)
-      wq[i] = __builtin_amdgcn_raw_buffer_load_b128(wrs, wv ? wo[i] + k0 : kPast, 0, 0);
+    for (int i = 0; i < WP; ++i) wq[i] = load_any(wbase, (unsigned)wo[i] + kw);
   };
   auto park = [&](u4* xq, const u4* wq, int stage, int k0) {
-    if (RAGGED && k0 + BK > klen) {                        // (uniform) the end of the rows
+    if (k0 + BK > klen) {                                  // (uniform) the end of the rows
       const int c16 = kbeg + k0 + 16 * (xc >> 1);
       const int z = c16 - min(c16, p.K - 16) - 8 * (xc & 1);
 #pragma unroll
       for (int i = 0; i < XP; ++i) xq[i] = zero_first(xq[i], z);
     }
 #pragma unroll
-    for (int i = 0; i < XP; ++i) {
-      if constexpr (F32) {
-        const f4 v = __builtin_bit_cast(f4, xq[i]);
-        h4 hi, lo;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          hi[e] = (_Float16)v[e];
-          lo[e] = (_Float16)(v[e] - (float)hi[e]);
-        }
-        *reinterpret_cast<h4*>(&xs[stage][xl[i]]) = hi;
-        *reinterpret_cast<h4*>(&xs[stage][BM * 128 + xl[i]]) = lo;
-      } else {
-        *reinterpret_cast<u4*>(&xs[stage][xl[i]]) = xq[i];
-      }
-    }
+    for (int i = 0; i < XP; ++i) *reinterpret_cast<u4*>(&xs[stage][xl[i]]) = xq[i];
 #pragma unroll
     for (int i = 0; i < WP; ++i) {
       h8 lo, hi;
@@ -419,69 +410,23 @@ __global__ void __launch_bounds__(WM * 128, sizeof(XT) == 4 ? 1 : 2)
   };
 
   // fragment rows of this wave
-  int xrow[FM], wrow[FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i) xrow[i] = (wm * FM + i) * 32 + r;
+  const int xrow = wm * 32 + r;
+  int wrow[FN];
 #pragma unroll
   for (int j = 0; j < FN; ++j) wrow[j] = (wn * FN + j) * 32 + r;
-  f16v acc[FM][FN];
+  f16v acc[FN];
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
+  for (int j = 0; j < FN; ++j)
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-
-  // (Reading the fragments of one 16-deep k step under the MFMAs of the step before, one LDS
-  // read scheduled between every two MFMAs, changed nothing measurable: 135.2 against 137.5 us
-  // at 4096^3 on 256 x 256 tiles.)
+    for (int v = 0; v < 16; ++v) acc[j][v] = 0.0f;
   auto multiply = [&](int st) {
-    if constexpr (FM * FN >= 8) {
-      // eight fragments per wave: one 16-deep k step at a time (this lane's 8 halves are chunk
-      // 4 (q / 2) + 2 g + q % 2), the registers do not hold more fragments than that
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        h8 a[FM], al[FM], w[FN];
-        const int c = 4 * (q >> 1) + 2 * g + (q & 1);
-#pragma unroll
-        for (int i = 0; i < FM; ++i) {
-          const int row = xrow[i], sx = (row ^ (row >> 3)) & 7;
-          a[i] = *reinterpret_cast<const h8*>(&xs[st][row * 128 + ((c ^ sx) << 4)]);
-          if constexpr (F32)
-            al[i] = *reinterpret_cast<const h8*>(&xs[st][BM * 128 + row * 128 + ((c ^ sx) << 4)]);
-        }
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          const int row = wrow[j], sw = (row ^ (row >> 3)) & 7;
-          w[j] = *reinterpret_cast<const h8*>(&ws[st][row * 128 + ((c ^ sw) << 4)]);
-        }
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < FN; ++j) {
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], w[j], acc[i][j], 0, 0, 0);
-            if constexpr (F32)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], w[j], acc[i][j], 0, 0, 0);
-          }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      return;
-    }
+    const int sx = (xrow ^ (xrow >> 3)) & 7;
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      h8 a0[FM], a1[FM], l0[FM], l1[FM], w0[FN], w1[FN];
       const int c0 = 4 * s + 2 * g;
-#pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        const int row = xrow[i], sx = (row ^ (row >> 3)) & 7;
-        a0[i] = *reinterpret_cast<const h8*>(&xs[st][row * 128 + ((c0 ^ sx) << 4)]);
-        a1[i] = *reinterpret_cast<const h8*>(&xs[st][row * 128 + (((c0 + 1) ^ sx) << 4)]);
-        if constexpr (F32) {
-          l0[i] = *reinterpret_cast<const h8*>(&xs[st][BM * 128 + row * 128 + ((c0 ^ sx) << 4)]);
-          l1[i] =
-              *reinterpret_cast<const h8*>(&xs[st][BM * 128 + row * 128 + (((c0 + 1) ^ sx) << 4)]);
-        }
-      }
+      const h8 a0 = *reinterpret_cast<const h8*>(&xs[st][xrow * 128 + ((c0 ^ sx) << 4)]);
+      const h8 a1 = *reinterpret_cast<const h8*>(&xs[st][xrow * 128 + (((c0 + 1) ^ sx) << 4)]);
+      h8 w0[FN], w1[FN];
 #pragma unroll
       for (int j = 0; j < FN; ++j) {
         const int row = wrow[j], sw = (row ^ (row >> 3)) & 7;
@@ -489,32 +434,21 @@ __global__ void __launch_bounds__(WM * 128, sizeof(XT) == 4 ? 1 : 2)
         w1[j] = *reinterpret_cast<const h8*>(&ws[st][row * 128 + (((c0 + 1) ^ sw) << 4)]);
       }
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0[i], w0[j], acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1[i], w1[j], acc[i][j], 0, 0, 0);
-          if constexpr (F32) {
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(l0[i], w0[j], acc[i][j], 0, 0, 0);
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(l1[i], w1[j], acc[i][j], 0, 0, 0);
-          }
-        }
+      for (int j = 0; j < FN; ++j) {
+        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, w0[j], acc[j], 0, 0, 0);
+        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, w1[j], acc[j], 0, 0, 0);
+      }
     }
   };
   // k tile t: set u = t % SETS has been handed to LDS stage t % 2 and takes tile t + SETS;
-  // tile t + 1 (zeros past the last) is handed over behind the multiplication
+  // tile t + 1 is handed over behind the multiplication
   // (the scheduling barriers keep a later step's arithmetic on loaded registers -- the first
   // instructions of widening -- from being moved up to where it would wait for their loads.  Between
   // a multiplication and the hand-over behind it there is none: the tile handed over left memory
-  // SETS - 1 tiles ago, and its widening and writes fill the gaps between the MFMAs: M = 1024,
-  // 4096 -> 4096 46.3 -> 44.3 us, M = 2048 75.0 -> 71.4, 8192 -> 2048 85.0 -> 81.0.  With the hand-over
-  // in front of the multiplication the fragment reads queue behind its writes: 49.6, 8192 -> 2048 91.1.
-  // It stays for 256 x 256 tiles, which have no registers for both at once, and for f32 on 64 x 64
-  // tiles, where nothing was gained: M = 64, 4096 -> 4096 15.9 against 16.3 us without.)
+  // SETS - 1 tiles ago, and its widening and writes fill the gaps between the MFMAs.)
   auto step = [&](int u, int t) {
     fetch(xr[u], wr[u], (t + SETS) * BK);
     multiply(u % 2);
-    if constexpr (FM * FN >= 8 || (F32 && FM * FN == 1)) __builtin_amdgcn_sched_barrier(0);
     park(xr[(u + 1) % SETS], wr[(u + 1) % SETS], (u + 1) % 2, (t + 1) * BK);
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
@@ -535,13 +469,419 @@ __global__ void __launch_bounds__(WM * 128, sizeof(XT) == 4 ? 1 : 2)
   for (int u = 0; u < SETS - 1; ++u)
     if (t + u < KT) step(u, t + u);                        // (uniform over the workgroup)
 #pragma unroll
+  for (int j = 0; j < FN; ++j)
+    if (p.partial)
+      store_partial(p, acc[j], blockIdx.y, m0 + xrow - r, n0 + wrow[j], lane);
+    else
+      store_frag<_Float16>(p, acc[j], m0 + xrow - r, n0 + wrow[j], lane);
+}
+
+// ---------------------------------------------------------------- tiles loaded straight into LDS
+// (32 FM) x (64 NCG) tile, NCG x KG waves, k tiles of BK in NST LDS stages.
+//
+// Staged as in the kernel above, every byte passes through registers and a ds_write on its way into
+// LDS, the widened weights are twice their bytes there and are read once per row of waves.  Here
+//  * both operands are loaded into LDS as they are in memory (buffer_load ... lds), NST - 1 tiles
+//    ahead: nothing waits in registers;
+//  * a wave multiplies all rows of the tile with 64 output channels, and its KG'th of every k
+//    tile: each weight byte is read from LDS by one wave only, as a byte, and widened once;
+//  * what a wave issues next to its MFMAs decides (a vector instruction of either of a SIMD's two
+//    waves runs next to an MFMA only while that is past its operand reads: about 3.5 of them per
+//    MFMA are free, the others add to it): widening is 16 instructions per 64 channels x 16 of k,
+//    shared by the 2 FM MFMAs that use them -- hence wave tiles of 128 rows where there are that
+//    many --, addresses advance in scalar registers, and reads, loads and widening are dealt out
+//    over the MFMAs.  Sent out together behind the barrier, the loads of all waves queue at the
+//    compute unit's address path (25 clocks apiece), the reads at the LDS, and every wave's MFMAs
+//    behind them;
+//  * one barrier per k tile, in the middle of the wave's last 32-deep unit of it: by then all
+//    fragments of the tile are in registers, its stage takes the tile NST further on, and the next
+//    tile's first fragments are read under the unit's second half.
+// The sums of the k groups meet in LDS at the end, which also puts the results into whole rows.
+// f32 activations stay f32 in LDS; a wave splits the fragments it reads (hi = half(x), lo = half(x
+// - hi)) and multiplies both.
+// LDS blocks as in the int8 kernels: 8 rows x 128 bytes, chunk c of row r in slot c ^ r ^ (block &
+// 1): whole lines for the loads, all banks for the fragment reads.
+// Against the staged kernel, f16: 1024 x 4096 -> 4096 42.9 -> 34.8 us (power: 24.6 on constant operands),
+// 256 x 4096 -> 11008 36.3 -> 28.0, 64 x 4096 -> 4096 13.5 -> 11.9, 290 x 1600 -> 752 10.5 -> 7.2, 4096^3
+// 133 -> 124; f32: 128 x 4096 -> 4096 23.1 -> 16.2, 1024 x 2048 -> 2048 31.6 -> 23.8, 1549 x 2208 -> 5628
+// 125 -> 95.5.
+template <typename XT, int FM, int NCG, int KG, int BK, int NST>
+struct DmaShape {
+  static constexpr int kBM = 32 * FM, kBN = 64 * NCG, kWaves = NCG * KG;
+  static constexpr int kStage = (kBM * (int)sizeof(XT) + kBN) * BK;
+  // the epilogue's sums: 64 rows (32 where the tile has no more) of every k group, rows padded by
+  // 16 bytes so that a fragment's writes spread over the banks
+  static constexpr int kPitch = kBN + 4, kRows = FM > 1 ? 64 : 32;
+  static constexpr int kSums = KG * kRows * kPitch * 4;
+  static constexpr int kTiles = NST * kStage > kSums ? NST * kStage : kSums;
+  // behind them: zero points (64 per wave), then the scale and the bias of every channel
+  static constexpr int kZp = kTiles, kFactors = kZp + kWaves * 256, kLds = kFactors + kBN * 8;
+};
+
+template <typename XT, bool SIGNED, int FM, int NCG, int KG, int BK, int NST>
+__global__ void __launch_bounds__(NCG* KG * 64, 2) wo_dma_kernel(const WoParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  using Shape = DmaShape<XT, FM, NCG, KG, BK, NST>;
+  constexpr bool F32 = sizeof(XT) == 4;
+  constexpr int BM = Shape::kBM, BN = Shape::kBN, NW = Shape::kWaves;
+  constexpr int SUBS = BK * (int)sizeof(XT) / 128;       // 128-byte wide pieces of an activation row's k tile
+  constexpr int WR = 1024 / BK;                          // weight rows per load
+  constexpr int A_LD = SUBS * (BM / 8) / NW, W_LD = (BN / WR) / NW, LD = A_LD + W_LD;
+  constexpr int A_BYTES = BM * 128 * SUBS, STAGE = Shape::kStage;
+  constexpr int U = BK / 32 / KG;                              // 32-deep units of a k tile per wave
+  constexpr int CH = F32 ? 2 : 1;                        // 16-byte chunks of an activation row per 16 of k and lane
+  constexpr unsigned kFlip = SIGNED ? 0x80808080u : 0u;
+  constexpr int kPast = (int)0x80000000;                 // an offset no descriptor covers
+  static_assert((BK == 64 || BK == 128) && U >= 1 && STAGE == A_BYTES + BN * BK && Shape::kLds <= 160 * 1024, "LDS");
+  static_assert((SUBS * (BM / 8)) % NW == 0 && (BM / 8) % 2 == 0 && NW % 2 == 0, "loads of a wave");
+  static_assert((BN / WR) % NW == 0 && NST * LD <= 63, "loads of a wave; vmcnt is a 6-bit counter");
+  extern __shared__ __attribute__((aligned(1024))) uint8_t wo_lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int cg = wave % NCG, kg = wave / NCG;
+  const int r = lane & 31, g = lane >> 5;
+
+  // Workgroups go to the 8 XCDs in turn, and each has its own L2: an XCD takes a contiguous range
+  // of tiles, walked in panels of 512 rows, so that what it has running at a time shares rows of
+  // both operands.
+  const int tiles_n = (p.N + BN - 1) / BN, tiles_m = (p.M + BM - 1) / BM;
+  int tile = blockIdx.x;
+  {
+    const int tiles = gridDim.x, q = tiles >> 3, rem = tiles & 7, x = tile & 7;
+    tile = x * q + min(x, rem) + (tile >> 3);
+  }
+  const int panel_rows = min(tiles_m, 512 / BM);
+  const int panel = tile / (panel_rows * tiles_n), in_panel = tile - panel * panel_rows * tiles_n;
+  const int rows_here = min(panel_rows, tiles_m - panel * panel_rows);
+  const int m0 = (panel * panel_rows + in_panel % rows_here) * BM, n0 = (in_panel / rows_here) * BN;
+  const int kbeg = blockIdx.y * p.k_split;               // this workgroup's k range
+  const int klen = min(p.K, kbeg + p.k_split) - kbeg;
+  const int KT = (klen + BK - 1) / BK;
+  // descriptors over the tile's rows from (first row, kbeg) on, moved on with the tiles that are
+  // loaded; the host has checked that the offsets below fit 31 bits
+  const int mrows = min(BM, p.M - m0), nrows = min(BN, p.N - n0);
+  const XT* xbase = static_cast<const XT*>(p.x) + (int64_t)m0 * p.ldx + kbeg;
+  const uint8_t* wbase = p.w + (int64_t)n0 * p.w_sn + kbeg;
+  const int xbytes = (int)(((int64_t)(mrows - 1) * p.ldx + klen) * (int)sizeof(XT));
+  const int wbytes = (int)((int64_t)(nrows - 1) * p.w_sn + klen);
+  const unsigned lds_base =
+      (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(size_t)(lds_void_t*)wo_lds);
+
+  // ---- loads.  Load q = wave + i NW of the workgroup fills 1 KiB block q: 8 rows x 128 bytes,
+  // lane -> row lane / 8, slot lane % 8.  The number of waves is even, so the parity of a block is
+  // the wave's and a lane takes the same chunk of a row in all its loads.
+  const int lr = lane >> 3;
+  const int ck = ((lane & 7) ^ lr ^ (wave & 1)) << 4;    // byte offset of that chunk
+  // (weight rows of 64 bytes: 16 to a block, chunk c of row r in slot c ^ (r / 4 & 3))
+  const int cw = BK == 128 ? ck : ((lane & 3) ^ (lane >> 4)) << 4;
+  int xo[A_LD], wo[W_LD];
+#pragma unroll
+  for (int i = 0; i < A_LD; ++i) {
+    const int q = wave + i * NW, row = (q % (BM / 8)) * 8 + lr;
+    // (rows past the last: zeros, no memory touched)
+    xo[i] = row < mrows ? (int)(row * p.ldx * (int)sizeof(XT)) + q / (BM / 8) * 128 + ck : kPast;
+  }
+#pragma unroll
+  for (int i = 0; i < W_LD; ++i) {
+    const int row = (wave + i * NW) * WR + lane / (BK / 16);
+    wo[i] = row < nrows ? (int)(row * p.w_sn) + cw : kPast;
+  }
+  // load l of tile t; FULL: the tile is whole (otherwise zeros past the range's end; K % 16 == 0)
+  auto issue_load = [&](auto full_c, auto l_c, int t, int st) {
+    constexpr bool FULL = decltype(full_c)::value != 0;
+    constexpr int l = decltype(l_c)::value;
+    const int k0 = t * BK;
+    const unsigned base = lds_base + st * STAGE + wave * 1024;
+    if constexpr (l < A_LD) {
+      const v4i rs = make_rsrc(xbase + k0, xbytes - k0 * (int)sizeof(XT));
+      const int first = ((wave + l * NW) / (BM / 8) * 128 + ck) / (int)sizeof(XT);   // the chunk's first element in the tile
+      buffer_load_lds_b128(rs, base + l * NW * 1024, FULL || k0 + first < klen ? xo[l] : kPast);
+    } else {
+      const v4i rs = make_rsrc(wbase + k0, wbytes - k0);
+      buffer_load_lds_b128(rs, base + A_BYTES + (l - A_LD) * NW * 1024, FULL || k0 + cw < klen ? wo[l - A_LD] : kPast);
+    }
+  };
+
+  // ---- fragments: row r of a 32-row block, 16 values of k from 16 g of a 32-deep unit on
+  const int swz = (r & 7) ^ ((r >> 3) & 1);
+  const int row_off = (r >> 3) * 1024 + (r & 7) * 128;
+  int a_off[U][2 * CH], w_off[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int unit = kg * U + u;
+    const int sub = F32 ? unit : unit >> 1, first = F32 ? 4 * g : 4 * (unit & 1) + 2 * g;
+#pragma unroll
+    for (int h = 0; h < 2 * CH; ++h) a_off[u][h] = sub * BM * 128 + row_off + (((first + h) ^ swz) << 4);
+    w_off[u] = A_BYTES + cg * 64 * BK + (BK == 128 ? row_off + (((2 * unit + g) ^ swz) << 4)
+                                                   : r * 64 + (((2 * unit + g) ^ ((r >> 2) & 3)) << 4));
+  }
+  h2 c[2];
+  u4 fa[2][FM][CH];                  // activations of the unit's two 16-deep steps
+  u4 fw[2][2];                       // weights of this unit and the next: both steps
+  h8 w[2][2];                        // widened: of this step and the next
+  // read q of a unit's fragments: the weights, then the activations of row block (q - 2) / (2 CH)
+  constexpr int READS = 2 + FM * 2 * CH;
+  auto read = [&](auto set_c, auto u_c, auto q_c, const uint8_t* base) {
+    constexpr int set = decltype(set_c)::value, u = decltype(u_c)::value, q = decltype(q_c)::value;
+    if constexpr (q < 2) {
+      fw[set][q] = *reinterpret_cast<const u4*>(base + w_off[u] + q * 32 * BK);
+    } else {
+      constexpr int i = (q - 2) / (2 * CH), h = (q - 2) % (2 * CH);
+      fa[h / CH][i][h % CH] = *reinterpret_cast<const u4*>(base + a_off[u][h] + i * 4096);
+    }
+  };
+  auto widen = [&](auto set_c, auto s_c, int j) {
+    constexpr int set = decltype(set_c)::value, s = decltype(s_c)::value;
+    w[s][j] = widen8(fw[set][j][2 * s], fw[set][j][2 * s + 1], kFlip, c[j]);
+  };
+  // (the low halves' products, 2^-11 of the others, on sums of their own: half the roundings at the
+  // size of the whole sum, 0.67 of the rms error against 64 bits that one sum for both gives)
+  f16v acc[FM][2], acc_lo[F32 ? FM : 1][2];
+#pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
-      if (p.partial)
-        store_partial(p, acc[i][j], blockIdx.y, m0 + xrow[i] - r, n0 + wrow[j], lane);
-      else
-        store_frag<XT>(p, acc[i][j], m0 + xrow[i] - r, n0 + wrow[j], lane);
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        acc[i][j][v] = 0.0f;
+        acc_lo[F32 ? i : 0][j][v] = 0.0f;
+      }
+  // One 16-deep step, a row block (two MFMAs per part) at a time, behind each of them hook(i) and a
+  // share of the widening of the next step's weights (of set `next`).
+  auto step = [&](auto s_c, auto next_c, auto&& hook) {
+    constexpr int s = decltype(s_c)::value;
+    static_for_n<FM>([&](auto i_c) {
+      constexpr int i = decltype(i_c)::value;
+      h8 a[F32 ? 2 : 1];
+      if constexpr (F32) {
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+          const f4 v = __builtin_bit_cast(f4, fa[s][i][e / 4 % CH]);
+          h2 hi, lo;
+          split2(v[e % 4], v[e % 4 + 1], hi, lo);
+          a[0][e] = hi.x, a[0][e + 1] = hi.y;
+          a[1][e] = lo.x, a[1][e + 1] = lo.y;
+        }
+      } else {
+        a[0] = __builtin_bit_cast(h8, fa[s][i][0]);
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[s][j], a[0], acc[i][j], 0, 0, 0);
+      if constexpr (F32) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc_lo[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[s][j], a[1], acc_lo[i][j], 0, 0, 0);
+      }
+      hook(i_c);
+      if constexpr (i == (FM > 1 ? FM - 2 : 0)) widen(next_c, Int<s ^ 1>(), 0);
+      if constexpr (i == FM - 1) widen(next_c, Int<s ^ 1>(), 1);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  // until tile t has landed: at most the tiles behind it of those issued so far are in flight
+  auto landed = [&](int behind) {
+    static_for_n<NST>([&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      if (behind == k) __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(k * LD));
+    });
+  };
+
+  // Scale and bias of channel tid, and the zero points of the wave's channels, ahead of the tiles: a
+  // use of a value loaded the ordinary way waits for every load before it, so the first are not
+  // touched until the end and the second go through LDS like the tiles.
+  // (As bits, and from the scales' place where there is no bias: nothing to be done to them here.)
+  using Raw = std::conditional_t<F32, uint32_t, uint16_t>;
+  const int own = n0 + min(tid, nrows - 1);
+  const Raw raw_s = static_cast<const Raw*>(p.scale)[own];
+  const Raw raw_b = static_cast<const Raw*>(p.bias ? p.bias : p.scale)[own];
+  if (p.zp)
+    buffer_load_lds_b32(make_rsrc(p.zp + n0, (int64_t)nrows * 4), lds_base + Shape::kZp + wave * 256, (cg * 64 + lane) * 4);
+  static_for_n<NST>([&](auto t_c) {
+    constexpr int t = decltype(t_c)::value;
+    if (t < KT) static_for_n<LD>([&](auto l_c) { issue_load(Int<0>(), l_c, t, t); });
+  });
+  landed(min(KT, NST) - 1);
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int zp = p.zp ? *reinterpret_cast<const int*>(wo_lds + Shape::kZp + wave * 256 + (j * 32 + r) * 4) : 0;
+    const _Float16 v = (_Float16)(float)(1024 + zp + (SIGNED ? 128 : 0));
+    c[j] = (h2){v, v};
+  }
+  static_for_n<READS>([&](auto q_c) { read(Int<0>(), Int<0>(), q_c, wo_lds); });
+  widen(Int<0>(), Int<0>(), 0);
+  widen(Int<0>(), Int<0>(), 1);
+
+  // Tile t's stage is free from the middle of its last unit on and takes tile t + NST, whose loads
+  // are dealt out from there to the same place of tile t + 1: over that unit's second step (SLOT 0)
+  // and the 2 U - 1 steps behind it.
+  auto spread = [&](auto count_c, auto slots_c, auto slot_c, auto&& body) {
+    constexpr int count = decltype(count_c)::value, slots = decltype(slots_c)::value, slot = decltype(slot_c)::value;
+    static_for_n<count>([&](auto l_c) {
+      if constexpr (decltype(l_c)::value * slots / count == slot) body(l_c);
+    });
+  };
+  constexpr int SLOTS = 2 * U * FM;
+  int st = 0;                                            // tile t's stage
+  // one k tile; PAR: the set its first unit's weights are in; MORE: the tiles loaded meanwhile are there, and whole
+  auto k_tile = [&](auto more_c, auto par_c, int t) {
+    constexpr int MORE = decltype(more_c)::value, PAR = decltype(par_c)::value;
+    const int pst = st == 0 ? NST - 1 : st - 1, nst = st + 1 == NST ? 0 : st + 1;
+    const uint8_t* here = wo_lds + st * STAGE;
+    const uint8_t* there = wo_lds + nst * STAGE;
+    const bool next = MORE || t + 1 < KT;                // (uniform)
+    static_for_n<U>([&](auto u_c) {
+      constexpr int u = decltype(u_c)::value;
+      constexpr bool last = u == U - 1;
+      using Set = Int<(PAR + u) & 1>;
+      using Next = Int<(PAR + u + 1) & 1>;
+      step(Int<0>(), Set(), [&](auto i_c) {
+        if (MORE || (t > 0 && t - 1 + NST < KT))
+          spread(Int<LD>(), Int<SLOTS>(), Int<(1 + 2 * u) * FM + decltype(i_c)::value>(),
+                 [&](auto l_c) { issue_load(Int<MORE>(), l_c, t - 1 + NST, pst); });
+      });
+      if constexpr (last) {
+        if (next) {
+          if constexpr (MORE)
+            __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0((NST - 2) * LD));
+          else
+            landed(min(KT - 2 - t, NST - 2));
+          __syncthreads();                               // tile t + 1 is in LDS; tile t is in registers
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      step(Int<1>(), Next(), [&](auto i_c) {
+        constexpr int i = decltype(i_c)::value;
+        // the next unit's fragments: the weights ahead of the others, a row block's activations behind
+        // its MFMAs, in their registers
+        if (!last || next)
+          static_for_n<READS>([&](auto q_c) {
+            constexpr int q = decltype(q_c)::value;
+            if constexpr (q < 2 ? i == 0 : (q - 2) / (2 * CH) == i)
+              read(Next(), Int<last ? 0 : u + 1>(), q_c, last ? there : here);
+          });
+        if constexpr (last) {
+          if (MORE || t + NST < KT)
+            spread(Int<LD>(), Int<SLOTS>(), i_c, [&](auto l_c) { issue_load(Int<MORE>(), l_c, t + NST, st); });
+        } else {
+          if (MORE || (t > 0 && t - 1 + NST < KT))
+            spread(Int<LD>(), Int<SLOTS>(), Int<(2 + 2 * u) * FM + i>(),
+                   [&](auto l_c) { issue_load(Int<MORE>(), l_c, t - 1 + NST, pst); });
+        }
+      });
+    });
+    st = nst;
+  };
+  // (the first step has no loads left over from one before it; then those whose loads are whole tiles;
+  // then the others)
+  const int whole = klen / BK - NST;
+  k_tile(Int<0>(), Int<0>(), 0);
+  int t = 1;
+  if constexpr (U % 2 == 0) {
+    for (; t < whole; ++t) k_tile(Int<1>(), Int<0>(), t);
+    for (; t < KT; ++t) k_tile(Int<0>(), Int<0>(), t);
+  } else {
+    for (; t + 1 < whole; t += 2) {
+      k_tile(Int<1>(), Int<1>(), t);
+      k_tile(Int<1>(), Int<0>(), t + 1);
+    }
+    for (; t + 1 < KT; t += 2) {
+      k_tile(Int<0>(), Int<1>(), t);
+      k_tile(Int<0>(), Int<0>(), t + 1);
+    }
+    if (t < KT) k_tile(Int<0>(), Int<1>(), t);
+  }
+
+  if constexpr (F32) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] += acc_lo[i][j];
+  }
+  // ---- the k groups' sums into LDS, 64 rows at a time, and out as rows: lane (r, g) holds of a
+  // fragment row r, channels 8 q + 4 g .. + 3
+  constexpr int P = Shape::kPitch, ROWS = Shape::kRows;
+  constexpr int CPR = BN / 8, RPP = NW * 64 / CPR;       // threads (8 channels each) per row, rows per pass
+  float* const sums = reinterpret_cast<float*>(wo_lds);
+  float* const factors = reinterpret_cast<float*>(wo_lds + Shape::kFactors);
+  const int n = n0 + (tid % CPR) * 8;
+  if (tid < BN) {
+    factors[tid] = to_f32(__builtin_bit_cast(XT, raw_s));
+    factors[BN + tid] = p.bias ? to_f32(__builtin_bit_cast(XT, raw_b)) : 0.0f;
+  }
+  float sc[8], bi[8];
+  // (16-byte pieces of any alignment: rows of N elements need not be multiples of 16 bytes)
+  typedef _Float16 h8_any __attribute__((ext_vector_type(8), aligned(2)));
+  typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));
+  const bool whole8 = n + 8 <= p.N;
+  static_for_n<(FM + 1) / 2>([&](auto h_c) {
+    constexpr int h = decltype(h_c)::value;
+    __syncthreads();                                     // the stages, or the rows before, have been read
+#pragma unroll
+    for (int i = 0; i < ROWS / 32; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<f4*>(&sums[(kg * ROWS + i * 32 + r) * P + cg * 64 + j * 32 + 8 * q + 4 * g]) =
+              (f4){acc[2 * h + i][j][4 * q], acc[2 * h + i][j][4 * q + 1], acc[2 * h + i][j][4 * q + 2],
+                   acc[2 * h + i][j][4 * q + 3]};
+    __syncthreads();
+    if (h == 0) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        sc[e] = factors[(tid % CPR) * 8 + e];
+        bi[e] = factors[BN + (tid % CPR) * 8 + e];
+      }
+    }
+#pragma unroll
+    for (int pass = 0; pass < ROWS / RPP; ++pass) {
+      const int row = tid / CPR + pass * RPP, m = m0 + 64 * h + row;
+      float s[8];
+#pragma unroll
+      for (int k = 0; k < KG; ++k) {
+        const f4* src = reinterpret_cast<const f4*>(&sums[(k * ROWS + row) * P + (tid % CPR) * 8]);
+        const f4 lo = src[0], hi = src[1];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          s[e] = k ? s[e] + lo[e] : lo[e];
+          s[4 + e] = k ? s[4 + e] + hi[e] : hi[e];
+        }
+      }
+      if (m >= p.M || n >= p.N) continue;
+      if (p.partial) {
+        float* dst = p.partial + ((int64_t)blockIdx.y * p.M + m) * p.N + n;
+        if (whole8) {
+          *reinterpret_cast<f4_any*>(dst) = (f4){s[0], s[1], s[2], s[3]};
+          *reinterpret_cast<f4_any*>(dst + 4) = (f4){s[4], s[5], s[6], s[7]};
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (n + e < p.N) dst[e] = s[e];
+        }
+        continue;
+      }
+      XT* dst = static_cast<XT*>(p.out) + (int64_t)m * p.ldo + n;
+      XT y[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] = (XT)(s[e] * sc[e] + bi[e]);
+      if (whole8) {
+        if constexpr (F32) {
+          *reinterpret_cast<f4_any*>(dst) = (f4){y[0], y[1], y[2], y[3]};
+          *reinterpret_cast<f4_any*>(dst + 4) = (f4){y[4], y[5], y[6], y[7]};
+        } else {
+          *reinterpret_cast<h8_any*>(dst) = (h8){y[0], y[1], y[2], y[3], y[4], y[5], y[6], y[7]};
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (n + e < p.N) dst[e] = y[e];
+      }
+    }
+  });
+#else
+  (void)p;
+#endif
 }
 
 // out = (sum over the k ranges, in their order) * scale + bias: the second half of a split
@@ -741,7 +1081,7 @@ typedef float f4v __attribute__((ext_vector_type(4)));
 // 13.9 with weights from HBM, 3.2 TB/s), f32 21.5 -> 12.7; 8192 -> 2048 11.3 -> 7.9; M = 32, 4096 -> 11008
 // 18.8 -> 12.1.  More units in registers were slower (D = 4 in place of 2: M = 32 14.0, f32 14.5)
 // except for the narrowest form (4096 -> 8192 9.5 against 10.6).
-// RAGGED (f16): as in wo_lds_kernel (M = 16, 3001 -> 4096, one output per thread before: 567 us).
+// RAGGED (f16): as in wo_ragged_kernel (M = 16, 3001 -> 4096, one output per thread before: 567 us).
 constexpr int kRowsWaves = 8;
 
 template <typename XT, int MT, int FN, int D, bool RAGGED = false>
@@ -828,14 +1168,11 @@ __global__ void __launch_bounds__(kRowsWaves * 64) wo_rows_kernel(const WoParams
     for (int i = 0; i < XP; ++i) {
       if constexpr (F32) {
         const f4 v = __builtin_bit_cast(f4, xq[i]);
-        h4 hi, lo;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          hi[e] = (_Float16)v[e];
-          lo[e] = (_Float16)(v[e] - (float)hi[e]);
-        }
-        *reinterpret_cast<h4*>(&xs[xl[i]]) = hi;
-        *reinterpret_cast<h4*>(&xs[MR * 128 + xl[i]]) = lo;
+        h2 hi[2], lo[2];
+        split2(v[0], v[1], hi[0], lo[0]);
+        split2(v[2], v[3], hi[1], lo[1]);
+        *reinterpret_cast<h4*>(&xs[xl[i]]) = (h4){hi[0].x, hi[0].y, hi[1].x, hi[1].y};
+        *reinterpret_cast<h4*>(&xs[MR * 128 + xl[i]]) = (h4){lo[0].x, lo[0].y, lo[1].x, lo[1].y};
       } else {
         *reinterpret_cast<u4*>(&xs[xl[i]]) = xq[i];
       }
@@ -1002,16 +1339,29 @@ __global__ void __launch_bounds__(256) wo_generic_kernel(const WoParams p) {
   static_cast<XT*>(p.out)[(int64_t)m * p.ldo + n] = (XT)(acc * s + b);
 }
 
-template <typename XT, int WM, int FM, int FN, int SETS, bool RAGGED = false>
-int launch_lds(dim3 grid, const WoParams& p, hipStream_t st) {
-  constexpr int lds = 2 * (WM * FM * 32 * (int)(sizeof(XT) / 2) + 2 * FN * 32) * 128;
-  static_assert(lds <= 160 * 1024, "the stages fit the LDS");
-  auto kern = wo_lds_kernel<XT, WM, FM, FN, SETS, RAGGED>;
-  static std::atomic<uint64_t> lds_allowed{0};
-  if (lds > 64 * 1024)
-    if (int s = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds, &lds_allowed)) return s;
-  hipLaunchKernelGGL(kern, grid, dim3(WM * 128), lds, st, p);
+template <int WM, int FN>
+int launch_ragged(dim3 grid, const WoParams& p, hipStream_t st) {
+  constexpr int lds = 2 * (WM * 32 + 2 * FN * 32) * 128;
+  static_assert(lds <= 64 * 1024, "the stages fit the LDS a launch has without asking");
+  hipLaunchKernelGGL((wo_ragged_kernel<WM, FN>), grid, dim3(WM * 128), lds, st, p);
   return check_hip(hipGetLastError(), "dq8_weight_only_qgemm launch");
+}
+
+template <typename XT, bool SIGNED, int FM, int NCG, int KG, int BK, int NST>
+int launch_dma_kind(const WoParams& p, int splits, hipStream_t st) {
+  using Shape = DmaShape<XT, FM, NCG, KG, BK, NST>;
+  auto kern = wo_dma_kernel<XT, SIGNED, FM, NCG, KG, BK, NST>;
+  static std::atomic<uint64_t> lds_allowed{0};
+  if (int s = allow_dynamic_lds(reinterpret_cast<const void*>(kern), Shape::kLds, &lds_allowed)) return s;
+  const int64_t tiles = ceil_div(p.M, Shape::kBM) * ceil_div(p.N, Shape::kBN);
+  hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)splits), dim3(Shape::kWaves * 64), Shape::kLds, st, p);
+  return check_hip(hipGetLastError(), "dq8_weight_only_qgemm launch");
+}
+
+template <typename XT, int FM, int NCG, int KG, int BK, int NST>
+int launch_dma(const WoParams& p, int splits, hipStream_t st) {
+  return p.flip ? launch_dma_kind<XT, true, FM, NCG, KG, BK, NST>(p, splits, st)
+                : launch_dma_kind<XT, false, FM, NCG, KG, BK, NST>(p, splits, st);
 }
 
 template <typename XT, int MR, int U>
@@ -1067,14 +1417,33 @@ int launch_rows(const WoParams& p, hipStream_t st) {
   return p.M <= 16 ? launch_rows_mt<XT, 1, RAGGED>(p, st) : launch_rows_mt<XT, 2, RAGGED>(p, st);
 }
 
-// The small tile forms of the LDS kernel, for problems whose tiles would leave most of the chip
-// idle.  A lone workgroup on a compute unit runs its k tiles as a chain of latencies (LDS
-// reads, MFMAs, hand-over of the next tile, barrier): 0.4 us per k tile with two 32 x 32
-// fragments per wave, 0.27 us with one -- so below a few rounds of tiles the 64 x 64 tile on
-// four waves beats every larger one, although it moves the most bytes per MFMA.
-enum { kForm128x128 = 0, kForm64x64, kNumForms };
-struct TileForm { int bm, bn; };
-constexpr TileForm kForms[kNumForms] = {{128, 128}, {64, 64}};
+// The tile forms.  Aligned rows: wo_dma_kernel's; f16 rows off 16 bytes: wo_ragged_kernel's.
+enum { kF16_32x64, kF16_64x64, kF16_64x128, kF16_128x128, kF16_128x128Wide, kF16_128x256,
+       kF32_32x64, kF32_32x128, kF32_64x128, kF32_64x128Wide, kF32_64x256,
+       kRagged64x64, kRagged128x128, kNumForms };
+
+// Estimated time of a plan in microseconds,
+//   t = c0 + kt (c1 + c2 (r - 1)) + c3 (r - 1) + [splits > 1] (c4 + c5 M N splits / 1e6) + c6 M N / 1e6
+// kt: 64-deep k tiles per workgroup; r: workgroups per compute unit, rounded up.  Fitted (least
+// squares on relative error, median error 4 %, 90th percentile 11 %) to 32800 timed launches of the
+// f16 forms and 24000 of the f32 forms: M = 33 .. 2048, K = 512 .. 8192, N = 512 .. 11008, odd sizes
+// among them, 1 .. 8 k ranges; the ragged forms to 3300 of their aligned forerunners.
+struct TileForm { int bm, bn; float c0, c1, c2, c3, c4, c5, c6; };
+constexpr TileForm kForms[kNumForms] = {
+    {32, 64, 4.034f, 0.119f, 0.104f, 0.002f, 2.743f, 1.841f, 1.814f},
+    {64, 64, 4.606f, 0.160f, 0.148f, -0.117f, 2.828f, 2.293f, 1.506f},
+    {64, 128, 5.183f, 0.249f, 0.239f, -0.407f, 2.746f, 2.327f, 1.052f},
+    {128, 128, 5.955f, 0.324f, 0.362f, -1.529f, 2.921f, 2.188f, 1.186f},
+    {128, 128, 6.834f, 0.291f, 0.428f, 0.751f, 2.880f, 2.369f, 1.249f},
+    {128, 256, 7.976f, 0.505f, 0.831f, -2.607f, 3.172f, 1.979f, 1.068f},
+    {32, 64, 4.606f, 0.175f, 0.185f, 1.795f, 2.426f, 2.974f, 2.336f},
+    {32, 128, 4.854f, 0.236f, 0.298f, 1.117f, 2.514f, 3.206f, 2.262f},
+    {64, 128, 5.656f, 0.402f, 0.407f, -1.281f, 2.713f, 2.353f, 1.852f},
+    {64, 128, 5.810f, 0.345f, 0.482f, 0.446f, 2.714f, 2.864f, 2.221f},
+    {64, 256, 6.141f, 0.614f, 0.895f, -2.083f, 2.916f, 2.498f, 2.051f},
+    {64, 64, 4.272f, 0.274f, 0.177f, 0.472f, 2.347f, 1.649f, 0.0f},
+    {128, 128, 7.616f, 0.569f, 0.484f, -0.948f, 1.629f, 1.696f, 0.0f},
+};
 
 // Plan: `splits` workgroups per tile of form `form`, each over k_split of the k range, and
 // (splits > 1) a reduction kernel behind them.  `us`: the estimate it was chosen by.
@@ -1085,116 +1454,85 @@ struct SplitPlan {
   float us;
 };
 
-// Estimated time of a plan in microseconds, fitted (least squares on relative error, median
-// error 4 %, 90th percentile 10 %) to 3300 timed launches of the 64 x 64 and 128 x 128 forms:
-// M = 40 .. 3072, nine weight shapes from 768 x 768 to 8192 x 8192, 1 .. 16 k ranges.
-//   t = c0 + kt (c1 + c2 (r - 1)) + c3 (r - 1) + [splits > 1] (c4 + c5 M N splits / 1e6)
-// kt: 64-deep k tiles per workgroup; r: workgroups per compute unit, rounded up.
-struct FormCost { float c0, c1, c2, c3, c4, c5; };
-constexpr FormCost kCost64x64[2] = {{4.272f, 0.274f, 0.177f, 0.472f, 2.347f, 1.649f},     // f16
-                                    {5.805f, 0.456f, 0.334f, 0.613f, 1.023f, 1.731f}};    // f32
-constexpr FormCost kCost128x128[2] = {{7.616f, 0.569f, 0.484f, -0.948f, 1.629f, 1.696f},
-                                      {8.471f, 0.919f, 1.175f, -1.589f, -1.035f, 2.310f}};
-
-// The cheapest of the 64 x 64 and 128 x 128 forms with 1, 2, 3, 4, 6 or 8 k ranges of at
-// least 192 (one range only unless `may_split`).  Choosing by this estimate comes within
-// 1.2 % (geometric mean; worst case 14 %) of the best timed plan of each of those problems.
-SplitPlan plan_split(int64_t M, int64_t N, int64_t K, int esz, bool may_split = true) {
-  SplitPlan best = {kForm128x128, 1, (int)K, 0.0f};
+// The cheapest of the type's forms with 1, 2, 3, 4, 6 or 8 k ranges of at least 192, from `least`
+// ranges on and up to `most`.  Choosing by this estimate comes within 0.8 % (geometric mean; 95 %
+// within 5 %) of the best timed plan of each of the 3400 problems it was fitted to.
+SplitPlan plan_split(int64_t M, int64_t N, int64_t K, int esz, bool ragged, int least, int most) {
+  SplitPlan best = {-1, 1, (int)K, 0.0f};
   const int64_t cus = compute_units();
-  for (int form : {(int)kForm64x64, (int)kForm128x128}) {
-    const FormCost& c = (form == kForm64x64 ? kCost64x64 : kCost128x128)[esz == 4];
-    const int64_t tiles = ceil_div(M, kForms[form].bm) * ceil_div(N, kForms[form].bn);
+  const int first = ragged ? kRagged64x64 : esz == 4 ? kF32_32x64 : kF16_32x64;
+  const int last = ragged ? kRagged128x128 : esz == 4 ? kF32_64x256 : kF16_128x256;
+  for (int form = first; form <= last; ++form) {
+    const TileForm& c = kForms[form];
+    const int64_t tiles = ceil_div(M, c.bm) * ceil_div(N, c.bn);
+    const float mn = (float)((double)M * (double)N * 1e-6);
     for (int want : {1, 2, 3, 4, 6, 8}) {
-      if (want > 1 && (!may_split || K / want < 192)) break;
+      if (want > most || (want > 1 && K / want < 192)) break;
       const int64_t k_split = ceil_div(ceil_div(K, (int64_t)want), 64) * 64;
       const int64_t splits = ceil_div(K, k_split);
+      if (splits < least) continue;
       const float kt = (float)(k_split / 64), r = (float)(ceil_div(tiles * splits, cus) - 1);
-      float us = c.c0 + kt * (c.c1 + c.c2 * r) + c.c3 * r;
-      if (splits > 1) us += c.c4 + c.c5 * (float)((double)M * (double)N * (double)splits * 1e-6);
-      if (best.us == 0.0f || us < best.us)
+      float us = c.c0 + kt * (c.c1 + c.c2 * r) + c.c3 * r + c.c6 * mn;
+      if (splits > 1) us += c.c4 + c.c5 * mn * (float)splits;
+      if (best.form < 0 || us < best.us)
         best = {form, (int)splits, splits > 1 ? (int)k_split : (int)K, us};
     }
   }
   return best;
 }
 
-// The 256-row tiles of f16 activations (eight waves, wave tiles 64 x 64 and 64 x 128: the
-// larger the wave tile, the fewer LDS bytes per MFMA) against 128 x 128 ones, by the measured
-// time of a round of each at 4096 of k: 128 x 128 tiles, two workgroups to a compute unit,
-// 82 us for a full round and 45 while one workgroup has the unit to itself; 256 x 128 tiles,
-// one to a unit, 75 us and 60 up to half a round; 256 x 256 tiles 135 us and 100.
-struct BigTiles {
-  int64_t n256x128, n256;     // tiles of the two shapes
-  int64_t cost128, cost256x128, cost256;
-  bool take256() const { return cost256 < cost128 && cost256 <= cost256x128; }
-  bool take256x128() const { return !take256() && cost256x128 < cost128; }
-};
-BigTiles big_tiles(int64_t M, int64_t N) {
-  const int64_t cus = compute_units();
-  auto rounds = [](int64_t tiles, int64_t slots, int64_t half, int full_us, int part_us) {
-    const int64_t rem = tiles % slots;
-    return tiles / slots * full_us + (rem == 0 ? 0 : rem <= half ? part_us : full_us);
-  };
-  BigTiles b;
-  b.n256x128 = ceil_div(M, 256) * ceil_div(N, 128);
-  b.n256 = ceil_div(M, 256) * ceil_div(N, 256);
-  b.cost128 = rounds(ceil_div(M, 128) * ceil_div(N, 128), 2 * cus, cus, 82, 45);
-  b.cost256x128 = rounds(b.n256x128, cus, cus / 2, 75, 60);
-  b.cost256 = rounds(b.n256, cus, cus / 2, 135, 100);
-  return b;
-}
-
-// Estimated time of whichever 256-row tile big_tiles prefers to 128 x 128: 8 us + 0.85 x its
-// rounds scaled to K (fitted to 70 timed launches, median error 9 %); 0 where it prefers none.
-float big_tile_us(int64_t M, int64_t N, int64_t K) {
-  const BigTiles b = big_tiles(M, N);
-  const int64_t cost = b.take256() ? b.cost256 : b.take256x128() ? b.cost256x128 : 0;
-  return cost ? 8.0f + 0.85f * (float)cost * (float)K / 4096.0f : 0.0f;
-}
-
-// The plan for M x N x K, or form = -1 where the small forms are not the choice: up to 32
-// rows (16 for f32 activations from 2048 of k on, where the staged kernel pays for two half
-// tiles: M = 32, 4096 -> 11008: 25.5 against 33.5 us; 4096^2: 15.7 against 17.9; 8192^2: 33.1
-// against 31.2) the kernels for few rows, and the 256-row tiles where they are estimated
-// cheaper.
-SplitPlan choose_small(int64_t M, int64_t N, int64_t K, int esz, bool ragged, bool may_split) {
+// The plan for M x N x K, or form = -1 where the kernels for few rows are the choice: up to 32 rows,
+// for f32 up to 16 from 2048 of k or 4096 channels on, where the staged kernel pays for two half tiles
+// (f32, tiles against the staged kernel, by geometric mean over 17 .. 32 rows: 1.14-1.48 times as fast
+// beyond 2048 of k, 1.03-1.06 beyond 4096 channels, 0.83-0.90 elsewhere; f16 0.65-0.95).
+SplitPlan choose_tiles(int64_t M, int64_t N, int64_t K, int esz, bool ragged, int most_splits) {
   const SplitPlan none = {-1, 1, (int)K, 0.0f};
-  // (rows off 16 bytes: f16 has the small tiles and the staged small-M kernel, f32 its own kernel)
-  if (ragged) return esz == 4 || M <= 32 ? none : plan_split(M, N, K, esz, may_split);
-  // (f32 from 17 rows on: the staged small-M kernel runs k as one chain per wave, the tiles split it: M =
-  // 24, 1024 -> 4096 7.4 against 8.9 us, 2048^2 10.3 / 11.2, 4096 -> 11008 21.8 / 25.6, but 3072 -> 768
-  // 13.0 / 11.9, 4096^2 16.4 / 16.3, 8192 -> 1024 27.4 / 17.0)
-  if (M <= (esz == 4 && K > 2048 && !(K <= 4096 && N >= 8192) ? 16 : 32)) return none;
-  const SplitPlan s = plan_split(M, N, K, esz, may_split);
-  if (esz == 2 && M > 128) {
-    const float big = big_tile_us(M, N, K);
-    if (big > 0.0f && big < s.us) return none;
-  }
-  return s;
+  // (rows off 16 bytes: f16 has tiles and the staged small-M kernel, f32 its own kernel)
+  if (ragged && (esz == 4 || M <= 32)) return none;
+  if (M <= (esz == 4 && (K > 2048 || N > 4096) ? 16 : 32)) return none;
+  return plan_split(M, N, K, esz, ragged, 1, most_splits);
 }
 
 size_t split_bytes(const SplitPlan& s, int64_t M, int64_t N) {
   return s.splits > 1 ? (size_t)s.splits * (size_t)(M * N) * sizeof(float) : 0;
 }
 
-// one launch of a small tile form over the whole k range (splits == 1) or its split
+// The scratch to ask a caller for, who has sizes but no pointers yet: what the plan for aligned rows
+// wants.  Where that plan is unsplit, what the plan for unaligned rows wants, whose k tiles are dearer,
+// or the cheapest split that is within the estimate's error (a tenth on either side): a scratch that
+// was sized once and kept should not depend on which of two near-equal plans the estimate prefers.
+size_t scratch_split_bytes(int64_t M, int64_t N, int64_t K, int esz) {
+  const size_t off16 = split_bytes(choose_tiles(M, N, K, esz, true, 8), M, N);
+  if (K % 16 != 0) return off16;
+  SplitPlan s = choose_tiles(M, N, K, esz, false, 8);
+  if (s.splits > 1 || s.form < 0) return split_bytes(s, M, N);
+  const SplitPlan split = plan_split(M, N, K, esz, false, 2, 8);
+  return std::max(off16, split.form >= 0 && split.us <= 1.2f * s.us ? split_bytes(split, M, N) : 0);
+}
+
+// one launch of a form over the whole k range (splits == 1) or its split
 template <typename XT>
 int launch_form(int form, int splits, const WoParams& p, hipStream_t st) {
-  constexpr int kSets = sizeof(XT) == 2 ? 4 : 2;         // (f32 rows are twice the registers)
-  const dim3 grid((unsigned)(ceil_div(p.M, kForms[form].bm) * ceil_div(p.N, kForms[form].bn)),
-                  (unsigned)splits);
-  if constexpr (sizeof(XT) == 2)
-    if (p.ragged)
-      return form == kForm128x128 ? launch_lds<XT, 4, 1, 2, kSets, true>(grid, p, st)
-                                  : launch_lds<XT, 2, 1, 1, kSets, true>(grid, p, st);
-  switch (form) {
-    case kForm128x128:
-      // (eight waves of two fragments: two waves per SIMD cover each other's reads and hand-overs, which
-      // is worth more than the LDS bytes that four waves of four fragments save -- M = 1024, 4096 -> 4096
-      // 42.9 against 44.3 us, M = 2048, 8192 -> 2048 78.9 / 81.0; unaligned rows, 4095 -> 4096 49.4 / 59.6)
-      return launch_lds<XT, 4, 1, 2, kSets>(grid, p, st);
-    case kForm64x64: return launch_lds<XT, 2, 1, 1, kSets>(grid, p, st);
+  if constexpr (sizeof(XT) == 2) {
+    const dim3 grid((unsigned)(ceil_div(p.M, kForms[form].bm) * ceil_div(p.N, kForms[form].bn)), (unsigned)splits);
+    switch (form) {
+      case kF16_32x64: return launch_dma<XT, 1, 1, 4, 128, 4>(p, splits, st);
+      case kF16_64x64: return launch_dma<XT, 2, 1, 4, 128, 3>(p, splits, st);
+      case kF16_64x128: return launch_dma<XT, 2, 2, 2, 64, 4>(p, splits, st);
+      case kF16_128x128: return launch_dma<XT, 4, 2, 2, 64, 3>(p, splits, st);
+      case kF16_128x128Wide: return launch_dma<XT, 4, 2, 4, 128, 3>(p, splits, st);
+      case kF16_128x256: return launch_dma<XT, 4, 4, 2, 64, 4>(p, splits, st);
+      case kRagged64x64: return launch_ragged<2, 1>(grid, p, st);
+      case kRagged128x128: return launch_ragged<4, 2>(grid, p, st);
+    }
+  } else {
+    switch (form) {
+      case kF32_32x64: return launch_dma<XT, 1, 1, 4, 128, 4>(p, splits, st);
+      case kF32_32x128: return launch_dma<XT, 1, 2, 4, 128, 4>(p, splits, st);
+      case kF32_64x128: return launch_dma<XT, 2, 2, 2, 64, 3>(p, splits, st);
+      case kF32_64x128Wide: return launch_dma<XT, 2, 2, 4, 128, 3>(p, splits, st);
+      case kF32_64x256: return launch_dma<XT, 2, 4, 2, 64, 4>(p, splits, st);
+    }
   }
   return fail("dq8_weight_only_qgemm: unknown tile form");
 }
@@ -1208,9 +1546,12 @@ int launch(WoParams& p, bool fast, void* scratch, size_t scratch_bytes, hipStrea
                       256 * p.w_sn + (int64_t)p.K + 4096 < (1LL << 31);
   if (fast && lds_ok) {
     const bool have = scratch && aligned(scratch, 16);
-    SplitPlan s = choose_small(p.M, p.N, p.K, (int)sizeof(XT), p.ragged, have);
+    const size_t planes = have ? scratch_bytes / ((size_t)p.M * (size_t)p.N * sizeof(float)) : 0;
+    // (unaligned rows whose scratch was sized for aligned ones: as many k ranges as it holds)
+    SplitPlan s = choose_tiles(p.M, p.N, p.K, (int)sizeof(XT), p.ragged,
+                               p.ragged ? (int)std::min<size_t>(std::max<size_t>(planes, 1), 8) : have ? 8 : 1);
     if (s.splits > 1 && scratch_bytes < split_bytes(s, p.M, p.N))
-      s = choose_small(p.M, p.N, p.K, (int)sizeof(XT), p.ragged, false);
+      s = choose_tiles(p.M, p.N, p.K, (int)sizeof(XT), p.ragged, 1);
     if (s.form >= 0 && s.splits > 1) {
       const int sp = s.splits;
       p.partial = static_cast<float*>(scratch);
@@ -1278,15 +1619,7 @@ int launch(WoParams& p, bool fast, void* scratch, size_t scratch_bytes, hipStrea
     else
       hipLaunchKernelGGL((wo_skinny_kernel<XT, 8, 4>), dim3(grid), dim3(512), 0, st, p);
   } else {
-    // (here: the plan above preferred a 256-row tile, or the LDS kernel cannot address the
-    // operands and the register kernel takes the problem)
-    if constexpr (sizeof(XT) == 2) {
-      const BigTiles b = big_tiles(p.M, p.N);
-      if (b.take256() && lds_ok)
-        return launch_lds<XT, 4, 2, 4, 2>(dim3((unsigned)b.n256), p, st);
-      if (b.take256x128() && lds_ok)
-        return launch_lds<XT, 4, 2, 2, 4>(dim3((unsigned)b.n256x128), p, st);
-    }
+    // (the LDS kernels cannot address the operands: the register kernel)
     const int64_t big = ceil_div(p.M, 128) * ceil_div(p.N, 128);
     if (big >= 192) {
       hipLaunchKernelGGL((wo_tile_kernel<XT, 2, 2>), dim3((unsigned)big), dim3(256), 0, st, p);
@@ -1344,7 +1677,7 @@ extern "C" size_t dq8_weight_only_qgemm_workspace_bytes_ex(int64_t M, int64_t N,
   size_t split = 0;
   if ((x_dtype == DQ8_DTYPE_F16 || x_dtype == DQ8_DTYPE_F32) && K >= 16 && M < (1LL << 31) &&
       N < (1LL << 31) && K < (1LL << 31))
-    split = split_bytes(choose_small(M, N, K, x_dtype == DQ8_DTYPE_F32 ? 4 : 2, K % 16 != 0, true), M, N);
+    split = scratch_split_bytes(M, N, K, x_dtype == DQ8_DTYPE_F32 ? 4 : 2);
   if (!split) return dq8_weight_only_qgemm_workspace_bytes(N, K, tp_b);
   return transposed_bytes(N, K, tp_b) + split;
 }

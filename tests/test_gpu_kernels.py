@@ -1907,6 +1907,38 @@ def test_weight_only_qgemm_few_rounds_of_small_tiles(K, dtype):
     assert unsplit_seen >= 5
 
 
+@pytest.mark.parametrize("dtype,m,k,n,signed", [
+    # 32 x 64 tiles: one k tile, shorter than 128; fewer k tiles than LDS stages; a split whose last
+    # k range is a part of a tile
+    (torch.float16, 33, 80, 17, False), (torch.float16, 102, 384, 65, True), (torch.float16, 85, 1888, 25, False),
+    # 64 x 64, 64 x 128, 128 x 128 (four and eight waves), 128 x 256: a part of a row and of a channel
+    # tile, k ending inside a k tile
+    (torch.float16, 292, 656, 1771, False), (torch.float16, 265, 656, 3662, True),
+    (torch.float16, 323, 672, 5777, False), (torch.float16, 274, 1936, 6689, True),
+    (torch.float16, 978, 1072, 4133, False),
+    (torch.float32, 45, 16, 27, True), (torch.float32, 58, 1312, 19, False), (torch.float32, 68, 144, 5877, False),
+    (torch.float32, 1425, 48, 671, True), (torch.float32, 1375, 560, 651, False),
+    (torch.float32, 356, 752, 5530, True)])
+def test_weight_only_qgemm_tiles_loaded_into_lds(K, dtype, m, k, n, signed):
+    """Every tile form of the kernel that loads both operands straight into LDS, at sizes its tiles do
+    not divide, with results whose rows start off 16 bytes and nothing written beside them; activations
+    and weights past the rows and the k range are NaN / 255, so that nothing outside may be used."""
+    rng = np.random.default_rng(m + k + n)
+    x, w, scale, zp, bias = _weight_only_case(rng, m, k, n, dtype, signed)
+    wide_x = torch.full((m + 1, k + 16), float("nan"), dtype=dtype, device="cuda")
+    wide_x[:m, :k] = dev(x)
+    wide_w = torch.full((n + 1, k + 16), -1 if signed else 255, dtype=torch.int8 if signed else torch.uint8,
+                        device="cuda")
+    wide_w[:n, :k] = dev(w)
+    frame = torch.full((m + 1, n + 5), 7.0, dtype=dtype, device="cuda")
+    out = frame[:m, 1:n + 1]
+    K.weight_only_qgemm(wide_x[:m, :k], wide_w[:n, :k], dev(scale), dev(zp), dev(bias), out=out)
+    _weight_only_check(out, x, w, scale, zp, bias, dtype)
+    assert bool((frame[:, 0] == 7).all()) and bool((frame[:, n + 1:] == 7).all()) and bool((frame[m] == 7).all())
+    got = K.weight_only_qgemm(dev(x), dev(w), dev(scale), workspace=False)
+    _weight_only_check(got, x, w, scale, None, None, dtype)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 def test_weight_only_qgemm_strided_rows_in_and_out(K, dtype):
     """Activation and result rows that are slices of wider buffers (ldx > K, ldo > N), one shape
