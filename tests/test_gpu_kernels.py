@@ -1482,6 +1482,32 @@ def test_qgemm_strided_rows_all_variants(K, m, n, k, pad):
         assert (got[:, n:] == 77).all(), "variant %d wrote past the row" % v
 
 
+@pytest.mark.parametrize("m,n,k", [(70, 33, 64), (300, 129, 256), (500, 1501, 80), (2100, 515, 128), (4200, 1027, 64)])
+def test_qgemm_4_byte_results_in_rows_at_any_word(K, m, n, k):
+    """int32 and f32 results in rows that begin at any multiple of four bytes, also with a residual at
+    another one: 16 bytes a lane, the row's end element by element, nothing beside the rows."""
+    rng = np.random.default_rng(m + n + k)
+    a, w = dev(rng.integers(-128, 128, (m, k), dtype=np.int8)), dev(rng.integers(-128, 128, (n, k), dtype=np.int8))
+    sw = dev(rng.uniform(0.001, 0.05, n).astype(np.float32))
+    sc = dict(sx=dev(np.array([0.02], np.float32)), sw=sw, so=dev(np.array([0.3], np.float32)))
+    bias = dev(rng.standard_normal(n).astype(np.float32))
+    wide = torch.zeros((m, n + 3), device="cuda")
+    res = wide[:, 2:n + 2]
+    res.copy_(dev(rng.standard_normal((m, n)).astype(np.float32)))
+    for epi, kw in ((K.EPI_ACC_S32, {}), (K.EPI_DEQUANT_F32, dict(sx=sc["sx"], sw=sw, bias=bias)),
+                    (K.EPI_REQUANT_CPU_DEQUANT_F32, dict(bias=bias, **sc))):
+        want = K.qgemm(a, w, epi, variant=0, **kw).view(torch.int32)
+        for lead in range(4):
+            frame = torch.full((m, n + 4), 77, dtype=torch.int32, device="cuda")
+            out = frame if epi == K.EPI_ACC_S32 else frame.view(torch.float32)
+            K.qgemm(a, w, epi, out=out[:, lead:lead + n], **kw)
+            assert torch.equal(frame[:, lead:lead + n], want), (epi, lead)
+            assert bool((frame[:, :lead] == 77).all()) and bool((frame[:, lead + n:] == 77).all()), (epi, lead)
+    y = K.qgemm(a, w, epi, variant=0, **kw)
+    got = K.qgemm(a, w, epi, post=K.make_postops(residual=res), **kw)
+    assert torch.equal(got.view(torch.int32), (y + res).view(torch.int32))
+
+
 @pytest.mark.parametrize("m,n,k,ldo", [(300, 200, 256, 208), (1000, 100, 768, 112), (513, 72, 128, 80),
                                        (4100, 1000, 768, 1008), (260, 328, 512, 336)])
 def test_qgemm_ragged_channels_in_16_byte_aligned_rows(K, m, n, k, ldo):
