@@ -91,25 +91,32 @@ namespace {
 // tile's patch again; `narrow` is a second width for layers with no more output channels than
 // that.  (1 x 1 x 256 with 128-channel slices spills; 1 x 1 x 512 was measured and lost to the
 // GEMM tiles at every size.)
+// `paired`: the width behind a residual, where it is set.  With the tail's arithmetic 128 channels take
+// 188 registers and a workgroup has the compute unit to itself; 64 leave room for a second one, which
+// multiplies and stores under the first one's loads: 32 x 56 x 56 x 64 -> 256 with an int8 residual, ReLU
+// and quantize 19.5 -> 17.5 us, batch 8 9.0 -> 7.7, 17 x 60 x 60 13.2 -> 11.3.  (From 128 input channels it
+// loses, each patch loaded eight times: 32 x 28 x 28 x 128 -> 512 13.4 -> 16.2, 20 x 33 x 33 11.2 -> 15.4.)
 struct StreamInstance {
-  int kh, kw, ci, ns, narrow;
+  int kh, kw, ci, ns, narrow, paired;
 };
 constexpr StreamInstance kStreamInstances[] = {
-    {3, 3, 64, 64, 0}, {3, 3, 128, 32, 0}, {1, 1, 64, 128, 64}, {1, 1, 128, 128, 0}, {4, 4, 16, 64, 0},
-    {1, 1, 256, 64, 0},
+    {3, 3, 64, 64, 0, 0}, {3, 3, 128, 32, 0, 0}, {1, 1, 64, 128, 64, 64}, {1, 1, 128, 128, 0, 0}, {4, 4, 16, 64, 0, 0},
+    {1, 1, 256, 64, 0, 0},
 };
-int stream_conv_slice(int Kh, int Kw, int Ci, int Co) {
+const StreamInstance* stream_conv_instance(int Kh, int Kw, int Ci) {
   for (const StreamInstance& s : kStreamInstances)
-    if (s.kh == Kh && s.kw == Kw && s.ci == Ci) return s.narrow && Co <= s.narrow ? s.narrow : s.ns;
-  return 0;
+    if (s.kh == Kh && s.kw == Kw && s.ci == Ci) return &s;
+  return nullptr;
 }
 }  // namespace
 
-bool stream_conv_has_instance(int Kh, int Kw, int Ci) { return stream_conv_slice(Kh, Kw, Ci, 1) != 0; }
+bool stream_conv_has_instance(int Kh, int Kw, int Ci) { return stream_conv_instance(Kh, Kw, Ci) != nullptr; }
 
 bool stream_conv_plan(DirectConvParams* p) {
-  const int ns = stream_conv_slice(p->Kh, p->Kw, p->Ci, p->Co);
-  if (ns == 0) return false;
+  const StreamInstance* inst = stream_conv_instance(p->Kh, p->Kw, p->Ci);
+  if (!inst) return false;
+  const bool paired = p->epi.resid_kind != 0 && inst->paired;
+  const int ns = paired ? inst->paired : inst->narrow && p->Co <= inst->narrow ? inst->narrow : inst->ns;
   if (p->NB <= 0 || p->Ho <= 0 || p->Wo <= 1 || p->Co <= 0) return false;
   const int K = p->Kh * p->Kw * p->Ci;
   const int64_t in_bytes = (int64_t)p->NB * p->H * p->Wd * p->Ci;
@@ -118,8 +125,9 @@ bool stream_conv_plan(DirectConvParams* p) {
   if (hw >= (1 << 24) || hw * p->Wo >= (1LL << 31)) return false;   // (exact umulhi division)
   const int64_t pitch = (p->Wo + p->Kw - 1 + 15) / 16 * 16;
   const int64_t tiles_n = ceil_div(p->Co, ns);
-  const int64_t cus = compute_units();
-  const int fixed = kLdsBytes - stream_conv_weight_lds(K, ns) - stream_conv_cp_bytes(ns);
+  const int64_t per_cu = paired ? 2 : 1;                   // workgroups a compute unit holds
+  const int64_t cus = compute_units() * per_cu;
+  const int fixed = kLdsBytes / (int)per_cu - stream_conv_weight_lds(K, ns) - stream_conv_cp_bytes(ns);
   // Time of a launch in cycles of a SIMD: rounds of workgroups x (blocks of 32 pixels of the
   // busiest SIMD -- it runs waves 0 and 4, which take blocks 0, 8, ... and 4, 12, ... -- each K / 32
   // MFMAs of 32 cycles per 32 channels plus the part of their requantisation that does not
@@ -139,7 +147,7 @@ bool stream_conv_plan(DirectConvParams* p) {
   for (int64_t tpi = p->Kh * p->Kw == 1 ? ceil_div(hw, most_1x1) : 1, next; tpi <= ceil_div(hw, 32); tpi = next) {
     const int64_t tile = ceil_div(hw, tpi);
     next = tile > 1 ? ceil_div(hw, tile - 1) : hw + 1;
-    if (best_cost >= 0 && ceil_div((int64_t)p->NB * tpi * tiles_n, cus) * (block_clk + fixed_clk) > best_cost) break;
+    if (best_cost >= 0 && ceil_div((int64_t)p->NB * tpi * tiles_n, cus) * (per_cu * block_clk + fixed_clk) > best_cost) break;
     // image rows a tile of `tile` consecutive pixels can span, wherever it starts in a row (an
     // upper bound for this tiling, in closed form: the planner is called per launch)
     const int64_t span = std::min<int64_t>((tile + p->Wo - 2) / p->Wo + 1, p->Ho);
@@ -151,7 +159,7 @@ bool stream_conv_plan(DirectConvParams* p) {
     const int64_t blocks = ceil_div(tile, 32);
     const int64_t simd0 = ceil_div(blocks, 8) + (blocks > 4 ? ceil_div(blocks - 4, 8) : 0);
     const int64_t wgs = (int64_t)p->NB * tpi * tiles_n;
-    const int64_t cost = ceil_div(wgs, cus) * (simd0 * block_clk + fixed_clk);
+    const int64_t cost = ceil_div(wgs, cus) * (per_cu * simd0 * block_clk + fixed_clk);
     if (best_cost < 0 || cost < best_cost || (cost == best_cost && wgs <= cus)) {
       best_cost = cost;
       best_tpi = tpi;

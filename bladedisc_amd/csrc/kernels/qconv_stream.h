@@ -57,6 +57,11 @@ constexpr int stream_conv_weight_lds(int K, int NS) {
 // tile per wave)
 constexpr int stream_conv_cp_bytes(int NS) { return NS * 8 + 256 + (NS >= 64 ? 8 * 32 * NS : 0); }
 
+// Behind a residual 1 x 1 filters on 64 channels run two workgroups to a compute unit: 128 registers.
+constexpr bool stream_conv_paired(int KH, int KW, int CI, int NS, int POST) {
+  return POST == 2 && KH == 1 && KW == 1 && CI == 64 && NS == 64;
+}
+
 // POST: the operators fused behind the convolution -- 0 none, 1 a table, 2 a residual (their code
 // and registers are kept out of each other's forms).  A table that only clamps costs nothing
 // (table_clamp).  The int8 residual of a block is fetched a block ahead, in row order, and meets
@@ -64,7 +69,7 @@ constexpr int stream_conv_cp_bytes(int NS) { return NS * 8 + 256 + (NS >= 64 ? 8
 // for a trip to memory (32 x 56 x 56 x 64 -> 256, 1 x 1, int8 residual + ReLU + quantize: 30 us,
 // of which 7 were arithmetic).
 template <int KH, int KW, int CI, int NS, int EPI, int POST>
-__global__ void __launch_bounds__(512) qconv_stream_kernel(const DirectConvParams p) {
+__global__ void __launch_bounds__(512, stream_conv_paired(KH, KW, CI, NS, POST) ? 4 : 2) qconv_stream_kernel(const DirectConvParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   static_assert(EPI == DQ8_EPI_REQUANT_CPU || EPI == DQ8_EPI_REQUANT_GPU, "int8 results only");
   static_assert(CI == 16 || CI == 32 || CI == 64 || CI == 128 || CI == 256 || CI == 512, "channels per pixel");
@@ -113,7 +118,10 @@ __global__ void __launch_bounds__(512) qconv_stream_kernel(const DirectConvParam
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // Blocks go to the waves in turn, so the first waves have one more of them where 8 does not divide
+  // the blocks; wave w runs on SIMD w % 4.  The second workgroup of a compute unit (256 further on, where
+  // two fit) starts one wave on, so that the two workgroups' longer waves do not meet on one SIMD.
+  const int wave = __builtin_amdgcn_readfirstlane(((tid >> 6) + (int)(blockIdx.x >> 8)) & 7);
   const EpiParams& e = p.epi;
 
   // workgroup -> (pixel tile, channel slice): consecutive workgroups go to the 8 XCDs in turn,

@@ -503,7 +503,9 @@ __device__ __forceinline__ ClampTable table_clamp(uint32_t word) {
 // result, unpacking it again and testing every step's special cases: 14 to 19 vector
 // instructions per result, requantisation included, where the general form below takes about 30.
 // With all three scales between 2^-40 and 2^40 every intermediate is finite, so that
-//  * q - zo is (c + magic) - (magic + zo): both steps exact (c is clamped to [-128, 127]);
+//  * q - zo is (c + magic) - (magic + zo): both steps exact (c is clamped to [-128, 127]); without a
+//    zero point q is the rounded c, whose zero may be negative: times so and added to r's product, which
+//    is no negative zero, it leaves the sum as it is;
 //  * the exact quotient by the reciprocal (elementwise::div4_by_constant) needs no probe;
 //  * ReLU before a quantize with a positive scale is a lower bound z2 of the final clamp:
 //    t < 0 gives t / s2 + z2 <= z2, t >= 0 gives >= z2, the same in every rounding.
@@ -549,7 +551,8 @@ __device__ __forceinline__ uint32_t resid_pack4(const EpiParams& p, const ResidT
       d = c[e].os * d;
       d = d + c[e].b;
     }
-    d = (__builtin_amdgcn_fmed3f(d, -128.0f, 127.0f) + magic) - (ZERO ? magic : t.mzo);
+    d = __builtin_amdgcn_fmed3f(d, -128.0f, 127.0f);
+    d = ZERO ? __builtin_rintf(d) : (d + magic) - t.mzo;
     float f = (float)(int)(int8_t)(r >> (8 * e));
     if (!ZERO) f = f - t.zr;
     const float x = d * t.so + f * t.rs;      // (separate roundings: the file has contraction off)

@@ -2228,6 +2228,30 @@ def test_clamping_tables_and_int8_residuals_equal_the_separate_operators(K, nb, 
             assert torch.equal(got, want), (epi, zo, rz, z2, s2, relu)
 
 
+@pytest.mark.parametrize("nb,h,w,co", [(1, 1, 2, 16), (1, 5, 7, 80), (2, 33, 31, 272), (3, 97, 64, 256), (9, 61, 59, 144)])
+def test_conv_1x1_64_behind_a_residual_in_paired_slices(K, nb, h, w, co):
+    """1 x 1 filters on 64 channels with an int8 residual: 64-channel slices, two workgroups to a compute
+    unit; slices and pixel tiles that end anywhere, one workgroup to several rounds of pairs, the f32
+    residual and the general tail (a scale outside the fast range) in the same slices."""
+    rng = np.random.default_rng(nb * h + co)
+    md = list(O.NHWC_OHWI_METADATA) + [1, 1, 1, 1, 1]
+    osh = [nb, h, w, co]
+    x = dev(rng.integers(-128, 128, (nb, h, w, 64), dtype=np.int8))
+    wt = dev(rng.integers(-128, 128, (co, 1, 1, 64), dtype=np.int8))
+    one = lambda v: dev(np.array([v], np.float32))  # noqa: E731
+    z = torch.zeros(1, dtype=torch.int32, device="cuda")
+    kw = dict(sx=one(0.02), so=one(0.043), bias=dev((rng.standard_normal(co) * 0.9).astype(np.float32)),
+              sw=dev((rng.uniform(0.7, 1.3, co) * (50 * 0.043 / 0.02 / (8 * 74 * 74))).astype(np.float32)))
+    y = K.dequantize(K.qconv2d(x, wt, [0] * 4, md, osh, K.EPI_REQUANT_CPU, **kw), kw["so"], z)
+    rq = dev(rng.integers(-128, 128, osh, dtype=np.int8))
+    rf = dev((rng.standard_normal(osh) * 2).astype(np.float32))
+    for res, rs, s2 in ((rq, 0.031, 0.05), (rq, 0.031, 2e12), (rf, None, 0.05)):
+        post = K.make_postops(residual=res, residual_scale=None if rs is None else one(rs), relu=True, out_scale=one(s2))
+        got = K.qconv2d(x, wt, [0] * 4, md, osh, K.EPI_REQUANT_CPU, post=post, **kw)
+        t = y + (res if rs is None else K.dequantize(res, one(rs), z))
+        assert torch.equal(got, K.quantize(torch.where(t < 0, torch.zeros_like(t), t), one(s2), z)), (rs, s2)
+
+
 @pytest.mark.parametrize("m,k,n", [(1, 64, 17), (3, 65, 1), (16, 79, 33), (17, 1000, 130), (32, 2049, 515), (200, 127, 70),
                                    (256, 260, 129), (65, 1001, 1501), (300, 100, 257), (513, 333, 64), (777, 1000, 1501),
                                    (1030, 4097, 260), (2100, 200, 3001), (4200, 72, 2100)])
