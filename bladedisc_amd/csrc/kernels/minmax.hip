@@ -21,6 +21,9 @@
 
 #include "dq8_common.h"
 #include "disc_q8.h"
+#include "q8_elementwise.h"
+
+#pragma clang fp contract(off)
 
 namespace dq8 {
 namespace {
@@ -188,7 +191,7 @@ struct QParamsOut {
   float range;
   int q_min, q_max;
 };
-__device__ __forceinline__ void qparams_one(const QParamsOut& q, int c, float lo, float hi) {
+__device__ __forceinline__ void qparams_of(const QParamsOut& q, float lo, float hi, float* scale, int* zero_point) {
   const float neg = lo < 0.0f ? lo : 0.0f, pos = hi > 0.0f ? hi : 0.0f;
   const float eps = std::numeric_limits<float>::epsilon();
   float s = (q.symmetric ? (-neg > pos ? -neg : pos) : pos - neg) / q.range;
@@ -198,6 +201,13 @@ __device__ __forceinline__ void qparams_one(const QParamsOut& q, int c, float lo
     z = q.q_min - (int)rintf(neg / s);
     z = z < q.q_min ? q.q_min : (z > q.q_max ? q.q_max : z);
   }
+  *scale = s;
+  *zero_point = z;
+}
+__device__ __forceinline__ void qparams_one(const QParamsOut& q, int c, float lo, float hi) {
+  float s;
+  int z;
+  qparams_of(q, lo, hi, &s, &z);
   q.scale[c] = s;
   q.zero_point[c] = z;
 }
@@ -296,6 +306,144 @@ minmax_fold_lastaxis(const float2* __restrict__ partial, int groups, int channel
     fold(m, MinMax{min_io[c], max_io[c]});
     min_io[c] = m.lo;
     max_io[c] = m.hi;
+  }
+}
+
+// ---- pass 2 and the fake quantization in one launch.  Every workgroup (per tensor) or wave (per
+// row) folds the pairs and the running values it needs itself, instead of waiting for a kernel that
+// does so once: at calibration sizes a step is launches and trips to memory, and the pairs come from
+// the L2 (a step in a loop, per row, 740 x 240 21.1 -> 17.5 us, 71 x 1328 20.7 -> 16.4; per tensor, where
+// one launch is saved and not two, 3072 x 768 18.2 -> 17.0).
+// Workgroup 0 also stores the running values, scale and zero point and gives the answer.  Others may
+// read a running value before or after it is stored: folding the same pairs into the result again
+// gives the result, bit for bit.
+struct FakeRange {
+  float s, y, lo, hi;
+  int z;
+  bool fast;
+  __device__ __forceinline__ FakeRange(const QParamsOut& q, const MinMax& m) {
+    qparams_of(q, m.lo, m.hi, &s, &z);
+    y = 1.0f / s;
+    fast = elementwise::divisor_in_fast_range(s);
+    lo = (float)q.q_min;
+    hi = (float)q.q_max;
+  }
+  __device__ __forceinline__ float4 operator()(const float4& v) const {
+    using namespace elementwise;
+    return fast ? fake4_by_constant<1>(v, s, y, z, lo, hi)
+                : make_float4(fake_one<1>(v.x, s, z, lo, hi), fake_one<1>(v.y, s, z, lo, hi),
+                              fake_one<1>(v.z, s, z, lo, hi), fake_one<1>(v.w, s, z, lo, hi));
+  }
+};
+
+// per tensor: n4 groups of four in tiles of 1024, `tiles` of them dealt over the workgroups
+__global__ void __launch_bounds__(kThreads)
+fold_fake_quant_tensor(const float4* __restrict__ x, float4* __restrict__ out, int64_t n4, int tiles,
+                       const float2* __restrict__ partial, int segs, float* min_io, float* max_io,
+                       const QParamsOut q) {
+  __shared__ MinMax all;
+  float4 v[4];
+  auto load = [&](int t) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t i = (int64_t)t * 1024 + u * kThreads + threadIdx.x;
+      v[u] = x[i < n4 ? i : n4 - 1];
+    }
+  };
+  load(blockIdx.x);                        // (the data on its way under the pairs)
+  MinMax m = identity();
+  for (int s0 = threadIdx.x; s0 < segs; s0 += 4 * kThreads) {
+    float2 pr[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) pr[u] = partial[s0 + u * kThreads < segs ? s0 + u * kThreads : s0];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) fold(m, MinMax{pr[u].x, pr[u].y});
+  }
+  m = block_reduce(m);
+  if (threadIdx.x == 0) {
+    fold(m, MinMax{min_io[0], max_io[0]});
+    all = m;
+  }
+  __syncthreads();
+  m = all;
+  const FakeRange f(q, m);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    min_io[0] = m.lo;
+    max_io[0] = m.hi;
+    q.scale[0] = f.s;
+    q.zero_point[0] = f.z;
+    signal(q.status, m.lo <= m.hi);
+  }
+  for (int t = blockIdx.x;;) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t i = (int64_t)t * 1024 + u * kThreads + threadIdx.x;
+      if (i < n4) dq8::st_stream(&out[i], f(v[u]));
+    }
+    t += gridDim.x;
+    if (t >= tiles) break;
+    load(t);
+  }
+}
+
+// per row (channel = row): a wave per piece of 256 groups of four of a row; workgroup 0 stores the
+// channels' results instead
+__device__ __forceinline__ MinMax row_range(const float2* __restrict__ partial, int segs, int first, int step,
+                                            int64_t row, const float* min_io, const float* max_io) {
+  const MinMax state = {min_io[row], max_io[row]};
+  MinMax m = identity();
+  for (int s = first; s < segs; s += step) {
+    const float2 pr = partial[row * segs + s];
+    fold(m, MinMax{pr.x, pr.y});
+  }
+  for (int off = step >> 1; off > 0; off >>= 1) {
+    MinMax o;
+    o.lo = __shfl_xor(m.lo, off, 64);
+    o.hi = __shfl_xor(m.hi, off, 64);
+    fold(m, o);
+  }
+  fold(m, state);
+  return m;
+}
+
+__global__ void __launch_bounds__(kThreads)
+fold_fake_quant_rows(const float4* __restrict__ x, float4* __restrict__ out, int rows, int inner4, int pieces,
+                     const float2* __restrict__ partial, int segs, float* min_io, float* max_io,
+                     const QParamsOut q) {
+  if (blockIdx.x == 0) {
+    bool ok = true;
+#pragma unroll 4
+    for (int c = threadIdx.x; c < rows; c += kThreads) {
+      const MinMax m = row_range(partial, segs, 0, 1, c, min_io, max_io);
+      ok = ok && m.lo <= m.hi;
+      min_io[c] = m.lo;
+      max_io[c] = m.hi;
+      qparams_one(q, c, m.lo, m.hi);
+    }
+    const bool every = __syncthreads_and(ok);
+    if (threadIdx.x == 0) signal(q.status, every);
+    return;
+  }
+  const int lane = threadIdx.x & 63;
+  const int64_t unit = (int64_t)(blockIdx.x - 1) * 4 + (threadIdx.x >> 6);
+  const int64_t row = unit / pieces;
+  if (row >= rows) return;
+  const int first = (int)(unit - row * pieces) * 256;
+  const float4* px = x + row * inner4;
+  float4 v[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int i = first + u * 64 + lane;
+    v[u] = px[i < inner4 ? i : inner4 - 1];
+  }
+  // (one pair a row: every lane reads it)
+  const MinMax m = segs == 1 ? row_range(partial, 1, 0, 1, row, min_io, max_io)
+                             : row_range(partial, segs, lane, 64, row, min_io, max_io);
+  const FakeRange f(q, m);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int i = first + u * 64 + lane;
+    if (i < inner4) dq8::st_stream(&out[row * inner4 + i], f(v[u]));
   }
 }
 
@@ -442,6 +590,55 @@ extern "C" int dq8_observe(const float* x, int64_t outer, int64_t channels, int6
   hipLaunchKernelGGL(minmax_qparams, dim3(1), dim3(1024), 0, (hipStream_t)stream, min_io, max_io,
                      (int)channels, q);
   return check_hip(hipGetLastError(), "minmax_qparams launch");
+}
+
+// The observation step and the fake quantization of the same tensor with its result.
+extern "C" int dq8_observe_fake_quant(const float* x, float* out, int64_t outer, int64_t channels, int64_t inner,
+                                      float* min_io, float* max_io, int symmetric, int32_t q_min, int32_t q_max,
+                                      float* scale, int32_t* zero_point, int32_t* status, void* workspace,
+                                      size_t workspace_bytes, void* stream) {
+  clear_error();
+  DQ8_REQUIRE(outer > 0 && channels > 0 && inner > 0, "dq8_observe_fake_quant: empty tensor");
+  DQ8_REQUIRE(x && out && min_io && max_io && scale && zero_point && status,
+              "dq8_observe_fake_quant: null pointer");
+  DQ8_REQUIRE(channels < (1LL << 31), "dq8_observe_fake_quant: too many channels");
+  DQ8_REQUIRE(q_min < q_max && q_min >= -32768 && q_max <= 65535,
+              "dq8_observe_fake_quant: quant_min/quant_max outside the 8- and 16-bit ranges");
+  const bool rows = outer == 1 && !(inner == 1 && channels > 1);     // (channels are rows, or one channel)
+  const bool vec = aligned(x, 16) && inner % 4 == 0;
+  Plan p;
+  // One launch behind pass 1 while what is folded more than once stays small: up to 4096 pairs of a
+  // tensor by at most 1024 workgroups (32 MB from the L2s), up to 2048 channels by workgroup 0.
+  // (Beyond, a kernel that folds once costs less than its share of the time: 6342 x 4016 57.8 us.)
+  if (rows && vec && aligned(out, 16) && make_plan(outer, channels, inner, true, &p) &&
+      (channels == 1 ? p.segs <= 4096 : channels <= 2048 && inner <= (1 << 20))) {
+    DQ8_REQUIRE(workspace && workspace_bytes >= (size_t)p.pairs * sizeof(float2),
+                "dq8_observe_fake_quant: workspace too small (see dq8_minmax_workspace_bytes)");
+    hipStream_t st = (hipStream_t)stream;
+    float2* partial = static_cast<float2*>(workspace);
+    const float full = (float)(q_max - q_min);
+    const QParamsOut q = {scale, zero_point, status, symmetric, symmetric ? full / 2 : full, q_min, q_max};
+    hipLaunchKernelGGL(minmax_rows<true>, dim3((unsigned)p.blocks), dim3(kThreads), 0, st, x, inner, p.segs,
+                       p.chunks, partial);
+    if (int s = check_hip(hipGetLastError(), "minmax_rows launch")) return s;
+    if (channels == 1) {
+      const int64_t tiles = ceil_div(inner / 4, 1024);
+      hipLaunchKernelGGL(fold_fake_quant_tensor, dim3((unsigned)std::min<int64_t>(tiles, 1024)), dim3(kThreads), 0,
+                         st, reinterpret_cast<const float4*>(x), reinterpret_cast<float4*>(out), inner / 4,
+                         (int)tiles, partial, p.segs, min_io, max_io, q);
+    } else {
+      const int64_t pieces = ceil_div(inner / 4, 256);
+      hipLaunchKernelGGL(fold_fake_quant_rows, dim3((unsigned)(1 + ceil_div(channels * pieces, 4))), dim3(kThreads),
+                         0, st, reinterpret_cast<const float4*>(x), reinterpret_cast<float4*>(out), (int)channels,
+                         (int)(inner / 4), (int)pieces, partial, p.segs, min_io, max_io, q);
+    }
+    return check_hip(hipGetLastError(), "fold_fake_quant launch");
+  }
+  if (int s = dq8_observe(x, outer, channels, inner, min_io, max_io, symmetric, q_min, q_max, scale, zero_point,
+                          status, workspace, workspace_bytes, stream))
+    return s;
+  return dq8_fake_quant(x, out, outer, channels, inner, scale, zero_point, channels, q_min, q_max,
+                        DQ8_ROUND_HALF_TO_EVEN, stream);
 }
 
 // ---- the same with the pairs in memory the library brings along -------------------------

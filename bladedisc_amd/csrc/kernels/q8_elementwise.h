@@ -117,6 +117,29 @@ __device__ __forceinline__ int quant_from_quotient(float t0, float lo, float hi)
   return (int)t3;
 }
 
+// quantize followed by dequantize without the 8-bit tensor in between: f32 in, f32 out,
+// the two functions' arithmetic unchanged (the integer result is subtracted from the zero
+// point as an integer, as dequantize does).
+template <int ROUND>
+__device__ __forceinline__ float fake_one(float x, float s, int zi, float lo, float hi) {
+  const int q = quant_one<ROUND>(x, s, (float)zi, lo, hi);
+  return (float)(q - zi) * s;
+}
+
+// fake_one on four values with one divisor through its reciprocal (the quotient's bits are those
+// of x / s, see div4_by_constant)
+template <int ROUND>
+__device__ __forceinline__ float4 fake4_by_constant(const float4& v, float s, float y, int zi,
+                                                    float lo, float hi) {
+  const float4 q = div4_by_constant(v, s, y);
+  const float z = (float)zi;
+  auto one = [&](float t0) {
+    const int qi = quant_from_quotient<ROUND>(t0 + z, lo, hi);
+    return (float)(qi - zi) * s;
+  };
+  return make_float4(one(q.x), one(q.y), one(q.z), one(q.w));
+}
+
 // Four quotients -> four int8 in one word, half-to-even rounding: clamp first (for integer
 // bounds clamp(rne(t)) = rne(clamp(t)); v_med3_f32 returns the smaller bound for a NaN, as
 // quant_one's fmaxf / fminf pair does), then one addition of 1.5 * 2^23 per value rounds to the

@@ -263,29 +263,6 @@ dequantize_rows(const uint32_t* __restrict__ q, float4* __restrict__ out,
 }
 
 // ------------------------------------------------------------------ fake quant
-// quantize followed by dequantize without the 8-bit tensor in between: f32 in, f32 out,
-// the two functions' arithmetic unchanged (the integer result is subtracted from the zero
-// point as an integer, as dequantize does).
-template <int ROUND>
-__device__ __forceinline__ float fake_one(float x, float s, int zi, float lo, float hi) {
-  const int q = quant_one<ROUND>(x, s, (float)zi, lo, hi);
-  return (float)(q - zi) * s;
-}
-
-// fake_one on four values with one divisor through its reciprocal (the quotient's bits are those
-// of x / s, see div4_by_constant)
-template <int ROUND>
-__device__ __forceinline__ float4 fake4_by_constant(const float4& v, float s, float y, int zi,
-                                                    float lo, float hi) {
-  const float4 q = div4_by_constant(v, s, y);
-  const float z = (float)zi;
-  auto one = [&](float t0) {
-    const int qi = quant_from_quotient<ROUND>(t0 + z, lo, hi);
-    return (float)(qi - zi) * s;
-  };
-  return make_float4(one(q.x), one(q.y), one(q.z), one(q.w));
-}
-
 template <int ROUND>
 __global__ void __launch_bounds__(kThreads)
 fake_quant_tensor_v4(const float4* __restrict__ x, float4* __restrict__ out, int64_t n,

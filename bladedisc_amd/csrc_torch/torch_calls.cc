@@ -308,7 +308,7 @@ dq8::StatusWords& status_words() {
 
 // observe(x, min_io, max_io, axis, symmetric, q_min, q_max, fake_quant)
 //   -> (min <= max everywhere, scale, zero_point, fake-quantized x or None)
-// One step of an observer: four kernels at most, the last of them the fake quantization, and one
+// One step of an observer: two to four kernels, the last of them with the fake quantization, and one
 // wait for the answer whether the observed range is sound.
 PyObject* py_observe(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
@@ -343,19 +343,18 @@ PyObject* py_observe(PyObject*, PyObject* const* a, Py_ssize_t n) {
       *own = pinned_words(1);
       return own->data_ptr<int32_t>();
     });
-    const char* what = "dq8_observe";
+    const char* what = fake ? "dq8_observe_fake_quant" : "dq8_observe";
     int failed;
     int32_t answer = 0;
     {
       const dq8::Unlocked unlocked;
       auto drain = [&] { st.synchronize(); };
-      failed = dq8_observe(xp, v.outer, v.nch, v.inner, lop, hip, symmetric, q_min, q_max,
-                           sp, zp, status.hand_out(), wsp, need, raw);
-      if (!failed && fake) {
-        what = "dq8_fake_quant";
-        failed = dq8_fake_quant(xp, yp, v.outer, v.nch, v.inner, sp, zp, v.nch, q_min, q_max,
-                                DQ8_ROUND_HALF_TO_EVEN, raw);
-      }
+      if (fake)
+        failed = dq8_observe_fake_quant(xp, yp, v.outer, v.nch, v.inner, lop, hip, symmetric, q_min, q_max,
+                                        sp, zp, status.hand_out(), wsp, need, raw);
+      else
+        failed = dq8_observe(xp, v.outer, v.nch, v.inner, lop, hip, symmetric, q_min, q_max,
+                             sp, zp, status.hand_out(), wsp, need, raw);
       if (!failed) {
         answer = status.wait(drain);
       } else {

@@ -152,6 +152,15 @@ int dq8_observe(const float* x, int64_t outer, int64_t channels, int64_t inner, 
                 int32_t* zero_point, int32_t* status, void* workspace, size_t workspace_bytes,
                 void* stream);
 
+/* dq8_observe, then dq8_fake_quant (half to even) of the same tensor with its scales and zero points
+ * into out (device f32, the shape of x, not x itself): the same bits, in two launches where the tensor
+ * is small and its channels are its rows or one.  status is set when everything but `out` has been
+ * written. */
+int dq8_observe_fake_quant(const float* x, float* out, int64_t outer, int64_t channels, int64_t inner,
+                           float* min_io, float* max_io, int symmetric, int32_t q_min, int32_t q_max,
+                           float* scale, int32_t* zero_point, int32_t* status, void* workspace,
+                           size_t workspace_bytes, void* stream);
+
 /* ---- quantize / dequantize -------------------------------------------- */
 
 /* x (device, f32) is viewed as [outer, nch, inner]; scale (device f32) and zp

@@ -231,3 +231,34 @@ def test_refused_steps_leave_the_next_one_its_answer(K):
     assert torch.equal(y, K.fake_quant(x, scale, zero_point))
     x[2, 64] = float("nan")
     assert not K.observe(x, lo, hi, True, -128, 127)[0]
+
+
+@pytest.mark.parametrize("shape,axis", [((4,), None), ((12, 3), None), ((1023, 4), None), ((64, 64), None),
+                                        ((1024, 16384), None), ((1025, 16384), None), ((4100, 4099), None),
+                                        ((1, 4), 0), ((5, 256), 0), ((9, 1028), 0), ((3, 20004), 0), ((2048, 64), 0),
+                                        ((2049, 64), 0), ((300, 4096), 0), ((31, 30), 0), ((2, 3, 40), 1)])
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_fake_quantization_in_the_observation_step(K, shape, axis, symmetric):
+    """dq8_observe_fake_quant, whose last kernel folds the pairs itself (aligned rows, up to 4096 pairs of
+    a tensor or 2048 rows) or is dq8_fake_quant's: the running values, scales, zero points and outputs of
+    the two calls, bit for bit, over steps that move the range, leave it, hold zeros of both signs,
+    infinities and a NaN in one channel."""
+    torch.manual_seed(sum(shape))
+    nch = 1 if axis is None else shape[axis]
+    lim = (-128, 127) if symmetric else (0, 255)
+    state = [fresh(nch), fresh(nch)]
+    for step in range(5):
+        x = torch.randn(shape, device="cuda") * (3.0, 5.0, 0.1, 1.0, 1.0)[step]
+        flat = x.reshape(-1)
+        if step == 2:
+            x = torch.where(x < 0, -0.0, 0.0).to(torch.float32).contiguous()
+        if step == 3:
+            flat[-1] = float("inf")
+        if step == 4:
+            flat[flat.numel() // 2] = float("nan")
+        sound, s, z, _ = K.observe(x, *state[0], symmetric, *lim, axis=axis)
+        want = K.fake_quant(x, s, z, axis=axis, qmin=lim[0], qmax=lim[1])
+        got = K.observe(x, *state[1], symmetric, *lim, axis=axis, fake_quant=True)
+        assert got[0] == sound == (step < 4)
+        for a, b in zip((s, z, want, *state[0]), (*got[1:], *state[1])):
+            assert torch.equal(a.view(torch.int32), b.view(torch.int32)), step
