@@ -247,6 +247,13 @@ class QuantBertLayer:
         linear in the kernel that produces its input, what follows a linear in its epilogue --
         eight launches, the bits of the separate operators."""
         f = self.f
+        if type(self.be) is RawBackend:
+            operands = [t[name] for name in LINEARS
+                        for t in (self.w_q, self.bias, self.s_in, self.sw, self.s_out)]
+            operands += self.gelu_table, f["ln1_g"], f["ln1_b"], f["ln2_g"], f["ln2_b"], self.be.z1
+            y = K.encoder_layer(h, self.heads, 1e-12, tuple(operands))
+            if y is not None:
+                return y
         b, s, c = h.shape
         h2 = h.reshape(-1, c)
         x_q = self.be.quantize(h2, self.s_in["qkv"])

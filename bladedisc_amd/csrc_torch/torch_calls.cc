@@ -597,6 +597,121 @@ PyObject* py_layer_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// encoder_layer(h [batch, seq, hidden], heads, eps, operands): operands holds, for the merged
+// projection, the attention output and the two feed-forward linears in turn, (int8 weights [N, K], f32
+// bias, input scale, weight scales, output scale), then the activation table between the last two, the
+// layer norms' weights and biases, and the zero point 0.  None where anything is of another form.
+// What kernels.py's quantize, qgemm, attention and layer_norm do one after the other for a layer with
+// everything fused that can be, the same eight launches: called one by one, with a view and a postops
+// structure between most of them, they take 45 to 48 us of the host's time, which is more than the GPU
+// needs below about 300 tokens.  A layer of hidden size 768: 48.1 -> 34.5 us at 1 x 19 tokens, 45.2 ->
+// 40.0 at 11 x 20, the same from 6 x 90 on; the first pass of a process 197 -> 137.
+PyObject* py_encoder_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    arguments("encoder_layer", n, 4);
+    const Tensor& h0 = device_tensor(a[0]);
+    const int64_t heads = integer(a[1]);
+    const float eps = (float)PyFloat_AsDouble(a[2]);
+    if (PyErr_Occurred()) throw PyFailure{};
+    constexpr int kLinears = 4, kEach = 5, kOperands = kLinears * kEach + 6;
+    if (!PyTuple_Check(a[3]) || PyTuple_GET_SIZE(a[3]) != kOperands)
+      raise(PyExc_TypeError, "encoder_layer takes a tuple of 26 operands");
+    if (h0.scalar_type() != ScalarType::Float || h0.dim() != 3 || heads <= 0 || h0.size(2) != heads * 64) Py_RETURN_NONE;
+    const int64_t batch = h0.size(0), seq = h0.size(1), hidden = h0.size(2), M = batch * seq;
+    const at::Device dev = h0.device();
+    const Tensor* t[kOperands];
+    for (int i = 0; i < kOperands; ++i) {
+      PyObject* o = PyTuple_GET_ITEM(a[3], i);
+      if (!THPVariable_Check(o)) Py_RETURN_NONE;
+      t[i] = &THPVariable_Unpack(o);
+      if (!t[i]->is_contiguous() || t[i]->device() != dev) Py_RETURN_NONE;
+    }
+    auto is = [](const Tensor& x, ScalarType type, int64_t numel) {
+      return x.scalar_type() == type && x.numel() == numel;
+    };
+    struct Linear {
+      const int8_t* w;
+      const float *bias, *sx, *sw, *so;
+      int64_t n, k;
+      size_t need;
+    } l[kLinears];
+    for (int i = 0; i < kLinears; ++i) {
+      const Tensor* const* o = t + i * kEach;
+      const int64_t k = i == 3 ? l[2].n : hidden, rows = o[0]->dim() == 2 ? o[0]->size(0) : 0;
+      if (rows <= 0 || !is(*o[0], ScalarType::Char, rows * k) || (i == 0 ? rows != 3 * hidden : i != 2 && rows != hidden) ||
+          !is(*o[1], ScalarType::Float, rows) || !is(*o[2], ScalarType::Float, 1) ||
+          !is(*o[3], ScalarType::Float, rows) || !is(*o[4], ScalarType::Float, 1))
+        Py_RETURN_NONE;
+      l[i] = {(const int8_t*)in(*o[0]), (const float*)in(*o[1]), (const float*)in(*o[2]), (const float*)in(*o[3]),
+              (const float*)in(*o[4]), rows, k, dq8_qgemm_workspace_bytes_zp(M, rows, k, 0, 1, 0, 0)};
+    }
+    const Tensor* const* last = t + kLinears * kEach;
+    if (!is(*last[0], ScalarType::Char, 256) || !is(*last[5], ScalarType::Int, 1)) Py_RETURN_NONE;
+    for (int i = 1; i < 5; ++i)
+      if (!is(*last[i], ScalarType::Float, hidden)) Py_RETURN_NONE;
+    const void* table = in(*last[0]);
+    const float *g1 = (const float*)in(*last[1]), *b1 = (const float*)in(*last[2]);
+    const float *g2 = (const float*)in(*last[3]), *b2 = (const float*)in(*last[4]);
+    const int32_t* zero = (const int32_t*)in(*last[5]);
+    const Tensor h = dense(h0);
+    const float* x = (const float*)in(h);
+    // the int8 input of each linear, and the f32 results: the merged projection, the sum in front of
+    // either layer norm (the second overwrites the first, which has been read by then), the first norm,
+    // the layer
+    Tensor q[kLinears], y[4];
+    for (int i = 0; i < kLinears; ++i) q[i] = empty({M, l[i].k}, ScalarType::Char, dev);
+    y[0] = empty({M, 3 * hidden}, ScalarType::Float, dev);
+    for (int i = 1; i < 3; ++i) y[i] = empty({M, hidden}, ScalarType::Float, dev);
+    y[3] = empty(h.sizes(), ScalarType::Float, dev);
+    int8_t* qp[kLinears];
+    float* yp[4];
+    for (int i = 0; i < 4; ++i) {
+      qp[i] = (int8_t*)inout(q[i]);
+      yp[i] = (float*)inout(y[i]);
+    }
+    size_t need = 0;
+    for (const Linear& i : l) need = std::max(need, i.need);
+    Tensor ws;
+    if (need) ws = empty({(int64_t)need}, ScalarType::Byte, dev);
+    void* wsp = inout(ws);
+    void* st = stream();
+    const char* what = "";
+    int failed = 0;
+    {
+      const dq8::Unlocked unlocked;
+      auto ok = [&](const char* name, int status) {
+        what = name;
+        failed = status;
+        return status == 0;
+      };
+      auto linear = [&](int i, void* out, int epilogue, const dq8_postops_t* post) {
+        return ok("dq8_qgemm", dq8_qgemm_fused(qp[i], l[i].k, l[i].w, l[i].k, out, l[i].n, M, l[i].n, l[i].k, 0, 1,
+                                               epilogue, l[i].bias, DQ8_BIAS_F32, l[i].sx, 1, l[i].sw, l[i].n,
+                                               l[i].so, 1, 0, 0, 0, wsp, l[i].need, post, st));
+      };
+      dq8_postops_t gelu = {}, add_x = {}, add_h1 = {};
+      gelu.table = table;
+      add_x.residual = x;
+      add_x.residual_kind = DQ8_RESIDUAL_F32;
+      add_x.ldr = hidden;
+      add_h1 = add_x;
+      add_h1.residual = yp[2];
+      ok("dq8_quantize", dq8_quantize_ex(x, DQ8_DTYPE_F32, qp[0], DQ8_I8, 1, 1, M * hidden, l[0].sx, zero, 1, -128,
+                                         127, DQ8_ROUND_HALF_TO_EVEN, st)) &&
+          linear(0, yp[0], DQ8_EPI_REQUANT_CPU_DEQUANT_F32, nullptr) &&
+          ok("dq8_attention_f32", dq8_attention_f32(yp[0], batch, seq, heads, 64, nullptr, qp[1], l[1].sx, st)) &&
+          linear(1, yp[1], DQ8_EPI_REQUANT_CPU_DEQUANT_F32, &add_x) &&
+          ok("dq8_layernorm_f32",
+             dq8_layernorm_f32(yp[1], M, hidden, g1, b1, eps, yp[2], qp[2], l[2].sx, st)) &&
+          linear(2, qp[3], DQ8_EPI_REQUANT_CPU, &gelu) &&
+          linear(3, yp[1], DQ8_EPI_REQUANT_CPU_DEQUANT_F32, &add_h1) &&
+          ok("dq8_layernorm_f32", dq8_layernorm_f32(yp[1], M, hidden, g2, b2, eps, yp[3], nullptr, nullptr, st));
+    }
+    check(failed, what);
+    return THPVariable_Wrap(y[3]);
+  });
+}
+
 PyMethodDef kMethods[] = {
 #define DQ8_METHOD(name, fn) {name, (PyCFunction)(void (*)(void))fn, METH_FASTCALL, nullptr}
     DQ8_METHOD("quantize", py_quantize),
@@ -611,6 +726,7 @@ PyMethodDef kMethods[] = {
     DQ8_METHOD("qconv2d", py_qconv2d),
     DQ8_METHOD("attention", py_attention),
     DQ8_METHOD("layer_norm", py_layer_norm),
+    DQ8_METHOD("encoder_layer", py_encoder_layer),
 #undef DQ8_METHOD
     {nullptr, nullptr, 0, nullptr}};
 

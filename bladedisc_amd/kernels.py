@@ -267,6 +267,17 @@ def layer_norm(x, weight, bias, eps=1e-5, scale=None):
     return _native().layer_norm(x, weight, bias, eps, scale)
 
 
+def encoder_layer(h, heads, eps, operands):
+    """A quantized encoder layer on h [B, S, 64 * heads] (f32): quantize, merged projection, attention,
+    output linear + h, layer norm, feed-forward linear with a 256-entry activation table, second
+    feed-forward linear + the first norm, layer norm -- the calls above in this order, eight launches.
+    operands: for the four linears in turn (int8 weights [N, K], f32 bias, input scale, weight scales,
+    output scale), then the table, the norms' (weight, bias, weight, bias) and an int32 zero; all
+    contiguous, one bias and weight scale per channel and one input and output scale.  None where an
+    operand is of another form: then the calls one by one decide."""
+    return _native().encoder_layer(h, heads, eps, operands)
+
+
 NHWC_OHWI = (0, 3, 1, 2, 3, 0, 1, 2, 0, 3, 1, 2)
 
 

@@ -308,6 +308,34 @@ def test_config5_bert_layer_in_eight_launches_has_the_bits_of_the_separate_opera
             ctx.close()
 
 
+@pytest.mark.parametrize("batch,seq", [(1, 1), (5, 13), (2, 300), (8, 509)])   # (512 positions at most)
+def test_encoder_layer_call_is_the_eight_calls(C, batch, seq, monkeypatch):
+    """The layer in one native call against its operators called one by one: the same bits, also for
+    an input that is a strided view; other forms of an operand are left to the separate calls."""
+    from bladedisc_amd import bert_layer as B
+    from bladedisc_amd import kernels as K
+    layer = B.QuantBertLayer(C.config5_weights(), B.RawBackend(), fuse_epilogue=True)
+    h = layer.embed(C.config5_tokens(batch, seq))
+    layer.calibrate(h)
+    native, returned = K.encoder_layer, []
+
+    def watched(*args):
+        returned.append(native(*args))
+        return returned[-1]
+
+    monkeypatch.setattr(K, "encoder_layer", watched)
+    strided = torch.cat([h, h], dim=-1)[..., : h.shape[-1]]
+    got = [layer.forward(h), layer.forward(strided)]
+    assert all(r is not None for r in returned) and strided.is_contiguous() == (batch * seq == 1)
+    scales = layer.s_out["qkv"]
+    layer.s_out["qkv"] = float(scales)               # a number is a scale of the separate calls
+    want = layer.forward(h)
+    assert returned[-1] is None
+    layer.s_out["qkv"] = scales
+    for y in got:
+        assert y.shape == want.shape and torch.equal(y.view(torch.int32), want.view(torch.int32))
+
+
 @pytest.mark.parametrize("backend", ["raw", "ral"])
 @pytest.mark.parametrize("fused", [False, True, "epilogue"])
 def test_config5_bert_layer_graph_replays_match_eager(C, fused, backend):
