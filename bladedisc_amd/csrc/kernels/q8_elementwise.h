@@ -83,18 +83,20 @@ __device__ __forceinline__ float4 div4_by_constant(const float4& x, float s, flo
   return q;
 }
 
-// The same with a divisor per component (per-channel scales on the last axis).
+// The same with a divisor per component (per-channel scales on the last axis); false where a quotient
+// is not finite and has to be had from the division.
+__device__ __forceinline__ bool div4_quick(const float4& x, const float4& s, const float4& y, float4& q) {
+  const float a = x.x * y.x, b = x.y * y.y, c = x.z * y.z, d = x.w * y.w;
+  q.x = __builtin_fmaf(__builtin_fmaf(-a, s.x, x.x), y.x, a);
+  q.y = __builtin_fmaf(__builtin_fmaf(-b, s.y, x.y), y.y, b);
+  q.z = __builtin_fmaf(__builtin_fmaf(-c, s.z, x.z), y.z, c);
+  q.w = __builtin_fmaf(__builtin_fmaf(-d, s.w, x.w), y.w, d);
+  const float probe = (q.x + q.y) + (q.z + q.w);
+  return probe == probe && __builtin_fabsf(probe) != __builtin_inff();
+}
 __device__ __forceinline__ float4 div4_by_constants(const float4& x, const float4& s, const float4& y) {
   float4 q;
-  {
-    const float a = x.x * y.x, b = x.y * y.y, c = x.z * y.z, d = x.w * y.w;
-    q.x = __builtin_fmaf(__builtin_fmaf(-a, s.x, x.x), y.x, a);
-    q.y = __builtin_fmaf(__builtin_fmaf(-b, s.y, x.y), y.y, b);
-    q.z = __builtin_fmaf(__builtin_fmaf(-c, s.z, x.z), y.z, c);
-    q.w = __builtin_fmaf(__builtin_fmaf(-d, s.w, x.w), y.w, d);
-  }
-  const float probe = (q.x + q.y) + (q.z + q.w);
-  if (__builtin_expect(!(probe == probe) || __builtin_fabsf(probe) == __builtin_inff(), 0)) {
+  if (__builtin_expect(!div4_quick(x, s, y, q), 0)) {
     q.x = x.x / s.x;
     q.y = x.y / s.y;
     q.z = x.z / s.z;

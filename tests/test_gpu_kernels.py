@@ -2622,3 +2622,43 @@ def test_fused_operators_behind_rows_of_any_length(K, shape, kernel):
     for a, w in forms:
         for zx in (0, -11):
             _fused_forms_equal_the_separate_operators(K, a, w, zx, rng)
+
+
+@pytest.mark.parametrize("rows,nch", [(4, 3), (5, 37), (1023, 255), (7, 256), (64, 257), (33, 511), (9, 1025),
+                                      (4, 3073), (517, 1537), (1021, 1)])
+@pytest.mark.parametrize("xt,qt", [(torch.float32, torch.uint8), (torch.float16, torch.int8),
+                                   (torch.float32, torch.int16), (torch.float16, torch.int16),
+                                   (torch.float32, torch.int32)])
+def test_quantize_by_channel_and_by_sweep_any_type(K, rows, nch, xt, qt):
+    """Per channel of the last axis and per tensor, at the edges of the four-row groups, of a workgroup's
+    1024, 2048 or 4096 elements and of the choice between the two kernels; with values whose quotients are
+    not finite and, in a second pass, scales that no reciprocal is used for.  Every step is one rounded
+    binary32 operation: equal bits."""
+    rng = np.random.default_rng(rows * 4096 + nch)
+    info = torch.iinfo(qt)
+    lo, hi = np.float32(info.min), np.float32(info.max)
+    x = (rng.standard_normal((rows, nch)) * 8).astype(np.float32)
+    x.reshape(-1)[rng.integers(0, x.size, 9)] = [np.nan, np.inf, -np.inf, 0.0, -0.0, 6e4, -6e4, 0.5, np.nan]
+    x = torch.from_numpy(x).to(xt)
+    for wild in (False, True):
+        scale = (rng.random(nch) * 0.05 + 0.01).astype(np.float32)
+        if wild:
+            scale[rng.integers(0, nch, 3)] = [1e-30, 1e30, 0.0]
+        zp = rng.integers(-3 if info.min < 0 else 0, 4, nch).astype(np.int32)
+        for axis in (1, None):
+            if axis is None and wild:
+                continue
+            s, z = (scale, zp) if axis == 1 and nch > 1 else (scale[:1], zp[:1])
+            ds, dz = torch.from_numpy(s).cuda(), torch.from_numpy(z).cuda()
+            q = K.quantize(x.cuda(), ds, dz, axis=axis, qmin=info.min, qmax=info.max, dtype=qt)
+            with np.errstate(all="ignore"):
+                t = np.rint(x.float().numpy() / s + z.astype(np.float32))
+            want = np.clip(np.fmin(np.fmax(t, lo), hi).astype(np.float64), info.min, info.max).astype(np.int64)
+            assert np.array_equal(q.cpu().numpy().astype(np.int64), want)
+            y = K.dequantize(q, ds, dz, axis=axis)
+            with np.errstate(all="ignore"):
+                back = (want.astype(np.int32) - z).astype(np.float32) * s
+            assert np.array_equal(y.cpu().numpy().view(np.int32), back.view(np.int32))
+            if xt == torch.float32 and qt in (torch.uint8, torch.int16):
+                f = K.fake_quant(x.cuda(), ds, dz, axis=axis, qmin=info.min, qmax=info.max)
+                assert np.array_equal(f.cpu().numpy(), back)
