@@ -2662,3 +2662,34 @@ def test_quantize_by_channel_and_by_sweep_any_type(K, rows, nch, xt, qt):
             if xt == torch.float32 and qt in (torch.uint8, torch.int16):
                 f = K.fake_quant(x.cuda(), ds, dz, axis=axis, qmin=info.min, qmax=info.max)
                 assert np.array_equal(f.cpu().numpy(), back)
+
+
+@pytest.mark.parametrize("outer,nch,inner", [(1, 400001, 4), (3, 70001, 9), (1, 1537, 1025), (2, 3, 400003),
+                                             (5, 300, 1024), (1, 7, 5), (700, 3, 1021)])
+@pytest.mark.parametrize("xt,qt", [(torch.float32, torch.uint8), (torch.float16, torch.int16),
+                                   (torch.float32, torch.int32)])
+def test_quantize_by_row_any_type(K, outer, nch, inner, xt, qt):
+    """The channel on an axis that is not the last, rows of any length from four elements on: groups across
+    the end of a row, several rows per workgroup, scales that no reciprocal is used for.  Equal bits."""
+    rng = np.random.default_rng(nch * 16 + inner)
+    info = torch.iinfo(qt)
+    x = (rng.standard_normal((outer, nch, inner)) * 8).astype(np.float32)
+    x.reshape(-1)[rng.integers(0, x.size, 6)] = [np.nan, np.inf, -np.inf, 0.0, 6e4, -6e4]
+    x = torch.from_numpy(x).to(xt)
+    s = (rng.random(nch) * 0.05 + 0.01).astype(np.float32)
+    s[rng.integers(0, nch, 3)] = [1e-30, 1e30, 0.0]
+    z = rng.integers(0, 4, nch).astype(np.int32)
+    ds, dz = torch.from_numpy(s).cuda(), torch.from_numpy(z).cuda()
+    q = K.quantize(x.cuda(), ds, dz, axis=1, qmin=info.min, qmax=info.max, dtype=qt)
+    with np.errstate(all="ignore"):
+        t = np.rint(x.float().numpy() / s[:, None] + z[:, None].astype(np.float32))
+    want = np.clip(np.fmin(np.fmax(t, np.float32(info.min)), np.float32(info.max)).astype(np.float64),
+                   info.min, info.max).astype(np.int64)
+    assert np.array_equal(q.cpu().numpy().astype(np.int64), want)
+    y = K.dequantize(q, ds, dz, axis=1).cpu().numpy()
+    with np.errstate(all="ignore"):
+        back = (want.astype(np.int32) - z[:, None]).astype(np.float32) * s[:, None]
+    assert np.array_equal(y.view(np.int32), back.view(np.int32))
+    if qt == torch.uint8:
+        f = K.fake_quant(x.cuda(), ds, dz, axis=1, qmin=0, qmax=255).cpu().numpy()
+        assert np.array_equal(f, back)
