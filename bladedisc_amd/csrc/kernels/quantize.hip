@@ -53,19 +53,42 @@ __device__ __forceinline__ uint32_t quant4_by_constants(const float4& v, const f
   return finish4_quotients<ROUND>(make_float4(q.x + z.x, q.y + z.y, q.z + z.z, q.w + z.w), lo, hi);
 }
 
+// The sweeps take pieces of 1024 groups whatever U, piece j on the accelerator die j % 8 (workgroups go to
+// the eight in turn; the 4 / U of a piece are eight apart): what one of them has just written the next one,
+// on the other type's U, finds in its die's L2.  With pieces of U * kThreads quantize and dequantize of
+// 1928 x 2451 f16 through int16 in one buffer took 12.9 us, 10.2 before there was a sweep.
+constexpr int kPiece = 4 * kThreads;
+template <int U>
+__device__ __forceinline__ uint32_t sweep_first_group() {
+  constexpr uint32_t R = 4 / U;
+  const uint32_t b = blockIdx.x, piece = b / (8 * R) * 8 + b % 8, part = b / 8 % R;
+  return piece * kPiece + part * (U * kThreads) + threadIdx.x;
+}
+template <int U>
+unsigned sweep_workgroups(int64_t n) {           // (one group more: the elements behind the last four)
+  const int64_t pieces = dq8::ceil_div(n / 4 + 1, (int64_t)kPiece);
+  return (unsigned)(U == 4 ? pieces : dq8::ceil_div(pieces, 8) * 8 * (4 / U));
+}
+
 // ---------------------------------------------------------------- per tensor
+// The 8-bit kernels walk the same pieces where the L2 holds what they leave: quantize and dequantize in
+// one buffer, f32 through int8, 1500 x 3072 11.2 -> 8.9 us, 3000 x 3072 16.4 -> 15.6 (from f16 19.5 -> 12.9),
+// 5000 x 3072 25.1 -> 24.4; 8000 x 3072 40.4 -> 40.8, and below four million elements the launches are all
+// there is (2.8 -> 2.9 at two million on buffers that change).
+inline bool pieces_pay(int64_t n) { return n >= (1 << 22) && n <= (1 << 24); }
+
 // One unit per thread and a grid that covers the tensor in one sweep (the loop only
 // runs again beyond 2^30 units): on this part a linear sweep by many small workgroups
 // reaches more of the HBM bandwidth than fewer workgroups that each keep several
 // far-apart streams in flight (measured on 1 GiB of f32: 6.2 TB/s against 4.7-5.2).
-template <int ROUND>
+template <int ROUND, bool PIECES>
 __global__ void __launch_bounds__(kThreads)
 quantize_tensor_v4(const float4* __restrict__ x, uint32_t* __restrict__ out,
                    int64_t n, const float* __restrict__ scale,
                    const int32_t* __restrict__ zp, float lo, float hi) {
   const int64_t n4 = n >> 2;
   const int64_t stride = (int64_t)gridDim.x * kThreads;
-  int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  int64_t i = PIECES ? (int64_t)sweep_first_group<1>() : (int64_t)blockIdx.x * kThreads + threadIdx.x;
   if (i < n4) {
     // The data load goes out first: a wave has one load to make, and behind the scalar loads of
     // the parameters and the reciprocal it would start a cache miss later.
@@ -115,7 +138,7 @@ __device__ __forceinline__ float4 dequant_word4(uint32_t w, const int4& z, const
 // [4096,768] 4.37 -> 3.35 us, [32,56,56,64] 6.3 -> 5.1 us, [65536,4096] 216 -> 187 us, which
 // is 7.2 TB/s; the same hint on the loads made every size slower, and on quantize's stores (a
 // fifth of its traffic) it helped some sizes and hurt others, so neither is used.
-template <bool SIGNED>
+template <bool SIGNED, bool PIECES>
 __global__ void __launch_bounds__(kThreads)
 dequantize_tensor_v4x2(const uint32_t* __restrict__ q, float4* __restrict__ out,
                        int64_t n, const float* __restrict__ scale,
@@ -124,7 +147,8 @@ dequantize_tensor_v4x2(const uint32_t* __restrict__ q, float4* __restrict__ out,
   const int z = zp[0];
   const int64_t n4 = n >> 2;
   const int64_t stride = (int64_t)gridDim.x * (2 * kThreads);
-  for (int64_t i = (int64_t)blockIdx.x * (2 * kThreads) + threadIdx.x; i < n4; i += stride) {
+  for (int64_t i = PIECES ? (int64_t)sweep_first_group<2>() : (int64_t)blockIdx.x * (2 * kThreads) + threadIdx.x; i < n4;
+       i += stride) {
     const bool two = i + kThreads < n4;
     const uint32_t w0 = q[i];
     const uint32_t w1 = two ? q[i + kThreads] : 0u;
@@ -553,23 +577,6 @@ lastaxis_any(const IN* __restrict__ in, OUT* __restrict__ out, int64_t n, int nc
   }
 }
 
-// The sweeps take pieces of 1024 groups whatever U, piece j on the accelerator die j % 8 (workgroups go to
-// the eight in turn; the 4 / U of a piece are eight apart): what one of them has just written the next one,
-// on the other type's U, finds in its die's L2.  With pieces of U * kThreads quantize and dequantize of
-// 1928 x 2451 f16 through int16 in one buffer took 12.9 us, 10.2 before there was a sweep.
-constexpr int kPiece = 4 * kThreads;
-template <int U>
-__device__ __forceinline__ uint32_t sweep_first_group() {
-  constexpr uint32_t R = 4 / U;
-  const uint32_t b = blockIdx.x, piece = b / (8 * R) * 8 + b % 8, part = b / 8 % R;
-  return piece * kPiece + part * (U * kThreads) + threadIdx.x;
-}
-template <int U>
-unsigned sweep_workgroups(int64_t n) {           // (one group more: the elements behind the last four)
-  const int64_t pieces = dq8::ceil_div(n / 4 + 1, (int64_t)kPiece);
-  return (unsigned)(U == 4 ? pieces : dq8::ceil_div(pieces, 8) * 8 * (4 / U));
-}
-
 // One linear sweep, n < 2^32: a workgroup takes U * kThreads groups of four that follow each other, a
 // thread kThreads apart.  PER_CHANNEL: the channels on the last axis, a group's parameters read with it
 // (advance = 4 kThreads mod nch); otherwise per tensor.
@@ -911,8 +918,12 @@ extern "C" int dq8_quantize(const float* x, void* out, int out_kind,
   } while (0)
 
   if (!per_channel && vec_ok) {
-    LAUNCH_RND(quantize_tensor_v4, dim3(sweep_grid(n / 4 + n % 4)), dim3(kThreads),
-               (const float4*)x, (uint32_t*)out, n, scale, zp, lo, hi);
+    const bool pieces = pieces_pay(n);
+    auto k = rne ? (pieces ? quantize_tensor_v4<DQ8_ROUND_HALF_TO_EVEN, true> : quantize_tensor_v4<DQ8_ROUND_HALF_TO_EVEN, false>)
+                 : (pieces ? quantize_tensor_v4<DQ8_ROUND_HALF_AWAY_FROM_ZERO, true>
+                           : quantize_tensor_v4<DQ8_ROUND_HALF_AWAY_FROM_ZERO, false>);
+    hipLaunchKernelGGL(k, dim3(pieces ? sweep_workgroups<1>(n) : sweep_grid(n / 4 + n % 4)), dim3(kThreads), 0, st,
+                       (const float4*)x, (uint32_t*)out, n, scale, zp, lo, hi);
   } else if (per_channel && vec_ok && inner == 1 && nch % 4 == 0 && nch / 4 < (1 << 30) &&
              dq8::aligned(scale, 16) && dq8::aligned(zp, 16)) {
     const int nch4 = (int)(nch / 4);
@@ -957,9 +968,11 @@ extern "C" int dq8_dequantize(const void* q, int in_kind, float* out,
   const bool vec_ok = dq8::aligned(q, 4) && dq8::aligned(out, 16);
 
   if (!per_channel && vec_ok) {
-    auto k = is_signed ? dequantize_tensor_v4x2<true> : dequantize_tensor_v4x2<false>;
-    hipLaunchKernelGGL(k, dim3(sweep_grid(dq8::ceil_div(n / 4, 2))), dim3(kThreads), 0, st,
-                       (const uint32_t*)q, (float4*)out, n, scale, zp);
+    const bool pieces = pieces_pay(n);
+    auto k = is_signed ? (pieces ? dequantize_tensor_v4x2<true, true> : dequantize_tensor_v4x2<true, false>)
+                       : (pieces ? dequantize_tensor_v4x2<false, true> : dequantize_tensor_v4x2<false, false>);
+    hipLaunchKernelGGL(k, dim3(pieces ? sweep_workgroups<2>(n) : sweep_grid(dq8::ceil_div(n / 4, 2))), dim3(kThreads),
+                       0, st, (const uint32_t*)q, (float4*)out, n, scale, zp);
   } else if (per_channel && vec_ok && inner == 1 && nch % 4 == 0 && nch / 4 < (1 << 30) &&
              dq8::aligned(scale, 16) && dq8::aligned(zp, 16)) {
     const int nch4 = (int)(nch / 4);

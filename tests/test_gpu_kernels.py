@@ -2625,7 +2625,7 @@ def test_fused_operators_behind_rows_of_any_length(K, shape, kernel):
 
 
 @pytest.mark.parametrize("rows,nch", [(4, 3), (5, 37), (1023, 255), (7, 256), (64, 257), (33, 511), (9, 1025),
-                                      (4, 3073), (517, 1537), (1021, 1)])
+                                      (4, 3073), (517, 1537), (1021, 1), (1723, 2501)])
 @pytest.mark.parametrize("xt,qt", [(torch.float32, torch.uint8), (torch.float16, torch.int8),
                                    (torch.float32, torch.int16), (torch.float16, torch.int16),
                                    (torch.float32, torch.int32)])
