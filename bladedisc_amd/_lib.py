@@ -66,6 +66,7 @@ _PROTOS = {
     "dq8_qconv2d_workspace_bytes_ex": (_SZ, [C.POINTER(_I64), C.POINTER(_I64), C.POINTER(_I64),
                                              C.POINTER(_I32)]),
     "dq8_mfma_probe": (_INT, [_VP] * 7),
+    "dq8_observe_folds_range": (_INT, [_I64] * 3),
     "dq8_lut8": (_INT, [_VP, _VP, _I64, _VP, _VP]),
     "dq8_weight_only_qgemm_workspace_bytes": (C.c_size_t, [_I64, _I64, _INT]),
     "dq8_weight_only_qgemm_workspace_bytes_ex": (C.c_size_t, [_I64, _I64, _I64, _INT, _INT]),
@@ -108,7 +109,7 @@ class PostOps(C.Structure):
 
 
 _HOOKS = ("dq8_qgemm_variant", "dq8_qgemm_num_variants", "dq8_qgemm_variant_name",
-          "dq8_qconv2d_variant", "dq8_mfma_probe")
+          "dq8_qconv2d_variant", "dq8_mfma_probe", "dq8_observe_folds_range")
 
 
 def _bind(L, skip=()):

@@ -493,7 +493,26 @@ bool make_plan(int64_t outer, int64_t channels, int64_t inner, bool vec, Plan* p
   return true;
 }
 
+// Whether the fake quantization folds the pairs itself, one launch behind pass 1: while what is folded
+// more than once, or by workgroup 0 on a thread a row, stays small.  A step in a loop, in one launch /
+// with a kernel that folds once:
+//  * a tensor, up to 4096 pairs folded by at most 1024 workgroups (32 MB from the L2s): 3 M elements 16.1 /
+//    16.4 us, 8 M 20.5 / 22.8, 16 M 37.5 / 38.5;
+//  * rows of up to six pairs, fewer than 1024 rows (from there on the other form folds a thread a row as
+//    well) and 8 M elements: 64 x 24576 14.7 / 16.8, 512 x 4096 15.4 / 17.0, 740 x 8192 21.0 / 21.6; beyond,
+//    2 x 1048576 39 / 18, 64 x 131072 28.5 / 25.0, 1024 x 3072 17.2 / 17.0, 2048 x 1024 17.9 / 16.7.
+bool fold_plan(int64_t outer, int64_t channels, int64_t inner, Plan* p) {
+  if (outer != 1 || inner % 4 != 0 || !make_plan(1, channels, inner, true, p)) return false;
+  return channels == 1 ? p->segs <= 4096 : channels < 1024 && p->segs <= 6 && channels * inner <= (1 << 23);
+}
+
 }  // namespace
+
+bool observe_folds_range(int64_t outer, int64_t channels, int64_t inner) {
+  Plan p;
+  return fold_plan(outer, channels, inner, &p);
+}
+
 }  // namespace dq8
 
 using namespace dq8;
@@ -604,14 +623,8 @@ extern "C" int dq8_observe_fake_quant(const float* x, float* out, int64_t outer,
   DQ8_REQUIRE(channels < (1LL << 31), "dq8_observe_fake_quant: too many channels");
   DQ8_REQUIRE(q_min < q_max && q_min >= -32768 && q_max <= 65535,
               "dq8_observe_fake_quant: quant_min/quant_max outside the 8- and 16-bit ranges");
-  const bool rows = outer == 1 && !(inner == 1 && channels > 1);     // (channels are rows, or one channel)
-  const bool vec = aligned(x, 16) && inner % 4 == 0;
   Plan p;
-  // One launch behind pass 1 while what is folded more than once stays small: up to 4096 pairs of a
-  // tensor by at most 1024 workgroups (32 MB from the L2s), up to 2048 channels by workgroup 0.
-  // (Beyond, a kernel that folds once costs less than its share of the time: 6342 x 4016 57.8 us.)
-  if (rows && vec && aligned(out, 16) && make_plan(outer, channels, inner, true, &p) &&
-      (channels == 1 ? p.segs <= 4096 : channels <= 2048 && inner <= (1 << 20))) {
+  if (aligned(x, 16) && aligned(out, 16) && fold_plan(outer, channels, inner, &p)) {
     DQ8_REQUIRE(workspace && workspace_bytes >= (size_t)p.pairs * sizeof(float2),
                 "dq8_observe_fake_quant: workspace too small (see dq8_minmax_workspace_bytes)");
     hipStream_t st = (hipStream_t)stream;

@@ -1626,6 +1626,10 @@ extern "C" int dq8_qconv2d(const int8_t* in, const int64_t in_sizes[4], const in
 }
 
 #ifdef DQ8_TEST_HOOKS
+extern "C" int dq8_observe_folds_range(int64_t outer, int64_t channels, int64_t inner) {
+  return observe_folds_range(outer, channels, inner);
+}
+
 extern "C" int dq8_mfma_probe(const int8_t* a, const int8_t* b, int32_t* d32,
                               const int8_t* a16, const int8_t* b16, int32_t* d16,
                               void* stream) {

@@ -51,6 +51,10 @@ int dq8_mfma_probe(const int8_t* a, const int8_t* b, int32_t* d32,
                    const int8_t* a16, const int8_t* b16, int32_t* d16,
                    void* stream);
 
+/* Whether dq8_observe_fake_quant (include/disc_q8.h) of a tensor with 16-byte aligned pointers folds
+ * the observed range in its last kernel (two launches); otherwise a kernel of its own does. */
+int dq8_observe_folds_range(int64_t outer, int64_t channels, int64_t inner);
+
 #ifdef __cplusplus
 }
 #endif

@@ -236,11 +236,12 @@ def test_refused_steps_leave_the_next_one_its_answer(K):
 @pytest.mark.parametrize("shape,axis", [((4,), None), ((12, 3), None), ((1023, 4), None), ((64, 64), None),
                                         ((1024, 16384), None), ((1025, 16384), None), ((4100, 4099), None),
                                         ((1, 4), 0), ((5, 256), 0), ((9, 1028), 0), ((3, 20004), 0), ((2048, 64), 0),
-                                        ((2049, 64), 0), ((300, 4096), 0), ((31, 30), 0), ((2, 3, 40), 1)])
+                                        ((2049, 64), 0), ((300, 4096), 0), ((31, 30), 0), ((2, 3, 40), 1),
+                                        ((1023, 64), 0), ((1024, 64), 0), ((7, 24576), 0), ((7, 24580), 0)])
 @pytest.mark.parametrize("symmetric", [True, False])
 def test_fake_quantization_in_the_observation_step(K, shape, axis, symmetric):
     """dq8_observe_fake_quant, whose last kernel folds the pairs itself (aligned rows, up to 4096 pairs of
-    a tensor or 2048 rows) or is dq8_fake_quant's: the running values, scales, zero points and outputs of
+    a tensor, or below 1024 rows of up to six pairs) or is dq8_fake_quant's: the running values, scales, zero points and outputs of
     the two calls, bit for bit, over steps that move the range, leave it, hold zeros of both signs,
     infinities and a NaN in one channel."""
     torch.manual_seed(sum(shape))
