@@ -36,6 +36,10 @@ int compute_units();
 // whether dq8_observe_fake_quant of an aligned tensor folds the range in its last kernel (minmax.hip)
 bool observe_folds_range(int64_t outer, int64_t channels, int64_t inner);
 
+// what dq8_weight_only_qgemm plans with all the scratch it wants (weight_only.hip): the tile form (-1: a
+// kernel for few rows), k ranges, rows and channels of a tile
+void weight_only_plan(int64_t M, int64_t N, int64_t K, int esz, bool ragged, int plan[4]);
+
 // Dynamic LDS above the default limit has to be allowed per kernel and per device.  `done`
 // is the kernel's bit set of devices (by ordinal) on which that has happened; two threads
 // racing on the first launch both set the attribute, which is harmless.

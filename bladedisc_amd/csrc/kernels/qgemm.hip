@@ -1630,6 +1630,10 @@ extern "C" int dq8_observe_folds_range(int64_t outer, int64_t channels, int64_t 
   return observe_folds_range(outer, channels, inner);
 }
 
+extern "C" void dq8_weight_only_plan(int64_t M, int64_t N, int64_t K, int x_dtype, int ragged, int plan[4]) {
+  weight_only_plan(M, N, K, x_dtype == DQ8_DTYPE_F32 ? 4 : 2, ragged != 0, plan);
+}
+
 extern "C" int dq8_mfma_probe(const int8_t* a, const int8_t* b, int32_t* d32,
                               const int8_t* a16, const int8_t* b16, int32_t* d16,
                               void* stream) {

@@ -1497,17 +1497,14 @@ size_t split_bytes(const SplitPlan& s, int64_t M, int64_t N) {
   return s.splits > 1 ? (size_t)s.splits * (size_t)(M * N) * sizeof(float) : 0;
 }
 
-// The scratch to ask a caller for, who has sizes but no pointers yet: what the plan for aligned rows
-// wants.  Where that plan is unsplit, what the plan for unaligned rows wants, whose k tiles are dearer,
-// or the cheapest split that is within the estimate's error (a tenth on either side): a scratch that
-// was sized once and kept should not depend on which of two near-equal plans the estimate prefers.
-size_t scratch_split_bytes(int64_t M, int64_t N, int64_t K, int esz) {
-  const size_t off16 = split_bytes(choose_tiles(M, N, K, esz, true, 8), M, N);
-  if (K % 16 != 0) return off16;
-  SplitPlan s = choose_tiles(M, N, K, esz, false, 8);
-  if (s.splits > 1 || s.form < 0) return split_bytes(s, M, N);
-  const SplitPlan split = plan_split(M, N, K, esz, false, 2, 8);
-  return std::max(off16, split.form >= 0 && split.us <= 1.2f * s.us ? split_bytes(split, M, N) : 0);
+// The operands' rows are not multiples of 16 bytes, 16-byte aligned.
+bool rows_ragged(const void* x, int esz, int64_t ldx, const void* w, int64_t w_sn, int64_t K) {
+  return !(K % 16 == 0 && aligned(x, 16) && (ldx * esz) % 16 == 0 && aligned(w, 16) && w_sn % 16 == 0);
+}
+
+// (the tiles address their rows by 31-bit byte offsets from the first)
+bool tiles_reach(int64_t ldx, int64_t w_sn, int64_t K) {
+  return 512 * ldx + 4 * K + 4096 < (1LL << 31) && 256 * w_sn + K + 4096 < (1LL << 31);
 }
 
 // one launch of a form over the whole k range (splits == 1) or its split
@@ -1541,10 +1538,7 @@ template <typename XT>
 int launch(WoParams& p, bool fast, void* scratch, size_t scratch_bytes, hipStream_t st) {
   p.partial = nullptr;
   p.k_split = p.K;
-  // (the LDS kernel addresses a tile's rows by 31-bit byte offsets from its first)
-  const bool lds_ok = 512 * p.ldx + 4 * (int64_t)p.K + 4096 < (1LL << 31) &&
-                      256 * p.w_sn + (int64_t)p.K + 4096 < (1LL << 31);
-  if (fast && lds_ok) {
+  if (fast && tiles_reach(p.ldx, p.w_sn, p.K)) {
     const bool have = scratch && aligned(scratch, 16);
     const size_t planes = have ? scratch_bytes / ((size_t)p.M * (size_t)p.N * sizeof(float)) : 0;
     // (unaligned rows whose scratch was sized for aligned ones: as many k ranges as it holds)
@@ -1632,6 +1626,15 @@ int launch(WoParams& p, bool fast, void* scratch, size_t scratch_bytes, hipStrea
 }
 
 }  // namespace
+
+void weight_only_plan(int64_t M, int64_t N, int64_t K, int esz, bool ragged, int plan[4]) {
+  const SplitPlan s = choose_tiles(M, N, K, esz, ragged, 8);
+  plan[0] = s.form;
+  plan[1] = s.splits;
+  plan[2] = s.form < 0 ? 0 : kForms[s.form].bm;
+  plan[3] = s.form < 0 ? 0 : kForms[s.form].bn;
+}
+
 }  // namespace dq8
 
 using namespace dq8;
@@ -1671,15 +1674,30 @@ extern "C" size_t dq8_weight_only_qgemm_workspace_bytes(int64_t N, int64_t K, in
   return (tp_b || N <= 0 || K <= 0) ? 0 : (size_t)(N * K);
 }
 
-extern "C" size_t dq8_weight_only_qgemm_workspace_bytes_ex(int64_t M, int64_t N, int64_t K,
-                                                           int tp_b, int x_dtype) {
+namespace {
+// The [N, K] copy of weights given as [K, N], and the partial sums of the plan that the call then takes.
+size_t scratch_bytes(int64_t M, int64_t N, int64_t K, int tp_b, int x_dtype, bool ragged) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   size_t split = 0;
   if ((x_dtype == DQ8_DTYPE_F16 || x_dtype == DQ8_DTYPE_F32) && K >= 16 && M < (1LL << 31) &&
       N < (1LL << 31) && K < (1LL << 31))
-    split = scratch_split_bytes(M, N, K, x_dtype == DQ8_DTYPE_F32 ? 4 : 2);
+    split = split_bytes(choose_tiles(M, N, K, x_dtype == DQ8_DTYPE_F32 ? 4 : 2, ragged, 8), M, N);
   if (!split) return dq8_weight_only_qgemm_workspace_bytes(N, K, tp_b);
   return transposed_bytes(N, K, tp_b) + split;
+}
+}  // namespace
+
+extern "C" size_t dq8_weight_only_qgemm_workspace_bytes_ex(int64_t M, int64_t N, int64_t K,
+                                                           int tp_b, int x_dtype) {
+  return scratch_bytes(M, N, K, tp_b, x_dtype, K % 16 != 0);
+}
+
+extern "C" size_t dq8_weight_only_qgemm_workspace_bytes_for(const void* x, int x_dtype, int64_t ldx, const void* w,
+                                                            int64_t ldw, int tp_b, int64_t M, int64_t N, int64_t K) {
+  const int64_t w_sn = tp_b ? ldw : K;                     // (the copy's rows follow each other)
+  if (!tiles_reach(ldx, w_sn, K)) return dq8_weight_only_qgemm_workspace_bytes(N, K, tp_b);
+  return scratch_bytes(M, N, K, tp_b, x_dtype,
+                       rows_ragged(x, x_dtype == DQ8_DTYPE_F32 ? 4 : 2, ldx, tp_b ? w : nullptr, w_sn, K));
 }
 
 extern "C" int dq8_weight_only_undo_compiler_layout(const uint8_t* reordered, uint8_t* w_nk,
@@ -1758,7 +1776,7 @@ extern "C" int dq8_weight_only_qgemm(const void* x, int x_dtype, int64_t ldx, co
     }
   }
   fast = fast && p.w_sk == 1;
-  p.ragged = !(K % 16 == 0 && aligned(x, 16) && (ldx * esz) % 16 == 0 && aligned(p.w, 16) && p.w_sn % 16 == 0);
+  p.ragged = rows_ragged(x, esz, ldx, p.w, p.w_sn, K);
   return x_dtype == DQ8_DTYPE_F32 ? launch<float>(p, fast, rest, rest_bytes, st)
                                   : launch<_Float16>(p, fast, rest, rest_bytes, st);
 }

@@ -1019,14 +1019,14 @@ MemRefType<T, N> weightOnlyQgemm(ExecutionContext* ctx, void* stream_handle,
   // (scratch for the transposed copy of a weight that is not cached and for the partial sums of
   // a launch split over k when m is small; handed back to the pool right after the launch,
   // which later work on the same stream is ordered behind)
-  size_t ws_bytes = dq8_weight_only_qgemm_workspace_bytes_ex(m, n, k, tp_b, WoDtype<T>::value);
+  const void* w = w_nk ? static_cast<const void*>(w_nk) : weight.data;
+  size_t ws_bytes = dq8_weight_only_qgemm_workspace_bytes_for(input.data, WoDtype<T>::value, k, w, tp_b ? k : n,
+                                                              tp_b, m, n, k);
   void* ws = ws_bytes ? drv->alloc(ctx, ws_bytes) : nullptr;
   if (!ws) ws_bytes = 0;                                   // (the call then runs unsplit)
   StreamTimer timer(stream);
-  const int st = dq8_weight_only_qgemm(input.data, WoDtype<T>::value, k,
-                                       w_nk ? static_cast<const void*>(w_nk) : weight.data, 0,
-                                       tp_b ? k : n, tp_b, scales.data, zeroPoints.data, bias, data,
-                                       n, m, n, k, ws, ws_bytes, stream);
+  const int st = dq8_weight_only_qgemm(input.data, WoDtype<T>::value, k, w, 0, tp_b ? k : n, tp_b, scales.data,
+                                       zeroPoints.data, bias, data, n, m, n, k, ws, ws_bytes, stream);
   if (ws) drv->dealloc(ctx, ws);
   if (timer.on() && st == 0) {
     const double ns = timer.stop();

@@ -424,7 +424,8 @@ PyObject* py_weight_only(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (THPVariable_Check(a[7])) {
       ws = THPVariable_Unpack(a[7]);
     } else if (truth(a[7])) {
-      const size_t need = dq8_weight_only_qgemm_workspace_bytes_ex(M, N, K, tp_b, xk);
+      const size_t need = dq8_weight_only_qgemm_workspace_bytes_for(in(x), xk, x.stride(0), in(w), w.stride(0), tp_b,
+                                                                    M, N, K);
       if (need) ws = empty({(int64_t)need}, ScalarType::Byte, x.device());
     }
     const size_t ws_bytes = ws.defined() ? ws.nbytes() : 0;

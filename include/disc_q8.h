@@ -388,9 +388,13 @@ size_t dq8_weight_only_qgemm_workspace_bytes(int64_t N, int64_t K, int tp_b);
  * M is too small for the tiles to fill the chip (f32 partial sums and a
  * reduction launch behind the GEMM; the sums of the k ranges are added in their order, so the
  * result does not depend on timing).  Includes the bytes of the function above; with less the
- * call still runs, unsplit. */
+ * call still runs, unsplit.  The first form is for operands whose rows are 16-byte aligned wherever K
+ * allows it; the second is told the operands that will be passed, whose k ranges may be others where
+ * rows start off 16 bytes. */
 size_t dq8_weight_only_qgemm_workspace_bytes_ex(int64_t M, int64_t N, int64_t K, int tp_b,
                                                 int x_dtype);
+size_t dq8_weight_only_qgemm_workspace_bytes_for(const void* x, int x_dtype, int64_t ldx, const void* w,
+                                                 int64_t ldw, int tp_b, int64_t M, int64_t N, int64_t K);
 int dq8_weight_only_qgemm(const void* x, int x_dtype, int64_t ldx, const void* w, int w_signed,
                           int64_t ldw, int tp_b, const void* scale, const int32_t* zero_points,
                           const void* bias, void* out, int64_t ldo, int64_t M, int64_t N,

@@ -55,6 +55,12 @@ int dq8_mfma_probe(const int8_t* a, const int8_t* b, int32_t* d32,
  * the observed range in its last kernel (two launches); otherwise a kernel of its own does. */
 int dq8_observe_folds_range(int64_t outer, int64_t channels, int64_t inner);
 
+/* What dq8_weight_only_qgemm (include/disc_q8.h) plans for a problem when it has all the scratch it
+ * wants: plan[0] the tile form (numbered as in weight_only.hip; -1 where a kernel for few rows runs),
+ * plan[1] the k ranges, plan[2], plan[3] the rows and channels of a tile.  ragged: rows that are not
+ * 16-byte aligned multiples of 16 bytes. */
+void dq8_weight_only_plan(int64_t M, int64_t N, int64_t K, int x_dtype, int ragged, int plan[4]);
+
 #ifdef __cplusplus
 }
 #endif

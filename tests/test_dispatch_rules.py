@@ -1,5 +1,8 @@
 """Which kernels a call gets, where the choice is made from sizes alone: asked of the library on the CPU
 (which then counts 256 compute units)."""
+import ctypes as C
+import random
+
 import pytest
 
 from bladedisc_amd import _lib
@@ -19,3 +22,43 @@ def test_the_observed_range_is_folded_with_the_fake_quantization_where_that_is_s
     L = _lib.hooks()
     assert bool(L.dq8_observe_folds_range(1, channels, inner)) == folds
     assert not L.dq8_observe_folds_range(2, channels, inner)
+
+
+def _weight_only_plan(m, n, k, dtype, ragged=False):
+    plan = (C.c_int * 4)()
+    _lib.hooks().dq8_weight_only_plan(m, n, k, dtype, int(ragged), plan)
+    return dict(form=plan[0], splits=plan[1], bm=plan[2], bn=plan[3])
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+def test_weight_only_scratch_is_what_the_plan_uses(dtype):
+    """The bytes asked for are the partial sums of the plan that the call then takes, none where it is
+    unsplit (1757 x 9360 -> 6560 in f32 asked for 131 MB that nothing used)."""
+    L = _lib.lib()
+    rng = random.Random(dtype)
+    sizes = [(1757, 6560, 9360), (64, 768, 3072), (33, 256, 1024)]
+    for _ in range(400):
+        m, n, k = (int(2 ** rng.uniform(low, 11.5)) for low in (0, 0, 5))
+        sizes.append((m, n, max(16, 2 * k) // 16 * 16 if rng.random() < 0.7 else 2 * k))
+    split = 0
+    for m, n, k in sizes:
+        want = {}
+        for ragged in (False, True):
+            plan = _weight_only_plan(m, n, k, dtype, ragged)
+            want[ragged] = 4 * m * n * plan["splits"] if plan["splits"] > 1 else 0
+            if k < 16:
+                want[ragged] = 0
+        esz = 2 if dtype else 4
+        assert L.dq8_weight_only_qgemm_workspace_bytes_ex(m, n, k, 1, dtype) == want[k % 16 != 0], (m, n, k)
+        # aligned operands; activations and weights off 16 bytes; rows off 16 bytes
+        for x, ldx, w, ldw, ragged in ((256, k, 512, k, k % 16 != 0), (256 + esz, k, 512, k, True),
+                                       (256, k, 513, k, True), (256, k + 1, 512, k, True), (256, k, 512, k + 1, True)):
+            got = L.dq8_weight_only_qgemm_workspace_bytes_for(x, dtype, ldx, w, ldw, 1, m, n, k)
+            assert got == want[ragged], (m, n, k, ldx, ldw)
+        # weights as [K, N]: their copy in front, which is aligned wherever K is
+        got = L.dq8_weight_only_qgemm_workspace_bytes_for(256, dtype, k, 513, n, 0, m, n, k)
+        assert got == ((n * k + 255) // 256 * 256 + want[k % 16 != 0] if want[k % 16 != 0] else n * k)
+        split += want[k % 16 != 0] > 0
+    assert split >= 40 and split < 300
+    # operands that the tiles cannot address run without a split
+    assert L.dq8_weight_only_qgemm_workspace_bytes_for(256, dtype, 1 << 23, 512, 3072, 1, 64, 768, 3072) == 0
