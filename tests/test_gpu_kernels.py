@@ -1717,6 +1717,39 @@ def _weight_only_case(rng, m, k, n, dtype, signed):
     return x, w, scale, zp, bias
 
 
+def _weight_only_plan(m, n, k, dtype, ragged=False):
+    """(tile form, k ranges) of a weight-only product that has all the scratch it wants."""
+    import ctypes as C
+    import bladedisc_amd._lib as _lib
+    plan = (C.c_int * 4)()
+    _lib.hooks().dq8_weight_only_plan(m, n, k, 1 if dtype == torch.float16 else 0, int(ragged), plan)
+    return plan[0], plan[1]
+
+
+def _weight_only_raw(x, w, scale, zp, bias, out, ws, ws_bytes):
+    """The C entry on device matrices whose rows may be pieces of wider ones, the weights' too (which
+    kernels.weight_only_qgemm makes contiguous first)."""
+    import bladedisc_amd._lib as _lib
+    L = _lib.lib()
+    (m, k), n = x.shape, w.shape[0]
+    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    _lib.check(L.dq8_weight_only_qgemm(
+        ptr(x), 1 if x.dtype == torch.float16 else 0, x.stride(0), ptr(w), int(w.dtype == torch.int8), w.stride(0), 1,
+        ptr(scale), ptr(zp), ptr(bias), ptr(out), out.stride(0), m, n, k, ptr(ws), ws_bytes,
+        torch.cuda.current_stream().cuda_stream), "dq8_weight_only_qgemm")
+
+
+def _weight_only_framed(x, w, dtype, signed):
+    """Device copies of both operands inside wider buffers of NaN / the largest byte."""
+    (m, k), n = x.shape, w.shape[0]
+    wide_x = torch.full((m + 1, k + 16), float("nan"), dtype=dtype, device="cuda")
+    wide_x[:m, :k] = dev(x)
+    wide_w = torch.full((n + 1, k + 16), -1 if signed else 255, dtype=torch.int8 if signed else torch.uint8,
+                        device="cuda")
+    wide_w[:n, :k] = dev(w)
+    return wide_x[:m, :k], wide_w[:n, :k]
+
+
 def _weight_only_check(got, x, w, scale, zp, bias, dtype):
     """|error| <= accumulation bound: products are exact in f32 (half activations; f32 ones
     enter as two halves, 2^-21 relative -- or 2^-25 absolute per activation where the low
@@ -1882,12 +1915,14 @@ def test_weight_only_qgemm_split_over_k(K, dtype):
     code = 1 if dtype == torch.float16 else 0
     split_seen = 0
     for (m, k, n) in [(33, 1024, 256), (64, 3072, 768), (100, 2064, 130), (128, 4096, 1024),
-                      (200, 1040, 333), (512, 2048, 640), (48, 1536, 4096)]:
+                      (200, 1040, 333), (512, 2048, 640), (48, 1536, 4096), (70, 4112, 520),
+                      (40, 3600, 203)]:
         x, w, scale, zp, bias = _weight_only_case(rng, m, k, n, dtype, signed=False)
         plain = L.dq8_weight_only_qgemm_workspace_bytes(n, k, 1)
         need = L.dq8_weight_only_qgemm_workspace_bytes_ex(m, n, k, 1, code)
-        assert plain == 0 and need % (4 * m * n) == 0
-        split_seen += need > 0
+        splits = _weight_only_plan(m, n, k, dtype)[1]
+        assert plain == 0 and need == (4 * m * n * splits if splits > 1 else 0)
+        split_seen += splits > 1
         args = (dev(x), dev(w), dev(scale), dev(zp), dev(bias))
         got = K.weight_only_qgemm(*args)
         _weight_only_check(got, x, w, scale, zp, bias, dtype)
@@ -1899,6 +1934,7 @@ def test_weight_only_qgemm_split_over_k(K, dtype):
             ws = torch.empty(need + 4096, dtype=torch.uint8, device="cuda")
             ws.fill_(0xff)                                   # (NaN patterns: nothing may leak)
             assert torch.equal(K.weight_only_qgemm(*args, workspace=ws), got)
+            assert bool((ws[:need].view(torch.int32) != -1).any()) and bool((ws[need:] == 0xff).all())
             assert torch.equal(K.weight_only_qgemm(*args, workspace=ws), got)
             # a scratch that is too small for the partial sums: the unsplit kernels
             assert torch.equal(K.weight_only_qgemm(*args, workspace=ws[:need - 16]), unsplit)
@@ -1951,18 +1987,49 @@ def test_weight_only_qgemm_tiles_loaded_into_lds(K, dtype, m, k, n, signed):
     and weights past the rows and the k range are NaN / 255, so that nothing outside may be used."""
     rng = np.random.default_rng(m + k + n)
     x, w, scale, zp, bias = _weight_only_case(rng, m, k, n, dtype, signed)
-    wide_x = torch.full((m + 1, k + 16), float("nan"), dtype=dtype, device="cuda")
-    wide_x[:m, :k] = dev(x)
-    wide_w = torch.full((n + 1, k + 16), -1 if signed else 255, dtype=torch.int8 if signed else torch.uint8,
-                        device="cuda")
-    wide_w[:n, :k] = dev(w)
+    wide_x, wide_w = _weight_only_framed(x, w, dtype, signed)
+    splits = _weight_only_plan(m, n, k, dtype)[1]
+    ws = torch.empty(max(4 * m * n * splits, 16), dtype=torch.uint8, device="cuda")
     frame = torch.full((m + 1, n + 5), 7.0, dtype=dtype, device="cuda")
     out = frame[:m, 1:n + 1]
-    K.weight_only_qgemm(wide_x[:m, :k], wide_w[:n, :k], dev(scale), dev(zp), dev(bias), out=out)
+    _weight_only_raw(wide_x, wide_w, dev(scale), dev(zp), dev(bias), out, ws, ws.nbytes)
     _weight_only_check(out, x, w, scale, zp, bias, dtype)
     assert bool((frame[:, 0] == 7).all()) and bool((frame[:, n + 1:] == 7).all()) and bool((frame[m] == 7).all())
     got = K.weight_only_qgemm(dev(x), dev(w), dev(scale), workspace=False)
     _weight_only_check(got, x, w, scale, None, None, dtype)
+
+
+@pytest.mark.parametrize("dtype,m,k,n,form,splits", [
+    (torch.float16, 33, 2064, 34, 0, 7), (torch.float16, 34, 7568, 1377, 1, 8), (torch.float16, 36, 7968, 4134, 2, 6),
+    (torch.float16, 66, 6240, 5481, 3, 4), (torch.float16, 129, 5456, 6579, 4, 2),
+    (torch.float16, 259, 7856, 6602, 5, 3),
+    (torch.float32, 33, 2096, 33, 6, 7), (torch.float32, 33, 2192, 2727, 7, 4), (torch.float32, 67, 6640, 5523, 8, 8),
+    (torch.float32, 33, 4752, 5469, 9, 4), (torch.float32, 66, 7344, 5614, 10, 4),
+    # rows off 16 bytes
+    (torch.float16, 33, 1131, 33, 11, 4), (torch.float16, 67, 4763, 4230, 12, 6)])
+def test_weight_only_qgemm_every_tile_form_split_over_k(K, dtype, m, k, n, form, splits):
+    """Every tile form with the k range split (the form and the ranges are asserted): M and N off the
+    tile, ranges that begin at odd multiples of 64, a last range that ends inside a k tile, operands in
+    frames of NaN / 255, a scratch of exactly the partial sums, filled with NaN patterns, and nothing
+    written behind it or beside the results."""
+    ragged = k % 16 != 0
+    assert _weight_only_plan(m, n, k, dtype, ragged) == (form, splits)
+    rng = np.random.default_rng(m + k + n)
+    x, w, scale, zp, bias = _weight_only_case(rng, m, k, n, dtype, signed=bool(form & 1))
+    wide_x, wide_w = _weight_only_framed(x, w, dtype, bool(form & 1))
+    need = 4 * m * n * splits
+    ws = torch.full((need + 4096,), 0xff, dtype=torch.uint8, device="cuda")
+    frame = torch.full((m + 1, n + 5), 7.0, dtype=dtype, device="cuda")
+    out = frame[:m, 1:n + 1]
+    _weight_only_raw(wide_x, wide_w, dev(scale), dev(zp), dev(bias), out, ws, need)
+    _weight_only_check(out, x, w, scale, zp, bias, dtype)
+    assert bool((frame[:, 0] == 7).all()) and bool((frame[:, n + 1:] == 7).all()) and bool((frame[m] == 7).all())
+    assert bool((ws[need:] == 0xff).all())
+    planes = ws[:need].view(torch.float32).reshape(splits, m, n)
+    assert bool(torch.isfinite(planes).all())
+    first = out.clone()
+    _weight_only_raw(wide_x, wide_w, dev(scale), dev(zp), dev(bias), out, ws, need)
+    assert torch.equal(out, first)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
@@ -2017,7 +2084,8 @@ def test_multi_kernel_paths_replay_from_a_captured_graph(K):
     import bladedisc_amd._lib as _lib
     L = _lib.lib()
     rng = np.random.default_rng(808)
-    m, k, n = 128, 2048, 512
+    m, k, n = 64, 3072, 768
+    assert _weight_only_plan(m, n, k, torch.float16)[1] > 1
     x, w, scale, zp, bias = _weight_only_case(rng, m, k, n, torch.float16, False)
     xd, wd, sd, zd, bd = dev(x), dev(w), dev(scale), dev(zp), dev(bias)
     need = L.dq8_weight_only_qgemm_workspace_bytes_ex(m, n, k, 1, 1)
