@@ -61,9 +61,6 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef unsigned u4 __attribute__((ext_vector_type(4)));
 
-// gfx9 raw buffer descriptor word 3: 32-bit data format, no swizzle
-constexpr int kBufferWord3 = 0x00020000;
-
 struct WoParams {
   const void* x;        // [M, K] activations, row stride ldx elements
   const uint8_t* w;     // weights; element (n, k) at w[n * w_sn + k * w_sk]
@@ -493,9 +490,9 @@ __global__ void __launch_bounds__(WM * 128, 2) wo_ragged_kernel(const WoParams p
 //    over the MFMAs.  Sent out together behind the barrier, the loads of all waves queue at the
 //    compute unit's address path (25 clocks apiece), the reads at the LDS, and every wave's MFMAs
 //    behind them;
-//  * one barrier per k tile, in the middle of the wave's last 32-deep unit of it: by then all
-//    fragments of the tile are in registers, its stage takes the tile NST further on, and the next
-//    tile's first fragments are read under the unit's second half.
+//  * a wave takes one 32-deep unit of every k tile (BK = 32 KG), and there is one barrier per k tile, in the
+//    middle of it: by then all fragments of the tile are in registers, its stage takes the tile NST
+//    further on, and the next tile's fragments are read under the unit's second half.
 // The sums of the k groups meet in LDS at the end, which also puts the results into whole rows.
 // f32 activations stay f32 in LDS; a wave splits the fragments it reads (hi = half(x), lo = half(x
 // - hi)) and multiplies both.
@@ -528,11 +525,11 @@ __global__ void __launch_bounds__(NCG* KG * 64, 2) wo_dma_kernel(const WoParams 
   constexpr int WR = 1024 / BK;                          // weight rows per load
   constexpr int A_LD = SUBS * (BM / 8) / NW, W_LD = (BN / WR) / NW, LD = A_LD + W_LD;
   constexpr int A_BYTES = BM * 128 * SUBS, STAGE = Shape::kStage;
-  constexpr int U = BK / 32 / KG;                              // 32-deep units of a k tile per wave
   constexpr int CH = F32 ? 2 : 1;                        // 16-byte chunks of an activation row per 16 of k and lane
   constexpr unsigned kFlip = SIGNED ? 0x80808080u : 0u;
   constexpr int kPast = (int)0x80000000;                 // an offset no descriptor covers
-  static_assert((BK == 64 || BK == 128) && U >= 1 && STAGE == A_BYTES + BN * BK && Shape::kLds <= 160 * 1024, "LDS");
+  static_assert((BK == 64 || BK == 128) && BK == 32 * KG, "a wave takes one 32-deep unit of a k tile");
+  static_assert(STAGE == A_BYTES + BN * BK && Shape::kLds <= 160 * 1024, "LDS");
   static_assert((SUBS * (BM / 8)) % NW == 0 && (BM / 8) % 2 == 0 && NW % 2 == 0, "loads of a wave");
   static_assert((BN / WR) % NW == 0 && NST * LD <= 63, "loads of a wave; vmcnt is a 6-bit counter");
   extern __shared__ __attribute__((aligned(1024))) uint8_t wo_lds[];
@@ -605,29 +602,27 @@ __global__ void __launch_bounds__(NCG* KG * 64, 2) wo_dma_kernel(const WoParams 
   // ---- fragments: row r of a 32-row block, 16 values of k from 16 g of a 32-deep unit on
   const int swz = (r & 7) ^ ((r >> 3) & 1);
   const int row_off = (r >> 3) * 1024 + (r & 7) * 128;
-  int a_off[U][2 * CH], w_off[U];
+  int a_off[2 * CH];
+  {
+    const int sub = F32 ? kg : kg >> 1, first = F32 ? 4 * g : 4 * (kg & 1) + 2 * g;
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int unit = kg * U + u;
-    const int sub = F32 ? unit : unit >> 1, first = F32 ? 4 * g : 4 * (unit & 1) + 2 * g;
-#pragma unroll
-    for (int h = 0; h < 2 * CH; ++h) a_off[u][h] = sub * BM * 128 + row_off + (((first + h) ^ swz) << 4);
-    w_off[u] = A_BYTES + cg * 64 * BK + (BK == 128 ? row_off + (((2 * unit + g) ^ swz) << 4)
-                                                   : r * 64 + (((2 * unit + g) ^ ((r >> 2) & 3)) << 4));
+    for (int h = 0; h < 2 * CH; ++h) a_off[h] = sub * BM * 128 + row_off + (((first + h) ^ swz) << 4);
   }
+  const int w_off = A_BYTES + cg * 64 * BK + (BK == 128 ? row_off + (((2 * kg + g) ^ swz) << 4)
+                                                        : r * 64 + (((2 * kg + g) ^ ((r >> 2) & 3)) << 4));
   h2 c[2];
   u4 fa[2][FM][CH];                  // activations of the unit's two 16-deep steps
-  u4 fw[2][2];                       // weights of this unit and the next: both steps
+  u4 fw[2][2];                       // weights of this k tile and the next: both steps
   h8 w[2][2];                        // widened: of this step and the next
   // read q of a unit's fragments: the weights, then the activations of row block (q - 2) / (2 CH)
   constexpr int READS = 2 + FM * 2 * CH;
-  auto read = [&](auto set_c, auto u_c, auto q_c, const uint8_t* base) {
-    constexpr int set = decltype(set_c)::value, u = decltype(u_c)::value, q = decltype(q_c)::value;
+  auto read = [&](auto set_c, auto q_c, const uint8_t* base) {
+    constexpr int set = decltype(set_c)::value, q = decltype(q_c)::value;
     if constexpr (q < 2) {
-      fw[set][q] = *reinterpret_cast<const u4*>(base + w_off[u] + q * 32 * BK);
+      fw[set][q] = *reinterpret_cast<const u4*>(base + w_off + q * 32 * BK);
     } else {
       constexpr int i = (q - 2) / (2 * CH), h = (q - 2) % (2 * CH);
-      fa[h / CH][i][h % CH] = *reinterpret_cast<const u4*>(base + a_off[u][h] + i * 4096);
+      fa[h / CH][i][h % CH] = *reinterpret_cast<const u4*>(base + a_off[h] + i * 4096);
     }
   };
   auto widen = [&](auto set_c, auto s_c, int j) {
@@ -708,67 +703,51 @@ __global__ void __launch_bounds__(NCG* KG * 64, 2) wo_dma_kernel(const WoParams 
     const _Float16 v = (_Float16)(float)(1024 + zp + (SIGNED ? 128 : 0));
     c[j] = (h2){v, v};
   }
-  static_for_n<READS>([&](auto q_c) { read(Int<0>(), Int<0>(), q_c, wo_lds); });
+  static_for_n<READS>([&](auto q_c) { read(Int<0>(), q_c, wo_lds); });
   widen(Int<0>(), Int<0>(), 0);
   widen(Int<0>(), Int<0>(), 1);
 
-  // Tile t's stage is free from the middle of its last unit on and takes tile t + NST, whose loads
-  // are dealt out from there to the same place of tile t + 1: over that unit's second step (SLOT 0)
-  // and the 2 U - 1 steps behind it.
+  // Tile t's stage is free from its middle on and takes tile t + NST, whose loads are dealt out from
+  // there to the middle of tile t + 1: over this tile's second step (SLOT 0 on) and the next one's first.
   auto spread = [&](auto count_c, auto slots_c, auto slot_c, auto&& body) {
     constexpr int count = decltype(count_c)::value, slots = decltype(slots_c)::value, slot = decltype(slot_c)::value;
     static_for_n<count>([&](auto l_c) {
       if constexpr (decltype(l_c)::value * slots / count == slot) body(l_c);
     });
   };
-  constexpr int SLOTS = 2 * U * FM;
+  constexpr int SLOTS = 2 * FM;
   int st = 0;                                            // tile t's stage
-  // one k tile; PAR: the set its first unit's weights are in; MORE: the tiles loaded meanwhile are there, and whole
+  // one k tile; PAR: the set its weights are in; MORE: the tiles loaded meanwhile are there, and whole
   auto k_tile = [&](auto more_c, auto par_c, int t) {
     constexpr int MORE = decltype(more_c)::value, PAR = decltype(par_c)::value;
+    using Next = Int<PAR ^ 1>;
     const int pst = st == 0 ? NST - 1 : st - 1, nst = st + 1 == NST ? 0 : st + 1;
-    const uint8_t* here = wo_lds + st * STAGE;
     const uint8_t* there = wo_lds + nst * STAGE;
     const bool next = MORE || t + 1 < KT;                // (uniform)
-    static_for_n<U>([&](auto u_c) {
-      constexpr int u = decltype(u_c)::value;
-      constexpr bool last = u == U - 1;
-      using Set = Int<(PAR + u) & 1>;
-      using Next = Int<(PAR + u + 1) & 1>;
-      step(Int<0>(), Set(), [&](auto i_c) {
-        if (MORE || (t > 0 && t - 1 + NST < KT))
-          spread(Int<LD>(), Int<SLOTS>(), Int<(1 + 2 * u) * FM + decltype(i_c)::value>(),
-                 [&](auto l_c) { issue_load(Int<MORE>(), l_c, t - 1 + NST, pst); });
-      });
-      if constexpr (last) {
-        if (next) {
-          if constexpr (MORE)
-            __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0((NST - 2) * LD));
-          else
-            landed(min(KT - 2 - t, NST - 2));
-          __syncthreads();                               // tile t + 1 is in LDS; tile t is in registers
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      step(Int<1>(), Next(), [&](auto i_c) {
-        constexpr int i = decltype(i_c)::value;
-        // the next unit's fragments: the weights ahead of the others, a row block's activations behind
-        // its MFMAs, in their registers
-        if (!last || next)
-          static_for_n<READS>([&](auto q_c) {
-            constexpr int q = decltype(q_c)::value;
-            if constexpr (q < 2 ? i == 0 : (q - 2) / (2 * CH) == i)
-              read(Next(), Int<last ? 0 : u + 1>(), q_c, last ? there : here);
-          });
-        if constexpr (last) {
-          if (MORE || t + NST < KT)
-            spread(Int<LD>(), Int<SLOTS>(), i_c, [&](auto l_c) { issue_load(Int<MORE>(), l_c, t + NST, st); });
-        } else {
-          if (MORE || (t > 0 && t - 1 + NST < KT))
-            spread(Int<LD>(), Int<SLOTS>(), Int<(2 + 2 * u) * FM + i>(),
-                   [&](auto l_c) { issue_load(Int<MORE>(), l_c, t - 1 + NST, pst); });
-        }
-      });
+    step(Int<0>(), Int<PAR>(), [&](auto i_c) {
+      if (MORE || (t > 0 && t - 1 + NST < KT))
+        spread(Int<LD>(), Int<SLOTS>(), Int<FM + decltype(i_c)::value>(),
+               [&](auto l_c) { issue_load(Int<MORE>(), l_c, t - 1 + NST, pst); });
+    });
+    if (next) {
+      if constexpr (MORE)
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0((NST - 2) * LD));
+      else
+        landed(min(KT - 2 - t, NST - 2));
+      __syncthreads();                                   // tile t + 1 is in LDS; tile t is in registers
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    step(Int<1>(), Next(), [&](auto i_c) {
+      constexpr int i = decltype(i_c)::value;
+      // the next tile's fragments: the weights ahead of the others, a row block's activations behind
+      // its MFMAs, in their registers
+      if (next)
+        static_for_n<READS>([&](auto q_c) {
+          constexpr int q = decltype(q_c)::value;
+          if constexpr (q < 2 ? i == 0 : (q - 2) / (2 * CH) == i) read(Next(), q_c, there);
+        });
+      if (MORE || t + NST < KT)
+        spread(Int<LD>(), Int<SLOTS>(), i_c, [&](auto l_c) { issue_load(Int<MORE>(), l_c, t + NST, st); });
     });
     st = nst;
   };
@@ -777,20 +756,15 @@ __global__ void __launch_bounds__(NCG* KG * 64, 2) wo_dma_kernel(const WoParams 
   const int whole = klen / BK - NST;
   k_tile(Int<0>(), Int<0>(), 0);
   int t = 1;
-  if constexpr (U % 2 == 0) {
-    for (; t < whole; ++t) k_tile(Int<1>(), Int<0>(), t);
-    for (; t < KT; ++t) k_tile(Int<0>(), Int<0>(), t);
-  } else {
-    for (; t + 1 < whole; t += 2) {
-      k_tile(Int<1>(), Int<1>(), t);
-      k_tile(Int<1>(), Int<0>(), t + 1);
-    }
-    for (; t + 1 < KT; t += 2) {
-      k_tile(Int<0>(), Int<1>(), t);
-      k_tile(Int<0>(), Int<0>(), t + 1);
-    }
-    if (t < KT) k_tile(Int<0>(), Int<1>(), t);
+  for (; t + 1 < whole; t += 2) {
+    k_tile(Int<1>(), Int<1>(), t);
+    k_tile(Int<1>(), Int<0>(), t + 1);
   }
+  for (; t + 1 < KT; t += 2) {
+    k_tile(Int<0>(), Int<1>(), t);
+    k_tile(Int<0>(), Int<0>(), t + 1);
+  }
+  if (t < KT) k_tile(Int<0>(), Int<1>(), t);
 
   if constexpr (F32) {
 #pragma unroll
@@ -1018,7 +992,7 @@ __global__ void __launch_bounds__(NW * 64) wo_gemv_kernel(const WoParams p) {
   __syncthreads();
   if (n >= p.N) return;                                  // (no barrier below)
   const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t*>(p.w + (int64_t)n * p.w_sn), 0, p.K, kBufferWord3);
+      const_cast<uint8_t*>(p.w + (int64_t)n * p.w_sn), 0, p.K, kBufferRsrcWord3);
   const h2 c = centre(p, n);
   float acc[MR];
 #pragma unroll
@@ -1106,10 +1080,10 @@ __global__ void __launch_bounds__(kRowsWaves * 64) wo_rows_kernel(const WoParams
   // checked that the byte offsets fit 31 bits
   const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<void*>(p.x), 0, (int)(((int64_t)(mrows - 1) * p.ldx + p.K) * sizeof(XT)),
-      kBufferWord3);
+      kBufferRsrcWord3);
   const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint8_t*>(p.w + (int64_t)n0 * p.w_sn), 0,
-      (int)((int64_t)(nrows - 1) * p.w_sn + p.K), kBufferWord3);
+      (int)((int64_t)(nrows - 1) * p.w_sn + p.K), kBufferRsrcWord3);
   constexpr int kPast = (int)0x80000000;                 // an offset no descriptor covers
 
   // global -> LDS assignment
