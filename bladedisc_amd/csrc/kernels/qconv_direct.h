@@ -44,6 +44,7 @@ struct DirectConvParams {
   int patch_pitch;      // (streaming kernel) pixels per patch row in LDS: Wo + Kw - 1 rounded up to 16
   unsigned wo_inv;      // (streaming kernel) floor(2^32 / Wo) + 1: pixel / Wo == umulhi(pixel, wo_inv)
   int slice_n;          // (streaming kernel) output channels per workgroup
+  int cus;              // (streaming kernel) compute units of the device
   int tiles_per_image;  // ceil(Ho * Wo / BM)
   int tiles_n;          // ceil(Co / BN)
   int patch_bytes;      // LDS reserved for the patch: (most rows a tile spans + Kh - 1) *

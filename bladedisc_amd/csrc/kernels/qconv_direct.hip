@@ -126,7 +126,8 @@ bool stream_conv_plan(DirectConvParams* p) {
   const int64_t pitch = (p->Wo + p->Kw - 1 + 15) / 16 * 16;
   const int64_t tiles_n = ceil_div(p->Co, ns);
   const int64_t per_cu = paired ? 2 : 1;                   // workgroups a compute unit holds
-  const int64_t cus = compute_units() * per_cu;
+  p->cus = compute_units();
+  const int64_t cus = p->cus * per_cu;
   const int fixed = kLdsBytes / (int)per_cu - stream_conv_weight_lds(K, ns) - stream_conv_cp_bytes(ns);
   // Time of a launch in cycles of a SIMD: rounds of workgroups x (blocks of 32 pixels of the
   // busiest SIMD -- it runs waves 0 and 4, which take blocks 0, 8, ... and 4, 12, ... -- each K / 32

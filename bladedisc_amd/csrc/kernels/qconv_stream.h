@@ -119,9 +119,11 @@ __global__ void __launch_bounds__(512, stream_conv_paired(KH, KW, CI, NS, POST) 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   // Blocks go to the waves in turn, so the first waves have one more of them where 8 does not divide
-  // the blocks; wave w runs on SIMD w % 4.  The second workgroup of a compute unit (256 further on, where
-  // two fit) starts one wave on, so that the two workgroups' longer waves do not meet on one SIMD.
-  const int wave = __builtin_amdgcn_readfirstlane(((tid >> 6) + (int)(blockIdx.x >> 8)) & 7);
+  // the blocks; wave w runs on SIMD w % 4.  Where two workgroups share a compute unit, the second (as
+  // many further on as there are units) starts one wave on, so that the longer waves of the two do not
+  // meet on one SIMD.
+  const int turn = stream_conv_paired(KH, KW, CI, NS, POST) ? (int)blockIdx.x / p.cus : 0;
+  const int wave = __builtin_amdgcn_readfirstlane(((tid >> 6) + turn) & 7);
   const EpiParams& e = p.epi;
 
   // workgroup -> (pixel tile, channel slice): consecutive workgroups go to the 8 XCDs in turn,
