@@ -53,42 +53,41 @@ __device__ __forceinline__ uint32_t quant4_by_constants(const float4& v, const f
   return finish4_quotients<ROUND>(make_float4(q.x + z.x, q.y + z.y, q.z + z.z, q.w + z.w), lo, hi);
 }
 
-// The sweeps take pieces of 1024 groups whatever U, piece j on the accelerator die j % 8 (workgroups go to
-// the eight in turn; the 4 / U of a piece are eight apart): what one of them has just written the next one,
-// on the other type's U, finds in its die's L2.  With pieces of U * kThreads quantize and dequantize of
-// 1928 x 2451 f16 through int16 in one buffer took 12.9 us, 10.2 before there was a sweep.
-constexpr int kPiece = 4 * kThreads;
+// Workgroups go to the eight accelerator dies in turn.  The sweeps take chunks of kThreads groups of four,
+// chunk j on die j % 8 whatever the type and however many chunks a thread takes (kHop groups apart): what
+// one of them has just written the next one finds in its die's L2, and one chunk to a workgroup is the
+// plain linear order.  Quantize and dequantize in one buffer, us, with contiguous chunks / with these, f32
+// through int8: 1000 x 3072 11.6 / 8.8, 2000 x 3072 20.6 / 9.7, 5400 x 3072 31.9 / 28.3, 8000 x 3072 41.5 /
+// 40.2; f16 through int8 3000 x 3072 17.8 / 11.4.
+constexpr int kHop = 8 * kThreads;
 template <int U>
 __device__ __forceinline__ uint32_t sweep_first_group() {
-  constexpr uint32_t R = 4 / U;
-  const uint32_t b = blockIdx.x, piece = b / (8 * R) * 8 + b % 8, part = b / 8 % R;
-  return piece * kPiece + part * (U * kThreads) + threadIdx.x;
+  const uint32_t b = blockIdx.x;
+  return (U == 1 ? b : b / 8 * (8 * U) + b % 8) * kThreads + threadIdx.x;
 }
 template <int U>
 unsigned sweep_workgroups(int64_t n) {           // (one group more: the elements behind the last four)
-  const int64_t pieces = dq8::ceil_div(n / 4 + 1, (int64_t)kPiece);
-  return (unsigned)(U == 4 ? pieces : dq8::ceil_div(pieces, 8) * 8 * (4 / U));
+  const int64_t chunks = dq8::ceil_div(n / 4 + 1, (int64_t)kThreads);
+  return (unsigned)(U == 1 ? chunks : dq8::ceil_div(chunks, (int64_t)(8 * U)) * 8);
 }
+// The 8-bit results of a tensor that the eight L2s, 4 MiB each, can still hold in part when the next
+// operator reads them.  (Beyond, dequantize's two chunks next to each other: 16000 x 3072 34.6 us, 35.0 with
+// them kHop apart.)
+inline bool l2s_hold(int64_t n) { return n <= (1 << 25); }
 
 // ---------------------------------------------------------------- per tensor
-// The 8-bit kernels walk the same pieces where the L2 holds what they leave: quantize and dequantize in
-// one buffer, f32 through int8, 1500 x 3072 11.2 -> 8.9 us, 3000 x 3072 16.4 -> 15.6 (from f16 19.5 -> 12.9),
-// 5000 x 3072 25.1 -> 24.4; 8000 x 3072 40.4 -> 40.8, and below four million elements the launches are all
-// there is (2.8 -> 2.9 at two million on buffers that change).
-inline bool pieces_pay(int64_t n) { return n >= (1 << 22) && n <= (1 << 24); }
-
 // One unit per thread and a grid that covers the tensor in one sweep (the loop only
 // runs again beyond 2^30 units): on this part a linear sweep by many small workgroups
 // reaches more of the HBM bandwidth than fewer workgroups that each keep several
 // far-apart streams in flight (measured on 1 GiB of f32: 6.2 TB/s against 4.7-5.2).
-template <int ROUND, bool PIECES>
+template <int ROUND>
 __global__ void __launch_bounds__(kThreads)
 quantize_tensor_v4(const float4* __restrict__ x, uint32_t* __restrict__ out,
                    int64_t n, const float* __restrict__ scale,
                    const int32_t* __restrict__ zp, float lo, float hi) {
   const int64_t n4 = n >> 2;
   const int64_t stride = (int64_t)gridDim.x * kThreads;
-  int64_t i = PIECES ? (int64_t)sweep_first_group<1>() : (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   if (i < n4) {
     // The data load goes out first: a wave has one load to make, and behind the scalar loads of
     // the parameters and the reciprocal it would start a cache miss later.
@@ -128,9 +127,9 @@ __device__ __forceinline__ float4 dequant_word4(uint32_t w, const int4& z, const
                      (float)(b.z - z.z) * s.z, (float)(b.w - z.w) * s.w);
 }
 
-// Two 4-byte words in, two 16-byte stores out per thread, one sweep.  A workgroup covers 512
-// consecutive words and a thread takes words t and t + 256 of them, so that every load and
-// store instruction of a wave covers one contiguous span (64 x 16 bytes per store).  With the
+// Two 4-byte words in, two 16-byte stores out per thread, one sweep.  A workgroup covers two chunks of
+// 256 consecutive words, HOP words apart (kThreads or kHop), and a thread takes word t of each, so that
+// every load and store instruction of a wave covers one contiguous span (64 x 16 bytes per store).  With the
 // two words of a thread next to each other (one 8-byte load, stores 32 bytes apart between
 // neighbouring lanes) tensors that fit the last-level cache ran a quarter slower:
 // [4096,768] 5.35 -> 4.3 us, [32,56,56,64] 8.1 -> 6.1 us, [65536,4096] 221 -> 210 us.
@@ -138,7 +137,7 @@ __device__ __forceinline__ float4 dequant_word4(uint32_t w, const int4& z, const
 // [4096,768] 4.37 -> 3.35 us, [32,56,56,64] 6.3 -> 5.1 us, [65536,4096] 216 -> 187 us, which
 // is 7.2 TB/s; the same hint on the loads made every size slower, and on quantize's stores (a
 // fifth of its traffic) it helped some sizes and hurt others, so neither is used.
-template <bool SIGNED, bool PIECES>
+template <bool SIGNED, int HOP>
 __global__ void __launch_bounds__(kThreads)
 dequantize_tensor_v4x2(const uint32_t* __restrict__ q, float4* __restrict__ out,
                        int64_t n, const float* __restrict__ scale,
@@ -147,13 +146,13 @@ dequantize_tensor_v4x2(const uint32_t* __restrict__ q, float4* __restrict__ out,
   const int z = zp[0];
   const int64_t n4 = n >> 2;
   const int64_t stride = (int64_t)gridDim.x * (2 * kThreads);
-  for (int64_t i = PIECES ? (int64_t)sweep_first_group<2>() : (int64_t)blockIdx.x * (2 * kThreads) + threadIdx.x; i < n4;
-       i += stride) {
-    const bool two = i + kThreads < n4;
+  for (int64_t i = HOP == kHop ? (int64_t)sweep_first_group<2>() : (int64_t)blockIdx.x * (2 * kThreads) + threadIdx.x;
+       i < n4; i += stride) {
+    const bool two = i + HOP < n4;
     const uint32_t w0 = q[i];
-    const uint32_t w1 = two ? q[i + kThreads] : 0u;
+    const uint32_t w1 = two ? q[i + HOP] : 0u;
     dq8::st_stream(&out[i], dequant_word<SIGNED>(w0, z, s));
-    if (two) dq8::st_stream(&out[i + kThreads], dequant_word<SIGNED>(w1, z, s));
+    if (two) dq8::st_stream(&out[i + HOP], dequant_word<SIGNED>(w1, z, s));
   }
   if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {        // the elements behind the last word
     const int64_t e = 4 * n4 + threadIdx.x;
@@ -255,6 +254,17 @@ quantize_rows_v4(const float4* __restrict__ x, uint32_t* __restrict__ out,
           ? quant4_by_constant<ROUND>(v, s, 1.0f / s, z, lo, hi)
           : pack4(quant_one<ROUND>(v.x, s, z, lo, hi), quant_one<ROUND>(v.y, s, z, lo, hi),
                   quant_one<ROUND>(v.z, s, z, lo, hi), quant_one<ROUND>(v.w, s, z, lo, hi));
+}
+
+// The grid of the row kernels: a workgroup per UNIT * kThreads groups of four of a row.
+struct RowsGrid {
+  unsigned x, y;
+  int64_t z;
+};
+template <int UNIT>
+RowsGrid rows_grid(int64_t rows, int64_t inner4) {
+  const unsigned y = (unsigned)std::min<int64_t>(rows, 32768);
+  return {(unsigned)dq8::ceil_div(inner4, UNIT * kThreads), y, dq8::ceil_div(rows, y)};
 }
 
 // One (outer, channel) row of `inner_words` 4-byte words per blockIdx.y; UNIT words per thread,
@@ -577,9 +587,9 @@ lastaxis_any(const IN* __restrict__ in, OUT* __restrict__ out, int64_t n, int nc
   }
 }
 
-// One linear sweep, n < 2^32: a workgroup takes U * kThreads groups of four that follow each other, a
-// thread kThreads apart.  PER_CHANNEL: the channels on the last axis, a group's parameters read with it
-// (advance = 4 kThreads mod nch); otherwise per tensor.
+// One linear sweep, n < 2^32: a workgroup takes U chunks of kThreads groups of four, kHop groups apart.
+// PER_CHANNEL: the channels on the last axis, a group's parameters read with it (advance = 4 kHop mod nch);
+// otherwise per tensor.
 // Bound: HBM.  U: 16 KiB of f32 or 8 KiB of a narrower type on their way per workgroup, less where the
 // results are 4 bytes wide and as many stores follow the loads (four instead of two or one: 2-5 % slower
 // on large tensors).  Us, 16000 x 3072 per tensor: f16 to uint8 44.0 -> 23.6 (6.2 TB/s) with one load of 8
@@ -596,7 +606,7 @@ sweep_any(const IN* __restrict__ in, OUT* __restrict__ out, uint32_t n, uint32_t
   Four<IN> x[U];
 #pragma unroll
   for (int k = 0; k < U; ++k)                    // (groups past the end are read as the last one)
-    x[k] = *reinterpret_cast<const Four<IN>*>(in + 4 * (size_t)min(g0 + k * kThreads, n4 - 1));
+    x[k] = *reinterpret_cast<const Four<IN>*>(in + 4 * (size_t)min(g0 + k * kHop, n4 - 1));
   __builtin_amdgcn_sched_barrier(0);
   float4 s[P];
   int4 z[P];
@@ -626,7 +636,7 @@ sweep_any(const IN* __restrict__ in, OUT* __restrict__ out, uint32_t n, uint32_t
   if (__builtin_expect(ok, 1)) {
 #pragma unroll
     for (int k = 0; k < U; ++k)
-      if (g0 + k * kThreads < n4) st_stream_four(out + 4 * (size_t)(g0 + k * kThreads), o[k]);
+      if (g0 + k * kHop < n4) st_stream_four(out + 4 * (size_t)(g0 + k * kHop), o[k]);
   } else {                                       // (one copy of the divisions, as in lastaxis_any)
 #pragma unroll 1
     for (int k = 0; k < U; ++k) {
@@ -642,10 +652,10 @@ sweep_any(const IN* __restrict__ in, OUT* __restrict__ out, uint32_t n, uint32_t
         }
       Four<OUT> w;
       each_of_four(op, v, sk, zk, w);
-      if (g0 + k * kThreads < n4) st_stream_four(out + 4 * (size_t)(g0 + k * kThreads), w);
+      if (g0 + k * kHop < n4) st_stream_four(out + 4 * (size_t)(g0 + k * kHop), w);
     }
   }
-  if ((n & 3) != 0 && (n4 - g0) % kThreads == 0 && n4 - g0 < U * kThreads) {
+  if ((n & 3) != 0 && (n4 - g0) % kHop == 0 && n4 - g0 < U * kHop) {
     // the up to three elements behind the last four
     for (uint32_t e = 4 * n4; e < n; ++e) {
       const uint32_t c = PER_CHANNEL ? e % nch : 0;
@@ -657,12 +667,26 @@ sweep_any(const IN* __restrict__ in, OUT* __restrict__ out, uint32_t n, uint32_t
 // The same sweep with the channel on another axis, rows of inner >= 4 elements: a group of four lies in
 // one row or across the end of one.  16000 x 3072, a channel a row, f16 to uint8 55.6 -> 31.5 us, f32 to
 // int16 61.1 -> 50.7 and back 55.3 -> 46.4; 16000 x 3073 to uint8 55.9 -> 42.0, 1000 x 3073 6.1 -> 5.15.
+// A workgroup's groups follow each other here, in pieces of 1024 groups whatever U, piece j on die j % 8
+// (the 4 / U workgroups of a piece are eight apart): kHop apart, f16 to uint8 in buffers that change took
+// 10.0-10.6 us at 4000 x 3072 in place of 9.55.
+template <int U>
+__device__ __forceinline__ uint32_t piece_first_group() {
+  constexpr uint32_t R = 4 / U;
+  const uint32_t b = blockIdx.x, piece = b / (8 * R) * 8 + b % 8, part = b / 8 % R;
+  return piece * (4 * kThreads) + part * (U * kThreads) + threadIdx.x;
+}
+template <int U>
+unsigned piece_workgroups(int64_t n) {           // (one group more: the elements behind the last four)
+  const int64_t pieces = dq8::ceil_div(n / 4 + 1, (int64_t)(4 * kThreads));
+  return (unsigned)(U == 4 ? pieces : dq8::ceil_div(pieces, 8) * 8 * (4 / U));
+}
 template <typename IN, typename OUT, typename OP, int U>
 __global__ void __launch_bounds__(kThreads)
 rows_any(const IN* __restrict__ in, OUT* __restrict__ out, uint32_t n, uint32_t nch, uint32_t inner,
          const float* __restrict__ scale, const int32_t* __restrict__ zp, const OP op) {
   const uint32_t n4 = n >> 2;
-  const uint32_t g0 = sweep_first_group<U>();
+  const uint32_t g0 = piece_first_group<U>();
   if (g0 > n4) return;
   Four<IN> x[U];
 #pragma unroll
@@ -803,7 +827,7 @@ int launch_sweep(const IN* in, OUT* out, int64_t n, int64_t nch, const float* sc
                  hipStream_t st) {
   constexpr int U = sizeof(OUT) < 4 ? 4 : PER_CHANNEL ? 2 : sizeof(IN) < 4 ? 2 : 1;
   hipLaunchKernelGGL((sweep_any<IN, OUT, OP, PER_CHANNEL, U>), dim3(sweep_workgroups<U>(n)),
-                     dim3(kThreads), 0, st, in, out, (uint32_t)n, (uint32_t)nch, (uint32_t)(4 * kThreads % nch), scale,
+                     dim3(kThreads), 0, st, in, out, (uint32_t)n, (uint32_t)nch, (uint32_t)(4 * kHop % nch), scale,
                      zp, op);
   return dq8::check_hip(hipGetLastError(), "quantize / dequantize launch");
 }
@@ -835,7 +859,7 @@ int launch_any(const IN* in, OUT* out, int64_t outer, int64_t nch, int64_t inner
   // against 3.47 us, 100 x 500 3.14 against 2.52; from 1.5 M on the sweep wins, 4000 x 513 3.9 against 4.3)
   if (vec && per_channel && inner >= 4 && sweep_takes(n) && (sizeof(OUT) == 4 || n >= 1500000)) {
     constexpr int U = sizeof(OUT) < 4 ? 4 : sizeof(IN) < 4 ? 2 : 1;
-    hipLaunchKernelGGL((rows_any<IN, OUT, OP, U>), dim3(sweep_workgroups<U>(n)),
+    hipLaunchKernelGGL((rows_any<IN, OUT, OP, U>), dim3(piece_workgroups<U>(n)),
                        dim3(kThreads), 0, st, in, out, (uint32_t)n, (uint32_t)nch, (uint32_t)inner, scale, zp, op);
     return dq8::check_hip(hipGetLastError(), "quantize / dequantize launch");
   }
@@ -918,12 +942,8 @@ extern "C" int dq8_quantize(const float* x, void* out, int out_kind,
   } while (0)
 
   if (!per_channel && vec_ok) {
-    const bool pieces = pieces_pay(n);
-    auto k = rne ? (pieces ? quantize_tensor_v4<DQ8_ROUND_HALF_TO_EVEN, true> : quantize_tensor_v4<DQ8_ROUND_HALF_TO_EVEN, false>)
-                 : (pieces ? quantize_tensor_v4<DQ8_ROUND_HALF_AWAY_FROM_ZERO, true>
-                           : quantize_tensor_v4<DQ8_ROUND_HALF_AWAY_FROM_ZERO, false>);
-    hipLaunchKernelGGL(k, dim3(pieces ? sweep_workgroups<1>(n) : sweep_grid(n / 4 + n % 4)), dim3(kThreads), 0, st,
-                       (const float4*)x, (uint32_t*)out, n, scale, zp, lo, hi);
+    LAUNCH_RND(quantize_tensor_v4, dim3(sweep_grid(n / 4 + n % 4)), dim3(kThreads),
+               (const float4*)x, (uint32_t*)out, n, scale, zp, lo, hi);
   } else if (per_channel && vec_ok && inner == 1 && nch % 4 == 0 && nch / 4 < (1 << 30) &&
              dq8::aligned(scale, 16) && dq8::aligned(zp, 16)) {
     const int nch4 = (int)(nch / 4);
@@ -935,11 +955,9 @@ extern "C" int dq8_quantize(const float* x, void* out, int out_kind,
     const int64_t rows = outer * nch;
     const int64_t inner4 = inner / 4;
     DQ8_REQUIRE(inner4 < (1LL << 38), "dq8_quantize: rows too long for one launch");
-    unsigned gx = (unsigned)dq8::ceil_div(inner4, kThreads);
-    int gy = (int)std::min<int64_t>(rows, 32768);
-    int64_t gz = dq8::ceil_div(rows, gy);
-    DQ8_REQUIRE(gz <= 65535, "dq8_quantize: too many rows for one launch");
-    LAUNCH_RND(quantize_rows_v4, dim3(gx, gy, (unsigned)gz), dim3(kThreads),
+    const RowsGrid g = rows_grid<1>(rows, inner4);
+    DQ8_REQUIRE(g.z <= 65535, "dq8_quantize: too many rows for one launch");
+    LAUNCH_RND(quantize_rows_v4, dim3(g.x, g.y, (unsigned)g.z), dim3(kThreads),
                (const float4*)x, (uint32_t*)out, (unsigned)rows, inner4, (unsigned)nch, scale,
                zp, lo, hi);
   } else {
@@ -968,10 +986,10 @@ extern "C" int dq8_dequantize(const void* q, int in_kind, float* out,
   const bool vec_ok = dq8::aligned(q, 4) && dq8::aligned(out, 16);
 
   if (!per_channel && vec_ok) {
-    const bool pieces = pieces_pay(n);
-    auto k = is_signed ? (pieces ? dequantize_tensor_v4x2<true, true> : dequantize_tensor_v4x2<true, false>)
-                       : (pieces ? dequantize_tensor_v4x2<false, true> : dequantize_tensor_v4x2<false, false>);
-    hipLaunchKernelGGL(k, dim3(pieces ? sweep_workgroups<2>(n) : sweep_grid(dq8::ceil_div(n / 4, 2))), dim3(kThreads),
+    const bool hops = l2s_hold(n);
+    auto k = is_signed ? (hops ? dequantize_tensor_v4x2<true, kHop> : dequantize_tensor_v4x2<true, kThreads>)
+                       : (hops ? dequantize_tensor_v4x2<false, kHop> : dequantize_tensor_v4x2<false, kThreads>);
+    hipLaunchKernelGGL(k, dim3(hops ? sweep_workgroups<2>(n) : sweep_grid(dq8::ceil_div(n / 4, 2))), dim3(kThreads),
                        0, st, (const uint32_t*)q, (float4*)out, n, scale, zp);
   } else if (per_channel && vec_ok && inner == 1 && nch % 4 == 0 && nch / 4 < (1 << 30) &&
              dq8::aligned(scale, 16) && dq8::aligned(zp, 16)) {
@@ -983,18 +1001,18 @@ extern "C" int dq8_dequantize(const void* q, int in_kind, float* out,
                        (const int4*)zp);
   } else if (per_channel && vec_ok && inner % 4 == 0 && outer * nch < (1LL << 31)) {
     const int64_t rows = outer * nch;
-    // two words per thread once a row is several workgroups -- except where one, as in quantize, keeps the
-    // words on the die that has just written them (both in one buffer, 1500 x 3072 11.2 -> 9.5 us, 3000 x
-    // 2432 15.1 -> 12.9, 5000 x 3072 25.4 -> 24.8, 3000 x 4096 20.6 -> 20.7)
-    const bool v8 = inner >= 2048 && !pieces_pay(n);
+    // Two words per thread once a row is several workgroups -- except where one, on quantize's grid, keeps
+    // the words on the die that has just written them.  Both in one buffer, two words / one: 1000 x 3072
+    // 12.2 / 9.2 us, 1500 x 3072 16.4 / 9.5, 5000 x 3072 29.9 / 26.8, 12000 x 2048 41.5 / 40.3; dequantize alone
+    // 4.9 / 4.7, 5.5 / 5.4, 12.7 / 12.1, 18.3 / 18.0 in buffers that change.
+    const bool two = inner >= 2048 && !l2s_hold(n);
     const int64_t units = inner / 4;
-    int gx = (int)std::min<int64_t>(dq8::ceil_div(units, kThreads * (v8 ? 2 : 1)), 65536);
-    int gy = (int)std::min<int64_t>(rows, 32768);
-    int64_t gz = dq8::ceil_div(rows, gy);
-    DQ8_REQUIRE(gz <= 65535, "dq8_dequantize: too many rows for one launch");
-    auto k = v8 ? (is_signed ? dequantize_rows<true, 2> : dequantize_rows<false, 2>)
-                : (is_signed ? dequantize_rows<true, 1> : dequantize_rows<false, 1>);
-    hipLaunchKernelGGL(k, dim3(gx, gy, (unsigned)gz), dim3(kThreads), 0, st,
+    RowsGrid g = two ? rows_grid<2>(rows, units) : rows_grid<1>(rows, units);
+    g.x = std::min(g.x, 65536u);
+    DQ8_REQUIRE(g.z <= 65535, "dq8_dequantize: too many rows for one launch");
+    auto k = two ? (is_signed ? dequantize_rows<true, 2> : dequantize_rows<false, 2>)
+                 : (is_signed ? dequantize_rows<true, 1> : dequantize_rows<false, 1>);
+    hipLaunchKernelGGL(k, dim3(g.x, g.y, (unsigned)g.z), dim3(kThreads), 0, st,
                        (const uint32_t*)q, (float4*)out, (unsigned)rows, units, (unsigned)nch,
                        scale, zp);
   } else {

@@ -2761,3 +2761,31 @@ def test_quantize_by_row_any_type(K, outer, nch, inner, xt, qt):
     if qt == torch.uint8:
         f = K.fake_quant(x.cuda(), ds, dz, axis=1, qmin=0, qmax=255).cpu().numpy()
         assert np.array_equal(f, back)
+
+
+@pytest.mark.parametrize("rows,inner", [
+    # per tensor: elements behind the last four; the edges of a chunk of 1024, of the sixteen chunks of eight
+    # workgroups, and of the sizes that are walked in chunks
+    (1, 1), (1, 3), (1, 1023), (1, 1025), (1, 8191), (1, 8193), (1, 16383), (1, 16384), (1, 16387), (1, 24577),
+    (1, (1 << 25) - 1), (1, 1 << 25), (1, (1 << 25) + 5),
+    # by row: rows on both sides of 2048, one and two words a thread
+    (3, 4), (5, 1024), (5, 1028), (7, 2044), (7, 2048), (7, 2052), (300, 16388), (8193, 4096), (16380, 2052)])
+@pytest.mark.parametrize("qt", [torch.int8, torch.uint8])
+def test_quantize_and_dequantize_in_every_order_of_the_words(K, rows, inner, qt):
+    """8-bit quantize and dequantize per tensor and by row, whose workgroups take the words in an order of
+    their own: every element once, nothing behind the last.  Each step is one rounded binary32 operation:
+    equal bits."""
+    torch.manual_seed(inner)
+    info = torch.iinfo(qt)
+    n = rows * inner
+    scale = torch.rand(rows, device="cuda") * 0.05 + 0.01
+    zp = torch.randint(0, 4, (rows,), dtype=torch.int32, device="cuda")
+    axis = 0 if rows > 1 else None
+    x = torch.randn((rows, inner), device="cuda")
+    buf = torch.full((n + 64,), 77, dtype=qt, device="cuda")
+    q = K.quantize(x, scale, zp, axis=axis, qmin=info.min, qmax=info.max, dtype=qt, out=buf[:n].view(rows, inner))
+    want = torch.clamp(torch.round(x / scale[:, None] + zp[:, None]), info.min, info.max).to(torch.int32)
+    assert torch.equal(q.to(torch.int32), want) and bool((buf[n:] == 77).all())
+    back = torch.full((n + 64,), 7.0, device="cuda")
+    y = K.dequantize(q, scale, zp, axis=axis, out=back[:n].view(rows, inner))
+    assert torch.equal(y, (want - zp[:, None]).float() * scale[:, None]) and bool((back[n:] == 7).all())
