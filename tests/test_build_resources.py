@@ -12,8 +12,9 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 OBJ = os.path.join(ROOT, "bladedisc_amd", "build")
 
 # mangled-name fragments of the kernels in question
-NO_SPILL = ("qconv_stream_kernel", "qgemm_persist_kernel", "qgemm_skinny_kernel", "qlinear",
-            "quantize", "dequantize", "lut_u8", "minmax")
+NO_SPILL = ("qconv_stream_kernel", "qgemm_persist_kernel", "qgemm_skinny_",
+            "quantize", "dequantize", "fake_quant", "sweep_any", "rows_any", "lastaxis_any", "flat_any", "lut_u8",
+            "minmax", "wo_", "attention_f32_kernel", "layernorm_f32_kernel")
 # the 256 x 256 tile on four waves keeps 256 accumulators per lane and spills part of their
 # indexing; it is a cross-check variant that the library never picks by itself
 ALLOWED = ("qgemm_pipe_kernelILi256ELi256ELi2ELi2E", "qgemm_mfma_kernelILi256ELi256E")
@@ -28,7 +29,7 @@ def test_register_resident_kernels_do_not_spill():
     files = sorted(glob.glob(os.path.join(OBJ, "*.o.resources.json")))
     if not files:
         pytest.skip("no resource records: the library was not built here")
-    seen, spilled = 0, []
+    seen, spilled, found = 0, [], set()
     for f in files:
         for name, res in json.load(open(f)).items():
             if "scratch_bytes_per_lane" not in res:
@@ -37,9 +38,11 @@ def test_register_resident_kernels_do_not_spill():
             if not watched or any(a in name for a in ALLOWED):
                 continue
             seen += 1
+            found.update(k for k in NO_SPILL if k in name)
             if res["scratch_bytes_per_lane"] > 0:
                 spilled.append((name, res))
     assert seen > 50, "too few kernels recorded (%d): are the records stale?" % seen
+    assert found == set(NO_SPILL), "no kernel is named %s" % sorted(set(NO_SPILL) - found)
     if spilled:
         pretty = _demangle([n for n, _ in spilled])
         raise AssertionError("kernels with scratch memory:\n" + "\n".join(
