@@ -24,10 +24,10 @@
 // so lane (row, g) takes the 16 consecutive k values k0 + 16 g .. of its row -- 16 weight bytes
 // (one dwordx4), 16 activations -- and feeds two MFMAs with them.
 //  * wo_dma_kernel: tiles loaded straight into LDS, everything above 32 rows (16 for f32 against deep or
-//    wide weights): 32 x 64 to 128 x 256 tiles, with several workgroups per tile, each over a part of
-//    k, and wo_splitk_reduce_kernel behind them, where that is estimated cheaper (1.1-1.2 PFLOP/s for
-//    f16 activations at 4096^2 .. 8192^2 weights, where the ROCm library's plain f16 GEMM reaches
-//    1.16-1.49);
+//    wide weights, f32_rows_on_tiles): 32 x 64 to 128 x 256 tiles, with several workgroups per tile, each
+//    over a part of k, and wo_splitk_reduce_kernel behind them, where that is estimated cheaper (1.1-1.2
+//    PFLOP/s for f16 activations at 4096^2 .. 8192^2 weights, where the ROCm library's plain f16 GEMM
+//    reaches 1.16-1.49);
 //  * wo_ragged_kernel: the same for f16 rows that are not multiples of 16 bytes, through registers;
 //  * wo_tile_kernel: 2 x 2 waves, wave tile (32 FM) x (32 FN), operands straight into registers:
 //    operands too large for the LDS kernel's 31-bit offsets;
@@ -1154,11 +1154,19 @@ __global__ void __launch_bounds__(kRowsWaves * 64) wo_rows_kernel(const WoParams
 #pragma unroll
     for (int i = 0; i < FN; ++i) *reinterpret_cast<u4*>(&ws[wl[i]]) = wq[i];
   };
-  f4v acc[MT][FN];
+  // f32, more than 16 rows and channels: the low halves' products on sums of their own, as in wo_dma_kernel,
+  // and the waves' sums added in pairs: 0.65-0.78 of the rms error against 64 bits of one sum added wave by
+  // wave, for 0-2 % of the time (1024 of k 0.87e-7 against 1.25e-7, tiles 0.96e-7; 2048 1.00e-7 / 1.53e-7 /
+  // 1.21e-7).  Up to 16 rows the registers would cost a compute unit its second workgroup.
+  constexpr bool kLowSums = F32 && MT == 2 && FN > 1;
+  f4v acc[MT][FN], acc_lo[kLowSums ? MT : 1][FN];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = (f4v){0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < FN; ++j) {
+      acc[i][j] = (f4v){0.f, 0.f, 0.f, 0.f};
+      acc_lo[kLowSums ? i : 0][j] = (f4v){0.f, 0.f, 0.f, 0.f};
+    }
   // lane (r, g): the unit's k values 16 g .. 16 g + 15 of row r of a fragment, as two k steps
   auto multiply = [&]() {
     h8 a[F32 ? 2 : 1][MT][2];
@@ -1182,8 +1190,9 @@ __global__ void __launch_bounds__(kRowsWaves * 64) wo_rows_kernel(const WoParams
       for (int part = 0; part < (F32 ? 2 : 1); ++part)
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[part][i][0], w0, acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[part][i][1], w1, acc[i][j], 0, 0, 0);
+          f4v& sum = kLowSums && part ? acc_lo[kLowSums ? i : 0][j] : acc[i][j];
+          sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[part][i][0], w0, sum, 0, 0, 0);
+          sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[part][i][1], w1, sum, 0, 0, 0);
         }
     }
   };
@@ -1204,6 +1213,12 @@ __global__ void __launch_bounds__(kRowsWaves * 64) wo_rows_kernel(const WoParams
       __builtin_amdgcn_sched_barrier(0);
     }
   }
+  if constexpr (kLowSums) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[i][j] += acc_lo[i][j];
+  }
   // partial sums of the waves through LDS (all waves are done with their pieces of it), a
   // fragment to each of the first MT x FN waves
   __syncthreads();
@@ -1214,11 +1229,19 @@ __global__ void __launch_bounds__(kRowsWaves * 64) wo_rows_kernel(const WoParams
     for (int v = 0; v < 4; ++v) red[((f * NW + wave) * 4 + v) * 64 + lane] = acc[f / FN][f % FN][v];
   __syncthreads();
   if (wave >= MT * FN) return;
-  f4v sum = {0.f, 0.f, 0.f, 0.f};
+  f4v part[NW];
 #pragma unroll
   for (int w = 0; w < NW; ++w)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) sum[v] += red[((wave * NW + w) * 4 + v) * 64 + lane];
+    for (int v = 0; v < 4; ++v) part[w][v] = red[((wave * NW + w) * 4 + v) * 64 + lane];
+  f4v sum = part[0];
+  if constexpr (kLowSums) {
+    static_assert(NW == 8, "three levels of pairs");
+    sum = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+  } else {
+#pragma unroll
+    for (int w = 1; w < NW; ++w) sum += part[w];
+  }
   // D of the 16x16 MFMA: column n = lane % 16, rows 4 (lane / 16) + v
   const int n = n0 + 16 * (wave % FN) + r, m0 = 16 * (wave / FN) + 4 * g;
   if (n >= p.N) return;
@@ -1455,15 +1478,26 @@ SplitPlan plan_split(int64_t M, int64_t N, int64_t K, int esz, bool ragged, int 
   return best;
 }
 
-// The plan for M x N x K, or form = -1 where the kernels for few rows are the choice: up to 32 rows,
-// for f32 up to 16 from 2048 of k or 4096 channels on, where the staged kernel pays for two half tiles
-// (f32, tiles against the staged kernel, by geometric mean over 17 .. 32 rows: 1.14-1.48 times as fast
-// beyond 2048 of k, 1.03-1.06 beyond 4096 channels, 0.83-0.90 elsewhere; f16 0.65-0.95).
+// Whether 17 .. 32 rows of f32 run on tiles.  us at 24 rows, staged / tiles: 4104 channels (from 4097 on the
+// staged kernel's workgroups are 32 wide) 256 of k 4.70 / 4.15, 448 5.0 / 5.05, 768 5.7 / 6.45, 1024 6.1 / 7.1,
+// 2048 8.7 / 9.9; 8192 channels 256 4.8 / 4.25, 512 5.3 / 5.4, 1024 6.7 / 7.3, 2304 9.7 / 10.8, 2816 equal, 4096
+// 16.3 / 14.4; 9216 and more equal at 768 to 2048, tiles 1.06-1.24 times as fast on either side.  Up to 4096
+// channels tiles win from 3584 of k on (4096^2 13.1 / 12.0); from 2048 on, and to 6143 channels, they are
+// taken for their sums: split over k, 0.97e-7 rms against 64 bits where the staged kernel has 1.6e-7 (one
+// sum for both halves) and 1.03e-7, for 0.05-0.2 of the time.
+bool f32_rows_on_tiles(int64_t N, int64_t K) {
+  if (N > 8192 || (N > 4096 && K < 400)) return true;
+  return K > (N >= 6144 ? 2816 : 2048);
+}
+
+// The plan for M x N x K, or form = -1 where the kernels for few rows are the choice: up to 32 rows, for
+// f32 up to 16 where the staged kernel, which multiplies two half tiles, is the slower or less exact one
+// (f16 up to 32 rows, tiles against the staged kernel: 0.65-0.95 times as fast).
 SplitPlan choose_tiles(int64_t M, int64_t N, int64_t K, int esz, bool ragged, int most_splits) {
   const SplitPlan none = {-1, 1, (int)K, 0.0f};
   // (rows off 16 bytes: f16 has tiles and the staged small-M kernel, f32 its own kernel)
   if (ragged && (esz == 4 || M <= 32)) return none;
-  if (M <= (esz == 4 && (K > 2048 || N > 4096) ? 16 : 32)) return none;
+  if (M <= (esz == 4 && f32_rows_on_tiles(N, K) ? 16 : 32)) return none;
   return plan_split(M, N, K, esz, ragged, 1, most_splits);
 }
 

@@ -2032,6 +2032,25 @@ def test_weight_only_qgemm_every_tile_form_split_over_k(K, dtype, m, k, n, form,
     assert torch.equal(out, first)
 
 
+@pytest.mark.parametrize("m,k,n,signed", [
+    (17, 400, 4097, False), (24, 1040, 4111, True), (32, 2048, 5000, False), (31, 784, 6161, True),
+    (17, 2816, 6144, False), (25, 1024, 8177, True), (32, 2064, 8192, False), (20, 384, 4097, True),
+    (32, 2832, 8192, False), (29, 512, 8193, True), (18, 2064, 4096, False)])
+def test_weight_only_qgemm_f32_rows_on_either_side_of_the_tiles_line(K, m, k, n, signed):
+    """17 to 32 rows of f32 on 32-channel workgroups of the staged kernel (low halves on sums of their own,
+    the waves' sums in pairs) and on tiles, at the edges of the rule between them, in frames of NaN / 255."""
+    rng = np.random.default_rng(m + k + n)
+    x, w, scale, zp, bias = _weight_only_case(rng, m, k, n, torch.float32, signed)
+    wide_x, wide_w = _weight_only_framed(x, w, torch.float32, signed)
+    splits = _weight_only_plan(m, n, k, torch.float32)[1]
+    ws = torch.empty(max(4 * m * n * splits, 16), dtype=torch.uint8, device="cuda")
+    frame = torch.full((m + 1, n + 5), 7.0, device="cuda")
+    out = frame[:m, 1:n + 1]
+    _weight_only_raw(wide_x, wide_w, dev(scale), dev(zp), dev(bias), out, ws, ws.nbytes)
+    _weight_only_check(out, x, w, scale, zp, bias, torch.float32)
+    assert bool((frame[:, 0] == 7).all()) and bool((frame[:, n + 1:] == 7).all()) and bool((frame[m] == 7).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 def test_weight_only_qgemm_strided_rows_in_and_out(K, dtype):
     """Activation and result rows that are slices of wider buffers (ldx > K, ldo > N), one shape
