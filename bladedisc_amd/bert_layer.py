@@ -150,11 +150,27 @@ class QuantBertLayer:
         64 channels, a hidden size its layer norm takes)."""
         return h == 64 * self.heads and h <= 2048
 
-    def _attention(self, qkv):
-        """attention() of the quantized layer: this library's kernel where it applies."""
-        if self._native_ops(qkv.shape[-1] // 3):
-            return K.attention(qkv, self.heads)
-        return self.attention(qkv)
+    def _context(self, qkv_in, shape, out_scale=None):
+        """attention() of the quantized layer on this library's kernel, from the projection's int8 input: on
+        the projection's int8 result where that has one scale."""
+        b, s, c = shape
+        if torch.as_tensor(self.s_out["qkv"]).numel() == 1:
+            qkv = self._gemm("qkv", qkv_in)
+            return K.attention(qkv.reshape(b, s, 3 * c), self.heads, out_scale, self.s_out["qkv"])
+        qkv = self.be.qlinear_dequantized(qkv_in, self.w_q["qkv"], self.bias["qkv"], self.s_in["qkv"],
+                                          self.sw["qkv"], self.s_out["qkv"])
+        return K.attention(qkv.reshape(b, s, 3 * c), self.heads, out_scale)
+
+    def _projected_attention(self, h, rec):
+        """The merged projection and attention() of the layer of separate operators."""
+        if not self._native_ops(h.shape[-1]):
+            return self.attention(self._qlinear("qkv", h, rec))
+        x2 = h.reshape(-1, h.shape[-1])
+        x_q = self.be.quantize(x2, self.s_in["qkv"])
+        if rec is not None:
+            y_q, y = self._gemm_dequantized("qkv", x_q)
+            rec["qkv"] = dict(x=x2, x_q=x_q, y_q=y_q, y=y)
+        return self._context(x_q, h.shape)
 
     def _norm(self, x, name):
         """The layer norms of the quantized layer, likewise."""
@@ -257,9 +273,7 @@ class QuantBertLayer:
         b, s, c = h.shape
         h2 = h.reshape(-1, c)
         x_q = self.be.quantize(h2, self.s_in["qkv"])
-        qkv = self.be.qlinear_dequantized(x_q, self.w_q["qkv"], self.bias["qkv"], self.s_in["qkv"],
-                                          self.sw["qkv"], self.s_out["qkv"])
-        ctx_q = K.attention(qkv.reshape(b, s, 3 * c), self.heads, self.s_in["out"])
+        ctx_q = self._context(x_q, h.shape, self.s_in["out"])
         pre1 = self._residual_gemm("out", ctx_q.reshape(-1, c), h2)
         h1, h1_q = K.layer_norm(pre1, f["ln1_g"], f["ln1_b"], 1e-12, self.s_in["ffn1"])
         mid_q = self.be.qlinear_table(h1_q, self.w_q["ffn1"], self.bias["ffn1"], self.s_in["ffn1"],
@@ -335,8 +349,7 @@ class QuantBertLayer:
             raise RuntimeError("calibrate() first")
         if self.fuse_epilogue and record is None and self._native_ops(h.shape[-1]):
             return self._forward_fused(h)
-        qkv = self._qlinear("qkv", h, record)
-        ctx = self._attention(qkv)
+        ctx = self._projected_attention(h, record)
         if self.fuse_epilogue:
             pre1 = self._qlinear_residual("out", ctx, h, record)
             h1 = self._norm(pre1, "ln1")

@@ -549,22 +549,31 @@ PyObject* py_qconv2d(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
-// attention(qkv [.., seq, 3 heads 64], heads, scale or None): int8 result with a scale, else f32
+// attention(qkv [.., seq, 3 heads 64], heads, scale or None, qkv_scale or None): int8 result with a scale, else
+// f32; qkv is f32, or with a qkv_scale int8
 PyObject* py_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
-    arguments("attention", n, 3);
+    arguments("attention", n, 4);
     const Tensor x = dense(device_tensor(a[0]));
-    if (x.scalar_type() != ScalarType::Float || x.dim() != 3)
-      raise(PyExc_TypeError, "attention takes a float32 tensor of rank 3");
+    const Tensor sx = scale(a[3], x.device());
+    if (x.scalar_type() != (sx.defined() ? ScalarType::Char : ScalarType::Float) || x.dim() != 3)
+      raise(PyExc_TypeError, "attention takes a float32 tensor of rank 3, or an int8 one and its scale");
+    if (sx.defined() && (!sx.is_cuda() || sx.numel() != 1))
+      raise(PyExc_ValueError, "attention takes one scale of its int8 input, on the device");
     const int64_t heads = integer(a[1]), h3 = x.size(2);
     if (heads <= 0 || h3 % (3 * heads) != 0) raise(PyExc_ValueError, "attention: heads do not divide the channels");
     const Tensor s = optional_device_tensor(a[2]);
     const Tensor out = empty({x.size(0), x.size(1), h3 / 3}, s.defined() ? ScalarType::Char : ScalarType::Float,
                              x.device());
     void* st = stream();
-    launch("dq8_attention_f32", dq8_attention_f32, (const float*)in(x), x.size(0), x.size(1), heads,
-           h3 / 3 / heads, s.defined() ? nullptr : (float*)inout(out),
-           s.defined() ? (int8_t*)inout(out) : nullptr, (const float*)in(s), st);
+    float* y = s.defined() ? nullptr : (float*)inout(out);
+    int8_t* y_q = s.defined() ? (int8_t*)inout(out) : nullptr;
+    if (sx.defined())
+      launch("dq8_attention_i8", dq8_attention_i8, (const int8_t*)in(x), (const float*)in(sx), x.size(0), x.size(1),
+             heads, h3 / 3 / heads, y, y_q, (const float*)in(s), st);
+    else
+      launch("dq8_attention_f32", dq8_attention_f32, (const float*)in(x), x.size(0), x.size(1), heads,
+             h3 / 3 / heads, y, y_q, (const float*)in(s), st);
     return THPVariable_Wrap(out);
   });
 }
@@ -656,20 +665,18 @@ PyObject* py_encoder_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int32_t* zero = (const int32_t*)in(*last[5]);
     const Tensor h = dense(h0);
     const float* x = (const float*)in(h);
-    // the int8 input of each linear, and the f32 results: the merged projection, the sum in front of
+    // the int8 input of each linear and the merged projection; the f32 results: the sum in front of
     // either layer norm (the second overwrites the first, which has been read by then), the first norm,
     // the layer
-    Tensor q[kLinears], y[4];
+    Tensor q[kLinears + 1], y[3];
     for (int i = 0; i < kLinears; ++i) q[i] = empty({M, l[i].k}, ScalarType::Char, dev);
-    y[0] = empty({M, 3 * hidden}, ScalarType::Float, dev);
-    for (int i = 1; i < 3; ++i) y[i] = empty({M, hidden}, ScalarType::Float, dev);
-    y[3] = empty(h.sizes(), ScalarType::Float, dev);
-    int8_t* qp[kLinears];
-    float* yp[4];
-    for (int i = 0; i < 4; ++i) {
-      qp[i] = (int8_t*)inout(q[i]);
-      yp[i] = (float*)inout(y[i]);
-    }
+    q[kLinears] = empty({M, 3 * hidden}, ScalarType::Char, dev);
+    for (int i = 0; i < 2; ++i) y[i] = empty({M, hidden}, ScalarType::Float, dev);
+    y[2] = empty(h.sizes(), ScalarType::Float, dev);
+    int8_t* qp[kLinears + 1];
+    float* yp[3];
+    for (int i = 0; i <= kLinears; ++i) qp[i] = (int8_t*)inout(q[i]);
+    for (int i = 0; i < 3; ++i) yp[i] = (float*)inout(y[i]);
     size_t need = 0;
     for (const Linear& i : l) need = std::max(need, i.need);
     Tensor ws;
@@ -696,20 +703,21 @@ PyObject* py_encoder_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
       add_x.residual_kind = DQ8_RESIDUAL_F32;
       add_x.ldr = hidden;
       add_h1 = add_x;
-      add_h1.residual = yp[2];
+      add_h1.residual = yp[1];
       ok("dq8_quantize", dq8_quantize_ex(x, DQ8_DTYPE_F32, qp[0], DQ8_I8, 1, 1, M * hidden, l[0].sx, zero, 1, -128,
                                          127, DQ8_ROUND_HALF_TO_EVEN, st)) &&
-          linear(0, yp[0], DQ8_EPI_REQUANT_CPU_DEQUANT_F32, nullptr) &&
-          ok("dq8_attention_f32", dq8_attention_f32(yp[0], batch, seq, heads, 64, nullptr, qp[1], l[1].sx, st)) &&
-          linear(1, yp[1], DQ8_EPI_REQUANT_CPU_DEQUANT_F32, &add_x) &&
+          linear(0, qp[kLinears], DQ8_EPI_REQUANT_CPU, nullptr) &&
+          ok("dq8_attention_i8",
+             dq8_attention_i8(qp[kLinears], l[0].so, batch, seq, heads, 64, nullptr, qp[1], l[1].sx, st)) &&
+          linear(1, yp[0], DQ8_EPI_REQUANT_CPU_DEQUANT_F32, &add_x) &&
           ok("dq8_layernorm_f32",
-             dq8_layernorm_f32(yp[1], M, hidden, g1, b1, eps, yp[2], qp[2], l[2].sx, st)) &&
+             dq8_layernorm_f32(yp[0], M, hidden, g1, b1, eps, yp[1], qp[2], l[2].sx, st)) &&
           linear(2, qp[3], DQ8_EPI_REQUANT_CPU, &gelu) &&
-          linear(3, yp[1], DQ8_EPI_REQUANT_CPU_DEQUANT_F32, &add_h1) &&
-          ok("dq8_layernorm_f32", dq8_layernorm_f32(yp[1], M, hidden, g2, b2, eps, yp[3], nullptr, nullptr, st));
+          linear(3, yp[0], DQ8_EPI_REQUANT_CPU_DEQUANT_F32, &add_h1) &&
+          ok("dq8_layernorm_f32", dq8_layernorm_f32(yp[0], M, hidden, g2, b2, eps, yp[2], nullptr, nullptr, st));
     }
     check(failed, what);
-    return THPVariable_Wrap(y[3]);
+    return THPVariable_Wrap(y[2]);
   });
 }
 

@@ -254,11 +254,12 @@ def qlinear_f32(x, w, epilogue, sx, sw=None, so=None, bias=None, zo=0,
     return _native().qlinear_f32(x, w, epilogue, sx, sw, so, bias, zo, round_mode, out)
 
 
-def attention(qkv, heads, scale=None):
+def attention(qkv, heads, scale=None, qkv_scale=None):
     """softmax(q k^T / sqrt(64)) v of a merged f32 projection [B, S, 3 * heads * 64] -> [B, S,
     heads * 64], f32 throughout; with a one-element device `scale` the result is quantized to int8
-    in the same pass (the bits of quantize(., scale, 0) behind it)."""
-    return _native().attention(qkv, heads, scale)
+    in the same pass (the bits of quantize(., scale, 0) behind it).  With a one-element device
+    `qkv_scale` the projection is int8, qkv_scale times which is what its products are of."""
+    return _native().attention(qkv, heads, scale, qkv_scale)
 
 
 def layer_norm(x, weight, bias, eps=1e-5, scale=None):
@@ -268,7 +269,7 @@ def layer_norm(x, weight, bias, eps=1e-5, scale=None):
 
 
 def encoder_layer(h, heads, eps, operands):
-    """A quantized encoder layer on h [B, S, 64 * heads] (f32): quantize, merged projection, attention,
+    """A quantized encoder layer on h [B, S, 64 * heads] (f32): quantize, merged projection (int8), attention,
     output linear + h, layer norm, feed-forward linear with a 256-entry activation table, second
     feed-forward linear + the first norm, layer norm -- the calls above in this order, eight launches.
     operands: for the four linears in turn (int8 weights [N, K], f32 bias, input scale, weight scales,

@@ -423,6 +423,11 @@ int dq8_weight_only_undo_compiler_layout(const uint8_t* reordered, uint8_t* w_nk
 int dq8_attention_f32(const float* qkv, int64_t batch, int64_t seq, int64_t heads, int64_t head_dim,
                       float* out, int8_t* out_q, const float* q_scale, void* stream);
 
+/* The same of an int8 projection (codes times qkv_scale[0], zero point 0), which is what dq8_qgemm leaves
+ * without its dequantize: the scores in whole numbers, the probabilities and their sums in f32. */
+int dq8_attention_i8(const int8_t* qkv, const float* qkv_scale, int64_t batch, int64_t seq, int64_t heads,
+                     int64_t head_dim, float* out, int8_t* out_q, const float* q_scale, void* stream);
+
 /* (x - mean) / sqrt(var + eps) * gamma + beta over the rows of x [rows, cols] (device f32), to
  * out (f32), to out_q = dq8_quantize of that, or to both.  Up to 2048 columns, a multiple of 4. */
 int dq8_layernorm_f32(const float* x, int64_t rows, int64_t cols, const float* gamma,

@@ -2416,6 +2416,39 @@ def test_attention_equals_softmax_of_the_scores(K, b, s, heads):
     assert torch.equal(K.attention(qkv.cuda(), heads, scale), K.quantize(got, scale, torch.zeros(1, dtype=torch.int32, device="cuda")))
 
 
+@pytest.mark.parametrize("b,s,heads", [(1, 1, 1), (2, 8, 12), (3, 17, 2), (1, 33, 3), (2, 64, 1), (1, 65, 12), (2, 97, 3), (2, 333, 5)])
+@pytest.mark.parametrize("step", [0.02, 0.1])
+def test_attention_of_an_int8_projection(K, b, s, heads, step):
+    """Edges of the 16-query, 32- and 64-key tiles with codes of the whole range, a wide and a narrow
+    softmax (scores up to 10 / up to 230), against the same in f64.  Bound: the scale's f32 square and product
+    move a difference of scores d by 3 ulp, its rounding and the exponential's ulp come on top, and d above 25
+    contributes nothing: 25 * 3 * 2^-24 + 2 * 2^-24 of each probability, twice (also in their sum), and
+    s / 8 roundings of sums of values up to 128 * step: below 1e-5 of that."""
+    g = torch.Generator().manual_seed(s)
+    codes = torch.randint(-128, 128, (b, s, 3 * heads * 64), generator=g, dtype=torch.int8)
+    codes[:, -1, -64:] = -128
+    scale = torch.full((1,), step)
+    q, k, v = (t.double().reshape(b, s, heads, 64).transpose(1, 2) for t in (codes.double() * scale.double()).chunk(3, dim=-1))
+    want = (torch.softmax(q @ k.transpose(2, 3) / 8.0, -1) @ v).transpose(1, 2).reshape(b, s, heads * 64)
+    got = K.attention(codes.cuda(), heads, qkv_scale=scale.cuda())
+    assert (got.cpu().double() - want).abs().max().item() <= 1e-5 * 128 * step
+    out_scale = torch.full((1,), 0.02, device="cuda")
+    zero = torch.zeros(1, dtype=torch.int32, device="cuda")
+    assert torch.equal(K.attention(codes.cuda(), heads, out_scale, float(scale)), K.quantize(got, out_scale, zero))
+    # a scale that is not a number, or infinite: of 0 * inf and inf - inf; zero: all keys alike
+    for bad in (float("nan"), float("inf")):
+        assert K.attention(codes.cuda(), heads, None, bad).isnan().all()
+    assert (K.attention(codes.cuda(), heads, None, 0.0) == 0).all()
+
+
+def test_attention_takes_an_int8_projection_with_its_scale_only(K):
+    codes = torch.zeros((1, 2, 192), dtype=torch.int8, device="cuda")
+    for args in ((codes, 1), (codes, 1, None, torch.ones(2, device="cuda")), (codes, 1, None, torch.ones(1)),
+                 (codes.float(), 1, None, 1.0)):
+        with pytest.raises((TypeError, ValueError)):
+            K.attention(*args)
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 4), (5, 252), (3, 260), (9, 768), (1026, 1000), (7, 1028), (2, 2048)])
 def test_layer_norm_with_and_without_its_quantize(K, rows, cols):
     g = torch.Generator().manual_seed(cols)
