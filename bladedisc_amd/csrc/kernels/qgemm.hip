@@ -435,7 +435,49 @@ int pick_k_split64(int64_t M, int64_t N, int64_t K) {
   return (K >= 8192 && t64 <= compute_units()) ? kPipe64k4 : kPipe64k2;
 }
 
-int pick_variant(int64_t M, int64_t N, int64_t K, bool pipe, int out_bytes = 1) {
+// The kernels whose waves share nothing until the end (qgemm_wave.h), or -1: the smallest tile of which the
+// launch has at most one per compute unit.  Against the best of the other tiles (us per launch):
+//  * 32 x 32, on eight waves from 1024 of k on, on four below: 343 x 512, 4608 of k 11.9 -> 7.1, 2048 of k 6.25 ->
+//    5.0, 644 x 192 x 4992 12.0 -> 7.0, 263 x 256 x 448 4.5 -> 4.0; 3 x 3 x 512 filters on 7 x 7 x 7 images 11.2 ->
+//    7.2, x 256 on 4 x 15 x 15 7.9 -> 6.1;
+//  * 32 x 64: 400 x 768 x 3072 9.9 -> 7.4, 438 x 640 x 2368 9.1 -> 6.8, 335 x 1152 x 320 4.4 -> 4.3, 32 x 9600 x 1600
+//    8.1 -> 6.8; with up to three rows of tiles in four empty and 5376 of k 14.3 -> 14.8 (81 x 4672);
+//  * 64 x 64 from 1280 of k on: 1000 x 768 x 3072 9.9 -> 9.05, 1155 x 640 x 1344 7.05 -> 6.55; 1933 x 512 x 1136 5.8 /
+//    6.7.  Of convolutions from 4096 of k on (3 x 3 x 512 on 28 x 8 x 8 13.5 -> 11.9, x 256 on 15 x 13 x 13 8.3 / 8.7:
+//    more instructions a load).
+// Launches of more tiles lose (two rounds; one workgroup to a compute unit).  int8 rows off 16 bytes and 8192 of k
+// and more stay with the tiles below, whose tests name them (343 x 513 x 2304 9.5 / 7.7, 256 x 512 x 8192 15.4 / 9.1).
+int pick_wave(int64_t M, int64_t N, int64_t K, bool conv, int out_bytes) {
+  if ((out_bytes == 1 && N % 16 != 0) || K >= 8192) return -1;
+  const int64_t cus = compute_units();
+  auto tiles = [&](int v) { return ceil_div(M, kVariants[v].bm) * ceil_div(N, kVariants[v].bn); };
+  if (tiles(kWave32) <= cus) return K >= 1024 ? kWave32 : kWave32w4;
+  if (tiles(kWave32x64) <= cus) return kWave32x64;
+  if (tiles(kWave64) <= cus && K >= (conv ? 4096 : 1280)) return kWave64;
+  return -1;
+}
+
+// Estimated us of a launch on one round of such tiles, and on the small-M kernel: least squares over 210 and
+// 300 launches (M 3 .. 300 / .. 2500, N 64 .. 12000, K 256 .. 8192), standard error 5 to 7 %.  Per wave-tiled
+// workgroup and in all, the bytes it loads.
+double wave_us(int v, int64_t M, int64_t N, int64_t K) {
+  const double each = (double)(kVariants[v].bm + kVariants[v].bn) * (double)K * 1e-6;    // MB
+  const double all = each * (double)(ceil_div(M, kVariants[v].bm) * ceil_div(N, kVariants[v].bn));
+  switch (v) {
+    case kWave64: return 4.50 + 7.8 * each + 0.032 * all;
+    case kWave32x64: return 3.86 + 7.5 * each + 0.041 * all;
+    case kWave32: return 3.86 + 6.6 * each + 0.034 * all;
+    default: return 3.75 + 7.9 * each + 0.031 * all;
+  }
+}
+double skinny_us(int64_t M, int64_t N, int64_t K) {
+  const int mt = skinny_row_tiles(M, N, K);
+  const double groups = (double)(ceil_div(M, 16 * mt) * ceil_div(N, 16));
+  return 3.03 + 0.066e-6 * groups * (double)(16 + 16 * mt) * (double)K + 0.285e-3 * (double)K + 0.09e-3 * groups;
+}
+
+int pick_variant(int64_t M, int64_t N, int64_t K, bool pipe, int out_bytes, int wave) {
+  if (pipe && wave >= 0) return wave;
   auto tiles = [&](int v) { return ceil_div(M, kVariants[v].bm) * ceil_div(N, kVariants[v].bn); };
   if (pipe) {
     const int64_t cus = compute_units();
@@ -513,23 +555,21 @@ int pick_variant(int64_t M, int64_t N, int64_t K, bool pipe, int out_bytes = 1) 
   return 3;
 }
 
-// The small-M kernel up to kSkinnyMaxM rows -- except against weights wide enough to give the
-// 64 x 64 tile with its k range split over two wave groups a workgroup for every second compute
-// unit or more: its time hardly depends on M, the small-M kernel's grows with it.  From 17 rows
-// at 128 tiles (M = 32, 8192 x 8192 weights: 18.5 against 24.6 us; 4096 x 4096: 9.1 against
-// 8.5), from 9 rows at 144 (M = 16, 4096 -> 11008: 12.0 against 14.2 us; at 128 tiles, 8192^2,
-// 18.7 against 17.9), from 3 rows at 224 (M = 4, 4096 -> 16384: 13.2 against 15.1 us; M = 16,
-// 8192 -> 16384: 22.0 against 32.0) -- and the tiled kernels above.
-int pick_any(int64_t M, int64_t N, int64_t K, bool pipe, int out_bytes) {
-  if (M <= kSkinnyMaxM) {
+// The small-M kernel up to kSkinnyMaxM rows and where skinny_takes_rows says so, unless one round of
+// tiles on waves of their own is estimated a tenth faster (34 x 3232 x 5392 16.4 -> 10.4 us, 118 x 1536 x 5248 13.2
+// -> 7.5, 72 x 2560 x 2432 6.9 -> 5.2) -- and the tiled kernels above.  Weights too wide for one round: from 3 rows
+// at 224 tiles of 64 channels on, the 64 x 64 tile with its k range split over two wave groups a workgroup, whose
+// time hardly depends on M (M = 16, 8192 -> 16384: 22.0 against 32.0).  `waves`: whether the operands are such
+// as those kernels take.
+int pick_any(int64_t M, int64_t N, int64_t K, bool pipe, int out_bytes, bool waves = true) {
+  const int wave = pipe && waves ? pick_wave(M, N, K, false, out_bytes) : -1;
+  if (wave < 0 && pipe && K >= 2048 && M <= kSkinnyMaxM) {
     const int64_t t64 = ceil_div(N, 64);
-    if (pipe && K >= 2048 &&
-        ((M > 16 && t64 >= 128) || (M >= 9 && t64 >= 144) || (M >= 3 && t64 >= 224)))
-      return pick_k_split64(M, N, K);
-    return kSkinnyVariant;
+    if ((M > 16 && t64 >= 128) || (M >= 9 && t64 >= 144) || (M >= 3 && t64 >= 224)) return pick_k_split64(M, N, K);
   }
-  if (skinny_takes_rows(M, N, K)) return kSkinnyVariant;
-  return pick_variant(M, N, K, pipe, out_bytes);
+  if (skinny_takes_rows(M, N, K))
+    return wave >= 0 && wave_us(wave, M, N, K) < 0.9 * skinny_us(M, N, K) ? wave : kSkinnyVariant;
+  return pick_variant(M, N, K, pipe, out_bytes, wave);
 }
 
 // Whether a 3x3 stride-1 convolution goes to the kernel that keeps the input patch in LDS
@@ -793,7 +833,7 @@ int qgemm_impl(int variant, const int8_t* A, int64_t lda, const int8_t* W, int64
     p.zx = zx;
     p.zw = zw;
     p.kzz = (int)((uint32_t)K * (uint32_t)zx * (uint32_t)zw);
-    const int v = pick_any(M, N, Kp, ragged_ok(p), es);
+    const int v = pick_any(M, N, Kp, ragged_ok(p), es, false);
     if (v == kSkinnyVariant) return launch_epi<false>(v, p, epilogue, st);
     // (rows at odd bytes: each load is served in pieces, about 0.25 us per k tile -- 777 x 1504, 1000
     // of k at any multiple of four 8.3 us, at odd bytes 11.5, copied first 12; 1000 x 768 with 3073
@@ -1517,7 +1557,7 @@ int qconv2d_impl(int variant, const int8_t* in, const int64_t in_sizes[4], const
       const int c = pick_direct_conv(NB, Ho * Wo, Ci, Co);
       if (c >= 0 && direct_conv_plan(c, &d)) return launch_direct_conv(c, epilogue, d, st);
     }
-    variant = pick_variant(Mg, Co, Kg, pipe_ok(256, 256, p, true), es);
+    variant = pick_variant(Mg, Co, Kg, pipe_ok(256, 256, p, true), es, pick_wave(Mg, Co, Kg, true, es));
     // (the persistent forms are tuned for the plain GEMM: with the convolution's row geometry
     // on top they run out of registers)
     if (variant == kPersist256) variant = kPipe256w8;

@@ -878,6 +878,30 @@ __global__ void __launch_bounds__(WM* WN * 64) qgemm_mfma_kernel(const MainParam
   mfma_epilogue<EPI, FM, FN, NT, BN>(acc, p.epi, smem, m0 + wm * TM, n0 + wn * TN, n0);
 }
 
+// The same in two halves, for a kernel whose loads are counted by hand: the loads, ahead of the first of
+// those, and the arithmetic, which must not be moved to where it would wait for all of them.
+template <int EPI, int NT, int BN>
+struct EarlyColRaw {
+  static constexpr int kPerThread = (BN + NT - 1) / NT;
+  ColRaw raw[kPerThread];
+  __device__ __forceinline__ void request(const EpiParams& e, int n_blk0) {
+#pragma unroll
+    for (int i = 0; i < kPerThread; ++i) {
+      raw[i] = ColRaw{1.f, 1.f, 1.f, 0};
+      if ((int)(threadIdx.x & ~63u) + i * NT >= BN) continue;
+      const int n = n_blk0 + (int)threadIdx.x + i * NT;
+      raw[i] = col_fetch<EPI>(e, n < e.N ? n : e.N - 1);
+    }
+  }
+  __device__ __forceinline__ void finish(const EpiParams& e, ColParams (&c)[kPerThread]) {
+#pragma unroll
+    for (int i = 0; i < kPerThread; ++i) {
+      asm volatile("" : "+v"(raw[i].sx), "+v"(raw[i].sw), "+v"(raw[i].so), "+v"(raw[i].bias));
+      c[i] = col_finish<EPI>(e, raw[i]);
+    }
+  }
+};
+
 // Epilogue shared by the MFMA kernels.  Accumulator v of fragment (i,j) belongs to
 // output row m_wave0 + i*32 + lane%32 and channel n_wave0 + j*32 + 8*(v/4) +
 // 4*(lane/32) + v%4.

@@ -14,6 +14,7 @@
 #include "qgemm_pipelined.h"
 #include "qgemm_persistent.h"
 #include "qgemm_skinny.h"
+#include "qgemm_wave.h"
 
 #pragma clang fp contract(off)
 
@@ -65,6 +66,11 @@ inline constexpr Variant kVariants[] = {
     // a filter slice held in registers (3 x 3 or 1 x 1 on 64 or 128 channels), pixel tile chosen
     // per problem (convolution only, int8 results)
     {"stream", 32, 64, 32, 512},
+    // k tiles dealt out over the waves of a workgroup, which share nothing until the end
+    {"wave_64x64_w4", 64, 64, 128, 256},
+    {"wave_32x64_w4", 32, 64, 128, 256},
+    {"wave_32x32_w8", 32, 32, 128, 512},
+    {"wave_32x32_w4", 32, 32, 128, 256},
 };
 constexpr int kPipe256 = 4, kPipe128 = 5, kPipe64 = 6, kPipe256x64 = 7;
 constexpr int kPipe64k2 = 8;
@@ -76,6 +82,7 @@ constexpr int kPipe256x192 = 16, kPersist256x192 = 17;
 constexpr int kDirectConv2 = 18;   // the third direct variant (configuration 2)
 constexpr int kPipe64k4 = 19;
 constexpr int kStreamConv = 20;
+constexpr int kWave64 = 21, kWave32x64 = 22, kWave32 = 23, kWave32w4 = 24;
 // largest M the heuristic hands to the small-M kernel
 constexpr int64_t kSkinnyMaxM = 32;
 // Above that many rows the small-M kernel still beats the 64 x 64 tiles while its workgroups
@@ -91,10 +98,11 @@ inline bool skinny_takes_rows(int64_t M, int64_t N, int64_t K) {
   return units <= (K >= 2048 ? 3072 : 1024);
 }
 
+inline bool is_wave_variant(int v) { return v == kWave64 || v == kWave32x64 || v == kWave32 || v == kWave32w4; }
 inline bool is_pipe_variant(int v) {
   return v == kPipe256 || v == kPipe128 || v == kPipe64 || v == kPipe256x64 || v == kPipe64k2 ||
          v == kPipe64k4 || v == kPipe256w8 || v == kPipe128w8 || v == kPersist256 ||
-         v == kPersist128 || v == kPipe256x192 || v == kPersist256x192;
+         v == kPersist128 || v == kPipe256x192 || v == kPersist256x192 || is_wave_variant(v);
 }
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
@@ -139,6 +147,19 @@ int launch_pipe(const MainParams& p, hipStream_t st) {
   return check_hip(hipGetLastError(), "qgemm_pipe launch");
 }
 
+template <int FM, int FN, int NW, int STAGES, bool CONV, int EPI, bool ROWMAP = false, bool ZP = false>
+int launch_wave(const MainParams& p, hipStream_t st) {
+  constexpr int lds = qgemm_wave_lds(FM, FN, NW, STAGES);
+  static_assert(lds >= FM * FN * (NW - 1) * 4096 && lds >= NW * 4096 + FN * 32 * 12 + 256, "sums, staging of the results");
+  DQ8_REQUIRE(pipe_ok(32 * FM, 32 * FN, p, CONV) && (!ROWMAP || p.conv_bytes < (1LL << 31)),
+              "qgemm on waves of their own needs K % 16 == 0 and operands that fit 32-bit buffer offsets");
+  auto kern = qgemm_wave_kernel<FM, FN, NW, STAGES, CONV, EPI, ROWMAP, ZP>;
+  static std::atomic<uint64_t> lds_allowed{0};
+  if (int s = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds, &lds_allowed)) return s;
+  hipLaunchKernelGGL(kern, dim3(p.tiles_m * p.tiles_n), dim3(NW * 64), lds, st, p);
+  return check_hip(hipGetLastError(), "qgemm_wave launch");
+}
+
 // `per_cu`: workgroups of this shape a compute unit holds at a time
 template <int BM, int BN, int WM, int WN, bool CONV, int EPI>
 int launch_persist(const MainParams& p, int per_cu, hipStream_t st) {
@@ -177,6 +198,14 @@ int launch_gemv_t(const MainParams& p, hipStream_t st) {
   return check_hip(hipGetLastError(), "qgemm_gemv launch");
 }
 
+// Row tiles of 16 that a workgroup of the small-M kernel takes (see launch_skinny): no more than there
+// are (4 x 5120 -> 4736, 24 MB of weights, with four row tiles of which three are empty 14.5 us, with one 9.3)
+inline int skinny_row_tiles(int64_t M, int64_t N, int64_t K) {
+  int mt = 1;
+  while (mt < 4 && M > 16 * mt && ceil_div(M, 16 * mt) * N * K > (20LL << 20)) mt *= 2;
+  return mt;
+}
+
 // rows per workgroup grow with M (fewer passes over W), waves with the depth of K
 template <int EPI>
 int launch_skinny(const MainParams& p, hipStream_t st) {
@@ -191,13 +220,11 @@ int launch_skinny(const MainParams& p, hipStream_t st) {
   // Waves: four, eight from 1024 of k on (M = 16, 3072 -> 768: 4.1 against 4.3 us).  Row tiles
   // of 16 per workgroup: one, i.e. as many workgroups as possible, while the weights, which
   // every block of rows streams again, stay below about 20 MB over all its passes; else two or
-  // four (us per launch, graph replays, for (waves, row tiles) = (4,1) (4,2) (4,4) / (8,1) (8,2)
+  // four, as far as there are rows for them (us per launch, graph replays, for (waves, row tiles) = (4,1) (4,2) (4,4) / (8,1) (8,2)
   // (8,4): M = 64, 768 -> 768: 3.2 3.9 4.9; M = 256, 768 -> 3072: 7.3 7.0 7.5; M = 32, 4096^2:
   // 7.2 6.3 7.3 (eight waves); M = 64, 4096^2: 10.7 9.4 8.7; M = 128, 3072 -> 768: 5.7 5.0 6.8).
   const bool deep = p.K >= 1024;
-  const int64_t weight_bytes = (int64_t)p.N * p.K;
-  int mt = 1;
-  while (mt < 4 && ceil_div(p.M, 16 * mt) * weight_bytes > (20LL << 20)) mt *= 2;
+  const int mt = skinny_row_tiles(p.M, p.N, p.K);
   // k-steps a wave keeps in flight: as many as it has altogether up to six -- a batch that is
   // not full still issues all its loads (3072 of k on eight waves, six steps each: 4.1 -> 3.8 us
   // at M = 16, 7.5 -> 6.9 at M = 256; 768 of k on four waves, three steps: M = 128, -> 3072 5.4 ->
@@ -258,6 +285,10 @@ int launch_variant(int variant, MainParams& p, hipStream_t st) {
     case kPipe256w8: return launch_pipe<256, 256, 2, 4, 1, CONV, EPI>(p, st);
     case kPipe128w8: return launch_pipe<128, 128, 2, 4, 1, CONV, EPI>(p, st);
     case kPipe256x192: return launch_pipe<256, 192, 4, 2, 1, CONV, EPI>(p, st);
+    case kWave64: return launch_wave<2, 2, 4, 2, CONV, EPI>(p, st);
+    case kWave32x64: return launch_wave<1, 2, 4, 2, CONV, EPI>(p, st);
+    case kWave32: return launch_wave<1, 1, 8, 2, CONV, EPI>(p, st);
+    case kWave32w4: return launch_wave<1, 1, 4, 4, CONV, EPI>(p, st);
   }
   if constexpr (!CONV) {   // GEMM only: the small-M kernel and the persistent forms
     if (variant == kSkinnyVariant) return launch_skinny<EPI>(p, st);
@@ -277,7 +308,7 @@ int launch_variant(int variant, MainParams& p, hipStream_t st) {
 // any length and alignment (qgemm_launch_zp_*.hip).
 inline bool zp_has_variant(int variant) {
   return variant == kPipe64 || variant == kPipe64k2 || variant == kPipe64k4 || variant == kPipe128 ||
-         variant == kPipe128w8 || variant == kPipe256w8 || variant == kPipe256x192;
+         variant == kPipe128w8 || variant == kPipe256w8 || variant == kPipe256x192 || is_wave_variant(variant);
 }
 inline bool ragged_has_variant(int variant) {
   return variant == kPipe64 || variant == kPipe64k2 || variant == kPipe64k4;
@@ -305,6 +336,10 @@ int launch_zp_ragged(int variant, MainParams& p, hipStream_t st) {
     case kPipe128w8: return launch_pipe<128, 128, 2, 4, 1, false, EPI, false, true>(p, st);
     case kPipe256w8: return launch_pipe<256, 256, 2, 4, 1, false, EPI, false, true>(p, st);
     case kPipe256x192: return launch_pipe<256, 192, 4, 2, 1, false, EPI, false, true>(p, st);
+    case kWave64: return launch_wave<2, 2, 4, 2, false, EPI, false, true>(p, st);
+    case kWave32x64: return launch_wave<1, 2, 4, 2, false, EPI, false, true>(p, st);
+    case kWave32: return launch_wave<1, 1, 8, 2, false, EPI, false, true>(p, st);
+    case kWave32w4: return launch_wave<1, 1, 4, 4, false, EPI, false, true>(p, st);
   }
   return fail("no kernel with a zero point in the k loop for this variant");
 }
@@ -313,7 +348,7 @@ int launch_zp_ragged(int variant, MainParams& p, hipStream_t st) {
 // next to the convolution kernels: CONV true; the GEMM files carry a stub).
 inline bool rowmap_has_variant(int variant) {
   return variant == kPipe128 || variant == kPipe128w8 || variant == kPipe64 || variant == kPipe64k2 ||
-         variant == kPipe256w8 || variant == kPipe256x192;
+         variant == kPipe256w8 || variant == kPipe256x192 || is_wave_variant(variant);
 }
 template <bool CONV, int EPI>
 int launch_rowmap(int variant, MainParams& p, hipStream_t st) {
@@ -328,6 +363,10 @@ int launch_rowmap(int variant, MainParams& p, hipStream_t st) {
       case kPipe64k2: return launch_pipe<64, 64, 2, 2, 2, false, EPI, true>(p, st);
       case kPipe256w8: return launch_pipe<256, 256, 2, 4, 1, false, EPI, true>(p, st);
       case kPipe256x192: return launch_pipe<256, 192, 4, 2, 1, false, EPI, true>(p, st);
+      case kWave64: return launch_wave<2, 2, 4, 2, false, EPI, true>(p, st);
+      case kWave32x64: return launch_wave<1, 2, 4, 2, false, EPI, true>(p, st);
+      case kWave32: return launch_wave<1, 1, 8, 2, false, EPI, true>(p, st);
+      case kWave32w4: return launch_wave<1, 1, 4, 4, false, EPI, true>(p, st);
     }
   }
   return fail("no kernel with rows mapped to pixels for this variant");

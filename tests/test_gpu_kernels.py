@@ -2722,6 +2722,48 @@ def test_fused_operators_behind_a_zero_point_in_the_k_loop(K, shape, kernel):
         _fused_forms_equal_the_separate_operators(K, a, w, zx, rng)
 
 
+# and of the tiles whose k tiles are dealt out over the waves: fewer k tiles than waves, one more than whole
+# rounds of them, rows and channels that end inside a tile
+WAVE_TILES = [((300, 272, 96), "wave_32x32_w4"), ((410, 560, 528), "wave_32x32_w4"), ((343, 512, 2064), "wave_32x32_w8"),
+              ((335, 1168, 320), "wave_32x64_w4"), ((519, 848, 1040), "wave_32x64_w4"), ((1100, 784, 2064), "wave_64x64_w4")]
+
+
+@pytest.mark.parametrize("shape,kernel", WAVE_TILES, ids=["%s-%d" % (t[1], t[0][2]) for t in WAVE_TILES])
+def test_fused_operators_behind_k_tiles_dealt_out_over_the_waves(K, shape, kernel):
+    m, n, k = shape
+    assert K._lib.lib().dq8_qgemm_kernel_name(m, n, k, 1).decode() == kernel
+    rng = np.random.default_rng(m + n + k)
+    a, w = dev(rng.integers(-128, 128, (m, k), dtype=np.int8)), dev(rng.integers(-128, 128, (n, k), dtype=np.int8))
+    for zx in (0, -11):
+        _fused_forms_equal_the_separate_operators(K, a, w, zx, rng)
+
+
+@pytest.mark.parametrize("nb,h,w_,ci,co,kk,stride,pad,dil", [
+    (1, 7, 7, 16, 32, 1, 1, 0, 1), (2, 9, 11, 48, 72, 3, 1, 1, 1), (3, 7, 7, 512, 48, 3, 1, 1, 1),
+    (1, 13, 10, 80, 33, 3, 2, 1, 1), (2, 12, 9, 32, 64, 5, 1, 2, 1), (1, 15, 15, 208, 96, 3, 1, 2, 2),
+    (5, 14, 14, 256, 65, 1, 2, 0, 1), (2, 20, 6, 144, 40, 2, 3, 1, 1)])
+def test_convolutions_on_k_tiles_dealt_out_over_the_waves(K, nb, h, w_, ci, co, kk, stride, pad, dil):
+    """Forced, against the generic kernel: taps in the padding, a k tile that begins inside a tap (the tap of a
+    wave's next tile is had by additions, several taps and a row of the filter on), images that end inside a
+    tile; and as the library runs them (a strided 1 x 1 filter as a GEMM over its pixels)."""
+    rng = np.random.default_rng(h * w_ + ci + co + kk)
+    x = dev(rng.integers(-128, 128, (nb, h, w_, ci), dtype=np.int8))
+    wt = dev(rng.integers(-128, 128, (co, kk, kk, ci), dtype=np.int8))
+    ho = (h + 2 * pad - dil * (kk - 1) - 1) // stride + 1
+    wo = (w_ + 2 * pad - dil * (kk - 1) - 1) // stride + 1
+    md = list(O.NHWC_OHWI_METADATA) + [stride, stride, dil, dil, 1]
+    sc = dict(sx=dev(np.array([0.02], np.float32)), sw=dev(rng.uniform(0.001, 0.05, co).astype(np.float32)),
+              so=dev(np.array([0.5], np.float32)), bias=dev(rng.standard_normal(co).astype(np.float32)))
+    waves = [i for i, nm in enumerate(K.variant_names()) if nm.startswith("wave_")]
+    assert len(waves) == 4
+    for epi in (K.EPI_ACC_S32, K.EPI_REQUANT_CPU, K.EPI_REQUANT_CPU_DEQUANT_F32):
+        kw = {} if epi == K.EPI_ACC_S32 else sc
+        want = K.qconv2d(x, wt, [pad] * 4, md, [nb, ho, wo, co], epi, variant=0, **kw)
+        for v in waves + [-1]:
+            got = K.qconv2d(x, wt, [pad] * 4, md, [nb, ho, wo, co], epi, variant=v, **kw)
+            assert torch.equal(got, want), (v, epi)
+
+
 # the same for operand rows of any length and alignment; K rounded up to 16 names the tile
 RAGGED_TILES = [((300, 261, 90), "pipe_64x64x128"), ((260, 130, 1001), "pipe_64x64x128"),
                 ((1100, 770, 2058), "pipe_64x64x128_k2"), ((320, 513, 8204), "pipe_64x64x128_k4"),
