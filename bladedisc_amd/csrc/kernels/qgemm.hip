@@ -445,38 +445,49 @@ int pick_k_split64(int64_t M, int64_t N, int64_t K) {
 //  * 64 x 64 from 1280 of k on: 1000 x 768 x 3072 9.9 -> 9.05, 1155 x 640 x 1344 7.05 -> 6.55; 1933 x 512 x 1136 5.8 /
 //    6.7.  Of convolutions from 4096 of k on (3 x 3 x 512 on 28 x 8 x 8 13.5 -> 11.9, x 256 on 15 x 13 x 13 8.3 / 8.7:
 //    more instructions a load).
-// Launches of more tiles lose (two rounds; one workgroup to a compute unit).  int8 rows off 16 bytes and 8192 of k
-// and more stay with the tiles below, whose tests name them (343 x 513 x 2304 9.5 / 7.7, 256 x 512 x 8192 15.4 / 9.1).
+//  * 96 x 64 where the 64 x 64 ones are just more than a round, from 2048 of k on: 1300 x 1024 x 3072 12.9 -> 11.3,
+//    777 x 1504 x 5120 18.8 -> 16.0; 4-byte results from 2560 on (1300 x 1024 x 3072 14.1 -> 13.05, x 2048 10.85 / 10.85).
+// Launches of more tiles lose (two rounds; one workgroup to a compute unit).  int8 rows off 16 bytes, whose stores
+// are dearer: from 1024 of k on, 64 x 64 from 2304, 96 x 64 from 2560 (258 x 159 x 3072 9.2 -> 4.9 small-M, 1048 x 187 x 1920
+// 9.3 -> 5.4, 1000 x 1002 x 1536 8.6 / 7.2).  8192 of k and more stay with the tiles below.
 int pick_wave(int64_t M, int64_t N, int64_t K, bool conv, int out_bytes) {
-  if ((out_bytes == 1 && N % 16 != 0) || K >= 8192) return -1;
+  const bool off16 = out_bytes == 1 && N % 16 != 0;
+  if (K >= 8192 || (off16 && (conv || K < 1024))) return -1;
   const int64_t cus = compute_units();
   auto tiles = [&](int v) { return ceil_div(M, kVariants[v].bm) * ceil_div(N, kVariants[v].bn); };
   if (tiles(kWave32) <= cus) return K >= 1024 ? kWave32 : kWave32w4;
   if (tiles(kWave32x64) <= cus) return kWave32x64;
-  if (tiles(kWave64) <= cus && K >= (conv ? 4096 : 1280)) return kWave64;
+  if (tiles(kWave64) <= cus) return K >= (conv ? 4096 : off16 ? 2304 : 1280) ? kWave64 : -1;
+  if (tiles(kWave96x64) <= cus && !conv && K >= (off16 || out_bytes == 4 ? 2560 : 2048)) return kWave96x64;
   return -1;
 }
 
-// Estimated us of a launch on one round of such tiles, and on the small-M kernel: least squares over 210 and
-// 300 launches (M 3 .. 300 / .. 2500, N 64 .. 12000, K 256 .. 8192), standard error 5 to 7 %.  Per wave-tiled
-// workgroup and in all, the bytes it loads.
-double wave_us(int v, int64_t M, int64_t N, int64_t K) {
-  const double each = (double)(kVariants[v].bm + kVariants[v].bn) * (double)K * 1e-6;    // MB
+// Estimated us of a launch on one round of such tiles, and on the small-M kernel: least squares over 11000 and 2400
+// launches (M 3 .. 16384 / .. 300, N 64 .. 5000, K 128 .. 5000), standard error 7 to 10 %.  Of a tile, the MB it
+// loads; of the launch, those of all tiles and of its result.  Rows that begin inside a 128-byte line are read
+// with a line more to a k tile, and one that another wave reads as well (1000 x 768: 3072 of k 8.65, 3136 9.8, 3088 10.6).
+double wave_us(int v, int64_t M, int64_t N, int64_t K, int out_bytes) {
+  const double each = (double)(kVariants[v].bm + kVariants[v].bn) * (double)K * 1e-6;
   const double all = each * (double)(ceil_div(M, kVariants[v].bm) * ceil_div(N, kVariants[v].bn));
+  const double out = (double)M * (double)N * out_bytes * 1e-6;
+  const int lines = K % 128 == 0 ? 0 : K % 64 == 0 ? 1 : 2;
+  const double more = (lines == 0 ? 0.0 : lines == 1 ? 0.6 : 1.15) * each + (lines == 0 ? 0.0 : lines == 1 ? 0.0125 : 0.020) * all +
+                      (out_bytes == 1 && N % 16 != 0 ? 0.55 : 0.0);
   switch (v) {
-    case kWave64: return 4.50 + 7.8 * each + 0.032 * all;
-    case kWave32x64: return 3.86 + 7.5 * each + 0.041 * all;
-    case kWave32: return 3.86 + 6.6 * each + 0.034 * all;
-    default: return 3.75 + 7.9 * each + 0.031 * all;
+    case kWave64: return more + 4.04 + 8.46 * each + 0.026 * all + 0.33 * out;
+    case kWave96x64: return more + 4.80 + 10.6 * each + 0.014 * all + 0.60 * out;
+    case kWave32x64: return more + 3.44 + 8.42 * each + 0.029 * all + 0.65 * out;
+    case kWave32: return more + 3.39 + 7.61 * each + 0.030 * all + 1.26 * out;
+    default: return more + 3.25 + 9.49 * each + 0.024 * all + 1.26 * out;
   }
 }
 double skinny_us(int64_t M, int64_t N, int64_t K) {
   const int mt = skinny_row_tiles(M, N, K);
   const double groups = (double)(ceil_div(M, 16 * mt) * ceil_div(N, 16));
-  return 3.03 + 0.066e-6 * groups * (double)(16 + 16 * mt) * (double)K + 0.285e-3 * (double)K + 0.09e-3 * groups;
+  return 2.31 + 0.0828e-6 * groups * (double)(16 + 16 * mt) * (double)K + 0.415e-3 * (double)K + 0.445e-3 * groups;
 }
 
-int pick_variant(int64_t M, int64_t N, int64_t K, bool pipe, int out_bytes, int wave) {
+int pick_variant(int64_t M, int64_t N, int64_t K, bool pipe, int out_bytes, int wave, bool conv = false) {
   if (pipe && wave >= 0) return wave;
   auto tiles = [&](int v) { return ceil_div(M, kVariants[v].bm) * ceil_div(N, kVariants[v].bn); };
   if (pipe) {
@@ -512,9 +523,9 @@ int pick_variant(int64_t M, int64_t N, int64_t K, bool pipe, int out_bytes, int 
     } else if (big256) {
       return kPipe256w8;
     }
-    // 128x128: eight waves while every tile has a compute unit to itself (more waves to cover
-    // the load latency: 6.3 against 7.1 us at M = 2048, 768 -> 768); with two tiles on a
-    // compute unit, or a deep K, four waves (10.0 against 11.2 us at M = 2048, 768 -> 3072)
+    // 128x128: eight waves (more waves to cover the load latency; over 700 products of more than a tile per
+    // compute unit 4 % faster than four, int8 rows off 16 bytes 18 %: 3485 x 1903 x 336 18.6 -> 13.9 us); four
+    // for a deep K, and for implicit-GEMM convolutions of more than a tile per compute unit
     const int64_t t128 = tiles(kPipe128);
     // 128 x 128 tiles, two to a compute unit, that end in a round of a few tiles (at most a
     // quarter of a round) pay a whole k loop for them: the larger tiles, whichever the estimate
@@ -539,8 +550,11 @@ int pick_variant(int64_t M, int64_t N, int64_t K, bool pipe, int out_bytes, int 
       // M = 256, 8192^2 weights: 28.5 against 33.1 us; M = 512, 4096^2: 16.4 against 18.0)
       if (K >= 4096)
         return (t128 < cus && tiles(kPipe64) <= 2 * cus) ? pick_k_split64(M, N, K) : kPipe128;
-      if (out_bytes == 1) return t128 <= cus ? kPipe128w8 : kPipe128;
-      return t128 > 2 * cus ? kPersist128 : kPipe128w8;
+      // (at most two 64 x 64 tiles to a compute unit: those, 2000 x 1024 x 768 6.9 -> 6.2 us, x 3072 14.8 -> 13.5, f32 results of
+      // 900 x 2048 x 768 8.5 -> 7.2; wide weights past 2048 of k are read by too many of them, 438 x 4032 x 2048 11.0 / 11.6)
+      if (!conv && tiles(kPipe64) <= 2 * cus && (K < 2048 || N <= 3 * M)) return kPipe64;
+      if (conv && out_bytes == 1 && t128 > cus) return kPipe128;
+      return out_bytes == 4 && t128 > 2 * cus ? kPersist128 : kPipe128w8;
     }
     // (64 x 64 tiles: the k range split over two wave groups while they come to at most one per
     // compute unit, from 4096 of k on at most two -- M = 384, 11008 -> 4096: 37.0 against 40.1 us)
@@ -555,10 +569,12 @@ int pick_variant(int64_t M, int64_t N, int64_t K, bool pipe, int out_bytes, int 
   return 3;
 }
 
-// The small-M kernel up to kSkinnyMaxM rows and where skinny_takes_rows says so, unless one round of
-// tiles on waves of their own is estimated a tenth faster (34 x 3232 x 5392 16.4 -> 10.4 us, 118 x 1536 x 5248 13.2
-// -> 7.5, 72 x 2560 x 2432 6.9 -> 5.2) -- and the tiled kernels above.  Weights too wide for one round: from 3 rows
-// at 224 tiles of 64 channels on, the 64 x 64 tile with its k range split over two wave groups a workgroup, whose
+// Up to 320 rows (256 for int8 rows off 16 bytes) the estimates decide between one round of tiles on waves of their
+// own and the small-M kernel (34 x 3232 x 5392 16.4 -> 10.4 us, 118 x 1536 x 5248 13.2 -> 7.5, 258 x 208 x 128 4.15 -> 2.6
+// small-M, 89 x 3200 x 576 5.6 -> 4.3): over 2000 launches 0.5 % slower than the better of the two, 1.3 % (int8 rows off 16
+// bytes 4) with the rows' limits below.  Without such a round: the small-M kernel up to
+// kSkinnyMaxM rows and where skinny_takes_rows says so, and the tiled kernels above.  Weights too wide for one round: from 3
+// rows at 224 tiles of 64 channels on, the 64 x 64 tile with its k range split over two wave groups a workgroup, whose
 // time hardly depends on M (M = 16, 8192 -> 16384: 22.0 against 32.0).  `waves`: whether the operands are such
 // as those kernels take.
 int pick_any(int64_t M, int64_t N, int64_t K, bool pipe, int out_bytes, bool waves = true) {
@@ -567,8 +583,9 @@ int pick_any(int64_t M, int64_t N, int64_t K, bool pipe, int out_bytes, bool wav
     const int64_t t64 = ceil_div(N, 64);
     if ((M > 16 && t64 >= 128) || (M >= 9 && t64 >= 144) || (M >= 3 && t64 >= 224)) return pick_k_split64(M, N, K);
   }
-  if (skinny_takes_rows(M, N, K))
-    return wave >= 0 && wave_us(wave, M, N, K) < 0.9 * skinny_us(M, N, K) ? wave : kSkinnyVariant;
+  if (wave >= 0 && M <= (out_bytes == 1 && N % 16 != 0 ? 256 : 320))
+    return 1.05 * wave_us(wave, M, N, K, out_bytes) < skinny_us(M, N, K) ? wave : kSkinnyVariant;
+  if (wave < 0 && skinny_takes_rows(M, N, K)) return kSkinnyVariant;
   return pick_variant(M, N, K, pipe, out_bytes, wave);
 }
 
@@ -1557,7 +1574,7 @@ int qconv2d_impl(int variant, const int8_t* in, const int64_t in_sizes[4], const
       const int c = pick_direct_conv(NB, Ho * Wo, Ci, Co);
       if (c >= 0 && direct_conv_plan(c, &d)) return launch_direct_conv(c, epilogue, d, st);
     }
-    variant = pick_variant(Mg, Co, Kg, pipe_ok(256, 256, p, true), es, pick_wave(Mg, Co, Kg, true, es));
+    variant = pick_variant(Mg, Co, Kg, pipe_ok(256, 256, p, true), es, pick_wave(Mg, Co, Kg, true, es), true);
     // (the persistent forms are tuned for the plain GEMM: with the convolution's row geometry
     // on top they run out of registers)
     if (variant == kPersist256) variant = kPipe256w8;

@@ -71,6 +71,7 @@ inline constexpr Variant kVariants[] = {
     {"wave_32x64_w4", 32, 64, 128, 256},
     {"wave_32x32_w8", 32, 32, 128, 512},
     {"wave_32x32_w4", 32, 32, 128, 256},
+    {"wave_96x64_w4", 96, 64, 128, 256},
 };
 constexpr int kPipe256 = 4, kPipe128 = 5, kPipe64 = 6, kPipe256x64 = 7;
 constexpr int kPipe64k2 = 8;
@@ -82,7 +83,7 @@ constexpr int kPipe256x192 = 16, kPersist256x192 = 17;
 constexpr int kDirectConv2 = 18;   // the third direct variant (configuration 2)
 constexpr int kPipe64k4 = 19;
 constexpr int kStreamConv = 20;
-constexpr int kWave64 = 21, kWave32x64 = 22, kWave32 = 23, kWave32w4 = 24;
+constexpr int kWave64 = 21, kWave32x64 = 22, kWave32 = 23, kWave32w4 = 24, kWave96x64 = 25;
 // largest M the heuristic hands to the small-M kernel
 constexpr int64_t kSkinnyMaxM = 32;
 // Above that many rows the small-M kernel still beats the 64 x 64 tiles while its workgroups
@@ -98,7 +99,7 @@ inline bool skinny_takes_rows(int64_t M, int64_t N, int64_t K) {
   return units <= (K >= 2048 ? 3072 : 1024);
 }
 
-inline bool is_wave_variant(int v) { return v == kWave64 || v == kWave32x64 || v == kWave32 || v == kWave32w4; }
+inline bool is_wave_variant(int v) { return v >= kWave64 && v <= kWave96x64; }
 inline bool is_pipe_variant(int v) {
   return v == kPipe256 || v == kPipe128 || v == kPipe64 || v == kPipe256x64 || v == kPipe64k2 ||
          v == kPipe64k4 || v == kPipe256w8 || v == kPipe128w8 || v == kPersist256 ||
@@ -149,8 +150,8 @@ int launch_pipe(const MainParams& p, hipStream_t st) {
 
 template <int FM, int FN, int NW, int STAGES, bool CONV, int EPI, bool ROWMAP = false, bool ZP = false>
 int launch_wave(const MainParams& p, hipStream_t st) {
-  constexpr int lds = qgemm_wave_lds(FM, FN, NW, STAGES);
-  static_assert(lds >= FM * FN * (NW - 1) * 4096 && lds >= NW * 4096 + FN * 32 * 12 + 256, "sums, staging of the results");
+  constexpr int lds = std::max(qgemm_wave_lds(FM, FN, NW, STAGES), FM * FN * (NW - 1) * 4096);
+  static_assert(lds >= NW * 4096 + FN * 32 * 12 + 256 && lds <= 160 * 1024, "staging of the results");
   DQ8_REQUIRE(pipe_ok(32 * FM, 32 * FN, p, CONV) && (!ROWMAP || p.conv_bytes < (1LL << 31)),
               "qgemm on waves of their own needs K % 16 == 0 and operands that fit 32-bit buffer offsets");
   auto kern = qgemm_wave_kernel<FM, FN, NW, STAGES, CONV, EPI, ROWMAP, ZP>;
@@ -158,6 +159,21 @@ int launch_wave(const MainParams& p, hipStream_t st) {
   if (int s = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds, &lds_allowed)) return s;
   hipLaunchKernelGGL(kern, dim3(p.tiles_m * p.tiles_n), dim3(NW * 64), lds, st, p);
   return check_hip(hipGetLastError(), "qgemm_wave launch");
+}
+
+// the tiles on waves of their own, by variant
+template <bool CONV, int EPI, bool ROWMAP = false, bool ZP = false>
+int launch_wave_variant(int variant, const MainParams& p, hipStream_t st) {
+  switch (variant) {
+    case kWave64: return launch_wave<2, 2, 4, 2, CONV, EPI, ROWMAP, ZP>(p, st);
+    case kWave32x64: return launch_wave<1, 2, 4, 2, CONV, EPI, ROWMAP, ZP>(p, st);
+    case kWave32: return launch_wave<1, 1, 8, 2, CONV, EPI, ROWMAP, ZP>(p, st);
+    case kWave32w4: return launch_wave<1, 1, 4, 4, CONV, EPI, ROWMAP, ZP>(p, st);
+  }
+  if constexpr (!CONV) {   // (one stage to a wave: four of two do not fit the LDS)
+    if (variant == kWave96x64) return launch_wave<3, 2, 4, 1, CONV, EPI, ROWMAP, ZP>(p, st);
+  }
+  return fail("no kernel on waves of their own for this variant");
 }
 
 // `per_cu`: workgroups of this shape a compute unit holds at a time
@@ -285,11 +301,8 @@ int launch_variant(int variant, MainParams& p, hipStream_t st) {
     case kPipe256w8: return launch_pipe<256, 256, 2, 4, 1, CONV, EPI>(p, st);
     case kPipe128w8: return launch_pipe<128, 128, 2, 4, 1, CONV, EPI>(p, st);
     case kPipe256x192: return launch_pipe<256, 192, 4, 2, 1, CONV, EPI>(p, st);
-    case kWave64: return launch_wave<2, 2, 4, 2, CONV, EPI>(p, st);
-    case kWave32x64: return launch_wave<1, 2, 4, 2, CONV, EPI>(p, st);
-    case kWave32: return launch_wave<1, 1, 8, 2, CONV, EPI>(p, st);
-    case kWave32w4: return launch_wave<1, 1, 4, 4, CONV, EPI>(p, st);
   }
+  if (is_wave_variant(variant)) return launch_wave_variant<CONV, EPI>(variant, p, st);
   if constexpr (!CONV) {   // GEMM only: the small-M kernel and the persistent forms
     if (variant == kSkinnyVariant) return launch_skinny<EPI>(p, st);
     if (variant == kPersist128) return launch_persist<128, 128, 2, 4, false, EPI>(p, 2, st);
@@ -336,11 +349,8 @@ int launch_zp_ragged(int variant, MainParams& p, hipStream_t st) {
     case kPipe128w8: return launch_pipe<128, 128, 2, 4, 1, false, EPI, false, true>(p, st);
     case kPipe256w8: return launch_pipe<256, 256, 2, 4, 1, false, EPI, false, true>(p, st);
     case kPipe256x192: return launch_pipe<256, 192, 4, 2, 1, false, EPI, false, true>(p, st);
-    case kWave64: return launch_wave<2, 2, 4, 2, false, EPI, false, true>(p, st);
-    case kWave32x64: return launch_wave<1, 2, 4, 2, false, EPI, false, true>(p, st);
-    case kWave32: return launch_wave<1, 1, 8, 2, false, EPI, false, true>(p, st);
-    case kWave32w4: return launch_wave<1, 1, 4, 4, false, EPI, false, true>(p, st);
   }
+  if (is_wave_variant(variant)) return launch_wave_variant<false, EPI, false, true>(variant, p, st);
   return fail("no kernel with a zero point in the k loop for this variant");
 }
 
@@ -363,11 +373,8 @@ int launch_rowmap(int variant, MainParams& p, hipStream_t st) {
       case kPipe64k2: return launch_pipe<64, 64, 2, 2, 2, false, EPI, true>(p, st);
       case kPipe256w8: return launch_pipe<256, 256, 2, 4, 1, false, EPI, true>(p, st);
       case kPipe256x192: return launch_pipe<256, 192, 4, 2, 1, false, EPI, true>(p, st);
-      case kWave64: return launch_wave<2, 2, 4, 2, false, EPI, true>(p, st);
-      case kWave32x64: return launch_wave<1, 2, 4, 2, false, EPI, true>(p, st);
-      case kWave32: return launch_wave<1, 1, 8, 2, false, EPI, true>(p, st);
-      case kWave32w4: return launch_wave<1, 1, 4, 4, false, EPI, true>(p, st);
     }
+    if (is_wave_variant(variant)) return launch_wave_variant<false, EPI, true>(variant, p, st);
   }
   return fail("no kernel with rows mapped to pixels for this variant");
 }

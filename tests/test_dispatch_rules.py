@@ -80,17 +80,26 @@ def test_weight_only_scratch_is_what_the_plan_uses(dtype):
 
 
 @pytest.mark.parametrize("m,n,k,out,kernel", [
-    # up to 256 tiles of 32 x 32, then of 32 x 64, then (from 1280 of k on) of 64 x 64
+    # up to 256 tiles of 32 x 32, then of 32 x 64, then (from 1280 of k on) of 64 x 64, of 96 x 64
     (512, 512, 1008, 1, "wave_32x32_w4"), (512, 512, 1024, 1, "wave_32x32_w8"), (512, 513, 1024, 4, "wave_32x64_w4"),
     (513, 512, 1024, 1, "wave_32x64_w4"), (513, 960, 2048, 1, "wave_32x64_w4"), (512, 1024, 256, 4, "wave_32x64_w4"),
     (1024, 1024, 1280, 1, "wave_64x64_w4"), (1024, 1024, 1264, 1, "pipe_64x64x128"), (1025, 1024, 1280, 1, "pipe_64x64x128"),
+    (1300, 1024, 2048, 1, "wave_96x64_w4"), (1300, 1024, 2032, 1, "pipe_64x64x128"), (1300, 1024, 2560, 4, "wave_96x64_w4"),
+    (1300, 1024, 2544, 4, "pipe_64x64x128"), (1537, 1024, 2048, 1, "pipe_64x64x128"),
     # int8 rows off 16 bytes, 8192 of k
-    (512, 504, 1024, 1, "pipe_64x64x128"), (512, 504, 1024, 4, "wave_32x32_w8"), (512, 512, 8176, 1, "wave_32x32_w8"),
-    (512, 512, 8192, 1, "pipe_64x64x128_k4"),
-    # few rows: the small-M kernel where it is not a tenth slower
-    (64, 768, 768, 1, "skinny_16"), (16, 4096, 1088, 1, "skinny_16"), (128, 512, 4608, 1, "skinny_16"),
+    (512, 504, 1024, 1, "wave_32x32_w8"), (512, 504, 1008, 1, "pipe_64x64x128"), (512, 504, 1024, 4, "wave_32x32_w8"),
+    (1024, 1000, 2288, 1, "pipe_64x64x128_k2"), (1024, 1000, 2304, 1, "wave_64x64_w4"), (1300, 1000, 2544, 1, "pipe_64x64x128"),
+    (1300, 1000, 2560, 1, "wave_96x64_w4"), (512, 512, 8176, 1, "wave_32x32_w8"), (512, 512, 8192, 1, "pipe_64x64x128_k4"),
+    # few rows: the small-M kernel where it is estimated as fast
+    (64, 768, 768, 1, "skinny_16"), (16, 4096, 1088, 1, "skinny_16"), (128, 384, 2048, 1, "skinny_16"),
+    (320, 64, 512, 1, "skinny_16"), (321, 64, 512, 1, "wave_32x32_w4"), (256, 72, 1024, 1, "skinny_16"),
+    (257, 72, 1024, 1, "wave_32x32_w8"),
     (118, 1536, 5248, 1, "wave_32x32_w8"), (34, 3232, 5392, 1, "wave_32x32_w8"), (30, 8640, 1088, 1, "wave_32x64_w4"),
-    (16, 16448, 4096, 1, "pipe_64x64x128_k2")])
+    (16, 16448, 4096, 1, "pipe_64x64x128_k2"),
+    # two 64 x 64 tiles to a compute unit, then 128 x 128 ones on eight waves, four for a deep k
+    (2048, 1024, 768, 1, "pipe_64x64x128"), (2049, 1024, 768, 1, "pipe_128x128x128_w8"), (512, 4096, 2032, 1, "pipe_64x64x128"),
+    (512, 4096, 2048, 1, "pipe_128x128x128_w8"), (1024, 2048, 3072, 4, "pipe_64x64x128"),
+    (4096, 1152, 768, 1, "pipe_128x128x128_w8"), (4096, 1152, 4096, 1, "pipe_128x128x128")])
 def test_few_tiles_run_on_waves_of_their_own(m, n, k, out, kernel):
     """The smallest tile of which a launch has one per compute unit: 343 x 512 x 4608 took 11.9 us on 64 x 64
     tiles, 7.1 on these; one more than that and a compute unit does two."""

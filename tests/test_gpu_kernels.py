@@ -2724,8 +2724,10 @@ def test_fused_operators_behind_a_zero_point_in_the_k_loop(K, shape, kernel):
 
 # and of the tiles whose k tiles are dealt out over the waves: fewer k tiles than waves, one more than whole
 # rounds of them, rows and channels that end inside a tile
-WAVE_TILES = [((300, 272, 96), "wave_32x32_w4"), ((410, 560, 528), "wave_32x32_w4"), ((343, 512, 2064), "wave_32x32_w8"),
-              ((335, 1168, 320), "wave_32x64_w4"), ((519, 848, 1040), "wave_32x64_w4"), ((1100, 784, 2064), "wave_64x64_w4")]
+WAVE_TILES = [((330, 272, 96), "wave_32x32_w4"), ((410, 560, 528), "wave_32x32_w4"), ((343, 512, 2064), "wave_32x32_w8"),
+              ((335, 1168, 320), "wave_32x64_w4"), ((519, 848, 1040), "wave_32x64_w4"), ((1100, 784, 2064), "wave_64x64_w4"),
+              ((1300, 1008, 2064), "wave_96x64_w4"), ((260, 130, 1040), "wave_32x32_w8"), ((519, 847, 1040), "wave_32x64_w4"),
+              ((1021, 1001, 2320), "wave_64x64_w4"), ((1250, 1006, 2576), "wave_96x64_w4")]
 
 
 @pytest.mark.parametrize("shape,kernel", WAVE_TILES, ids=["%s-%d" % (t[1], t[0][2]) for t in WAVE_TILES])
@@ -2755,7 +2757,7 @@ def test_convolutions_on_k_tiles_dealt_out_over_the_waves(K, nb, h, w_, ci, co, 
     sc = dict(sx=dev(np.array([0.02], np.float32)), sw=dev(rng.uniform(0.001, 0.05, co).astype(np.float32)),
               so=dev(np.array([0.5], np.float32)), bias=dev(rng.standard_normal(co).astype(np.float32)))
     waves = [i for i, nm in enumerate(K.variant_names()) if nm.startswith("wave_")]
-    assert len(waves) == 4
+    assert len(waves) == 5 and K.variant_names()[waves.pop()] == "wave_96x64_w4"   # (products only)
     for epi in (K.EPI_ACC_S32, K.EPI_REQUANT_CPU, K.EPI_REQUANT_CPU_DEQUANT_F32):
         kw = {} if epi == K.EPI_ACC_S32 else sc
         want = K.qconv2d(x, wt, [pad] * 4, md, [nb, ho, wo, co], epi, variant=0, **kw)
