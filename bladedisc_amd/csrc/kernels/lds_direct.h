@@ -60,6 +60,15 @@ __device__ __forceinline__ void buffer_load_lds_b32(v4i rsrc, unsigned lds_addr,
       : "memory", "m0");
 }
 
+// The last chunk of rows of K bytes (K % 4 == 0, not a multiple of 16), loaded as the last 16 bytes of the row:
+// the words that belong to the chunk before it set to zero.  A fragment of 32 bytes of k has the chunk in the lanes of half
+// (K / 16) % 2 of the wave.
+__device__ __forceinline__ void clear_row_end(v4i& fragment, int K, int lane) {
+  const int drop = (lane >> 5) == ((K >> 4) & 1) ? 4 - ((K >> 2) & 3) : 0;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) fragment[c] = c < drop ? 0 : fragment[c];
+}
+
 // s_waitcnt immediate for gfx9: vmcnt = n (6 bits, split), lgkmcnt = 0, expcnt = any
 constexpr int waitcnt_vm_lgkm0(int n) { return (n & 0xf) | ((n >> 4) << 14) | (0x7 << 4); }
 

@@ -348,6 +348,10 @@ extern template int launch_zp_ragged<DQ8_EPI_ACC_S32>(int, MainParams&, hipStrea
 extern template int launch_zp_ragged<DQ8_EPI_REQUANT_CPU>(int, MainParams&, hipStream_t);
 extern template int launch_zp_ragged<DQ8_EPI_REQUANT_GPU>(int, MainParams&, hipStream_t);
 extern template int launch_zp_ragged<DQ8_EPI_DEQUANT_F32>(int, MainParams&, hipStream_t);
+extern template int launch_words<DQ8_EPI_ACC_S32>(int, MainParams&, hipStream_t);
+extern template int launch_words<DQ8_EPI_REQUANT_CPU>(int, MainParams&, hipStream_t);
+extern template int launch_words<DQ8_EPI_REQUANT_GPU>(int, MainParams&, hipStream_t);
+extern template int launch_words<DQ8_EPI_DEQUANT_F32>(int, MainParams&, hipStream_t);
 
 int compute_units() {
   static std::atomic<int> cached{0};
@@ -383,6 +387,16 @@ int launch_zp_ragged_epi(int variant, MainParams& p, int epilogue, hipStream_t s
     case DQ8_EPI_REQUANT_CPU: return launch_zp_ragged<DQ8_EPI_REQUANT_CPU>(variant, p, st);
     case DQ8_EPI_REQUANT_GPU: return launch_zp_ragged<DQ8_EPI_REQUANT_GPU>(variant, p, st);
     case DQ8_EPI_DEQUANT_F32: return launch_zp_ragged<DQ8_EPI_DEQUANT_F32>(variant, p, st);
+  }
+  return fail("unknown epilogue");
+}
+
+int launch_words_epi(int variant, MainParams& p, int epilogue, hipStream_t st) {
+  switch (epilogue) {
+    case DQ8_EPI_ACC_S32: return launch_words<DQ8_EPI_ACC_S32>(variant, p, st);
+    case DQ8_EPI_REQUANT_CPU: return launch_words<DQ8_EPI_REQUANT_CPU>(variant, p, st);
+    case DQ8_EPI_REQUANT_GPU: return launch_words<DQ8_EPI_REQUANT_GPU>(variant, p, st);
+    case DQ8_EPI_DEQUANT_F32: return launch_words<DQ8_EPI_DEQUANT_F32>(variant, p, st);
   }
   return fail("unknown epilogue");
 }
@@ -850,11 +864,18 @@ int qgemm_impl(int variant, const int8_t* A, int64_t lda, const int8_t* W, int64
     p.zx = zx;
     p.zw = zw;
     p.kzz = (int)((uint32_t)K * (uint32_t)zx * (uint32_t)zw);
+    // (rows on four bytes: the tiles chosen as for aligned rows, operands straight into LDS -- 5525 x 336, 1292 of k
+    // 22.3 -> 11.8 us and 835 x 3488 x 696 14.4 -> 9.0, copied first before; 489 x 416 x 1220 8.1 -> 5.2 and 777 x 1501 x
+    // 1000 with a zero point 9.6 -> 8.2, through registers before; 150 drawn products 1.10 times the speed)
+    if (words_ok(256, 256, p) && zw == 0) {
+      const int vw = words_variant(pick_any(M, N, Kp, true, es));
+      if (vw >= 0) return launch_words_epi(vw, p, epilogue, st);
+    }
     const int v = pick_any(M, N, Kp, ragged_ok(p), es, false);
     if (v == kSkinnyVariant) return launch_epi<false>(v, p, epilogue, st);
     // (rows at odd bytes: each load is served in pieces, about 0.25 us per k tile -- 777 x 1504, 1000
-    // of k at any multiple of four 8.3 us, at odd bytes 11.5, copied first 12; 1000 x 768 with 3073
-    // of k 13.8, copied 12.7)
+    // of k at odd bytes 11.5, copied first 12; 1000 x 768 with 3073 of k 13.8, copied 12.7; rows on four
+    // bytes, K not a multiple of it: any depth)
     const bool words = aligned(A, 4) && aligned(W, 4) && lda % 4 == 0 && ldw % 4 == 0;
     if (ragged_has_variant(v) && ragged_ok(p) && zw == 0 && (words || K <= 2048))
       return launch_zp_ragged_epi(v, p, epilogue, st);

@@ -134,27 +134,37 @@ inline bool ragged_ok(const MainParams& p) {
   return p.K >= 16 && 64 * std::max(p.lda, p.ldw) + p.K + 512 < (1LL << 31);
 }
 
+// What the WORDS form of a tile asks of them.
+inline bool words_ok(int bm, int bn, const MainParams& p) {
+  constexpr int BK = 128;
+  return p.K >= 16 && p.K % 4 == 0 && p.lda % 4 == 0 && p.ldw % 4 == 0 && aligned(p.A, 4) && aligned(p.W, 4) &&
+         std::max(bm * p.lda, bn * p.ldw) + p.K + 2 * BK < (1LL << 31);
+}
+
 template <int BM, int BN, int WM, int WN, int KSPLIT, bool CONV, int EPI, bool ROWMAP = false,
-          bool ZP = false, bool RAGGED = false>
+          bool ZP = false, bool RAGGED = false, bool WORDS = false>
 int launch_pipe(const MainParams& p, hipStream_t st) {
   constexpr int BK = 128;
   constexpr int lds = KSPLIT * 2 * (BM + BN) * BK;
-  DQ8_REQUIRE(RAGGED ? ragged_ok(p) : pipe_ok(BM, BN, p, CONV) && (!ROWMAP || p.conv_bytes < (1LL << 31)),
+  DQ8_REQUIRE(RAGGED ? ragged_ok(p)
+              : WORDS ? words_ok(BM, BN, p)
+                      : pipe_ok(BM, BN, p, CONV) && (!ROWMAP || p.conv_bytes < (1LL << 31)),
               "pipelined qgemm needs K % 16 == 0 and operands that fit 32-bit buffer offsets");
-  auto kern = qgemm_pipe_kernel<BM, BN, WM, WN, KSPLIT, CONV, EPI, ROWMAP, ZP, RAGGED>;
+  auto kern = qgemm_pipe_kernel<BM, BN, WM, WN, KSPLIT, CONV, EPI, ROWMAP, ZP, RAGGED, WORDS>;
   static std::atomic<uint64_t> lds_allowed{0};
   if (int s = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds, &lds_allowed)) return s;
   hipLaunchKernelGGL(kern, dim3(p.tiles_m * p.tiles_n), dim3(WM * WN * KSPLIT * 64), lds, st, p);
   return check_hip(hipGetLastError(), "qgemm_pipe launch");
 }
 
-template <int FM, int FN, int NW, int STAGES, bool CONV, int EPI, bool ROWMAP = false, bool ZP = false>
+template <int FM, int FN, int NW, int STAGES, bool CONV, int EPI, bool ROWMAP = false, bool ZP = false, bool WORDS = false>
 int launch_wave(const MainParams& p, hipStream_t st) {
   constexpr int lds = std::max(qgemm_wave_lds(FM, FN, NW, STAGES), FM * FN * (NW - 1) * 4096);
   static_assert(lds >= NW * 4096 + FN * 32 * 12 + 256 && lds <= 160 * 1024, "staging of the results");
-  DQ8_REQUIRE(pipe_ok(32 * FM, 32 * FN, p, CONV) && (!ROWMAP || p.conv_bytes < (1LL << 31)),
+  DQ8_REQUIRE(WORDS ? words_ok(32 * FM, 32 * FN, p)
+                    : pipe_ok(32 * FM, 32 * FN, p, CONV) && (!ROWMAP || p.conv_bytes < (1LL << 31)),
               "qgemm on waves of their own needs K % 16 == 0 and operands that fit 32-bit buffer offsets");
-  auto kern = qgemm_wave_kernel<FM, FN, NW, STAGES, CONV, EPI, ROWMAP, ZP>;
+  auto kern = qgemm_wave_kernel<FM, FN, NW, STAGES, CONV, EPI, ROWMAP, ZP, WORDS>;
   static std::atomic<uint64_t> lds_allowed{0};
   if (int s = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds, &lds_allowed)) return s;
   hipLaunchKernelGGL(kern, dim3(p.tiles_m * p.tiles_n), dim3(NW * 64), lds, st, p);
@@ -354,6 +364,40 @@ int launch_zp_ragged(int variant, MainParams& p, hipStream_t st) {
   return fail("no kernel with a zero point in the k loop for this variant");
 }
 
+// Tiles on operand rows that begin on four bytes (qgemm_launch_words_*.hip): those that the choice comes down to
+// most, each also in the place of the forms next to it that carry no such rows; -1: none.
+inline int words_variant(int variant) {
+  switch (variant) {
+    case kPipe64: case kPipe64k2: case kPipe128w8: case kPipe256w8: case kWave64: case kWave32x64: case kWave32:
+      return variant;
+    case kPipe64k4: return kPipe64k2;
+    case kPipe128: case kPersist128: return kPipe128w8;
+    case kPersist256: case kPipe256x192: case kPersist256x192: return kPipe256w8;
+    case kWave32w4: return kWave32;
+    case kWave96x64: return kPipe64;
+  }
+  return -1;
+}
+template <int EPI, bool ZP>
+int launch_words_zp(int variant, MainParams& p, hipStream_t st) {
+  switch (variant) {
+    case kPipe64: return launch_pipe<64, 64, 2, 2, 1, false, EPI, false, ZP, false, true>(p, st);
+    case kPipe64k2: return launch_pipe<64, 64, 2, 2, 2, false, EPI, false, ZP, false, true>(p, st);
+    case kPipe128w8: return launch_pipe<128, 128, 2, 4, 1, false, EPI, false, ZP, false, true>(p, st);
+    case kPipe256w8: return launch_pipe<256, 256, 2, 4, 1, false, EPI, false, ZP, false, true>(p, st);
+    case kWave64: return launch_wave<2, 2, 4, 2, false, EPI, false, ZP, true>(p, st);
+    case kWave32x64: return launch_wave<1, 2, 4, 2, false, EPI, false, ZP, true>(p, st);
+    case kWave32: return launch_wave<1, 1, 8, 2, false, EPI, false, ZP, true>(p, st);
+  }
+  return fail("no kernel for rows on four bytes for this variant");
+}
+template <int EPI>
+int launch_words(int variant, MainParams& p, hipStream_t st) {
+  p.tiles_m = (int)ceil_div(p.M, kVariants[variant].bm);
+  p.tiles_n = (int)ceil_div(p.N, kVariants[variant].bn);
+  return p.zx ? launch_words_zp<EPI, true>(variant, p, st) : launch_words_zp<EPI, false>(variant, p, st);
+}
+
 // The tiles a strided 1 x 1 convolution runs on as a GEMM over the pixels it reads (instantiated
 // next to the convolution kernels: CONV true; the GEMM files carry a stub).
 inline bool rowmap_has_variant(int variant) {
@@ -393,6 +437,12 @@ int launch_rowmap(int variant, MainParams& p, hipStream_t st) {
 #define DQ8_INSTANTIATE_LAUNCH_ZP(EPI) \
   namespace dq8 {                       \
   template int launch_zp_ragged<EPI>(int, MainParams&, hipStream_t); \
+  }
+
+// the body of one qgemm_launch_words_*.hip
+#define DQ8_INSTANTIATE_LAUNCH_WORDS(EPI) \
+  namespace dq8 {                          \
+  template int launch_words<EPI>(int, MainParams&, hipStream_t); \
   }
 
 #endif  // DQ8_QGEMM_LAUNCH_H_

@@ -1,0 +1,4 @@
+// Launchers of the int8 GEMM tiles on operand rows that begin on four bytes, epilogue ACC_S32.
+#include "qgemm_launch.h"
+
+DQ8_INSTANTIATE_LAUNCH_WORDS(DQ8_EPI_ACC_S32)

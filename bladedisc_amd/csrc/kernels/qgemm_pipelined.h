@@ -79,9 +79,14 @@ namespace dq8 {
 // k tile further ahead, and the chunk that holds the end of a row is shifted into place and
 // filled up with zeros.  For the 64 x 64 tiles, where copying the operands to aligned rows first
 // costs as much as the product (777 x 1000 x 1501: 13.3 us with the copy, 9.6 without).
+//
+// WORDS: operand rows that begin on four bytes, K % 4 == 0: loaded straight into LDS like aligned ones.  A chunk
+// that holds the end of a row is loaded as the row's last 16 bytes, of both operands, and the words of it
+// that the chunk before holds already are cleared in the weights' fragment: no load leaves its row.  What a
+// 64 x 64 tile pays for RAGGED is its waves' instructions (777 x 1501, 1000 of k, a zero point: 9.6 us, so 8.2).
 typedef int v4i_any_t __attribute__((ext_vector_type(4), aligned(1)));
 template <int BM, int BN, int WM, int WN, int KSPLIT, bool CONV, int EPI, bool ROWMAP = false,
-          bool ZP = false, bool RAGGED = false>
+          bool ZP = false, bool RAGGED = false, bool WORDS = false>
 __global__ void __launch_bounds__(WM* WN* KSPLIT * 64) qgemm_pipe_kernel(const MainParams p) {
   // The inline assembly only assembles in the device compilation; the host pass
   // just needs the kernel's stub.
@@ -209,7 +214,7 @@ __global__ void __launch_bounds__(WM* WN* KSPLIT * 64) qgemm_pipe_kernel(const M
   auto tile_setup = [&](int kt) {
     const int k = (kt0 + kt) * BK + kc;
     const bool in = kt < KT && k < p.K;
-    t_koff = in ? (kt0 + kt) * BK : kOutOfRange;
+    t_koff = in ? (kt0 + kt) * BK - (WORDS ? max(k + 16 - p.K, 0) : 0) : kOutOfRange;
     if (CONV) {
       t_dh = c_kh * p.dh;
       t_dw = c_kw * p.dw;
@@ -386,6 +391,9 @@ __global__ void __launch_bounds__(WM* WN* KSPLIT * 64) qgemm_pipe_kernel(const M
 #pragma unroll
   for (int j = 0; j < (ZP ? FN : 1); ++j) w_sum[j] = 0;
 
+  // WORDS: the k-step (of this group) whose fragments hold the end of the rows, in one half of the lanes
+  const int end_step = WORDS && (p.K & 15) != 0 ? __builtin_amdgcn_readfirstlane(p.K / 32 - kt0 * NKS) : -1;
+
   // One k tile out of stage `cur` (an int, or a compile-time constant: see below).
   auto k_tile = [&](auto cur_v, int kt) {
     const int cur = cur_v, nxt = cur ^ 1;
@@ -402,6 +410,12 @@ __global__ void __launch_bounds__(WM* WN* KSPLIT * 64) qgemm_pipe_kernel(const M
           fetch_tile(kt + 3, held);
         } else {
           tile_setup(kt + 2);
+        }
+      }
+      if constexpr (WORDS) {
+        if (kt * NKS + ks == end_step) {
+#pragma unroll
+          for (int j = 0; j < FN; ++j) clear_row_end(fb[ks][j], p.K, lane);
         }
       }
       if (ks == 3 && !RAGGED) {

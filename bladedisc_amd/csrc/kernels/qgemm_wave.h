@@ -17,7 +17,7 @@
 // bytes apart, which puts rows r and r + 8 of a fragment into different halves of the banks and leaves
 // every lane with the same chunk in every block it loads.
 // Requires what the pipelined kernel does: K % 16 == 0, 16-byte aligned, k-contiguous operands, 32-bit
-// offsets.  ROWMAP, ZP: see qgemm_pipelined.h.
+// offsets.  ROWMAP, ZP, WORDS (rows on four bytes): see qgemm_pipelined.h.
 #ifndef DQ8_QGEMM_WAVE_H_
 #define DQ8_QGEMM_WAVE_H_
 
@@ -29,7 +29,7 @@ namespace dq8 {
 constexpr int kWaveBlock = 1152;   // bytes between two blocks of 8 rows
 constexpr int qgemm_wave_lds(int fm, int fn, int nw, int stages) { return nw * stages * (fm + fn) * 4 * kWaveBlock; }
 
-template <int FM, int FN, int NW, int STAGES, bool CONV, int EPI, bool ROWMAP = false, bool ZP = false>
+template <int FM, int FN, int NW, int STAGES, bool CONV, int EPI, bool ROWMAP = false, bool ZP = false, bool WORDS = false>
 __global__ void __launch_bounds__(NW * 64) qgemm_wave_kernel(const MainParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int BK = 128, NKS = BK / 32;
@@ -112,7 +112,7 @@ __global__ void __launch_bounds__(NW * 64) qgemm_wave_kernel(const MainParams p)
     d_kw = d_tap - d_kh * p.Kw;
   }
   auto tile_setup = [&]() {
-    t_koff = k_next + kc < p.K ? k_next : kOutOfRange;
+    t_koff = k_next + kc < p.K ? k_next - (WORDS ? max(k_next + kc + 16 - p.K, 0) : 0) : kOutOfRange;
     k_next += NW * BK;
     if (CONV) {
       t_dh = c_kh * p.dh;
@@ -166,8 +166,11 @@ __global__ void __launch_bounds__(NW * 64) qgemm_wave_kernel(const MainParams p)
       for (int i = 0; i < LD; ++i) issue_load(i, lds_base + t * STAGE);
     }
 
+  // WORDS: whether the end of the rows is in this wave's last tile
+  const bool row_end = WORDS && (p.K & 15) != 0 && nt > 0 && wave + (nt - 1) * NW == KT - 1;
+
   // MORE: tile t + STAGES exists and is loaded; else at most `behind` tiles are on their way behind tile t
-  auto k_tile = [&](auto more_c, int st) {
+  auto k_tile = [&](auto more_c, int st, bool last) {
     constexpr bool more = decltype(more_c)::value != 0;
     const int8_t* base = smem + st * STAGE;
     v4i fa[NKS][FM], fb[NKS][FN];
@@ -183,6 +186,13 @@ __global__ void __launch_bounds__(NW * 64) qgemm_wave_kernel(const MainParams p)
       // the stage is this wave's alone: free once its fragments are in registers
       __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(63));
       __builtin_amdgcn_sched_barrier(0);
+    }
+    if (WORDS && !more && last && row_end) {
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks)
+        if (ks == (p.K & (BK - 1)) / 32)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) clear_row_end(fb[ks][j], p.K, lane);
     }
     constexpr int MF = NKS * FM * FN;
     static_for<MF>([&](auto mc) {
@@ -204,7 +214,7 @@ __global__ void __launch_bounds__(NW * 64) qgemm_wave_kernel(const MainParams p)
     // (tile t: older than the STAGES - 1 behind it)
     __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0((STAGES - 1) * LD));
     asm volatile("" ::: "memory");
-    k_tile(IntC<1>(), st);
+    k_tile(IntC<1>(), st, false);
     st = st + 1 == STAGES ? 0 : st + 1;
   }
   for (; t < nt; ++t) {
@@ -213,7 +223,7 @@ __global__ void __launch_bounds__(NW * 64) qgemm_wave_kernel(const MainParams p)
       if (a == nt - t - 1) __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(a * LD));
     });
     asm volatile("" ::: "memory");
-    k_tile(IntC<0>(), st);
+    k_tile(IntC<0>(), st, t == nt - 1);
     st = st + 1 == STAGES ? 0 : st + 1;
   }
   ColParams col[EarlyColRaw<EPI, NT, BN>::kPerThread];

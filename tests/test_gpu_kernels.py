@@ -2788,6 +2788,36 @@ def test_fused_operators_behind_rows_of_any_length(K, shape, kernel):
             _fused_forms_equal_the_separate_operators(K, a, w, zx, rng)
 
 
+# operand rows on four bytes: (m, n, k) and the tile named for k rounded up to 16
+WORD_TILES = [((400, 256, 500), "wave_32x32_w4"), ((300, 257, 1036), "wave_32x32_w8"), ((335, 1152, 324), "wave_32x64_w4"),
+              ((1023, 897, 4108), "wave_64x64_w4"), ((777, 1501, 1000), "pipe_64x64x128"), ((640, 513, 124), "pipe_64x64x128"),
+              ((513, 1023, 2052), "pipe_64x64x128_k2"), ((4097, 1281, 264), "pipe_128x128x128_w8"),
+              ((4090, 3500, 396), "pipe_256x256x128_w8"), ((1300, 1024, 2500), "wave_96x64_w4"), ((777, 1501, 1024), "pipe_64x64x128")]
+
+
+@pytest.mark.parametrize("shape,kernel", WORD_TILES, ids=["%s-%d" % (t[1], t[0][2]) for t in WORD_TILES])
+def test_qgemm_on_rows_that_begin_on_four_bytes(K, shape, kernel):
+    """Rows of whole words, contiguous and out of wider rows whose other bytes are not zero: every place of the
+    rows' end in a k tile's steps, a wave's half and a chunk.  Sums of whole numbers: equal bits."""
+    m, n, k = shape
+    assert K._lib.lib().dq8_qgemm_kernel_name(m, n, (k + 15) // 16 * 16, 1).decode() == kernel
+    rng = np.random.default_rng(m + n + k)
+    wide_a = dev(rng.integers(-128, 128, (m, k + 12), dtype=np.int8))
+    wide_w = dev(rng.integers(-128, 128, (n, k + 20), dtype=np.int8))
+    sc = dict(sx=dev(np.array([0.02], np.float32)), sw=dev(rng.uniform(0.001, 0.05, n).astype(np.float32)),
+              so=dev(np.array([3.0], np.float32)), bias=dev(rng.standard_normal(n).astype(np.float32)))
+    last = [k] if k > 1500 else [k, k - 4, k - 8, k - 12, k - 20, k - 36]
+    for kk in last:
+        for a, w in ((wide_a[:, :kk].contiguous(), wide_w[:, :kk].contiguous()),
+                     (wide_a[:, 4:4 + kk], wide_w[:, 8:8 + kk])):
+            for zx in (0, -11):
+                acc = K.qgemm(a, w, K.EPI_ACC_S32, variant=0, zx=zx)
+                assert torch.equal(K.qgemm(a, w, K.EPI_ACC_S32, zx=zx), acc)
+                for epi in (K.EPI_REQUANT_CPU, K.EPI_REQUANT_GPU, K.EPI_REQUANT_CPU_DEQUANT_F32):
+                    want = K.qgemm(a, w, epi, variant=0, zx=zx, **sc)
+                    assert torch.equal(K.qgemm(a, w, epi, zx=zx, **sc), want), (kk, zx, epi)
+
+
 @pytest.mark.parametrize("rows,nch", [(4, 3), (5, 37), (1023, 255), (7, 256), (64, 257), (33, 511), (9, 1025),
                                       (4, 3073), (517, 1537), (1021, 1), (1723, 2501)])
 @pytest.mark.parametrize("xt,qt", [(torch.float32, torch.uint8), (torch.float16, torch.int8),
