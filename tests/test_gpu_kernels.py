@@ -2032,6 +2032,29 @@ def test_weight_only_qgemm_every_tile_form_split_over_k(K, dtype, m, k, n, form,
     assert torch.equal(out, first)
 
 
+@pytest.mark.parametrize("m,k,n,form,splits", [
+    (35, 72, 140, 0, 1), (42, 1868, 32, 0, 8), (92, 2700, 105, 0, 8), (227, 412, 2227, 1, 1), (1018, 68, 1282, 2, 1),
+    (286, 216, 4074, 2, 1), (1727, 280, 3699, 3, 1), (1030, 4100, 4090, 5, 1), (1021, 4100, 4090, 4, 1),
+    (66, 6236, 2481, 0, 2)])
+@pytest.mark.parametrize("signed", [False, True])
+def test_weight_only_qgemm_rows_that_begin_on_four_bytes(K, m, k, n, form, splits, signed):
+    """Rows of whole words on the tiles of aligned rows: 4, 8 and 12 k in the last group of 16, in each half of a
+    unit, a last range of 4 to 12 k (92 x 2700), in frames of NaN / 255, with the scratch that is asked for."""
+    assert _weight_only_plan(m, n, k, torch.float16) == (form, splits)
+    rng = np.random.default_rng(m + k + n)
+    x, w, scale, zp, bias = _weight_only_case(rng, m, k, n, torch.float16, signed)
+    wide_x, wide_w = _weight_only_framed(x, w, torch.float16, signed)
+    ws = torch.full((4 * m * n * 8,), 0xff, dtype=torch.uint8, device="cuda")
+    frame = torch.full((m + 1, n + 5), 7.0, dtype=torch.float16, device="cuda")
+    out = frame[:m, 1:n + 1]
+    _weight_only_raw(wide_x, wide_w, dev(scale), dev(zp), dev(bias), out, ws, ws.nbytes)
+    _weight_only_check(out, x, w, scale, zp, bias, torch.float16)
+    assert bool((frame[:, 0] == 7).all()) and bool((frame[:, n + 1:] == 7).all()) and bool((frame[m] == 7).all())
+    for workspace in (True, False):
+        got = K.weight_only_qgemm(dev(x), dev(w), dev(scale), zero_points=dev(zp), workspace=workspace)
+        _weight_only_check(got, x, w, scale, zp, None, torch.float16)
+
+
 @pytest.mark.parametrize("m,k,n,signed", [
     (17, 400, 4097, False), (24, 1040, 4111, True), (32, 2048, 5000, False), (31, 784, 6161, True),
     (17, 2816, 6144, False), (25, 1024, 8177, True), (32, 2064, 8192, False), (20, 384, 4097, True),
