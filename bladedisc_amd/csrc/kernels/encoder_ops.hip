@@ -200,8 +200,10 @@ attention_f32_kernel(const float* __restrict__ qkv, int S, uint32_t all_heads, i
 // quantized: q, k and v are codes times one scale s, and nothing of them is widened to f32.
 //  * S^T = K Q^T in whole numbers, one v_mfma_i32_16x16x64_i8 for 16 keys x 16 queries x 64 channels (in
 //    f32 sixteen v_mfma_f32_16x16x4 of twice its time); lanes hold what they hold in the f32 kernel.  The
-//    maxima are whole numbers too, and exp2(acc f - max f), f = s^2 log2(e) / sqrt(64), is rounded once
-//    in front of the exponential.
+//    maxima are whole numbers too, and so is the difference in exp2((acc - max) f), f = s^2 log2(e) /
+//    sqrt(64): at most 2^21, exact in f32.  The best key's probability is 1 whatever the scale.  (Of
+//    max f, rounded, taken off acc f the best key keeps that rounding: several powers of two from scales
+//    of 15 on, beyond the largest half.)
 //  * O^T = V^T P^T on v_mfma_f32_16x16x32_f16: a code is a half as it is, and a probability, times 2^14,
 //    is the sum of two halves to 2^-23 of itself (24 bits in 11 + 11 and a sign; the factor keeps the
 //    second half of all that matter out of the subnormals).  16 instead of 128 matrix instructions for 64
@@ -302,15 +304,14 @@ attention_i8_kernel(const int8_t* __restrict__ qkv, const float* __restrict__ qk
       x = __builtin_amdgcn_permlane32_swap(top, top, false, false);
       top = max((int)x[0], (int)x[1]);
     }
-    const float ref = (float)top * f;
-    const float keep = __builtin_amdgcn_exp2f((float)m * f - ref);
+    const float keep = __builtin_amdgcn_exp2f((float)(m - top) * f);
     m = top;
     float p[4][4];
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
       for (int v = 0; v < 4; ++v)
-        p[kt][v] = __builtin_amdgcn_exp2f(__builtin_fmaf((float)a[kt][v], f, -ref)) * 16384.0f;
+        p[kt][v] = __builtin_amdgcn_exp2f((float)(a[kt][v] - top) * f) * 16384.0f;
     if (ragged) {
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt)

@@ -2440,11 +2440,11 @@ def test_attention_equals_softmax_of_the_scores(K, b, s, heads):
 
 
 @pytest.mark.parametrize("b,s,heads", [(1, 1, 1), (2, 8, 12), (3, 17, 2), (1, 33, 3), (2, 64, 1), (1, 65, 12), (2, 97, 3), (2, 333, 5)])
-@pytest.mark.parametrize("step", [0.02, 0.1])
+@pytest.mark.parametrize("step", [0.02, 0.1, 20.0, 50.0, 1000.0])
 def test_attention_of_an_int8_projection(K, b, s, heads, step):
     """Edges of the 16-query, 32- and 64-key tiles with codes of the whole range, a wide and a narrow
-    softmax (scores up to 10 / up to 230), against the same in f64.  Bound: the scale's f32 square and product
-    move a difference of scores d by 3 ulp, its rounding and the exponential's ulp come on top, and d above 25
+    softmax (scores up to 10 / up to 230) and the best key alone (up to 2e10), against the same in f64.  Bound:
+    the scale's f32 square and product move a difference of scores d by 3 ulp, its rounding and the exponential's ulp come on top, and d above 25
     contributes nothing: 25 * 3 * 2^-24 + 2 * 2^-24 of each probability, twice (also in their sum), and
     s / 8 roundings of sums of values up to 128 * step: below 1e-5 of that."""
     g = torch.Generator().manual_seed(s)
@@ -2454,6 +2454,7 @@ def test_attention_of_an_int8_projection(K, b, s, heads, step):
     q, k, v = (t.double().reshape(b, s, heads, 64).transpose(1, 2) for t in (codes.double() * scale.double()).chunk(3, dim=-1))
     want = (torch.softmax(q @ k.transpose(2, 3) / 8.0, -1) @ v).transpose(1, 2).reshape(b, s, heads * 64)
     got = K.attention(codes.cuda(), heads, qkv_scale=scale.cuda())
+    assert got.isfinite().all()
     assert (got.cpu().double() - want).abs().max().item() <= 1e-5 * 128 * step
     out_scale = torch.full((1,), 0.02, device="cuda")
     zero = torch.zeros(1, dtype=torch.int32, device="cuda")
