@@ -11,9 +11,7 @@ namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef int v4i __attribute__((ext_vector_type(4)));
-typedef float f2 __attribute__((ext_vector_type(2)));
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 
 // int8 of four values, dq8_quantize's bits (zero point 0, half to even)
 __device__ __forceinline__ uint32_t quantize4(const v4f& v, float s, float y, bool fast) {
@@ -196,6 +194,14 @@ attention_f32_kernel(const float* __restrict__ qkv, int S, uint32_t all_heads, i
   store_context<QUANT>(y, ((int64_t)b * S + q0 + r) * heads * kHead + h * kHead + 16 * g, out, out_q, q_scale);
 }
 
+__device__ __forceinline__ float upper_half(float x) {
+  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & 0xffff0000u);
+}
+// the bf16 of two floats, cut off
+__device__ __forceinline__ uint32_t upper_halves(float x, float y) {
+  return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, y), __builtin_bit_cast(uint32_t, x), 0x07060302u);
+}
+
 // The same on the int8 result of the merged projection and its scale, for a layer whose projection is
 // quantized: q, k and v are codes times one scale s, and nothing of them is widened to f32.
 //  * S^T = K Q^T in whole numbers, one v_mfma_i32_16x16x64_i8 for 16 keys x 16 queries x 64 channels (in
@@ -204,20 +210,26 @@ attention_f32_kernel(const float* __restrict__ qkv, int S, uint32_t all_heads, i
 //    sqrt(64): at most 2^21, exact in f32.  The best key's probability is 1 whatever the scale.  (Of
 //    max f, rounded, taken off acc f the best key keeps that rounding: several powers of two from scales
 //    of 15 on, beyond the largest half.)
-//  * O^T = V^T P^T on v_mfma_f32_16x16x32_f16: a code is a half as it is, and a probability, times 2^14,
-//    is the sum of two halves to 2^-23 of itself (24 bits in 11 + 11 and a sign; the factor keeps the
-//    second half of all that matter out of the subnormals).  16 instead of 128 matrix instructions for 64
-//    keys, of half the time each, and sums round a quarter as often: the rms error against 64 bits is 0.14 to
-//    0.97 of the f32 kernel's on the dequantized projection (8 to 384 tokens, scores of 0.5 to 30).
+//  * O^T = V^T P^T on v_mfma_f32_16x16x32_bf16: a code is a bf16 as it is, and a probability the sum of
+//    three, its 24 bits eight by eight, cut off and not rounded, so that every product is that of the f32
+//    probability.  (Times 2^64: the last part of the smallest that the exponential gives is a normal number
+//    then.  The sum of two halves has 22 to 24 of the bits and none below 2^-38 of the largest -- values
+//    behind a key that has all the weight and is zero itself came out 1e-1 off at 2^-31 -- and is 0.3 us less
+//    at 8 x 128 tokens, 2.5 at 8 x 384.)  24 instead of 128 matrix instructions for 64 keys, of half the time
+//    each, and sums round a quarter as often: the rms error against 64 bits, over 24 scales from 0.003 to 0.3
+//    at each of 8 to 384 tokens, is 0.14 to 1.0 of the f32 kernel's on the dequantized projection, the smaller
+//    the wider the scores spread; of the int8 results of eight encoder layers' attention 52 in 14.4 million
+//    differ from those of 64 bits, with the f32 kernel 73.
 //  * Values are widened and transposed once, on their way into LDS: a thread takes 4 channels of 4 keys.
 //    A row of 64 keys is a channel, keys 32 j + 16 i + 4 g + v at 32 j + 8 g + 4 i + v, so that the eight
 //    a lane multiplies are one 16-byte read; channel 4 r + t is row 16 t + r, 144 bytes apart, which spreads
 //    the 16 channels of a read over all banks.  Keys lie in 64-byte rows, 16-byte chunk c of row r in slot
 //    c ^ (r / 4 % 4), likewise.
 //  * Two stages of 64 keys, one barrier a block.
-// What is left is the vector work of the softmax, ten instructions per score, and at encoder sizes the
-// launch and the trips to memory.  8 x 128 tokens, 12 heads 12.0 -> 5.5 us, and the projection in front of it
-// 10.4 -> 7.6 (2.4 MB of int8 results in place of 9.4 MB); the layer 57.6 -> 49.0, at 4 x 336 85 -> 61.
+// What is left is the vector work of the softmax, fourteen instructions per score, and at encoder sizes the
+// launch and the trips to memory.  us, one after the other in a graph, this kernel / the f32 one: 12 heads of
+// 8 x 128 tokens 4.8 / 9.7, 4 x 336 11.0 / 31.8, 8 x 384 15.4 / 49.0; the projection in front of it 7.6 / 10.4 at
+// 8 x 128 (2.4 MB of int8 results in place of 9.4 MB of f32).
 template <bool QUANT>
 __global__ void __launch_bounds__(256, 2)
 attention_i8_kernel(const int8_t* __restrict__ qkv, const float* __restrict__ qkv_scale, int S, uint32_t all_heads,
@@ -258,11 +270,8 @@ attention_i8_kernel(const int8_t* __restrict__ qkv, const float* __restrict__ qk
     for (int t = 0; t < 4; ++t) {                            // channel 4 vc + t of four keys
       uint32_t w[2];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        // 0x6400 | (code ^ 0x80) is the half 1024 + 128 + code
-        w[i] = __builtin_amdgcn_perm(vreg[2 * i + 1], vreg[2 * i], 0x0c000c00u + ((4u + t) << 16) + t) ^ 0x64806480u;
-        w[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, w[i]) - (h2){(_Float16)1152.f, (_Float16)1152.f});
-      }
+      for (int i = 0; i < 2; ++i)
+        w[i] = upper_halves((float)(int8_t)(vreg[2 * i] >> (8 * t)), (float)(int8_t)(vreg[2 * i + 1] >> (8 * t)));
       *reinterpret_cast<uint2*>(vdst + stage * kStage + 16 * t * kValPitch) = make_uint2(w[0], w[1]);
     }
   };
@@ -311,7 +320,7 @@ attention_i8_kernel(const int8_t* __restrict__ qkv, const float* __restrict__ qk
     for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
       for (int v = 0; v < 4; ++v)
-        p[kt][v] = __builtin_amdgcn_exp2f((float)(a[kt][v] - top) * f) * 16384.0f;
+        p[kt][v] = __builtin_amdgcn_exp2f((float)(a[kt][v] - top) * f) * 0x1p64f;
     if (ragged) {
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt)
@@ -327,25 +336,23 @@ attention_i8_kernel(const int8_t* __restrict__ qkv, const float* __restrict__ qk
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       if (key0 + 32 * j >= S) continue;                      // (uniform: keys past the sequence)
-      h8 hi, lo;
+      v4i part[3];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float x = p[2 * j + (e >> 1)][2 * (e & 1)], y = p[2 * j + (e >> 1)][2 * (e & 1) + 1];
-        const h2 top2 = __builtin_convertvector((f2){x, y}, h2);
-        f2 rest;                               // what a half leaves over, exact
-        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(rest.x) : "v"(top2), "v"(x));
-        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(rest.y) : "v"(top2), "v"(y));
-        const h2 low2 = __builtin_convertvector(rest, h2);
-        hi[2 * e] = top2[0];
-        hi[2 * e + 1] = top2[1];
-        lo[2 * e] = low2[0];
-        lo[2 * e + 1] = low2[1];
+        float x = p[2 * j + (e >> 1)][2 * (e & 1)], y = p[2 * j + (e >> 1)][2 * (e & 1) + 1];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          part[c][e] = (int)upper_halves(x, y);
+          x -= upper_half(x);                  // (exact)
+          y -= upper_half(y);
+        }
       }
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        const h8 vv = *reinterpret_cast<const h8*>(vp + 16 * t * kValPitch + 64 * j);
-        o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv, hi, o[t], 0, 0, 0);
-        o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv, lo, o[t], 0, 0, 0);
+        const b8 vv = *reinterpret_cast<const b8*>(vp + 16 * t * kValPitch + 64 * j);
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+          o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, __builtin_bit_cast(b8, part[c]), o[t], 0, 0, 0);
       }
     }
     if (key0 + kBlock < S) {
@@ -358,13 +365,13 @@ attention_i8_kernel(const int8_t* __restrict__ qkv, const float* __restrict__ qk
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
   if (q0 + r >= S) return;
-  const float inv = 1.0f / l;
+  const float inv = s / (l * 0x1p-64f);
   // channel 16 g + 4 v + t is element v of tile t
   v4f y[4];
 #pragma unroll
   for (int v = 0; v < 4; ++v)
 #pragma unroll
-    for (int t = 0; t < 4; ++t) y[v][t] = o[t][v] * inv * s;
+    for (int t = 0; t < 4; ++t) y[v][t] = (o[t][v] * 0x1p-64f) * inv;
   store_context<QUANT>(y, ((int64_t)b * S + q0 + r) * heads * kHead + h * kHead + 16 * g, out, out_q, q_scale);
 }
 

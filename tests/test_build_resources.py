@@ -14,7 +14,7 @@ OBJ = os.path.join(ROOT, "bladedisc_amd", "build")
 # mangled-name fragments of the kernels in question
 NO_SPILL = ("qconv_stream_kernel", "qgemm_persist_kernel", "qgemm_skinny_",
             "quantize", "dequantize", "fake_quant", "sweep_any", "rows_any", "lastaxis_any", "flat_any", "lut_u8",
-            "minmax", "wo_", "attention_f32_kernel", "layernorm_f32_kernel")
+            "minmax", "wo_", "attention_f32_kernel", "attention_i8_kernel", "layernorm_f32_kernel", "qgemm_wave_kernel")
 # the 256 x 256 tile on four waves keeps 256 accumulators per lane and spills part of their
 # indexing; it is a cross-check variant that the library never picks by itself
 ALLOWED = ("qgemm_pipe_kernelILi256ELi256ELi2ELi2E", "qgemm_mfma_kernelILi256ELi256E")

@@ -2465,6 +2465,25 @@ def test_attention_of_an_int8_projection(K, b, s, heads, step):
     assert (K.attention(codes.cuda(), heads, None, 0.0) == 0).all()
 
 
+@pytest.mark.parametrize("gap", [5, 17, 31, 60, 100, 120])
+def test_attention_keeps_small_probabilities_of_an_int8_projection(K, gap):
+    """One key takes all the weight and has values of zero; what the others, 2^-gap of it each, add up to, against
+    f64.  Bound, relative: the scale's square, its factor and their product with the difference of scores are 3.5
+    roundings of an exponent of -gap, 3.5 * ln 2 * gap; the exponential, the sums of 80 positive products and of
+    80 probabilities, the division and the last product on top."""
+    keys = 80
+    g = torch.Generator().manual_seed(gap)
+    q = torch.full((1, keys, 64), 100, dtype=torch.int8)
+    k = torch.randint(-1, 2, (1, keys, 64), generator=g, dtype=torch.int8)
+    v = torch.randint(1, 128, (1, keys, 64), generator=g, dtype=torch.int8)
+    k[0, 0], v[0, 0] = 100, 0
+    scale = torch.tensor([(gap * 8 * np.log(2) / 640000) ** 0.5], dtype=torch.float32)
+    qd, kd, vd = (t.double() * scale.double() for t in (q, k, v))
+    want = torch.softmax(qd @ kd.transpose(1, 2) / 8.0, -1) @ vd
+    got = K.attention(torch.cat([q, k, v], -1).cuda(), 1, qkv_scale=scale.cuda()).cpu().double()
+    assert ((got - want) / want).abs().max().item() <= (2.5 * gap + 170) * 2.0 ** -24
+
+
 def test_attention_takes_an_int8_projection_with_its_scale_only(K):
     codes = torch.zeros((1, 2, 192), dtype=torch.int8, device="cuda")
     for args in ((codes, 1), (codes, 1, None, torch.ones(2, device="cuda")), (codes, 1, None, torch.ones(1)),
