@@ -67,6 +67,7 @@ _PROTOS = {
                                              C.POINTER(_I32)]),
     "dq8_mfma_probe": (_INT, [_VP] * 7),
     "dq8_observe_folds_range": (_INT, [_I64] * 3),
+    "dq8_qgemm_rows_kernel": (C.c_char_p, [_I64] * 5 + [_INT] * 4 + [C.POINTER(_INT)]),
     "dq8_weight_only_plan": (None, [_I64, _I64, _I64, _INT, _INT, C.POINTER(_INT)]),
     "dq8_lut8": (_INT, [_VP, _VP, _I64, _VP, _VP]),
     "dq8_weight_only_qgemm_workspace_bytes": (C.c_size_t, [_I64, _I64, _INT]),
@@ -111,7 +112,8 @@ class PostOps(C.Structure):
 
 
 _HOOKS = ("dq8_qgemm_variant", "dq8_qgemm_num_variants", "dq8_qgemm_variant_name",
-          "dq8_qconv2d_variant", "dq8_mfma_probe", "dq8_observe_folds_range", "dq8_weight_only_plan")
+          "dq8_qconv2d_variant", "dq8_mfma_probe", "dq8_observe_folds_range", "dq8_weight_only_plan",
+          "dq8_qgemm_rows_kernel")
 
 
 def _bind(L, skip=()):

@@ -603,6 +603,38 @@ int pick_any(int64_t M, int64_t N, int64_t K, bool pipe, int out_bytes, bool wav
   return pick_variant(M, N, K, pipe, out_bytes, wave);
 }
 
+// What takes operand rows off 16 bytes as they are (k-contiguous, p.K and pitches as the caller's): tiles on
+// rows of whole words (words_variant's), the small-M kernel, the 64 x 64 tiles through registers, or nothing --
+// they are copied to aligned rows first, where there is scratch for that.
+enum RowsForm { kRowsCopied, kRowsWords, kRowsSmallM, kRowsRegisters };
+struct RowsPlan { RowsForm form; int variant; };
+RowsPlan plan_rows(const MainParams& p, int out_bytes) {
+  const int64_t M = p.M, N = p.N, Kp = (p.K + 15) / 16 * 16;
+  const bool words = aligned(p.A, 4) && aligned(p.W, 4) && p.lda % 4 == 0 && p.ldw % 4 == 0;
+  const int any = pick_any(M, N, Kp, ragged_ok(p), out_bytes, false);
+  // (rows on four bytes: the tiles chosen as for aligned rows, operands straight into LDS -- 5525 x 336, 1292 of k
+  // 22.3 -> 11.8 us and 835 x 3488 x 696 14.4 -> 9.0, copied first before; 489 x 416 x 1220 8.1 -> 5.2 and 777 x 1501 x
+  // 1000 with a zero point 9.6 -> 8.2, through registers before; 150 drawn products 1.10 times the speed)
+  if (words_ok(256, 256, p) && p.zw == 0) {
+    int v = pick_any(M, N, Kp, true, out_bytes);
+    // The small-M kernel estimated as fast as the round of tiles on waves of their own, outside the limits that
+    // it has by itself (its loads of such rows are served in pieces): those tiles, where there is a k tile for a
+    // wave.  150 such products of 33 to 320 rows, 68 to 7000 of k, against 64 x 64 tiles through registers:
+    // geometric mean 0.75 of the time, 0.71 from 192 of k on, none slower by more than 2 %; below 128 of k 1.0 to
+    // 1.1.  (f32 results of 283 x 618 x 2628 9.1 -> 6.1 us, int8 ones of 130 x 1306 x 1416 8.0 -> 4.8.)  On the small-M
+    // kernel 0.87 from 192 of k on, 48 of the 150 slower than before.
+    if (v == kSkinnyVariant && any != kSkinnyVariant && p.K >= 128) v = pick_wave(M, N, Kp, false, out_bytes);
+    const int vw = v < 0 ? -1 : words_variant(v);
+    if (vw >= 0) return {kRowsWords, vw};
+  }
+  if (any == kSkinnyVariant) return {kRowsSmallM, any};
+  // (rows at odd bytes: each load is served in pieces, about 0.25 us per k tile -- 777 x 1504, 1000
+  // of k at odd bytes 11.5, copied first 12; 1000 x 768 with 3073 of k 13.8, copied 12.7; rows on four
+  // bytes, K not a multiple of it: any depth)
+  if (ragged_has_variant(any) && ragged_ok(p) && p.zw == 0 && (words || p.K <= 2048)) return {kRowsRegisters, any};
+  return {kRowsCopied, -1};
+}
+
 // Whether a 3x3 stride-1 convolution goes to the kernel that keeps the input patch in LDS
 // (and with which tile), or to the implicit GEMM.  Measured on ResNet / VGG shaped layers
 // with batch 1 .. 128: with at most 64 input and output channels the implicit GEMM is bound
@@ -864,21 +896,13 @@ int qgemm_impl(int variant, const int8_t* A, int64_t lda, const int8_t* W, int64
     p.zx = zx;
     p.zw = zw;
     p.kzz = (int)((uint32_t)K * (uint32_t)zx * (uint32_t)zw);
-    // (rows on four bytes: the tiles chosen as for aligned rows, operands straight into LDS -- 5525 x 336, 1292 of k
-    // 22.3 -> 11.8 us and 835 x 3488 x 696 14.4 -> 9.0, copied first before; 489 x 416 x 1220 8.1 -> 5.2 and 777 x 1501 x
-    // 1000 with a zero point 9.6 -> 8.2, through registers before; 150 drawn products 1.10 times the speed)
-    if (words_ok(256, 256, p) && zw == 0) {
-      const int vw = words_variant(pick_any(M, N, Kp, true, es));
-      if (vw >= 0) return launch_words_epi(vw, p, epilogue, st);
+    const RowsPlan plan = plan_rows(p, es);
+    switch (plan.form) {
+      case kRowsWords: return launch_words_epi(plan.variant, p, epilogue, st);
+      case kRowsSmallM: return launch_epi<false>(plan.variant, p, epilogue, st);
+      case kRowsRegisters: return launch_zp_ragged_epi(plan.variant, p, epilogue, st);
+      case kRowsCopied: break;
     }
-    const int v = pick_any(M, N, Kp, ragged_ok(p), es, false);
-    if (v == kSkinnyVariant) return launch_epi<false>(v, p, epilogue, st);
-    // (rows at odd bytes: each load is served in pieces, about 0.25 us per k tile -- 777 x 1504, 1000
-    // of k at odd bytes 11.5, copied first 12; 1000 x 768 with 3073 of k 13.8, copied 12.7; rows on four
-    // bytes, K not a multiple of it: any depth)
-    const bool words = aligned(A, 4) && aligned(W, 4) && lda % 4 == 0 && ldw % 4 == 0;
-    if (ragged_has_variant(v) && ragged_ok(p) && zw == 0 && (words || K <= 2048))
-      return launch_zp_ragged_epi(v, p, epilogue, st);
   }
   const bool repack_a = K > 0 && (tp_a || K % 16 != 0);
   const bool repack_w = K > 0 && (!tp_b || K % 16 != 0);
@@ -1704,6 +1728,22 @@ extern "C" int dq8_qconv2d(const int8_t* in, const int64_t in_sizes[4], const in
 }
 
 #ifdef DQ8_TEST_HOOKS
+extern "C" const char* dq8_qgemm_rows_kernel(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int a_at,
+                                             int w_at, int zw, int out_bytes, int* form) {
+  MainParams p = {};
+  p.A = reinterpret_cast<const int8_t*>((uintptr_t)(256 + a_at));
+  p.W = reinterpret_cast<const int8_t*>((uintptr_t)(256 + w_at));
+  p.lda = lda;
+  p.ldw = ldw;
+  p.M = (int)M;
+  p.N = (int)N;
+  p.K = (int)K;
+  p.zw = zw;
+  const RowsPlan plan = plan_rows(p, out_bytes);
+  *form = plan.form;
+  return plan.variant < 0 ? "" : kVariants[plan.variant].name;
+}
+
 extern "C" int dq8_observe_folds_range(int64_t outer, int64_t channels, int64_t inner) {
   return observe_folds_range(outer, channels, inner);
 }

@@ -61,6 +61,13 @@ int dq8_observe_folds_range(int64_t outer, int64_t channels, int64_t inner);
  * 16-byte aligned multiples of 16 bytes. */
 void dq8_weight_only_plan(int64_t M, int64_t N, int64_t K, int x_dtype, int ragged, int plan[4]);
 
+/* What dq8_qgemm runs for A [M, K] and W [N, K], k-contiguous rows that are not all 16-byte aligned multiples
+ * of 16 bytes, K at least 64: the kernel's name, and form[0] = 1 tiles on rows of whole words, 2 the small-M
+ * kernel, 3 the 64 x 64 tiles through registers, 0 (name "") a copy to aligned rows first.  a_at, w_at: the
+ * operands' addresses modulo 16; zw: the weights' zero point; out_bytes: of a result element, 1 or 4. */
+const char* dq8_qgemm_rows_kernel(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int a_at,
+                                  int w_at, int zw, int out_bytes, int* form);
+
 #ifdef __cplusplus
 }
 #endif

@@ -104,3 +104,40 @@ def test_few_tiles_run_on_waves_of_their_own(m, n, k, out, kernel):
     """The smallest tile of which a launch has one per compute unit: 343 x 512 x 4608 took 11.9 us on 64 x 64
     tiles, 7.1 on these; one more than that and a compute unit does two."""
     assert _lib.hooks().dq8_qgemm_kernel_name(m, n, k, out).decode() == kernel
+
+
+WORDS, SMALL_M, REGISTERS, COPIED = 1, 2, 3, 0
+
+
+def rows_kernel(m, n, k, lda=0, ldw=0, a_at=0, w_at=0, zw=0, out_bytes=1):
+    form = C.c_int()
+    name = _lib.hooks().dq8_qgemm_rows_kernel(m, n, k, lda or k, ldw or k, a_at, w_at, zw, out_bytes, C.byref(form))
+    return form.value, name.decode()
+
+
+@pytest.mark.parametrize("m,n,k,form,kernel", [
+    # tiles on waves of their own estimated at or below the small-M kernel, in the forms next to them too
+    (400, 256, 500, WORDS, "wave_32x32_w8"), (335, 1152, 324, WORDS, "wave_32x64_w4"), (1023, 897, 4108, WORDS, "wave_64x64_w4"),
+    (1300, 1024, 2500, WORDS, "pipe_64x64x128"), (320, 513, 8204, WORDS, "pipe_64x64x128_k2"),
+    (4097, 1281, 264, WORDS, "pipe_128x128x128_w8"), (4090, 3500, 396, WORDS, "pipe_256x256x128_w8"),
+    # the small-M kernel estimated below them: within the limits it has by itself, else those tiles from 128 of k on
+    (256, 64, 2000, SMALL_M, "skinny_16"), (16, 768, 500, SMALL_M, "skinny_16"), (257, 64, 2000, WORDS, "wave_32x32_w8"),
+    (283, 618, 2628, WORDS, "wave_32x32_w8"), (130, 1306, 1416, WORDS, "wave_32x32_w8"), (320, 64, 500, WORDS, "wave_32x32_w8"),
+    (32, 8640, 2052, WORDS, "wave_32x64_w4"), (320, 64, 132, WORDS, "wave_32x32_w8"), (320, 64, 124, REGISTERS, "pipe_64x64x128"),
+    # rows at other bytes
+    (283, 618, 2029, REGISTERS, "pipe_64x64x128"), (283, 618, 2629, COPIED, ""), (4097, 1281, 265, COPIED, "")])
+def test_rows_off_16_bytes_keep_the_choice_that_was_made_for_them(m, n, k, form, kernel):
+    """Of 33 to 330 rows on four bytes an eighth had the small-M kernel chosen against the tiles and then ran on
+    neither, but on 64 x 64 tiles through registers: 297 x 530 x 4892 13.2 us in place of 7.1."""
+    assert rows_kernel(m, n, k) == (form, kernel)
+
+
+def test_rows_of_drawn_products_run_on_what_was_compared():
+    """Whole words, 128 of k and more: nothing through registers or copied first where a form for words exists."""
+    rng = random.Random(5)
+    for _ in range(2000):
+        m, n = (int(2 ** rng.uniform(1, 12)) for _ in range(2))
+        k = 4 * int(2 ** rng.uniform(5, 11))
+        assert rows_kernel(m, n, k, k + 4, k + 12, 4, 8, out_bytes=rng.choice((1, 4)))[0] in (WORDS, SMALL_M), (m, n, k)
+        assert rows_kernel(m, n, k, k + 4, k + 12, 4, 8, zw=3)[0] in (COPIED, SMALL_M)
+        assert rows_kernel(m, n, k, k + 4, k + 12, 4, 9)[0] in (COPIED, SMALL_M, REGISTERS)
