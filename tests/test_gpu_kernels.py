@@ -2783,6 +2783,24 @@ def test_fused_operators_behind_k_tiles_dealt_out_over_the_waves(K, shape, kerne
         _fused_forms_equal_the_separate_operators(K, a, w, zx, rng)
 
 
+@pytest.mark.parametrize("shape,kernel", [WAVE_TILES[i] for i in (1, 2, 3, 5, 6, 8, 9, 10)],
+                         ids=["%s-%d" % (t[1], t[0][2]) for t in (WAVE_TILES[i] for i in (1, 2, 3, 5, 6, 8, 9, 10))])
+def test_zero_point_of_the_weights_behind_k_tiles_dealt_out_over_the_waves(K, shape, kernel):
+    """The row sums of both operands, added by the owner of each fragment -- rows and channels of every fragment of
+    the tile, and those past the edges."""
+    m, n, k = shape
+    rng = np.random.default_rng(m + n + k)
+    a, w = dev(rng.integers(-128, 128, (m, k), dtype=np.int8)), dev(rng.integers(-128, 128, (n, k), dtype=np.int8))
+    sc = dict(sx=dev(np.array([0.02], np.float32)), sw=dev(rng.uniform(0.001, 0.05, n).astype(np.float32)),
+              so=dev(np.array([3.0], np.float32)), bias=dev(rng.standard_normal(n).astype(np.float32)))
+    assert K._lib.lib().dq8_qgemm_kernel_name(m, n, k, 1).decode() == kernel
+    for epi in (K.EPI_REQUANT_CPU, K.EPI_REQUANT_GPU, K.EPI_ACC_S32, K.EPI_REQUANT_CPU_DEQUANT_F32):
+        kw = {} if epi == K.EPI_ACC_S32 else sc
+        for zx, zw in ((0, 5), (-11, -7)):
+            want = K.qgemm(a, w, epi, variant=0, zx=zx, zw=zw, **kw)
+            assert torch.equal(K.qgemm(a, w, epi, zx=zx, zw=zw, **kw), want), (epi, zx, zw)
+
+
 @pytest.mark.parametrize("nb,h,w_,ci,co,kk,stride,pad,dil", [
     (1, 7, 7, 16, 32, 1, 1, 0, 1), (2, 9, 11, 48, 72, 3, 1, 1, 1), (3, 7, 7, 512, 48, 3, 1, 1, 1),
     (1, 13, 10, 80, 33, 3, 2, 1, 1), (2, 12, 9, 32, 64, 5, 1, 2, 1), (1, 15, 15, 208, 96, 3, 1, 2, 2),
@@ -2809,16 +2827,28 @@ def test_convolutions_on_k_tiles_dealt_out_over_the_waves(K, nb, h, w_, ci, co, 
             assert torch.equal(got, want), (v, epi)
 
 
-# the same for operand rows of any length and alignment; K rounded up to 16 names the tile
+WORDS, SMALL_M, REGISTERS = 1, 2, 3
+
+
+def _rows_kernel(a, w, out_bytes):
+    """(form, kernel) that dq8_qgemm plans for these operands' rows off 16 bytes."""
+    import ctypes as C
+    import bladedisc_amd._lib as _lib
+    form = C.c_int()
+    name = _lib.hooks().dq8_qgemm_rows_kernel(a.shape[0], w.shape[0], a.shape[1], a.stride(0), w.stride(0), a.data_ptr() % 16,
+                                         w.data_ptr() % 16, 0, out_bytes, C.byref(form))
+    return form.value, name.decode()
+
+
+# the same for operand rows of any length and alignment
 RAGGED_TILES = [((300, 261, 90), "pipe_64x64x128"), ((260, 130, 1001), "pipe_64x64x128"),
-                ((1100, 770, 2058), "pipe_64x64x128_k2"), ((320, 513, 8204), "pipe_64x64x128_k4"),
+                ((1100, 770, 2058), "pipe_64x64x128_k2"), ((320, 513, 8206), "pipe_64x64x128_k4"),
                 ((33, 257, 79), "skinny_16")]
 
 
 @pytest.mark.parametrize("shape,kernel", RAGGED_TILES, ids=["%s-%d" % (t[1], t[0][2]) for t in RAGGED_TILES])
 def test_fused_operators_behind_rows_of_any_length(K, shape, kernel):
     m, n, k = shape
-    assert K._lib.lib().dq8_qgemm_kernel_name(m, n, (k + 15) // 16 * 16, 1).decode() == kernel
     rng = np.random.default_rng(m + n + k)
     wide_a = dev(rng.integers(-128, 128, (m, (k + 11) // 4 * 4), dtype=np.int8))
     wide_w = dev(rng.integers(-128, 128, (n, (k + 15) // 4 * 4), dtype=np.int8))
@@ -2827,15 +2857,18 @@ def test_fused_operators_behind_rows_of_any_length(K, shape, kernel):
         ([(wide_a[:, :k].contiguous(), wide_w[:, :k].contiguous()), (wide_a[:, 3:3 + k], wide_w[:, 1:1 + k])]
          if k <= 2048 else [])
     for a, w in forms:
+        assert _rows_kernel(a, w, 1) == (SMALL_M if kernel == "skinny_16" else REGISTERS, kernel)
         for zx in (0, -11):
             _fused_forms_equal_the_separate_operators(K, a, w, zx, rng)
 
 
-# operand rows on four bytes: (m, n, k) and the tile named for k rounded up to 16
-WORD_TILES = [((400, 256, 500), "wave_32x32_w4"), ((300, 257, 1036), "wave_32x32_w8"), ((335, 1152, 324), "wave_32x64_w4"),
+# operand rows on four bytes: (m, n, k) and the tile that an int8 result gets
+WORD_TILES = [((400, 256, 500), "wave_32x32_w8"), ((300, 257, 1036), "wave_32x32_w8"), ((335, 1152, 324), "wave_32x64_w4"),
               ((1023, 897, 4108), "wave_64x64_w4"), ((777, 1501, 1000), "pipe_64x64x128"), ((640, 513, 124), "pipe_64x64x128"),
               ((513, 1023, 2052), "pipe_64x64x128_k2"), ((4097, 1281, 264), "pipe_128x128x128_w8"),
-              ((4090, 3500, 396), "pipe_256x256x128_w8"), ((1300, 1024, 2500), "wave_96x64_w4"), ((777, 1501, 1024), "pipe_64x64x128")]
+              ((4090, 3500, 396), "pipe_256x256x128_w8"), ((1300, 1024, 2500), "pipe_64x64x128"), ((777, 1501, 1024), "pipe_64x64x128"),
+              # the small-M kernel chosen and not taken
+              ((283, 618, 2628), "wave_32x32_w8"), ((130, 1306, 1416), "wave_32x32_w8"), ((32, 8640, 2052), "wave_32x64_w4")]
 
 
 @pytest.mark.parametrize("shape,kernel", WORD_TILES, ids=["%s-%d" % (t[1], t[0][2]) for t in WORD_TILES])
@@ -2843,7 +2876,6 @@ def test_qgemm_on_rows_that_begin_on_four_bytes(K, shape, kernel):
     """Rows of whole words, contiguous and out of wider rows whose other bytes are not zero: every place of the
     rows' end in a k tile's steps, a wave's half and a chunk.  Sums of whole numbers: equal bits."""
     m, n, k = shape
-    assert K._lib.lib().dq8_qgemm_kernel_name(m, n, (k + 15) // 16 * 16, 1).decode() == kernel
     rng = np.random.default_rng(m + n + k)
     wide_a = dev(rng.integers(-128, 128, (m, k + 12), dtype=np.int8))
     wide_w = dev(rng.integers(-128, 128, (n, k + 20), dtype=np.int8))
@@ -2853,12 +2885,29 @@ def test_qgemm_on_rows_that_begin_on_four_bytes(K, shape, kernel):
     for kk in last:
         for a, w in ((wide_a[:, :kk].contiguous(), wide_w[:, :kk].contiguous()),
                      (wide_a[:, 4:4 + kk], wide_w[:, 8:8 + kk])):
+            form, name = _rows_kernel(a, w, 1)       # (of what is not aligned after all another kernel runs)
+            assert form == _rows_kernel(a, w, 4)[0] == WORDS and (kk != k or name == kernel)
             for zx in (0, -11):
                 acc = K.qgemm(a, w, K.EPI_ACC_S32, variant=0, zx=zx)
                 assert torch.equal(K.qgemm(a, w, K.EPI_ACC_S32, zx=zx), acc)
                 for epi in (K.EPI_REQUANT_CPU, K.EPI_REQUANT_GPU, K.EPI_REQUANT_CPU_DEQUANT_F32):
                     want = K.qgemm(a, w, epi, variant=0, zx=zx, **sc)
                     assert torch.equal(K.qgemm(a, w, epi, zx=zx, **sc), want), (kk, zx, epi)
+
+
+@pytest.mark.parametrize("shape,kernel", [
+    ((335, 1168, 324), "wave_32x64_w4"), ((300, 261, 1036), "wave_32x32_w8"), ((1023, 897, 2316), "wave_64x64_w4"),
+    ((777, 1501, 516), "pipe_64x64x128"), ((320, 513, 8204), "pipe_64x64x128_k2"), ((4097, 1281, 268), "pipe_128x128x128_w8"),
+    ((4090, 3500, 264), "pipe_256x256x128_w8")])
+def test_fused_operators_behind_rows_of_whole_words(K, shape, kernel):
+    """Every tile that has a form for such rows."""
+    m, n, k = shape
+    rng = np.random.default_rng(m + n + k)
+    a = dev(rng.integers(-128, 128, (m, k + 12), dtype=np.int8))[:, 4:4 + k]
+    w = dev(rng.integers(-128, 128, (n, k + 20), dtype=np.int8))[:, 8:8 + k]
+    assert _rows_kernel(a, w, 1) == (WORDS, kernel)
+    for zx in (0, -11):
+        _fused_forms_equal_the_separate_operators(K, a, w, zx, rng)
 
 
 @pytest.mark.parametrize("rows,nch", [(4, 3), (5, 37), (1023, 255), (7, 256), (64, 257), (33, 511), (9, 1025),
