@@ -152,13 +152,12 @@ class QuantBertLayer:
 
     def _context(self, qkv_in, shape, out_scale=None):
         """attention() of the quantized layer on this library's kernel, from the projection's int8 input: on
-        the projection's int8 result where that has one scale."""
+        the projection's int8 result where that has one scale, else on what its dequantize makes of it."""
         b, s, c = shape
         if torch.as_tensor(self.s_out["qkv"]).numel() == 1:
             qkv = self._gemm("qkv", qkv_in)
             return K.attention(qkv.reshape(b, s, 3 * c), self.heads, out_scale, self.s_out["qkv"])
-        qkv = self.be.qlinear_dequantized(qkv_in, self.w_q["qkv"], self.bias["qkv"], self.s_in["qkv"],
-                                          self.sw["qkv"], self.s_out["qkv"])
+        _, qkv = self._gemm_dequantized("qkv", qkv_in)
         return K.attention(qkv.reshape(b, s, 3 * c), self.heads, out_scale)
 
     def _projected_attention(self, h, rec):

@@ -336,6 +336,26 @@ def test_encoder_layer_call_is_the_eight_calls(C, batch, seq, monkeypatch):
         assert y.shape == want.shape and torch.equal(y.view(torch.int32), want.view(torch.int32))
 
 
+@pytest.mark.parametrize("fused", ["", "fuse_dequant", "fuse_gelu", "fuse_epilogue"])
+def test_encoder_layer_whose_projection_has_more_than_one_output_scale(C, fused):
+    """Attention on the dequantized projection, as its dequantize is a pass of its own; the fused one refuses it."""
+    from bladedisc_amd import bert_layer as B
+    from bladedisc_amd import kernels as K
+    layer = B.QuantBertLayer(C.config5_weights(), B.RawBackend(), **({fused: True} if fused else {}))
+    h = layer.embed(C.config5_tokens(2, 5))
+    layer.calibrate(h)
+    layer.s_out["qkv"] = layer.s_out["qkv"].expand(2304).contiguous()
+    if layer.fuse_dequant:
+        for record in (None, {}):
+            with pytest.raises(RuntimeError, match="per-tensor output scale"):
+                layer.forward(h, record)
+        return
+    record = {}
+    y = layer.forward(h, record)
+    assert torch.equal(y, layer.forward(h))
+    assert torch.equal(record["out"]["x"].reshape(h.shape), K.attention(record["qkv"]["y"].reshape(2, 5, 2304), layer.heads))
+
+
 @pytest.mark.parametrize("backend", ["raw", "ral"])
 @pytest.mark.parametrize("fused", [False, True, "epilogue"])
 def test_config5_bert_layer_graph_replays_match_eager(C, fused, backend):
