@@ -463,7 +463,12 @@ int pick_k_split64(int64_t M, int64_t N, int64_t K) {
 //    777 x 1504 x 5120 18.8 -> 16.0; 4-byte results from 2560 on (1300 x 1024 x 3072 14.1 -> 13.05, x 2048 10.85 / 10.85).
 // Launches of more tiles lose (two rounds; one workgroup to a compute unit).  int8 rows off 16 bytes, whose stores
 // are dearer: from 1024 of k on, 64 x 64 from 2304, 96 x 64 from 2560 (258 x 159 x 3072 9.2 -> 4.9 small-M, 1048 x 187 x 1920
-// 9.3 -> 5.4, 1000 x 1002 x 1536 8.6 / 7.2).  8192 of k and more stay with the tiles below.
+// 9.3 -> 5.4, 1000 x 1002 x 1536 8.6 / 7.2).  The lines are drawn for operands that change from launch to launch: of
+// 2400 products that this choice moved to other tiles 39 are slower by 3 % or more, 1.17 times the speed in
+// geometric mean.  On operands still in the L2 from a launch before 200, 1.08 times: the 64 x 64 tile with a
+// barrier per k tile is 4 to 10 % faster then between 1280 and 1900 of k.  8192 of k and more are none of the
+// products that the estimates are fitted to and stay with the tiles below, which the tests of the k range split
+// over four wave groups name there; 256 x 512 x 8192 would run in 8.8 us in place of 15.2.
 int pick_wave(int64_t M, int64_t N, int64_t K, bool conv, int out_bytes) {
   const bool off16 = out_bytes == 1 && N % 16 != 0;
   if (K >= 8192 || (off16 && (conv || K < 1024))) return -1;

@@ -653,7 +653,8 @@ __device__ __forceinline__ void fused_tail16(const EpiParams& e, const uint8_t* 
 
 // Stores int8 result rows that begin at any byte: `rows` rows of W bytes, of which the first
 // N - n_first exist, from LDS to out + m * ldo + n_first, by the threads t = 0 .. nt - 1.
-// `at(row, byte)`: where a byte of a row lies in LDS, 4-byte pieces of a row being contiguous.
+// `at(row, byte)`: where a byte of a row lies in LDS; the 16 bytes from a multiple of 16 on are contiguous and
+// 16-byte aligned (they are read at once; of the chunk behind them, the first word).
 // Each row is written from its first whole 4-byte word in memory on, 16 bytes a lane, what remains as
 // words and single bytes, and up to three bytes in front.  (Byte by byte straight from the registers, 64
 // lanes on 32 rows, the stores of 777 x 1501 took as long as the rest of the kernel; a word a lane, with the

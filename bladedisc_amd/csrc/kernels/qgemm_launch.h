@@ -84,10 +84,12 @@ constexpr int kDirectConv2 = 18;   // the third direct variant (configuration 2)
 constexpr int kPipe64k4 = 19;
 constexpr int kStreamConv = 20;
 constexpr int kWave64 = 21, kWave32x64 = 22, kWave32 = 23, kWave32w4 = 24, kWave96x64 = 25;
-// largest M the heuristic hands to the small-M kernel
+// The small-M kernel's limits where there is no round of tiles on waves of their own to compare it with
+// (pick_any; with one, estimates decide up to 320 rows, 256 for int8 rows off 16 bytes): all products up to
+// this many rows but those with very wide weights,
 constexpr int64_t kSkinnyMaxM = 32;
-// Above that many rows the small-M kernel still beats the 64 x 64 tiles while its workgroups
-// (16 rows x 16 channels, each over all of k) are few: up to 256 rows and
+// and above that, against the 64 x 64 tiles, while its workgroups (16 rows x 16 channels, each over
+// all of k) are few: up to 256 rows and
 // ceil(M / 16) ceil(N / 16) ceil(K / 768) <= 1024, or 3072 from 2048 of k on, where the tiles'
 // k loop is long (us per launch, small-M kernel against tiles: M = 64, 768 -> 768: 3.2 / 4.8;
 // M = 256: 4.1 / 4.7; M = 64, 768 -> 3072: 4.1 / 4.6; M = 128: 5.1 / 4.9; M = 64, 3072 -> 768:
