@@ -217,7 +217,8 @@ __device__ __forceinline__ uint32_t upper_halves(float x, float y) {
 //    behind a key that has all the weight and is zero itself came out 1e-1 off at 2^-31 -- and is 0.3 us less
 //    at 8 x 128 tokens, 2.5 at 8 x 384.)  24 instead of 128 matrix instructions for 64 keys, of half the time
 //    each, and sums round a quarter as often: the rms error against 64 bits, over 24 scales from 0.003 to 0.3
-//    at each of 8 to 384 tokens, is 0.14 to 1.0 of the f32 kernel's on the dequantized projection, the smaller
+//    at each of 8 to 384 tokens (300 where the codes are of three or five levels and one scale's few distinct
+//    probabilities round one way), is 0.14 to 0.99 of the f32 kernel's on the dequantized projection, the smaller
 //    the wider the scores spread; of the int8 results of eight encoder layers' attention 52 in 14.4 million
 //    differ from those of 64 bits, with the f32 kernel 73.
 //  * Values are widened and transposed once, on their way into LDS: a thread takes 4 channels of 4 keys.
